@@ -227,6 +227,7 @@ struct GenL {
    // global, read with scalar loads: per xform the count of nonzero weights,
    // then (variation id, float weight bits) pairs (fl3_job_hdr::off_vl)
    const __attribute__((address_space(4))) int32_t *vlc;
+   const __attribute__((address_space(4))) uint32_t *wt;   // the walker table, likewise
    int nxf, nstd, final_index, chaos_enable, nunion, cmap_size, palette_mode, rotate, width, height;
    R b0, b1, b2, b3, rot00, rot01, rot10, rot11, rc0, rc1, ws0, wb0s0, hs1, hb1s1, final_opacity;
 };
@@ -317,6 +318,7 @@ __device__ void load_genome(const unsigned char *job, unsigned char *lds, GenL<R
    G.xf = xf; G.w = w; G.starts = st; G.uid = uid; G.dmap = dmap; G.dmapu = dmapu; G.dmapd = dmapd;
    G.vlist = vl; G.vcount = vc;
    G.vlc = (const __attribute__((address_space(4))) int32_t *)(job + h->off_vl);
+   G.wt = (const __attribute__((address_space(4))) uint32_t *)(job + h->off_wt);
 }
 
 #include "fl3_variations.inc"
@@ -336,7 +338,6 @@ __device__ __forceinline__ int select_xform(const GenL<R> &G, int row, uint32_t 
 // Variation tiers of the walker kernels.  Tier 0 holds the classic ids
 // 0-13 (linear .. julia); tier t in 1..FL3_NBLOCKS adds block t-1 of the
 // remaining ids; FL3_TIER_FULL holds all of them.
-#define FL3_CLASSIC 14
 #define FL3_BLOCK 17
 #define FL3_NBLOCKS 5
 #define FL3_TIER_FULL (FL3_NBLOCKS + 1)

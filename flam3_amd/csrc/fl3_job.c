@@ -9,6 +9,8 @@
  * in the same order as the reference's active-variation list
  * (variations.c:2043-2048, 2177-2381).
  */
+#include <float.h>
+#include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -97,6 +99,35 @@ static void pack_xform(const flam3_xform *x, fl3_xform_pack *d) {
    p[P_WAVES_DX2] = x->waves_dx2; p[P_WAVES_DY2] = x->waves_dy2;
 }
 
+/* Row of the walker table (fl3_pack.h) of xform d, whose variation list
+ * vl (count, 0, then id and weight pairs) is complete. */
+static void pack_walker_row(const fl3_xform_pack *d, const int32_t *vl, uint32_t *t) {
+   int k;
+   uint32_t mask = 0, flags = (uint32_t)d->flags;
+   float v[6 + 1 + 1], post[6], vis = (float)d->vis, preblur = (float)d->preblur;
+   for (k = 0; k < 6; k++) {
+      v[k] = (float)d->c[k];
+      post[k] = (float)d->post[k];
+   }
+   v[FL3_WT_COLOR] = (float)d->color;
+   v[FL3_WT_CSPEED] = (float)d->color_speed;
+   /* (the walkers flush subnormals: such a weight is zero to them) */
+   if (!(fabsf(preblur) < FLT_MIN)) flags |= FL3_HAS_PREBLUR;
+   for (k = 0; k < vl[0]; k++) {
+      const int id = vl[2 + 2 * k];
+      if (id >= FL3_CLASSIC) continue;
+      mask |= 1u << id;
+      t[FL3_WT_W + id] = (uint32_t)vl[3 + 2 * k];
+   }
+   memcpy(t + FL3_WT_C, v, sizeof(v));
+   memcpy(t + FL3_WT_POST, post, sizeof(post));
+   memcpy(t + FL3_WT_VIS, &vis, sizeof(vis));
+   memcpy(t + FL3_WT_PREBLUR, &preblur, sizeof(preblur));
+   t[FL3_WT_FLAGS] = flags;
+   t[FL3_WT_MASK] = mask;
+   t[FL3_WT_COUNT] = (uint32_t)vl[0];
+}
+
 static size_t align8(size_t n) { return (n + 7) & ~(size_t)7; }
 
 /* distrib: the selection table, or starts: its breakpoints
@@ -139,7 +170,7 @@ static void *pack_job(const flam3_genome *cp, const unsigned short *distrib, con
 
    off = align8(sizeof(fl3_job_hdr));
    {
-      size_t o_xf = off, o_w, o_st, o_dm, o_vl;
+      size_t o_xf = off, o_w, o_st, o_dm, o_vl, o_wt;
       off += sizeof(fl3_xform_pack) * nxf;
       o_w = off;
       off = align8(off + sizeof(double) * nxf * (nunion > 0 ? nunion : 1));
@@ -151,6 +182,8 @@ static void *pack_job(const flam3_genome *cp, const unsigned short *distrib, con
       /* (and four pairs of padding: a walker reads an xform's first four
        * pairs at once, whatever its count) */
       off = align8(off + sizeof(int32_t) * nxf * (2 + 2 * (size_t)nunion) + 8 * sizeof(int32_t));
+      o_wt = off = (off + 63) & ~(size_t)63;
+      off += sizeof(uint32_t) * FL3_WT_WORDS * (size_t)nxf;
       total = off;
       blob = (unsigned char *)calloc(1, total);
       if (!blob) { free(own); return NULL; }
@@ -160,6 +193,7 @@ static void *pack_job(const flam3_genome *cp, const unsigned short *distrib, con
       h->off_starts = (int64_t)o_st;
       h->off_dmap = (int64_t)o_dm;
       h->off_vl = (int64_t)o_vl;
+      h->off_wt = (int64_t)o_wt;
    }
    h->bytes = (int32_t)total;
    h->nxf = nxf;
@@ -215,6 +249,7 @@ static void *pack_job(const flam3_genome *cp, const unsigned short *distrib, con
          }
          vl[0] = k;
          vl[1] = 0;
+         pack_walker_row(&px[i], vl, (uint32_t *)(blob + h->off_wt) + (size_t)i * FL3_WT_WORDS);
       }
    }
 

@@ -60,6 +60,22 @@ enum fl3_param {
 #define FL3_PRE_ATAN_YX 4
 #define FL3_HAS_POST 8
 #define FL3_DRAWS_JULIA 16   /* julia (variation 13) is among the xform's nonzero float weights */
+#define FL3_HAS_PREBLUR 32   /* walker table only: a pre_blur weight that is not zero (or subnormal) as a float */
+
+/* One xform as the wavefront that applies it reads it with scalar loads
+ * (off_wt): 48 words, floats as the walkers' own conversions give them. */
+#define FL3_WT_WORDS 48
+#define FL3_WT_C 0           /* c00 c01 c10 c11 c20 c21 */
+#define FL3_WT_COLOR 6
+#define FL3_WT_CSPEED 7
+#define FL3_WT_FLAGS 8       /* fl3_xform_pack::flags, FL3_HAS_PREBLUR */
+#define FL3_WT_MASK 9        /* bit v: classic variation v (0..13) has a nonzero float weight */
+#define FL3_WT_COUNT 10      /* variations in the xform's off_vl list, the classic ones first */
+#define FL3_WT_VIS 11
+#define FL3_WT_PREBLUR 12
+#define FL3_WT_W 16          /* weights of variations 0..13 */
+#define FL3_WT_POST 32       /* as FL3_WT_C */
+#define FL3_CLASSIC 14       /* classic variation ids 0..13 (linear .. julia) */
 
 typedef struct {
    double c[6];        /* c00 c01 c10 c11 c20 c21 (x' = c00 x + c10 y + c20) */
@@ -98,6 +114,7 @@ typedef struct {
                               number of its weights that are nonzero as floats, 0,
                               then (variation id, the weight's float bits) for each,
                               in union order */
+   int64_t off_wt;         /* uint32[nxf][FL3_WT_WORDS], 64-byte aligned */
 } fl3_job_hdr;
 
 #endif

@@ -116,3 +116,31 @@ def test_frames_sharing_a_palette_equal_fl3h_render_alone(prod):
         assert got[k][1]["num_iters"] == ws["num_iters"]
         assert np.array_equal(got[k][0], want), it["seed"]
         assert np.array_equal(mixed[k if k < 3 else k + 1][0], want), it["seed"]
+
+
+@pytest.fixture
+def chunks_of(prod):
+    """Sets the samples per chunk of the binned deposit for one test."""
+    from flam3_amd import autotune
+    old = autotune._get("chunk_samples")
+    yield lambda n: autotune._set("chunk_samples", n)
+    autotune._set("chunk_samples", old)
+
+
+@pytest.mark.parametrize("nxf", [1, 3, 12])
+def test_short_renders_beside_long_ones_in_chunks(prod, chunks_of, nxf):
+    """Shared launches of several chunks: a short render's walkers are done
+    chunks before the longest one's and plot nothing more, and every walker
+    takes up its draws at the step where the chunk before ended."""
+    chunks_of(1 << 20)
+    items = []
+    for k, (size, quality) in enumerate([(64, 12), (256, 90), (65, 300), (128, 40)]):
+        it = _preview(700 + k, size=size, quality=quality)
+        rng = np.random.default_rng(720 + k)
+        it["genomes"].xforms = [G._mixed_xform(rng, G.WORKLOAD_VARS, 3, -1.2, 1.2) for _ in range(nxf)]
+        items.append(it)
+    got = prod.render_many(items)
+    for it, (img, st) in zip(items, got):
+        want, ws = _alone(prod, it)
+        assert st["badvals"] == ws["badvals"]
+        assert np.array_equal(img, want), it["seed"]
