@@ -108,6 +108,322 @@ __global__ __launch_bounds__(64) void k_iterate_points(PointsArgs a) {
    a.badvals[wid] = bad;
 }
 
+// ---- one walker per wavefront
+//
+// A few walkers (the bounding box of a genome is one) are a serial chain of
+// FP64 steps, bound by a step's latency.  k_iterate_points takes 33 us a step
+// for such a walker: ISAAC's arrays are indexed by their contents, so they
+// live in scratch memory, and the 196 KB of apply_xform with every variation
+// do not stay in the instruction cache beside it.  Here every lane of a
+// wavefront holds the same walker: the xform, the branches and ISAAC run in
+// scalar registers (its two arrays across the lanes of a register each), the
+// variations are the wavefront's own xform's only, and a genome of classic
+// variations runs code that holds no others; the sines and cosines of an
+// xform's classic variations are one evaluation (lone_classic).  The arithmetic is apply_xform's,
+// operation by operation.  20000 points of a genome of six xforms and a final
+// one: 690 -> 62 ms.
+
+// IsaacRng in a wavefront: word k of an array in lane k.
+struct WaveIsaac {
+   uint32_t rsl, mem, a, b, c, cnt;
+
+   __device__ static uint32_t word(uint32_t v, uint32_t k) {
+      return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)k);
+   }
+   // x into lane k of v
+   __device__ __forceinline__ static void put(uint32_t &v, uint32_t x, uint32_t k) {
+      v = threadIdx.x == k ? x : v;
+   }
+   __device__ void load(const uint32_t *s, unsigned lane) {
+      rsl = s[1 + (lane & 15u)];
+      mem = s[17 + (lane & 15u)];
+      cnt = (uint32_t)__builtin_amdgcn_readfirstlane((int)s[0]);
+      a = (uint32_t)__builtin_amdgcn_readfirstlane((int)s[33]);
+      b = (uint32_t)__builtin_amdgcn_readfirstlane((int)s[34]);
+      c = (uint32_t)__builtin_amdgcn_readfirstlane((int)s[35]);
+   }
+   __device__ void store(uint32_t *s, unsigned lane) const {
+      if (lane < 16) {
+         s[1 + lane] = rsl;
+         s[17 + lane] = mem;
+      }
+      if (lane == 0) {
+         s[0] = cnt;
+         s[33] = a;
+         s[34] = b;
+         s[35] = c;
+      }
+   }
+   __device__ __forceinline__ void refill() {
+      uint32_t aa = a, bb = b + (++c);
+#pragma unroll
+      for (uint32_t i = 0; i < 16; i++) {
+         const uint32_t x = word(mem, i);
+         const uint32_t mixv = (i & 3) == 0 ? aa << 13 : (i & 3) == 1 ? aa >> 6 : (i & 3) == 2 ? aa << 2 : aa >> 16;
+         aa = (aa ^ mixv) + word(mem, (i + 8) & 15);
+         const uint32_t y = word(mem, (x >> 2) & 15) + aa + bb;
+         put(mem, y, i);
+         bb = word(mem, (y >> 6) & 15) + x;
+         put(rsl, bb, i);
+      }
+      a = aa;
+      b = bb;
+   }
+   __device__ __forceinline__ uint32_t next() {
+      if (cnt-- == 0) {
+         refill();
+         cnt = 15;
+      }
+      return word(rsl, cnt);
+   }
+};
+
+__device__ __forceinline__ double uniform_f64(double v) {
+   return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                           __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+
+__device__ __forceinline__ double lane_f64(double v, int lane) {
+   return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                           __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// The classic variations of an xform (weight of variation v: w[v]).  A double
+// sine and cosine take some 200 instructions and most variations ask for
+// them, each for arguments of its own: lane v takes variation v's (lane 16 + v
+// its second), so that all of them cost one evaluation.  Returns how many
+// there are.
+__device__ __forceinline__ int lone_classic(const double *w, Pre<double> &f, WaveIsaac &rng) {
+   const unsigned lane = threadIdx.x, id = lane & 15u;
+   const bool second = lane & 16u;
+   const double wl = w[id];
+   const uint32_t mask = (uint32_t)__builtin_amdgcn_ballot_w64(wl != 0.0) & 0x3fffu;
+   const double EPS = 1e-10, PI = M_PI, a = f.atan, r = f.sq;
+   uint32_t word = 0;
+   if (mask & (1u << 13)) word = rng.next();   // julia's random bit, the classic variations' only draw
+   double s = 0.0, c = 0.0;
+   if (mask & 0x3bcau) {   // sinusoidal, swirl, handkerchief .. spiral, diamond .. julia
+      const double sum = a + r, dif = a - r;
+      double ja = 0.5 * a;
+      if (word & 1u) ja += PI;
+      double x = second ? f.ty : f.tx;                 // 1: sinusoidal
+      x = id == 3 ? f.sumsq : x;                       // swirl
+      x = id == 6 || id == 12 ? (second ? dif : sum) : x;   // handkerchief, ex
+      x = id == 7 ? r * a : x;                         // heart
+      x = id == 8 ? PI * r : x;                        // disc
+      x = id == 9 ? r + EPS : x;                       // spiral
+      x = id == 11 ? r : x;                            // diamond
+      x = id == 13 ? ja : x;                           // julia
+      m_sincos(x, &s, &c);
+   }
+#define LONE_VAR(v) if (mask & (1u << (v)))
+#define LONE_W(v) const double w = lane_f64(wl, v)
+   LONE_VAR(0) {  // linear :142
+      LONE_W(0);
+      f.p0 += w * f.tx;
+      f.p1 += w * f.ty;
+   }
+   LONE_VAR(1) {  // sinusoidal :153
+      LONE_W(1);
+      f.p0 += w * lane_f64(s, 1);
+      f.p1 += w * lane_f64(s, 17);
+   }
+   LONE_VAR(2) {  // spherical :164
+      LONE_W(2);
+      const double r2 = w / (f.sumsq + EPS);
+      f.p0 += r2 * f.tx;
+      f.p1 += r2 * f.ty;
+   }
+   LONE_VAR(3) {  // swirl :178
+      LONE_W(3);
+      const double c1 = lane_f64(s, 3), c2 = lane_f64(c, 3);
+      f.p0 += w * (c1 * f.tx - c2 * f.ty);
+      f.p1 += w * (c2 * f.tx + c1 * f.ty);
+   }
+   LONE_VAR(4) {  // horseshoe :202
+      LONE_W(4);
+      const double h = w / (r + EPS);
+      f.p0 += (f.tx - f.ty) * (f.tx + f.ty) * h;
+      f.p1 += 2.0 * f.tx * f.ty * h;
+   }
+   LONE_VAR(5) {  // polar :218
+      LONE_W(5);
+      f.p0 += w * (a * M_1_PI);
+      f.p1 += w * (r - 1.0);
+   }
+   LONE_VAR(6) {  // handkerchief :232
+      LONE_W(6);
+      f.p0 += w * r * lane_f64(s, 6);
+      f.p1 += w * r * lane_f64(c, 22);
+   }
+   LONE_VAR(7) {  // heart :246
+      LONE_W(7);
+      const double h = w * r;
+      f.p0 += h * lane_f64(s, 7);
+      f.p1 += (-h) * lane_f64(c, 7);
+   }
+   LONE_VAR(8) {  // disc :264
+      LONE_W(8);
+      const double h = a * M_1_PI;
+      f.p0 += w * lane_f64(s, 8) * h;
+      f.p1 += w * lane_f64(c, 8) * h;
+   }
+   LONE_VAR(9) {  // spiral :282
+      LONE_W(9);
+      const double r1 = w / (r + EPS);
+      f.p0 += r1 * (f.cosa + lane_f64(s, 9));
+      f.p1 += r1 * (f.sina - lane_f64(c, 9));
+   }
+   LONE_VAR(10) {  // hyperbolic :298
+      LONE_W(10);
+      const double h = r + EPS;
+      f.p0 += w * f.sina / h;
+      f.p1 += w * f.cosa * h;
+   }
+   LONE_VAR(11) {  // diamond :311
+      LONE_W(11);
+      f.p0 += w * f.sina * lane_f64(c, 11);
+      f.p1 += w * f.cosa * lane_f64(s, 11);
+   }
+   LONE_VAR(12) {  // ex :326
+      LONE_W(12);
+      const double n0 = lane_f64(s, 12), n1 = lane_f64(c, 28);
+      const double m0 = n0 * n0 * n0 * r, m1 = n1 * n1 * n1 * r;
+      f.p0 += w * (m0 + m1);
+      f.p1 += w * (m0 - m1);
+   }
+   LONE_VAR(13) {  // julia :350
+      LONE_W(13);
+      const double h = w * m_sqrt(r);
+      f.p0 += h * lane_f64(c, 13);
+      f.p1 += h * lane_f64(s, 13);
+   }
+#undef LONE_VAR
+#undef LONE_W
+   return __popc(mask);
+}
+
+// apply_xform<double> for a wavefront whose lanes all hold the same walker
+// (wd: the classic weights by xform and variation, 16 each).
+template <int TIER>
+__device__ __forceinline__ bool lone_apply(const GenL<double> &G, const double *wd, int fn, const double *p, double *q,
+                                           WaveIsaac &rng) {
+   const XfL<double> &X = G.xf[fn];
+   Pre<double> f;
+   const double s1 = X.cspeed;
+   q[2] = s1 * X.color + (1.0 - s1) * p[2];
+   q[3] = X.vis;
+   f.tx = X.c[0] * p[0] + X.c[2] * p[1] + X.c[4];
+   f.ty = X.c[1] * p[0] + X.c[3] * p[1] + X.c[5];
+   const double preblur = uniform_f64(X.preblur);
+   if (preblur != 0.0) {
+      const double g0 = u01<double>(rng), g1 = u01<double>(rng), g2 = u01<double>(rng), g3 = u01<double>(rng);
+      const double rndG = preblur * (g0 + g1 + g2 + g3 - 2.0);
+      const double rndA = u01<double>(rng) * 2.0 * M_PI;
+      double sA, cA;
+      m_sincos(rndA, &sA, &cA);
+      f.tx += rndG * cA;
+      f.ty += rndG * sA;
+   }
+   f.sumsq = f.tx * f.tx + f.ty * f.ty;
+   f.sq = m_sqrt(f.sumsq);
+   f.atan = f.sina = f.cosa = f.atanyx = 0.0;
+   const int flags = __builtin_amdgcn_readfirstlane(X.flags);
+   if (flags & FL3_PRE_ATAN_XY) f.atan = m_atan2(f.tx, f.ty);
+   if (flags & FL3_PRE_ANGLES) {
+      f.sina = m_div(f.tx, f.sq);
+      f.cosa = m_div(f.ty, f.sq);
+   }
+   if (flags & FL3_PRE_ATAN_YX) f.atanyx = m_atan2(f.ty, f.tx);
+   f.p0 = 0.0;
+   f.p1 = 0.0;
+   const int classic = lone_classic(wd + fn * 16, f, rng);
+   if constexpr (TIER != 0) {
+      // (ascending ids: the classic ones come first in the list too)
+      const int nv = __builtin_amdgcn_readfirstlane(G.vcount[fn]);
+      for (int k = classic; k < nv; k++) {
+         const int u = __builtin_amdgcn_readfirstlane((int)G.vlist[fn * G.nunion + k]);
+         const int v = __builtin_amdgcn_readfirstlane(G.uid[u]);
+         const double w = uniform_f64(G.w[fn * G.nunion + u]);
+         fl3_var<double, WaveIsaac, FL3_CLASSIC, FL3_NVAR>(v, w, X, f, rng);
+      }
+   }
+   if (flags & FL3_HAS_POST) {
+      q[0] = X.post[0] * f.p0 + X.post[2] * f.p1 + X.post[4];
+      q[1] = X.post[1] * f.p0 + X.post[3] * f.p1 + X.post[5];
+   } else {
+      q[0] = f.p0;
+      q[1] = f.p1;
+   }
+   if (__builtin_amdgcn_ballot_w64(fl3_bad(q[0]) || fl3_bad(q[1]))) {
+      q[0] = u11<double>(rng);
+      q[1] = u11<double>(rng);
+      return true;
+   }
+   return false;
+}
+
+// k_iterate_points, walker w in wavefront w.
+template <int TIER>
+__global__ __launch_bounds__(64) void k_iterate_lone(PointsArgs a) {
+   GenL<double> G;
+   load_genome<double>(a.job, fl3_lds, G, false);
+   __shared__ double wd[16 * FL3_MAX_XFORMS];
+   for (int e = threadIdx.x; e < 16 * G.nxf; e += 64) wd[e] = 0.0;
+   __syncthreads();
+   for (int e = threadIdx.x; e < G.nxf * G.nunion; e += 64) {
+      const int id = G.uid[e % G.nunion];
+      if (id < FL3_CLASSIC) wd[e / G.nunion * 16 + id] = G.w[e];
+   }
+   __syncthreads();
+   const int wid = blockIdx.x;
+   const unsigned lane = threadIdx.x;
+   WaveIsaac rng;
+   rng.load(a.isaac + 36 * wid, lane);
+   double p[4], q[4];
+   for (int k = 0; k < 4; k++) p[k] = a.start[4 * wid + k];
+   int lastxf = 0, consec = 0, bad = 0;
+   const int final_index = __builtin_amdgcn_readfirstlane(G.final_index);
+   double *out = a.out + (size_t)wid * a.n * 4;
+   int i = -a.fuse, fn = 0;
+   bool fin = false;   // the xform to apply next is the final one, to p's point
+   while (i < a.n) {
+      if (!fin) {
+         // (select_xform, a breakpoint per lane: at most 63 after the first)
+         const uint32_t slot = rng.next() & 16383u;
+         const int *st = G.starts + (G.chaos_enable ? lastxf : 0) * G.nstd;
+         fn = __popcll(__builtin_amdgcn_ballot_w64(lane >= 1 && (int)lane < G.nstd &&
+                                                   slot >= (uint32_t)st[min((int)lane, G.nstd - 1)]));
+      }
+      const bool isbad = lone_apply<TIER>(G, wd, fin ? final_index : fn, p, q, rng);
+      if (!fin) {
+         if (isbad) {
+            consec++;
+            bad++;
+            if (consec < 5) {
+               for (int k = 0; k < 4; k++) p[k] = q[k];
+               continue;
+            }
+         }
+         consec = 0;
+         lastxf = fn + 1;
+         for (int k = 0; k < 4; k++) p[k] = q[k];
+         if (final_index >= 0) {
+            fin = true;
+            if (uniform_f64(G.final_opacity) == 1.0) continue;
+            if (u01<double>(rng) < uniform_f64(G.final_opacity)) continue;
+         }
+      } else
+         q[3] = p[3];
+      fin = false;
+      if (i >= 0 && lane == 0)
+         for (int k = 0; k < 4; k++) out[4 * (size_t)i + k] = q[k];
+      i++;
+   }
+   rng.store(a.isaac + 36 * wid, lane);
+   if (lane == 0) a.badvals[wid] = bad;
+}
+
 // Apply xform xi `depth` times to each point of a grid (flam3.c:301-349).
 __global__ __launch_bounds__(64) void k_xform_preview(const unsigned char *job, int xi, double range,
                                                       int numvals, int depth, double *result,
@@ -624,8 +940,20 @@ extern "C" int fl3k_launch_replay(const IterArgs *a, unsigned grid, size_t lds, 
    return hipGetLastError() != hipSuccess;
 }
 
-extern "C" int fl3k_launch_points(const PointsArgs *a, unsigned grid, size_t lds, hipStream_t s) {
-   hipLaunchKernelGGL(k_iterate_points, dim3(grid), dim3(64), lds, s, *a);
+// Up to this many walkers one per wavefront (k_iterate_lone), more of them one
+// per lane (k_iterate_points).  220 steps of 1 / 1024 / 4096 / 16384 walkers of
+// a genome of six xforms and a final one: 0.74 / 1.6 / 5.3 / 19 ms per
+// wavefront, 9.1 / 9.8 / 10.7 / 15.8 ms per lane.
+#define FL3_LONE_WALKERS 4096
+
+// lds, lds_lone: the genome's LDS image with and without the palette
+extern "C" int fl3k_launch_points(const PointsArgs *a, size_t lds, size_t lds_lone, hipStream_t s, int tier) {
+   if (a->nwalkers > FL3_LONE_WALKERS)
+      hipLaunchKernelGGL(k_iterate_points, dim3((a->nwalkers + 63) / 64), dim3(64), lds, s, *a);
+   else if (tier == 0)
+      hipLaunchKernelGGL(k_iterate_lone<0>, dim3(a->nwalkers), dim3(64), lds_lone, s, *a);
+   else
+      hipLaunchKernelGGL(k_iterate_lone<FL3_TIER_FULL>, dim3(a->nwalkers), dim3(64), lds_lone, s, *a);
    return hipGetLastError() != hipSuccess;
 }
 
