@@ -106,6 +106,9 @@ struct Ctx {
    void *de_up_p = nullptr;
    size_t de_up_cap = 0;
    int de_up_nf = 0, de_up_ks = 0;   // its row count in use (max_filter_index + 1) and row length
+   int de_up_kind = 0;               // 1 the exact gather's coefficients, 2 / 3 double / float tables
+   size_t de_up_tab = 0;             // the tables' bytes, and how many of them LDS takes
+   int de_up_lds = 0;
    DevBuf crec[FL3_CHUNK_BUFS], cblk[FL3_CHUNK_BUFS], ctot[FL3_CHUNK_BUFS];   // tile-binned deposit
    DevBuf sorted, wstate, bins, jobtab, soff;
    DevBuf srcv, srcl;                  // density estimation per-source values
@@ -1381,96 +1384,114 @@ static int iterate_replay(const void *job, size_t job_bytes, uint32_t *isaac_hos
    return read_counters(badvals, nullptr);
 }
 
-// The rows of a filter bank cut to the coefficients a tap can reach (row i,
-// radius r = ceil(width) - 1 as the gather computes it: its first
-// (r + 1)(r + 2) / 2 entries), back to back as floats (rounded to nearest,
-// as the device's conversion) into cf, each row's start into off (both
-// skipped if cf is null: the count alone).  Returns the float count, or 0
-// (the gather then reads the full table) if a row would need more entries
-// than the table's rows hold or the cut bank exceeds FL3_DE_LDS_COEFS floats.
-static int de_cut_bank(const fl3_de_filters *de, int *off, float *cf) {
-   const int nf = de->max_filter_index + 1;
-   long n = 0;
-   for (int i = 0; i < nf; i++) {
-      const long r = (long)ceil(de->filter_widths[i]) - 1;
-      const long len = (r + 1) * (r + 2) / 2;
-      if (r < 0 || len > de->kernel_size || n + len > FL3_DE_LDS_COEFS) return 0;
-      if (cf) {
-         off[i] = (int)n;
-         for (long t = 0; t < len; t++) cf[n + t] = (float)de->filter_coefs[(size_t)i * de->kernel_size + (size_t)t];
+static size_t align16(size_t n) { return (n + 15) & ~(size_t)15; }
+
+// Entries of a bank's tables (DeTables), and whether the production gather's
+// 32-bit byte offsets reach them all; a larger bank takes the exact gather.
+static double de_table_entries(const fl3_de_filters *de) {
+   double n = 0;
+   for (int i = 0; i <= de->max_filter_index; i++) {
+      const double side = ceil(de->filter_widths[i]) + 1;
+      if (side > 0) n += side * side;
+   }
+   return n;
+}
+static bool de_tables_ok(const fl3_de_filters *de, size_t entry) {
+   return de_table_entries(de) * (double)entry < 0x7fff0000;
+}
+
+// A filter bank as the production gather reads it (DEArgs::tab, info): of
+// kernel i, radius r = ceil(width) - 1, a square of the coefficients by |dy|,
+// |dx| with a row and a column of zeros beyond the radius.  (A bank whose rows
+// are shorter than their radius asks for goes on in the next row, as the
+// reference's index does; past its end there are zeros.)
+template <typename T>
+struct DeTables {
+   std::vector<T> tab;
+   std::vector<int> info;
+   int lds_bytes = 0;   // what a gather workgroup copies: all of tab, or nothing if it doesn't fit
+   void make(const fl3_de_filters *de) {
+      const int nf = de->max_filter_index + 1;
+      const size_t nc = (size_t)de->nfilters * de->kernel_size;
+      size_t n = 0;
+      info.resize(2 * (size_t)nf);
+      for (int i = 0; i < nf; i++) {
+         int r = (int)ceil(de->filter_widths[i]) - 1;
+         if (r < -1) r = -1;   // (reaches nothing, whatever its width below zero)
+         info[2 * i] = (int)n;
+         info[2 * i + 1] = r;
+         n += (size_t)(r + 2) * (r + 2);
       }
-      n += len;
+      if (n * sizeof(T) + 8 * (size_t)(nf + 1) <= FL3_DE_LDS_BYTES) lds_bytes = (int)align16(n * sizeof(T));
+      tab.assign(n, (T)0);
+      for (int i = 0; i < nf; i++) {
+         const int r = info[2 * i + 1], side = r + 2;
+         T *t = tab.data() + info[2 * i];
+         for (int y = 0; y <= r; y++)
+            for (int x = 0; x <= r; x++) {
+               const int hi = x > y ? x : y, lo = x > y ? y : x;
+               const size_t e = (size_t)i * de->kernel_size + (size_t)hi * (hi + 1) / 2 + lo;
+               if (e < nc) t[y * side + x] = (T)de->filter_coefs[e];
+            }
+      }
    }
-   return (int)n;
-}
+};
 
-// A cut bank as the batched tables hold it: row starts, then the floats,
-// each part padded to 16 bytes.  Bytes of the row starts, and of the whole
-// (0 without a cut bank).
-static size_t de_cut_rows_bytes(const fl3_de_filters *de) {
-   return (sizeof(int) * (size_t)(de->max_filter_index + 1) + 15) & ~(size_t)15;
-}
-static size_t de_cut_bytes(const fl3_de_filters *de, int ncut) {
-   if (ncut <= 0) return 0;
-   return de_cut_rows_bytes(de) + ((sizeof(float) * (size_t)ncut + 15) & ~(size_t)15);
-}
-
-// DE tables on the device: coefficients (double), widths (double) and, for
-// the float accumulator, a float copy of the coefficients and the cut bank
-// (de_cut_bank; *ncoef 0 if there is none).
-static int upload_de(const fl3_de_filters *de, double **coefs, double **widths, float **coefs_f,
-                     const int **coff = nullptr, const float **ccoef = nullptr, int *ncoef = nullptr) {
-   size_t nc = (size_t)de->nfilters * de->kernel_size, nw = de->nfilters;
-   const int ncut = de_cut_bank(de, nullptr, nullptr);
-   std::vector<int> off(ncut ? (size_t)de->max_filter_index + 1 : 0);
-   std::vector<float> cf((size_t)ncut);
-   if (ncut) de_cut_bank(de, off.data(), cf.data());
-   const size_t cut0 = (sizeof(double) * (nc + nw) + sizeof(float) * nc + 15) & ~(size_t)15;
-   const size_t cut1 = cut0 + sizeof(int) * off.size();
-   const void *p0 = g_ctx.table.p;
-   const size_t cap0 = g_ctx.table.cap;
-   if (g_ctx.table.ensure(cut1 + sizeof(float) * (size_t)ncut)) {
-      g_ctx.de_up_p = nullptr;
-      return 1;
-   }
-   if (g_ctx.table.p != p0 || g_ctx.table.cap != cap0) g_ctx.de_up_p = nullptr;   // (a new allocation)
-   *coefs = (double *)g_ctx.table.p;
-   *widths = *coefs + nc;
-   *coefs_f = (float *)(*widths + nw);
-   if (ncoef) {
-      *coff = (const int *)((unsigned char *)g_ctx.table.p + cut0);
-      *ccoef = (const float *)((unsigned char *)g_ctx.table.p + cut1);
-      *ncoef = ncut;
-   }
+// DE tables on the device, into a: the widths, the coefficients (exact
+// gather; also, with the double accumulator, for the one that stands by) and
+// the production gather's tables and info.
+static int upload_de(const fl3_de_filters *de, int exact, DEArgs &a) {
+   const size_t nc = (size_t)de->nfilters * de->kernel_size, nw = de->nfilters;
+   const int nf = de->max_filter_index + 1, kind = exact ? 1 : g_ctx.bits == 64 ? 2 : 3;
+   const size_t o_coefs = align16(sizeof(double) * nw);
+   const size_t o_tab = o_coefs + (kind == 3 ? 0 : align16(sizeof(double) * nc));
    // the same tables as the last upload (equal estimator parameters, as in
    // every frame of a still or an animation): they are on the device
    // already, so no copies, conversion or wait
-   if (g_ctx.de_up_p == g_ctx.table.p && g_ctx.de_up_cap == g_ctx.table.cap && g_ctx.de_up.size() == nc + nw &&
-       g_ctx.de_up_nf == de->max_filter_index + 1 && g_ctx.de_up_ks == de->kernel_size &&
-       memcmp(g_ctx.de_up.data(), de->filter_coefs, sizeof(double) * nc) == 0 &&
-       memcmp(g_ctx.de_up.data() + nc, de->filter_widths, sizeof(double) * nw) == 0)
-      return 0;
-   g_ctx.de_up_p = nullptr;
-   HIPCHK(hipMemcpyAsync(*coefs, de->filter_coefs, sizeof(double) * nc, hipMemcpyHostToDevice, g_ctx.stream));
-   HIPCHK(hipMemcpyAsync(*widths, de->filter_widths, sizeof(double) * nw, hipMemcpyHostToDevice, g_ctx.stream));
-   if (ncut) {
-      HIPCHK(hipMemcpyAsync((unsigned char *)g_ctx.table.p + cut0, off.data(), sizeof(int) * off.size(),
-                            hipMemcpyHostToDevice, g_ctx.stream));
-      HIPCHK(hipMemcpyAsync((unsigned char *)g_ctx.table.p + cut1, cf.data(), sizeof(float) * (size_t)ncut,
-                            hipMemcpyHostToDevice, g_ctx.stream));
+   const bool same = g_ctx.de_up_p && g_ctx.de_up_p == g_ctx.table.p && g_ctx.de_up_cap == g_ctx.table.cap &&
+                     g_ctx.de_up_kind == kind && g_ctx.de_up.size() == nc + nw && g_ctx.de_up_nf == nf &&
+                     g_ctx.de_up_ks == de->kernel_size &&
+                     memcmp(g_ctx.de_up.data(), de->filter_coefs, sizeof(double) * nc) == 0 &&
+                     memcmp(g_ctx.de_up.data() + nc, de->filter_widths, sizeof(double) * nw) == 0;
+   if (!same) {
+      DeTables<double> td;
+      DeTables<float> tf;
+      g_ctx.de_up_p = nullptr;
+      if (kind == 2) td.make(de);
+      if (kind == 3) tf.make(de);
+      const size_t tb = sizeof(double) * td.tab.size() + sizeof(float) * tf.tab.size();
+      const std::vector<int> &info = kind == 2 ? td.info : tf.info;
+      const size_t ib = sizeof(int) * info.size();
+      if (g_ctx.table.ensure(o_tab + align16(tb) + ib + 16)) return 1;
+      unsigned char *t = (unsigned char *)g_ctx.table.p;
+      HIPCHK(hipMemcpyAsync(t, de->filter_widths, sizeof(double) * nw, hipMemcpyHostToDevice, g_ctx.stream));
+      if (kind != 3)
+         HIPCHK(hipMemcpyAsync(t + o_coefs, de->filter_coefs, sizeof(double) * nc, hipMemcpyHostToDevice, g_ctx.stream));
+      if (kind != 1) {
+         const void *src = kind == 2 ? (const void *)td.tab.data() : (const void *)tf.tab.data();
+         HIPCHK(hipMemcpyAsync(t + o_tab, src, tb, hipMemcpyHostToDevice, g_ctx.stream));
+         HIPCHK(hipMemcpyAsync(t + o_tab + align16(tb), info.data(), ib, hipMemcpyHostToDevice, g_ctx.stream));
+      }
+      // the caller may free its host tables once this returns
+      HIPCHK(hipStreamSynchronize(g_ctx.stream));
+      g_ctx.de_up.assign(de->filter_coefs, de->filter_coefs + nc);
+      g_ctx.de_up.insert(g_ctx.de_up.end(), de->filter_widths, de->filter_widths + nw);
+      g_ctx.de_up_p = g_ctx.table.p;
+      g_ctx.de_up_cap = g_ctx.table.cap;
+      g_ctx.de_up_nf = nf;
+      g_ctx.de_up_ks = de->kernel_size;
+      g_ctx.de_up_kind = kind;
+      g_ctx.de_up_tab = tb;
+      g_ctx.de_up_lds = kind == 2 ? td.lds_bytes : tf.lds_bytes;
    }
-   if (fl3k_launch_f64_to_f32(*coefs, *coefs_f, (long)nc, g_ctx.stream)) {
-      set_err("k_f64_to_f32 launch failed");
-      return 1;
+   const unsigned char *t = (const unsigned char *)g_ctx.table.p;
+   a.widths = (const double *)t;
+   if (kind != 3) a.coefs = (const double *)(t + o_coefs);
+   if (kind != 1) {
+      a.tab = t + o_tab;
+      a.info = (const int *)(t + o_tab + align16(g_ctx.de_up_tab));
+      a.tab_bytes = g_ctx.de_up_lds;
    }
-   // the caller may free its host tables once this returns
-   HIPCHK(hipStreamSynchronize(g_ctx.stream));
-   g_ctx.de_up.assign(de->filter_coefs, de->filter_coefs + nc);
-   g_ctx.de_up.insert(g_ctx.de_up.end(), de->filter_widths, de->filter_widths + nw);
-   g_ctx.de_up_p = g_ctx.table.p;
-   g_ctx.de_up_cap = g_ctx.table.cap;
-   g_ctx.de_up_nf = de->max_filter_index + 1;
-   g_ctx.de_up_ks = de->kernel_size;
    return 0;
 }
 
@@ -1478,22 +1499,14 @@ extern "C" int fl3d_density(const fl3d_de_params *p, const fl3_de_filters *de) {
    std::lock_guard<std::recursive_mutex> lk(g_mu);
    DEArgs a;
    memset(&a, 0, sizeof(a));
-   double *coefs, *widths;
-   float *coefs_f;
-   const int *coff;
-   const float *ccoef;
-   int ncoef;
-   if (upload_de(de, &coefs, &widths, &coefs_f, &coff, &ccoef, &ncoef)) return 1;
+   const int exact = p->exact || !de_tables_ok(de, g_ctx.bits == 64 ? 8 : 4);
+   if (de->max_filter_index >= 1024) {
+      set_err("density estimation: more than 1024 kernels");
+      return 1;
+   }
+   if (upload_de(de, exact, a)) return 1;
    a.buckets = cur_buckets();
    a.accum = cur_accum();
-   a.coefs = coefs;
-   a.widths = widths;
-   a.coefs_t = g_ctx.bits == 64 ? (const void *)coefs : (const void *)coefs_f;
-   if (g_ctx.bits != 64) {
-      a.coff = coff;
-      a.ccoef = ccoef;
-      a.ncoef = ncoef;
-   }
    a.width = g_ctx.width;
    a.height = g_ctx.height;
    a.oversample = p->oversample;
@@ -1506,10 +1519,6 @@ extern "C" int fl3d_density(const fl3d_de_params *p, const fl3_de_filters *de) {
    int half = 0;
    while ((half + 1) * (half + 2) / 2 < de->kernel_size) half++;
    a.half = half;
-   if (de->max_filter_index >= 1024) {
-      set_err("density estimation: more than 1024 kernels");
-      return 1;
-   }
    if (g_ctx.width >= 65536 || g_ctx.height >= 65536) {
       set_err("density estimation: histogram side above 65535 cells");
       return 1;
@@ -1520,17 +1529,16 @@ extern "C" int fl3d_density(const fl3d_de_params *p, const fl3_de_filters *de) {
    if (g_ctx.srcl.ensure(sizeof(double) * (size_t)g_ctx.width * g_ctx.height)) return 1;
    a.srcv = g_ctx.srcv.p;
    a.srcl = (double *)g_ctx.srcl.p;
-   a.exact = p->exact || g_ctx.bits == 64;   // (the FP64 gather is the exact one)
+   a.exact = exact || g_ctx.bits == 64;   // (the log terms, which the exact gather reads)
    a.taps = de_taps();   // gather footprint, for the stage profile
    tune_init();
-   if (g_tune.de_halo) {
-      a.nbx = (g_ctx.width + DG_REGION_HOST - 1) / DG_REGION_HOST;
-      const size_t nblk = (size_t)a.nbx * ((g_ctx.height + DG_REGION_HOST - 1) / DG_REGION_HOST);
-      if (g_ctx.deblk.ensure(sizeof(int) * nblk)) return 1;
-      a.blkmax = (int *)g_ctx.deblk.p;
-   }
+   a.nbx = (g_ctx.width + DG_REGION_HOST - 1) / DG_REGION_HOST;
+   const size_t nblk = (size_t)a.nbx * ((g_ctx.height + DG_REGION_HOST - 1) / DG_REGION_HOST);
+   if (g_ctx.deblk.ensure(sizeof(int) * (nblk + 1))) return 1;
+   if (g_tune.de_halo) a.blkmax = (int *)g_ctx.deblk.p;
+   if (!exact && g_ctx.bits == 64) a.nonfinite = (int *)g_ctx.deblk.p + (a.blkmax ? nblk : 0);
    const int pk = prof_begin(ST_DE);
-   const int lrc = fl3k_launch_de_tiled(&a, g_ctx.stream, g_ctx.bits);
+   const int lrc = fl3k_launch_de_tiled(&a, g_ctx.stream, g_ctx.bits, exact);
    prof_end(pk);
    g_prof.cells = (long long)g_ctx.width * g_ctx.height;
    if (lrc) {
@@ -1541,7 +1549,7 @@ extern "C" int fl3d_density(const fl3d_de_params *p, const fl3_de_filters *de) {
 }
 
 static int de_many_batch(const fl3d_de_params *p, const fl3_de_filters *const *de, const std::vector<int> &dej,
-                         size_t tab, long long tcells);
+                         long long tcells);
 
 // Density estimation of renders 0..n-1 of the begun histograms in one
 // launch pair (FP32 accumulators; renders without DE filters, or with bits
@@ -1556,21 +1564,17 @@ extern "C" int fl3d_density_many(const fl3d_de_params *p, const fl3_de_filters *
    }
    const bool batched = g_ctx.bits != 64;
    std::vector<int> dej;
-   size_t tab = 0;
    long long tcells = 0;
    for (int i = 0; i < n; i++) {
       tcells += (long long)g_ctx.rwidth[i] * g_ctx.rheight[i];
       const bool has = de[i] && de[i]->max_filter_index > 0;
       if (has && batched && !p[i].exact && de[i]->max_filter_index < 1024 && g_ctx.rwidth[i] < 65536 &&
-          g_ctx.rheight[i] < 65536) {
+          g_ctx.rheight[i] < 65536 && de_tables_ok(de[i], sizeof(float))) {
          dej.push_back(i);
-         const size_t nc = (size_t)de[i]->nfilters * de[i]->kernel_size, nw = de[i]->nfilters;
-         tab += (nc + nw) * sizeof(double) + ((nc * sizeof(float) + 15) & ~(size_t)15) +
-                de_cut_bytes(de[i], de_cut_bank(de[i], nullptr, nullptr));
       }
    }
    const int nd = (int)dej.size();
-   if (nd > 0 && de_many_batch(p, de, dej, tab, tcells)) return 1;
+   if (nd > 0 && de_many_batch(p, de, dej, tcells)) return 1;
    // then the renders outside the batch, one by one
    for (int i = 0; i < n; i++) {
       const bool has = de[i] && de[i]->max_filter_index > 0;
@@ -1585,12 +1589,10 @@ extern "C" int fl3d_density_many(const fl3d_de_params *p, const fl3_de_filters *
 }
 
 // The batched part of fl3d_density_many: renders dej of the begun
-// histograms, tab bytes of coefficient tables, tcells cells in all.
+// histograms, tcells cells in all.
 static int de_many_batch(const fl3d_de_params *p, const fl3_de_filters *const *de, const std::vector<int> &dej,
-                         size_t tab, long long tcells) {
+                         long long tcells) {
    const int nd = (int)dej.size();
-   // coefficient tables (double, then the float copy) of every render
-   if (g_ctx.detab.ensure(tab)) return 1;
    if (g_ctx.findex.ensure(sizeof(uint16_t) * (size_t)tcells) || g_ctx.srcv.ensure(16 * (size_t)tcells) ||
        g_ctx.srcl.ensure(sizeof(double) * (size_t)tcells))
       return 1;
@@ -1607,66 +1609,71 @@ static int de_many_batch(const fl3d_de_params *p, const fl3_de_filters *const *d
    long long blk0 = 0;
    unsigned *pf = first.data(), *gf = first.data() + nd + 1;
    unsigned long long pb = 0, gb = 0;
-   std::vector<unsigned char> hostt(tab);
-   size_t off = 0;
    // renders with equal filter banks (the same estimator parameters and
-   // oversampling) share one uploaded table
-   // (with its cut bank after the float copy, if it has one)
+   // oversampling) share one uploaded bank: widths, tables, info
    struct Uniq {
       const fl3_de_filters *d;
-      size_t off;
-      int ncut;
+      size_t off, tab;   // byte offset, bytes of its tables
    };
    std::vector<Uniq> uniq;
-   int ncut_max = 0;
+   std::vector<int> bank((size_t)nd);
+   size_t off = 0;
+   std::vector<DeTables<float>> tabs;
    for (int k = 0; k < nd; k++) {
-      const int i = dej[k];
-      const fl3_de_filters *d = de[i];
+      const fl3_de_filters *d = de[dej[k]];
       const size_t nc = (size_t)d->nfilters * d->kernel_size, nw = d->nfilters;
-      const size_t base = (nc + nw) * sizeof(double) + ((nc * sizeof(float) + 15) & ~(size_t)15);
-      size_t toff = off;
-      int ncut = 0;
-      bool found = false;
-      for (const auto &u : uniq) {
-         const fl3_de_filters *e = u.d;
+      size_t u = 0;
+      for (; u < uniq.size(); u++) {
+         const fl3_de_filters *e = uniq[u].d;
          if (e->nfilters == d->nfilters && e->kernel_size == d->kernel_size &&
              e->max_filter_index == d->max_filter_index &&
              !memcmp(e->filter_coefs, d->filter_coefs, nc * sizeof(double)) &&
-             !memcmp(e->filter_widths, d->filter_widths, nw * sizeof(double))) {
-            toff = u.off;
-            ncut = u.ncut;
-            found = true;
+             !memcmp(e->filter_widths, d->filter_widths, nw * sizeof(double)))
             break;
-         }
       }
-      if (!found) {
-         memcpy(hostt.data() + off, d->filter_coefs, nc * sizeof(double));
-         memcpy(hostt.data() + off + nc * sizeof(double), d->filter_widths, nw * sizeof(double));
-         // the float copy, rounded to nearest as a device conversion would
-         float *ft = (float *)(hostt.data() + off + (nc + nw) * sizeof(double));
-         for (size_t e = 0; e < nc; e++) ft[e] = (float)d->filter_coefs[e];
-         ncut = de_cut_bank(d, nullptr, nullptr);
-         if (ncut)
-            de_cut_bank(d, (int *)(hostt.data() + off + base),
-                        (float *)(hostt.data() + off + base + de_cut_rows_bytes(d)));
-         uniq.push_back({d, off, ncut});
-         off += base + de_cut_bytes(d, ncut);
-      }
-      ncut_max = ncut > ncut_max ? ncut : ncut_max;
-      unsigned char *tb = (unsigned char *)g_ctx.detab.p + toff;
+      bank[k] = (int)u;
+      if (u < uniq.size()) continue;
+      tabs.emplace_back();
+      tabs.back().make(d);
+      const size_t tb = sizeof(float) * tabs.back().tab.size();
+      uniq.push_back({d, off, tb});
+      off += align16(sizeof(double) * nw) + align16(tb) + align16(sizeof(int) * tabs.back().info.size());
+   }
+   std::vector<unsigned char> hostt(off);
+   for (size_t u = 0; u < uniq.size(); u++) {
+      unsigned char *t = hostt.data() + uniq[u].off;
+      const size_t nw = uniq[u].d->nfilters;
+      memcpy(t, uniq[u].d->filter_widths, nw * sizeof(double));
+      memcpy(t + align16(sizeof(double) * nw), tabs[u].tab.data(), uniq[u].tab);
+      memcpy(t + align16(sizeof(double) * nw) + align16(uniq[u].tab), tabs[u].info.data(),
+             sizeof(int) * tabs[u].info.size());
+   }
+   if (g_ctx.detab.ensure(off)) return 1;
+   // 16x16 blocks of all renders: how the gather's workgroups divide them
+   long long blocks = 0;
+   for (int k = 0; k < nd; k++)
+      blocks += (long long)((g_ctx.rwidth[dej[k]] + DG_REGION_HOST - 1) / DG_REGION_HOST) *
+                ((g_ctx.rheight[dej[k]] + DG_REGION_HOST - 1) / DG_REGION_HOST);
+   const int cells = fl3k_de_cells(blocks);
+   int rw, rh;   // a gather workgroup's region
+   fl3k_de_region(cells, &rw, &rh);
+   size_t lds = 0;
+   for (int k = 0; k < nd; k++) {
+      const int i = dej[k];
+      const fl3_de_filters *d = de[i];
+      const Uniq &u = uniq[bank[k]];
+      const size_t o_tab = align16(sizeof(double) * d->nfilters);
+      unsigned char *tb = (unsigned char *)g_ctx.detab.p + u.off;
       DEArgs &a = as[k];
       memset(&a, 0, sizeof(a));
       const long long c0 = g_ctx.rcell0[i];
       a.buckets = (unsigned char *)g_ctx.buckets.p + c0 * bucket_bytes(g_ctx.bits);
       a.accum = (unsigned char *)g_ctx.accum.p + c0 * accum_bytes(g_ctx.bits);
-      a.coefs = (const double *)tb;
-      a.widths = (const double *)(tb + nc * sizeof(double));
-      a.coefs_t = tb + (nc + nw) * sizeof(double);
-      if (ncut) {
-         a.coff = (const int *)(tb + base);
-         a.ccoef = (const float *)(tb + base + de_cut_rows_bytes(d));
-         a.ncoef = ncut;
-      }
+      a.widths = (const double *)tb;
+      a.tab = tb + o_tab;
+      a.info = (const int *)(tb + o_tab + align16(u.tab));
+      a.tab_bytes = tabs[bank[k]].lds_bytes;
+      lds = std::max(lds, (size_t)a.tab_bytes + 8 * (size_t)(d->max_filter_index + 2));
       a.findex = (uint16_t *)g_ctx.findex.p + c0;
       a.srcv = (unsigned char *)g_ctx.srcv.p + c0 * 16;
       a.srcl = (double *)g_ctx.srcl.p + c0;
@@ -1692,8 +1699,7 @@ static int de_many_batch(const fl3d_de_params *p, const fl3_de_filters *const *d
       pf[k] = (unsigned)pb;
       gf[k] = (unsigned)gb;
       pb += (unsigned long long)((a.width + 255) / 256) * a.height;
-      gb += (unsigned long long)((a.width + DG_REGION_HOST - 1) / DG_REGION_HOST) *
-            ((a.height + DG_REGION_HOST - 1) / DG_REGION_HOST);
+      gb += (unsigned long long)((a.width + rw - 1) / rw) * ((a.height + rh - 1) / rh);
    }
    if (pb > 0x7fffffffULL || gb > 0x7fffffffULL) {
       set_err("fl3d_density_many: too many workgroups");
@@ -1710,7 +1716,7 @@ static int de_many_batch(const fl3d_de_params *p, const fl3_de_filters *const *d
    const unsigned *dfirst = (const unsigned *)((unsigned char *)g_ctx.deargs.p + ab);
    const int lrc = fl3k_launch_de_many((const DEArgs *)g_ctx.deargs.p, dfirst, (unsigned)pb, dfirst + nd + 1,
                                        (unsigned)gb, nd, g_ctx.stream, halo ? (int *)g_ctx.deblk.p : nullptr,
-                                       (long)nblk, sizeof(float) * (size_t)ncut_max);
+                                       (long)nblk, lds, cells);
    prof_end(pk);
    if (lrc) {
       set_err("density estimation launch failed");
@@ -2346,7 +2352,6 @@ extern "C" int fl3h_density_estimate_noalloc(const void *buckets, int width, int
    // index, the log terms and the values
    double *coefs = (double *)base;
    double *widths = coefs + nc;
-   float *coefs_f = (float *)(base + align256(sizeof(double) * (nc + nw)));
    int *blkmax = (int *)(base + FL3_SCRATCH_TABLES);
    unsigned char *cellp = base + FL3_SCRATCH_TABLES + FL3_SCRATCH_BLOCKS;
    uint16_t *findex = (uint16_t *)cellp;
@@ -2354,17 +2359,12 @@ extern "C" int fl3h_density_estimate_noalloc(const void *buckets, int width, int
    void *srcv = (void *)((unsigned char *)srcl + align256(sizeof(double) * cells));
    HIPCHK(hipMemcpyAsync(coefs, filter_coefs, sizeof(double) * nc, hipMemcpyHostToDevice, 0));
    HIPCHK(hipMemcpyAsync(widths, filter_widths, sizeof(double) * nw, hipMemcpyHostToDevice, 0));
-   if (fl3k_launch_f64_to_f32(coefs, coefs_f, (long)nc, 0)) {
-      set_err("k_f64_to_f32 launch failed");
-      return 1;
-   }
    DEArgs a;
    memset(&a, 0, sizeof(a));
    a.buckets = buckets;
    a.accum = accum;
    a.coefs = coefs;
    a.widths = widths;
-   a.coefs_t = bits == 64 ? (const void *)coefs : (const void *)coefs_f;
    a.width = width;
    a.height = height;
    a.oversample = oversample;
@@ -2387,7 +2387,7 @@ extern "C" int fl3h_density_estimate_noalloc(const void *buckets, int width, int
       return 1;
    }
    a.blkmax = blkmax;
-   if (fl3k_launch_de_tiled(&a, 0, bits)) {
+   if (fl3k_launch_de_tiled(&a, 0, bits, 1)) {
       set_err("density estimation launch failed");
       return 1;
    }

@@ -142,7 +142,6 @@ struct DEArgs {
    const double *widths;
    uint16_t *findex;        // per cell filter index, 0xffff = no contribution
    void *srcv;              // per cell AT[4]: colour x k1 log(1 + c3 k2) / c3
-   const void *coefs_t;     // the kernel coefficients in the accumulator type
    double *srcl;            // per cell k1 log(1 + c3 k2) (the reference's per-tap numerator)
    int exact;               // sum each contribution as the reference does (double, in source order)
    int width, height, oversample;
@@ -155,14 +154,19 @@ struct DEArgs {
    int *blkmax;
    int nbx;                 // blocks per row
    unsigned long long *taps;   // if set: 64 counters, summed: the gather footprint (2r + 1)^2 of all sources
-   // float accumulator, ncoef > 0: the rows cut to what a tap reaches (row i
-   // from ccoef[coff[i]], (r + 1)(r + 2) / 2 entries for radius r), which the
-   // gather stages in ncoef floats of dynamic LDS; 0: taps read coefs_t
-   const float *ccoef;
-   const int *coff;
-   int ncoef;
+   // production gather: kernel i as a table of (r + 2)^2 coefficients by
+   // |dy|, |dx| in 0..r + 1 (the last row and column zero), in the
+   // accumulator type from tab[info[2 i]], r = info[2 i + 1]; tab_bytes: of
+   // all tables when a workgroup holds them in LDS, 0 if it reads tab
+   const void *tab;
+   const int *info;
+   int tab_bytes;
+   // double accumulator: set by the preparation pass if a source's values
+   // are not finite (the production gather multiplies them by zero, so the
+   // exact one takes over)
+   int *nonfinite;
 };
-#define FL3_DE_LDS_COEFS 8192   // most floats of a cut filter bank the gather stages in LDS
+#define FL3_DE_LDS_BYTES 49152   // most LDS bytes of tables and info a gather workgroup takes
 
 struct TMArgs {
    const void *accum;

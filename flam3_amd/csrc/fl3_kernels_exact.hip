@@ -536,6 +536,10 @@ __device__ __forceinline__ unsigned de_prep_cell(const DEArgs &a, int i, int j, 
          v[1] = (AT)((double)b[cell * 5 + 1] * sc);
          v[2] = (AT)((double)b[cell * 5 + 2] * sc);
          v[3] = (AT)(c3 * sc);
+         if constexpr (sizeof(AT) == 8) {
+            // (a NaN or an infinity in any of them leaves no zero)
+            if (a.nonfinite && v[0] * 0.0 + v[1] * 0.0 + v[2] * 0.0 + v[3] * 0.0 != 0.0) *a.nonfinite = 1;
+         }
       }
    }
    a.findex[cell] = out;
@@ -570,6 +574,35 @@ __device__ __forceinline__ void de_prep_body(const DEArgs &a, int bx, int by) {
    }
 }
 
+#define DG_REGION 16
+#define DG_CHUNK 256
+
+// The halo a workgroup's 16x16 region needs: the largest radius among the 16x16 blocks whose widest source can reach it (-1:
+// none can), from the preparation pass's per-block maxima; without them the
+// widest kernel's.  A smaller halo holds the same reaching sources in the same
+// row-major order.  Ends with a barrier.
+__device__ __forceinline__ int de_halo(const DEArgs &a, int bx, int by, int rx0, int rx1, int ry0, int ry1) {
+   __shared__ int s_ext;
+   const int R = a.half;
+   if (a.blkmax) {
+      if (threadIdx.x == 0) s_ext = -1;
+      __syncthreads();
+      const int nbx = a.nbx, nby = (a.height + DG_REGION - 1) / DG_REGION;
+      const int span = (R + DG_REGION - 1) / DG_REGION, side = 2 * span + 1;
+      for (int k = threadIdx.x; k < side * side; k += DG_CHUNK) {
+         const int qx = bx + k % side - span, qy = by + k / side - span;
+         if (qx < 0 || qy < 0 || qx >= nbx || qy >= nby) continue;
+         const int bm = a.blkmax[qy * nbx + qx] - 1;
+         const int qx0 = qx * DG_REGION, qy0 = qy * DG_REGION;
+         const int gx = max(max(rx0 - (qx0 + DG_REGION - 1), qx0 - rx1), 0);
+         const int gy = max(max(ry0 - (qy0 + DG_REGION - 1), qy0 - ry1), 0);
+         if (bm >= 0 && gx <= bm && gy <= bm) atomicMax(&s_ext, min(bm, R));
+      }
+   }
+   __syncthreads();
+   return a.blkmax ? s_ext : R;
+}
+
 // Gather form: each thread owns one output cell and adds, in registers,
 // the contribution of every source whose kernel reaches it, sources taken
 // in row-major order -- the order in which the reference's single DE thread
@@ -581,22 +614,19 @@ __device__ __forceinline__ void de_prep_body(const DEArgs &a, int bx, int by) {
 // 256 cells, compacts the sources that reach it into LDS in order, and lists
 // for each wavefront, in the same order, those that reach its block, so a
 // wavefront loops over its own sources only.  No atomics.
-#define DG_REGION 16
-#define DG_CHUNK 256
-template <typename AT, bool EXACT>
+// This is the exact form (verification, replay, and sources whose values are
+// not finite); production renders take de_taps_body.
+template <typename AT>
 __device__ __forceinline__ void de_gather_body(const DEArgs &a, int bx, int by) {
-   // per source: packed position, kernel index and values -- doubles
-   // (4 channels and the log term) in the exact mode, the accumulator type
-   // (4 pre-scaled channels) otherwise
-   typedef typename std::conditional<EXACT, double, AT>::type VT;
-   constexpr int NV = EXACT ? 5 : 4;
+   // per source: position, first coefficient of its kernel and radius; its
+   // channels and log term
    __shared__ int radius[1024];
-   __shared__ int4 s_src[DG_CHUNK];   // per source: x, y, first coefficient of its kernel, radius
-   __shared__ VT s_val[DG_CHUNK][NV];
+   __shared__ int4 s_src[DG_CHUNK];
+   __shared__ double s_val[DG_CHUNK][5];
    __shared__ unsigned wave_cnt[DG_CHUNK / 64];
    __shared__ unsigned short s_list[4][DG_CHUNK];   // per 8x8 block: indices into the chunk's sources
    __shared__ unsigned list_cnt[4][DG_CHUNK / 64];  // [block][wavefront that listed them]
-   const int W = a.width, H = a.height, R = a.half;
+   const int W = a.width, H = a.height;
    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
    const int rx0 = bx * DG_REGION, ry0 = by * DG_REGION;
    const int rx1 = min(rx0 + DG_REGION, W) - 1, ry1 = min(ry0 + DG_REGION, H) - 1;
@@ -608,38 +638,10 @@ __device__ __forceinline__ void de_gather_body(const DEArgs &a, int bx, int by) 
    if (live)
       for (int c = 0; c < 4; c++) acc[c] = accp[c];
    for (int e = tid; e <= a.max_filter_index && e < 1024; e += DG_CHUNK) radius[e] = (int)ceil(a.widths[e]) - 1;
-   // The halo this region needs: the largest radius among the 16x16 blocks
-   // whose widest source can reach it (-1: none can), from the preparation
-   // pass's per-block maxima; without them the widest kernel's.  A smaller
-   // halo holds the same reaching sources in the same row-major order.
-   __shared__ int s_ext;
-   int E = R;
-   if (a.blkmax) {
-      if (tid == 0) s_ext = -1;
-      __syncthreads();
-      const int nbx = a.nbx, nby = (H + DG_REGION - 1) / DG_REGION;
-      const int span = (R + DG_REGION - 1) / DG_REGION, side = 2 * span + 1;
-      for (int k = tid; k < side * side; k += DG_CHUNK) {
-         const int qx = bx + k % side - span, qy = by + k / side - span;
-         if (qx < 0 || qy < 0 || qx >= nbx || qy >= nby) continue;
-         const int bm = a.blkmax[qy * nbx + qx] - 1;
-         const int qx0 = qx * DG_REGION, qy0 = qy * DG_REGION;
-         const int gx = max(max(rx0 - (qx0 + DG_REGION - 1), qx0 - rx1), 0);
-         const int gy = max(max(ry0 - (qy0 + DG_REGION - 1), qy0 - ry1), 0);
-         if (bm >= 0 && gx <= bm && gy <= bm) atomicMax(&s_ext, min(bm, R));
-      }
-   }
-   // the cut filter bank (float accumulator), for the taps below
-   float *s_coef = (float *)fl3_lds;
-   constexpr bool CUT = !EXACT && std::is_same<AT, float>::value;
-   if (CUT && a.ncoef > 0)
-      for (int e = tid; e < a.ncoef; e += DG_CHUNK) s_coef[e] = a.ccoef[e];
-   __syncthreads();
-   if (a.blkmax) E = s_ext;
+   const int E = de_halo(a, bx, by, rx0, rx1, ry0, ry1);
    const int hx0 = max(0, rx0 - E), hx1 = min(W, rx1 + 1 + E);
    const int hy0 = max(0, ry0 - E), hy1 = min(H, ry1 + 1 + E);
    const int hw = hx1 - hx0, nh = E < 0 ? 0 : hw * (hy1 - hy0);
-   const AT *srcv = (const AT *)a.srcv;
    for (int base = 0; base < nh; base += DG_CHUNK) {
       const int s = base + tid;
       int flag = 0, sx = 0, sy = 0, fi = 0;
@@ -678,18 +680,9 @@ __device__ __forceinline__ void de_gather_body(const DEArgs &a, int bx, int by) 
       if (flag) {
          const unsigned idx = off + rank;
          const long cell = sx + (long)sy * W;
-         if constexpr (EXACT)
-            s_src[idx] = make_int4(sx, sy, fi * a.kernel_size, radius[fi]);
-         else   // (as floats: every value here is an integer below 2^24)
-            s_src[idx] = make_int4(__float_as_int((float)sx), __float_as_int((float)sy),
-                                   __float_as_int((float)(CUT && a.ncoef > 0 ? a.coff[fi] : fi * a.kernel_size)),
-                                   __float_as_int((float)radius[fi]));
-         if constexpr (EXACT) {
-            for (int c = 0; c < 4; c++) s_val[idx][c] = bucket_value(a.buckets, cell * 5 + c, (AT)0);
-            s_val[idx][4] = a.srcl[cell];
-         } else {
-            for (int c = 0; c < 4; c++) s_val[idx][c] = srcv[cell * 4 + c];
-         }
+         s_src[idx] = make_int4(sx, sy, fi * a.kernel_size, radius[fi]);
+         for (int c = 0; c < 4; c++) s_val[idx][c] = bucket_value(a.buckets, cell * 5 + c, (AT)0);
+         s_val[idx][4] = a.srcl[cell];
       }
       __syncthreads();
       unsigned nb = 0;
@@ -701,63 +694,207 @@ __device__ __forceinline__ void de_gather_body(const DEArgs &a, int bx, int by) 
       }
       for (int w = 0; w < DG_CHUNK / 64; w++) nb += list_cnt[wave][w];
       __syncthreads();
-      if constexpr (EXACT) {
-         // (the coefficient is loaded for every listed source, from index 0
-         // when the tap misses this cell, so that the loads of consecutive
-         // sources overlap; a missed tap adds nothing)
+      // (the coefficient is loaded for every listed source, from index 0
+      // when the tap misses this cell, so that the loads of consecutive
+      // sources overlap; a missed tap adds nothing)
 #pragma unroll 4
-         for (unsigned i = 0; i < nb; i++) {
-            const unsigned k = s_list[wave][i];
-            const int4 src = s_src[k];
-            const int dx = abs(x - src.x), dy = abs(y - src.y);
-            const int hi = max(dx, dy), lo = min(dx, dy);
-            const bool tap = live && hi <= src.w;
-            const long ci = tap ? (long)src.z + hi * (hi + 1) / 2 + lo : 0;
-            const double coef = a.coefs[ci];
-            if (tap && coef != 0.0) {
-               const double c3 = s_val[k][3];
-               const double ls = coef * s_val[k][4] / c3;
-               for (int c = 0; c < 4; c++) acc[c] = (AT)((double)acc[c] + s_val[k][c] * ls);
-            }
+      for (unsigned i = 0; i < nb; i++) {
+         const unsigned k = s_list[wave][i];
+         const int4 src = s_src[k];
+         const int dx = abs(x - src.x), dy = abs(y - src.y);
+         const int hi = max(dx, dy), lo = min(dx, dy);
+         const bool tap = live && hi <= src.w;
+         const long ci = tap ? (long)src.z + hi * (hi + 1) / 2 + lo : 0;
+         const double coef = a.coefs[ci];
+         if (tap && coef != 0.0) {
+            const double c3 = s_val[k][3];
+            const double ls = coef * s_val[k][4] / c3;
+            for (int c = 0; c < 4; c++) acc[c] = (AT)((double)acc[c] + s_val[k][c] * ls);
          }
-      } else {
-         // Straight-line taps, no branches, so that the coefficient loads of
-         // consecutive sources are in flight together: a tap that misses
-         // this cell loads index 0 and adds it times 0 (the per-source
-         // values are finite), in 32-bit index arithmetic, fused
-         // multiply-adds.
-         // (distances in float, exact for these integers below 2^24, so
-         // that |.| comes free with the max and min; the tap's index
-         // z + hi (hi + 1) / 2 + lo by exact fused multiply-adds; a missed
-         // tap's index cleared by a mask, so that the body has no branch)
-         // (coefficients from the cut bank in LDS when it is there, else
-         // from the full table: one loop each, no per-tap choice)
-         const AT *ct = (const AT *)a.coefs_t;
-         const float fx = (float)x, fy = (float)y;
-         auto taps = [&](auto coef_at) {
-#pragma unroll 4
-            for (unsigned i = 0; i < nb; i++) {
-               const unsigned k = s_list[wave][i];
-               const int4 src = s_src[k];
-               const float ax = fx - __int_as_float(src.x), ay = fy - __int_as_float(src.y);
-               const float hi = fmaxf(fabsf(ax), fabsf(ay)), lo = fminf(fabsf(ax), fabsf(ay));
-               const bool tap = live && hi <= __int_as_float(src.w);
-               const float cf = fmaf(fmaf(hi, hi, hi), 0.5f, lo) + __int_as_float(src.z);
-               const unsigned ci = (unsigned)cf & (0u - (unsigned)tap);
-               const AT cv = coef_at(ci);
-               const AT coef = tap ? cv : (AT)0;
-               for (int c = 0; c < 4; c++) acc[c] = fma(coef, s_val[k][c], acc[c]);
-            }
-         };
-         if (CUT && a.ncoef > 0)
-            taps([&](unsigned c) { return (AT)s_coef[c]; });
-         else
-            taps([&](unsigned c) { return ct[c]; });
       }
       __syncthreads();
    }
    if (live)
       for (int c = 0; c < 4; c++) accp[c] = acc[c];
+}
+
+// The production gather: the sums of de_gather_body in the same row-major
+// order, each contribution one fused multiply-add of the kernel's coefficient
+// and the source's pre-scaled channels.  Bound by vector instructions, those
+// of the taps and those that scan the halo for sources that reach.  A kernel's
+// coefficients lie in a square table with a zero row and column at its edge,
+// and the distances are clamped to that edge, so a tap costs three
+// instructions for its address, without tests (a missed tap adds zero); the tables are in LDS where they fit (a wavefront
+// reads 64 scattered coefficients per source).  A lane holds CELLS cells, 8
+// rows apart, which share the source's read and the x distance.  In FP32 the
+// four channels are one matrix instruction, an outer product of four cells'
+// coefficients and four channels whose every sum is one fused multiply-add
+// with the bits of fmaf.  Each
+// wavefront scans its own block's halo and lists its sources in LDS of its
+// own: no barriers, and a tighter halo than a workgroup's.
+// At 1920x1080 with 2x2 supersampling (8.4M cells, radius 9): 876 us with a
+// workgroup's shared lists and tests per tap, 671 us so (2.75e8 vector
+// instructions instead of 5.7e8; LDS is active for 60% of the time); 3840x2160
+// with 3x3 in FP64 44.0 ms (each term formed per tap) against 21.2 ms.
+// Wavefronts of a workgroup: they share the tables, NW / 2 blocks across and two
+// down.
+constexpr int de_waves(int cells) { return cells == 2 ? 8 : 4; }
+template <typename AT, int CELLS>
+__device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
+   constexpr int SH = sizeof(AT) == 4 ? 2 : 3, BH = 8 * CELLS, NW = de_waves(CELLS), TURN = 32, CAP = TURN + 64;
+   typedef typename std::conditional<sizeof(AT) == 4, float4, double4>::type V4;
+   __shared__ int4 s_src[NW][CAP];   // per wavefront: x, y, its table's place, radius + 1
+   __shared__ unsigned s_stride[NW][CAP];   // bytes of a row of its square
+   __shared__ V4 s_val[NW][CAP];
+   __shared__ int s_ext[NW];
+   // the tables (tab_bytes), then per kernel its table's place (LDS address, or
+   // byte offset in tab) and radius, and one that reaches nothing
+   int2 *s_info = (int2 *)(fl3_lds + a.tab_bytes);
+   typedef const __attribute__((address_space(3))) AT lds_at;
+   const int nf = a.max_filter_index + 1;
+   const int lds0 = a.tab_bytes ? (int)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)fl3_lds : 0;
+   const int W = a.width, H = a.height;
+   const int tid = threadIdx.x, lane = tid & 63;
+   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // (so that what depends on it is scalar)
+   const int mx0 = (bx * (NW / 2) + wave % (NW / 2)) * 8, my0 = (by * 2 + wave / (NW / 2)) * BH;
+   const int mx1 = min(mx0 + 8, W) - 1, my1 = min(my0 + BH, H) - 1;
+   const int x = mx0 + (lane & 7), y = my0 + (lane >> 3);
+#pragma unroll 4
+   for (int e = tid; e < a.tab_bytes / 16; e += 64 * NW) ((uint4 *)fl3_lds)[e] = ((const uint4 *)a.tab)[e];
+   for (int e = tid; e <= nf; e += 64 * NW)
+      s_info[e] = e < nf ? make_int2((a.info[2 * e] << SH) + lds0, a.info[2 * e + 1]) : make_int2(lds0, -(1 << 20));
+   // acc[j][i]: FP32, channel lane & 3 of cell (px + i, y + 8 j) of this lane's
+   // four, as the matrix instruction leaves them; FP64, channel i of (x, y + 8 j)
+   constexpr bool MAT = sizeof(AT) == 4;
+   const int px = MAT ? mx0 + (lane & 4) : x;
+   typedef AT AV __attribute__((ext_vector_type(4)));
+   AV acc[CELLS];
+   auto at_acc = [&](int j, int i) {
+      return (AT *)a.accum + ((px + (MAT ? i : 0)) + (long)(y + 8 * j) * W) * 4 + (MAT ? lane & 3 : i);
+   };
+   for (int j = 0; j < CELLS; j++)
+      for (int i = 0; i < 4; i++)
+         acc[j][i] = px + (MAT ? i : 0) < W && y + 8 * j < H ? *at_acc(j, i) : (AT)0;
+   // this block's halo, as de_halo finds a region's
+   int E = a.half;
+   if (a.blkmax) {
+      if (lane == 0) s_ext[wave] = -1;
+      const int span = (a.half + DG_REGION - 1) / DG_REGION;
+      const int bx0 = mx0 / DG_REGION - span, by0 = my0 / DG_REGION - span;
+      const int cols = 2 * span + 1, rows = (my0 + BH - 1) / DG_REGION + span - by0 + 1;
+      const int nby = (H + DG_REGION - 1) / DG_REGION;
+      for (int k = lane; k < cols * rows; k += 64) {
+         const int qx = bx0 + k % cols, qy = by0 + k / cols;
+         if (qx < 0 || qy < 0 || qx >= a.nbx || qy >= nby) continue;
+         const int bm = a.blkmax[qy * a.nbx + qx] - 1;
+         const int gx = max(max(mx0 - (qx * DG_REGION + DG_REGION - 1), qx * DG_REGION - mx1), 0);
+         const int gy = max(max(my0 - (qy * DG_REGION + DG_REGION - 1), qy * DG_REGION - my1), 0);
+         if (bm >= 0 && gx <= bm && gy <= bm) atomicMax(&s_ext[wave], min(bm, a.half));
+      }
+   }
+   __syncthreads();
+   if (a.blkmax) E = __builtin_amdgcn_readfirstlane(s_ext[wave]);
+   const int hx0 = max(0, mx0 - E), hx1 = min(W, mx1 + 1 + E);
+   const int hy0 = max(0, my0 - E), hy1 = min(H, my1 + 1 + E);
+   const int hw = hx1 - hx0, nh = E < 0 || mx0 >= W || my0 >= H ? 0 : hw * (hy1 - hy0);
+   const V4 *srcv = (const V4 *)a.srcv;
+   auto taps = [&](int n, auto coef_at) {
+#pragma unroll 4
+      for (int i = 0; i < n; i++) {
+         const int4 src = s_src[wave][i];
+         const unsigned w = (unsigned)src.w;
+         // (|x - y| of coordinates below 65536, whose high halves are zero)
+         const unsigned ax = min(__builtin_amdgcn_sad_u16((unsigned)x, (unsigned)src.x, 0u), w);
+         const unsigned row = (ax << SH) + (unsigned)src.z, stride = s_stride[wave][i];
+         for (int j = 0; j < CELLS; j++) {
+            const unsigned ay = min(__builtin_amdgcn_sad_u16((unsigned)(y + 8 * j), (unsigned)src.y, 0u), w);
+            const AT coef = coef_at(__umul24(ay, stride) + row);
+            if constexpr (MAT)
+               acc[j] = __builtin_amdgcn_mfma_f32_4x4x1f32(coef, ((const float *)&s_val[wave][i])[lane & 3], acc[j], 0, 0, 0);
+            else {
+               const V4 v = s_val[wave][i];
+               acc[j][0] = fma(coef, v.x, acc[j][0]);
+               acc[j][1] = fma(coef, v.y, acc[j][1]);
+               acc[j][2] = fma(coef, v.z, acc[j][2]);
+               acc[j][3] = fma(coef, v.w, acc[j][3]);
+            }
+         }
+      }
+   };
+   auto scan = [&](auto coef_at) {
+      // the lane's cell of the next 64 halo cells (its place, its index), and
+      // its kernel; the source it found among the 64 before, whose channels are
+      // on their way
+      int sx = hx0, sy = hy0, stepx = 0, stepy = 0;
+      if (nh > 0) {
+         sx += lane % hw;
+         sy += lane / hw;
+         stepx = 64 % hw;
+         stepy = 64 / hw;
+      }
+      unsigned cell = (unsigned)(sx + sy * W);   // (histograms stay below 2^31 cells)
+      const unsigned step = (unsigned)(stepx + stepy * W), wrap = (unsigned)(W - hw);
+      auto kernel_at = [&](int k, unsigned c) {
+         return k < nh ? (int)*(const uint16_t *)((const unsigned char *)a.findex + (size_t)(c * 2u)) : (int)DE_SKIP;
+      };
+      int fnext = kernel_at(lane, cell);
+      int listed = 0, found = 0, at = -1;   // sources in the list, and with the last 64's
+      int4 src = make_int4(0, 0, 0, 0);
+      V4 val = {(AT)0, (AT)0, (AT)0, (AT)0};
+      // (a block reaches as far as its distances from twice its middle)
+      const unsigned mid2x = (unsigned)(2 * mx0 + 7), mid2y = (unsigned)(2 * my0 + BH - 1);
+      for (int base = 0; base < nh + 64; base += 64) {   // (one turn more for the last 64's)
+         const int f = fnext, cx = sx, cy = sy;
+         const unsigned cc = cell;
+         sx += stepx;
+         sy += stepy;
+         cell += step;
+         if (sx >= hx1) {
+            sx -= hw;
+            sy++;
+            cell += wrap;
+         }
+         fnext = kernel_at(base + 64 + lane, cell);
+         const int2 in = s_info[min(f, nf)];
+         if (at >= 0) {
+            s_src[wave][at] = src;
+            s_stride[wave][at] = ((unsigned)src.w << SH) + (1u << SH);
+            s_val[wave][at] = val;
+         }
+         listed = found;
+         at = -1;
+         const int dx2 = abs(2 * cx - (int)mid2x), dy2 = abs(2 * cy - (int)mid2y);
+         const bool reach = dx2 <= 2 * in.y + 7 && dy2 <= 2 * in.y + BH - 1;
+         const unsigned long long m = __builtin_amdgcn_ballot_w64(reach);
+         if (listed >= TURN) {
+            __builtin_amdgcn_wave_barrier();
+            const int n = listed & ~(TURN - 1);
+            taps(n, coef_at);
+            __builtin_amdgcn_wave_barrier();
+            listed -= n;
+            if (lane < listed) {
+               s_src[wave][lane] = s_src[wave][n + lane];
+               s_stride[wave][lane] = s_stride[wave][n + lane];
+               s_val[wave][lane] = s_val[wave][n + lane];
+            }
+         }
+         if (reach) {
+            at = listed + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+            src = make_int4(cx, cy, in.x, in.y + 1);
+            val = srcv[cc];
+         }
+         found = listed + __popcll(m);
+      }
+      __builtin_amdgcn_wave_barrier();
+      taps(listed, coef_at);
+   };
+   if (a.tab_bytes)
+      scan([&](unsigned o) { return *(lds_at *)(uintptr_t)o; });
+   else
+      scan([&](unsigned o) { return *(const AT *)((const unsigned char *)a.tab + o); });
+   for (int j = 0; j < CELLS; j++)
+      for (int i = 0; i < 4; i++)
+         if (px + (MAT ? i : 0) < W && y + 8 * j < H) *at_acc(j, i) = acc[j][i];
 }
 
 __global__ __launch_bounds__(256) void k_fill_i32(int *p, long n, int v) {
@@ -770,9 +907,16 @@ __global__ __launch_bounds__(256) void k_de_prep(DEArgs a) {
    de_prep_body<BT, AT>(a, blockIdx.x, blockIdx.y);
 }
 
-template <typename AT, bool EXACT>
+template <typename AT>
 __global__ __launch_bounds__(DG_CHUNK) void k_de_gather(DEArgs a) {
-   de_gather_body<AT, EXACT>(a, blockIdx.x, blockIdx.y);
+   if (a.nonfinite && !*a.nonfinite) return;   // (the production gather has run)
+   de_gather_body<AT>(a, blockIdx.x, blockIdx.y);
+}
+
+template <typename AT, int CELLS>
+__global__ __launch_bounds__(64 * de_waves(CELLS)) void k_de_taps(DEArgs a) {
+   if (a.nonfinite && *a.nonfinite) return;   // (k_de_gather takes over)
+   de_taps_body<AT, CELLS>(a, blockIdx.x, blockIdx.y);
 }
 
 // Several renders in one launch: workgroup b belongs to the render j with
@@ -796,29 +940,43 @@ __global__ __launch_bounds__(256) void k_de_prep_many(const DEArgs *as, const un
    de_prep_body<BT, AT>(a, (int)(local % cols), (int)(local / cols));
 }
 
-template <typename AT, bool EXACT>
-__global__ __launch_bounds__(DG_CHUNK) void k_de_gather_many(const DEArgs *as, const unsigned *first, int n) {
+template <int CELLS>
+__global__ __launch_bounds__(64 * de_waves(CELLS)) void k_de_taps_many(const DEArgs *as, const unsigned *first, int n) {
    const int j = de_job(first, n, blockIdx.x);
    const DEArgs a = as[j];
-   const unsigned local = blockIdx.x - first[j], cols = (unsigned)(a.width + DG_REGION - 1) / DG_REGION;
-   de_gather_body<AT, EXACT>(a, (int)(local % cols), (int)(local / cols));
+   const unsigned local = blockIdx.x - first[j], cols = (unsigned)(a.width + 4 * de_waves(CELLS) - 1) / (4 * de_waves(CELLS));
+   de_taps_body<float, CELLS>(a, (int)(local % cols), (int)(local / cols));
+}
+
+// Cells a lane of the production gather holds, for regions of `blocks` 16x16
+// blocks of cells in all: two where that leaves every CU several workgroups,
+// one otherwise, where the gather is bound by how long a workgroup takes.
+// Kernel time with one and two: 640x480 (1271 blocks) 40 and 59 us; 7.7k blocks
+// 263 and 235 us, 32k blocks 838 and 672 us.
+extern "C" int fl3k_de_cells(long long blocks) { return blocks >= 4096 ? 2 : 1; }
+// Cells across and down of a workgroup's region.
+extern "C" void fl3k_de_region(int cells, int *w, int *h) {
+   *w = 4 * de_waves(cells);
+   *h = 16 * cells;
 }
 
 // Density estimation of n renders: per-render arguments in device memory,
 // workgroup prefixes prep_first[n + 1] (rows of 256 cells) and
-// gather_first[n + 1] (16x16 regions).  bits 32/33 with the FP32
-// accumulator (exact = 0) only.
+// gather_first[n + 1] (regions of 16 x 16 cells, 16 x 32 for cells 2).  bits
+// 32/33 with the FP32 accumulator (production arithmetic) only.
 // blkmax: a device array of nblk ints the renders' blkmax pointers point
 // into (cleared here), or nullptr.
 extern "C" int fl3k_launch_de_many(const DEArgs *as, const unsigned *prep_first, unsigned prep_blocks,
                                    const unsigned *gather_first, unsigned gather_blocks, int n, hipStream_t s,
-                                   int *blkmax, long nblk, size_t gather_lds) {
+                                   int *blkmax, long nblk, size_t gather_lds, int cells) {
    if (n <= 0) return 0;
    if (blkmax)
       hipLaunchKernelGGL(k_fill_i32, dim3((unsigned)((nblk + 255) / 256)), dim3(256), 0, s, blkmax, nblk, 0);
    hipLaunchKernelGGL((k_de_prep_many<uint32_t, float>), dim3(prep_blocks), dim3(256), 0, s, as, prep_first, n);
-   hipLaunchKernelGGL((k_de_gather_many<float, false>), dim3(gather_blocks), dim3(DG_CHUNK), gather_lds, s, as,
-                      gather_first, n);
+   if (cells == 2)
+      hipLaunchKernelGGL(k_de_taps_many<2>, dim3(gather_blocks), dim3(64 * de_waves(2)), gather_lds, s, as, gather_first, n);
+   else
+      hipLaunchKernelGGL(k_de_taps_many<1>, dim3(gather_blocks), dim3(64 * de_waves(1)), gather_lds, s, as, gather_first, n);
    return hipGetLastError() != hipSuccess;
 }
 
@@ -972,37 +1130,37 @@ extern "C" int fl3k_launch_deposit(const unsigned char *job, const double *pts, 
    return hipGetLastError() != hipSuccess;
 }
 
-extern "C" int fl3k_launch_de_tiled(const DEArgs *a, hipStream_t s, int bits) {
-   const dim3 g1((a->width + 255) / 256, a->height), b1(256);
+// exact: the reference's contributions one by one; else the production
+// gather (a->tab ..., and, for the double accumulator, a->nonfinite)
+extern "C" int fl3k_launch_de_tiled(const DEArgs *a, hipStream_t s, int bits, int exact) {
+   const dim3 g1((a->width + 255) / 256, a->height), b1(256), b3(DG_CHUNK);
    const dim3 g3((a->width + DG_REGION - 1) / DG_REGION, (a->height + DG_REGION - 1) / DG_REGION);
-   if (a->blkmax) {   // per-block radii, cleared here and marked by the preparation pass
-      const long nblk = (long)g3.x * g3.y;
-      hipLaunchKernelGGL(k_fill_i32, dim3((unsigned)((nblk + 255) / 256)), dim3(256), 0, s, a->blkmax, nblk, 0);
-   }
+   const int cells = fl3k_de_cells((long long)g3.x * g3.y);
+   int tw, th;
+   fl3k_de_region(cells, &tw, &th);
+   const dim3 gt((a->width + tw - 1) / tw, (a->height + th - 1) / th), bt(64 * de_waves(cells));
+   const size_t lds = exact ? 0 : (size_t)a->tab_bytes + 8 * (size_t)(a->max_filter_index + 2);
+   // per-block radii, cleared here and marked by the preparation pass, and
+   // the flag behind them
+   const long nblk = (a->blkmax ? (long)g3.x * g3.y : 0) + (a->nonfinite ? 1 : 0);
+   int *clear = a->blkmax ? a->blkmax : a->nonfinite;
+   if (nblk) hipLaunchKernelGGL(k_fill_i32, dim3((unsigned)((nblk + 255) / 256)), dim3(256), 0, s, clear, nblk, 0);
    if (bits == 64) {
       hipLaunchKernelGGL((k_de_prep<double, double>), g1, b1, 0, s, *a);
-      hipLaunchKernelGGL((k_de_gather<double, true>), g3, dim3(DG_CHUNK), 0, s, *a);
+      if (!exact && cells == 2)
+         hipLaunchKernelGGL((k_de_taps<double, 2>), gt, bt, lds, s, *a);
+      else if (!exact)
+         hipLaunchKernelGGL((k_de_taps<double, 1>), gt, bt, lds, s, *a);
+      hipLaunchKernelGGL(k_de_gather<double>, g3, b3, 0, s, *a);
    } else {
       hipLaunchKernelGGL((k_de_prep<uint32_t, float>), g1, b1, 0, s, *a);
-      if (a->exact)
-         hipLaunchKernelGGL((k_de_gather<float, true>), g3, dim3(DG_CHUNK), 0, s, *a);
+      if (exact)
+         hipLaunchKernelGGL(k_de_gather<float>, g3, b3, 0, s, *a);
+      else if (cells == 2)
+         hipLaunchKernelGGL((k_de_taps<float, 2>), gt, bt, lds, s, *a);
       else
-         hipLaunchKernelGGL((k_de_gather<float, false>), g3, dim3(DG_CHUNK),
-                            a->ncoef > 0 ? sizeof(float) * (size_t)a->ncoef : 0, s, *a);
+         hipLaunchKernelGGL((k_de_taps<float, 1>), gt, bt, lds, s, *a);
    }
-   return hipGetLastError() != hipSuccess;
-}
-
-// Double to float copy of a table on the device (the density-estimation
-// coefficients of the FP32 accumulator path).
-__global__ __launch_bounds__(256) void k_f64_to_f32(const double *src, float *dst, long n) {
-   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-   if (i < n) dst[i] = (float)src[i];
-}
-
-extern "C" int fl3k_launch_f64_to_f32(const double *src, float *dst, long n, hipStream_t s) {
-   if (n <= 0) return 0;
-   hipLaunchKernelGGL(k_f64_to_f32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, src, dst, n);
    return hipGetLastError() != hipSuccess;
 }
 

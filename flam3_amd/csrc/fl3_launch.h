@@ -34,11 +34,12 @@ int fl3k_launch_preview(const unsigned char *job, int xi, double range, int numv
                         uint32_t *isaac, size_t lds, hipStream_t s);
 int fl3k_launch_deposit(const unsigned char *job, const double *pts, long long n, void *buckets, uint32_t *sat,
                         unsigned grid, size_t lds, hipStream_t s, int bits);
-int fl3k_launch_de_tiled(const DEArgs *a, hipStream_t s, int bits);
+int fl3k_launch_de_tiled(const DEArgs *a, hipStream_t s, int bits, int exact);
+int fl3k_de_cells(long long blocks);
+void fl3k_de_region(int cells, int *w, int *h);
 int fl3k_launch_de_many(const DEArgs *as, const unsigned *prep_first, unsigned prep_blocks,
                         const unsigned *gather_first, unsigned gather_blocks, int n, hipStream_t s,
-                        int *blkmax, long nblk, size_t gather_lds);
-int fl3k_launch_f64_to_f32(const double *src, float *dst, long n, hipStream_t s);
+                        int *blkmax, long nblk, size_t gather_lds, int cells);
 int fl3k_launch_logscale(const void *b, void *acc, long n, double k1, double k2, hipStream_t s, int bits);
 int fl3k_launch_earlyclip(void *acc, long n, const TMArgs *a, hipStream_t s, int bits);
 int fl3k_launch_tonemap(const TMArgs *a, hipStream_t s, int bits);
