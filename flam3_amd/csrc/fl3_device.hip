@@ -110,7 +110,7 @@ struct Ctx {
    size_t de_up_tab = 0;             // the tables' bytes, and how many of them LDS takes
    int de_up_lds = 0;
    DevBuf crec[FL3_CHUNK_BUFS], cblk[FL3_CHUNK_BUFS], ctot[FL3_CHUNK_BUFS];   // tile-binned deposit
-   DevBuf sorted, wstate, bins, jobtab, soff;
+   DevBuf sorted, wstate, bins, jobtab, soff, partial;
    DevBuf srcv, srcl;                  // density estimation per-source values
    DevBuf detab, deargs;               // batched density estimation: tables, per-render arguments
    DevBuf deblk;                       // DE: widest source kernel per 16x16 block
@@ -170,7 +170,7 @@ extern "C" int fl3d_device_memory(double *avail, double *total) {
    size_t fr = 0, tot = 0;
    HIPCHK(hipMemGetInfo(&fr, &tot));
    const DevBuf *bufs[] = {&g_ctx.buckets, &g_ctx.accum, &g_ctx.job, &g_ctx.table, &g_ctx.image, &g_ctx.isaac,
-                           &g_ctx.points, &g_ctx.misc, &g_ctx.findex, &g_ctx.sorted, &g_ctx.wstate, &g_ctx.bins,
+                           &g_ctx.points, &g_ctx.misc, &g_ctx.findex, &g_ctx.sorted, &g_ctx.partial, &g_ctx.wstate, &g_ctx.bins,
                            &g_ctx.jobtab, &g_ctx.soff, &g_ctx.srcv, &g_ctx.srcl, &g_ctx.detab, &g_ctx.deargs,
                            &g_ctx.rcount, &g_ctx.descs, &g_ctx.deblk};
    double held = 0.0;
@@ -676,10 +676,10 @@ static int upload_job_tables(const fl3_job_hdr *const *h, int n, int nxf_max, Bi
 
 // Job records carry the colour (and take the packed accumulation) when
 // every job that writes them has full visibility and a stepped palette of
-// entries below 256, the tiles hold 2048 or 4096 cells and the walker's LDS
+// entries below 256, the tiles hold 4096 cells and the walker's LDS
 // has room for the palette after its tile counts.
 static bool colour_records(const fl3_job_hdr *const *h, int n, const uint32_t *pal8, int shift, size_t lds_walker) {
-   return pal8 && (shift == 11 || shift == 12) && job_records_packed(h, n) &&
+   return pal8 && shift == FL3_PACKED_SHIFT && job_records_packed(h, n) &&
           ((lds_walker + 15) & ~(size_t)15) + 1024 <= g_ctx.lds_max;
 }
 
@@ -699,6 +699,22 @@ static int narrow_round(const fl3_job_hdr *const *h, int n) {
    return (int)(lim / pass * pass);
 }
 
+// The alpha that every entry of the jobs' palettes truncates to, if all
+// entries are bytes (so that a cell's alpha is that times its count); else -1.
+static int narrow_alpha(const fl3_job_hdr *const *h, int n) {
+   int alpha = -1;
+   for (int j = 0; j < n; j++) {
+      const double *dm = (const double *)((const unsigned char *)h[j] + h[j]->off_dmap);
+      for (int e = 0; e < 1024; e++) {
+         if (!(dm[e] >= 0.0 && dm[e] < 256.0)) return -1;
+         if ((e & 3) != 3) continue;
+         if (alpha >= 0 && (int)dm[e] != alpha) return -1;
+         alpha = (int)dm[e];
+      }
+   }
+   return alpha;
+}
+
 // Largest records per accumulation work item: a cell's sums must fit 32
 // bits (and the packed pairs must not carry): at most 2^18 records, fewer
 // if a palette entry exceeds 255.  Double buckets (fixed64) sum multiples of
@@ -715,6 +731,21 @@ static int item_records(const fl3_job_hdr *const *h, int n, int fixed64 = 0) {
    const double lim = (fixed64 ? 2147483647.0 : 4294967295.0) / (maxd + 1.0);
    const int c = lim < (double)FL3_BIN_ITEM_RECORDS ? (int)lim : FL3_BIN_ITEM_RECORDS;
    return c < 1 ? 1 : c;
+}
+
+// Work items of the packed accumulation for chunks of up to `records`, and
+// room for their partial sums: one for each of two workgroups a CU, of at least
+// two of their steps and at most 2^17 records.  (3.6M records on 256 CUs: items
+// of 2^14 take 17 us with the merge, of 2^13 24 us, of 2^18 69 us.  2^28 records:
+// of 2^17 470 us, of 2^16 535 us, as more partial sums are written and read,
+// of 2^18 486 us, as the last ones run alone.)
+static int packed_items(BinArgs *b, long long records) {
+   const int step = fl3k_bin_pass_records();
+   const long long c = records / (2 * g_ctx.ncu) / step * step;
+   b->chunk = (int)std::min((long long)b->chunk, std::min(std::max(c, 2LL * step), 1LL << 17));
+   if (g_ctx.partial.ensure(fl3k_bin_partial_bytes(b, records))) return 1;
+   b->partial = g_ctx.partial.p;
+   return 0;
 }
 
 // Genomes whose walkers draw the xform per wavefront: no xaos, and room in
@@ -800,6 +831,8 @@ static int bin_banded(const BinArgs &b1, int format, int band, int shift, hipStr
       b.item_start = bw + 2 * FL3_MAX_BINS + 1;
       b.item_counter = bw + 3 * FL3_MAX_BINS + 2;
       b.cursor = bw + 3 * FL3_MAX_BINS + 4;
+      b.tile_part = bw + 4 * FL3_MAX_BINS + 4;
+      b.multi = bw + 5 * FL3_MAX_BINS + 4;
       b.sorted = (void *)b1.rec;                                // the walker buffer, free after the band pass
       b.final = (unsigned char *)b1.sorted + rsz * st[t0];      // the band's own range
       if (fl3k_launch_bin_count(&b, narrow, bs) || fl3k_launch_bin(&b, g_ctx.ncu, format, bs)) return 1;
@@ -852,9 +885,9 @@ static int iterate_binned(IterArgs a, long long W, long long Wj, const JobSet &j
    if (ensure_chunk_bufs(nchunks, rec_bytes, sizeof(unsigned) * (size_t)nblk * nsup, sizeof(unsigned) * (size_t)nbins))
       return 1;
    const int nsuper = (nbins + (1 << FL3_SUPER_SHIFT) - 1) >> FL3_SUPER_SHIFT;
-   if (g_ctx.bins.ensure(sizeof(unsigned) * (4 * (size_t)nbins + 8))) return 1;
+   if (g_ctx.bins.ensure(sizeof(unsigned) * (6 * (size_t)nbins + 16))) return 1;
    if (band) {
-      if (g_ctx.bins2.ensure(sizeof(unsigned) * (4 * (size_t)FL3_MAX_BINS + 8))) return 1;
+      if (g_ctx.bins2.ensure(sizeof(unsigned) * (6 * (size_t)FL3_MAX_BINS + 16))) return 1;
       HIPCHK(hipMemsetAsync(g_ctx.bins2.p, 0, sizeof(unsigned) * FL3_MAX_BINS, g_ctx.stream));
    }
    if (g_ctx.soff.ensure(sizeof(unsigned) * (size_t)nblk * nsuper)) return 1;
@@ -873,6 +906,8 @@ static int iterate_binned(IterArgs a, long long W, long long Wj, const JobSet &j
    b.item_start = bw + 2 * nbins + 1;
    b.item_counter = bw + 3 * nbins + 2;
    b.cursor = bw + 3 * nbins + 4;
+   b.tile_part = bw + 4 * nbins + 4;
+   b.multi = bw + 5 * nbins + 4;
    b.soff = (unsigned *)g_ctx.soff.p;
    b.nsuper = nsuper;
    b.shift = wshift;
@@ -895,6 +930,8 @@ static int iterate_binned(IterArgs a, long long W, long long Wj, const JobSet &j
    if (colour) lds_rec = a.pal_off + 1024;
    lds_rec = with_shuffle(a, lds_rec, jobs_wave_ok(js.h, js.n));
    b.round = narrow || colour ? narrow_round(js.h, js.n) : 0;
+   b.alpha = b.round > 0 ? narrow_alpha(js.h, js.n) : -1;
+   if (b.round > 0 && packed_items(&b, W * per)) return 1;
    // chunk k: walkers on the render stream, then its sort and accumulation
    // on the bin stream, which chunk k + 2's walkers wait for before they
    // overwrite the same record buffer
@@ -1243,7 +1280,7 @@ extern "C" int fl3d_iterate_multi(const fl3d_multi_job *jobs, int njobs, int fus
                             sizeof(unsigned) * (size_t)nbins))
          return 1;
       const int nsuper = (nbins + (1 << FL3_SUPER_SHIFT) - 1) >> FL3_SUPER_SHIFT;
-      if (g_ctx.bins.ensure(sizeof(unsigned) * (4 * (size_t)nbins + 8))) return 1;
+      if (g_ctx.bins.ensure(sizeof(unsigned) * (6 * (size_t)nbins + 16))) return 1;
       if (g_ctx.soff.ensure(sizeof(unsigned) * (size_t)nblk * nsuper)) return 1;
       unsigned *bw = (unsigned *)g_ctx.bins.p;
       BinArgs b;
@@ -1258,6 +1295,8 @@ extern "C" int fl3d_iterate_multi(const fl3d_multi_job *jobs, int njobs, int fus
       b.item_start = bw + 2 * nbins + 1;
       b.item_counter = bw + 3 * nbins + 2;
       b.cursor = bw + 3 * nbins + 4;
+      b.tile_part = bw + 4 * nbins + 4;
+      b.multi = bw + 5 * nbins + 4;
       b.soff = (unsigned *)g_ctx.soff.p;
       b.nsuper = nsuper;
       b.shift = shift;
@@ -1286,6 +1325,8 @@ extern "C" int fl3d_iterate_multi(const fl3d_multi_job *jobs, int njobs, int fus
          ar.pal_off = (unsigned)((lds_r + 15) & ~(size_t)15);
          if (colour) lds_r = ar.pal_off + 1024;
          b.round = narrow || colour ? narrow_round(rh.data(), (int)rh.size()) : 0;
+         b.alpha = b.round > 0 ? narrow_alpha(rh.data(), (int)rh.size()) : -1;
+         if (b.round > 0 && packed_items(&b, Wrec * per)) return 1;
       }
       const size_t lds_r_lane = lds_r;
       lds_r = with_shuffle(ar, lds_r, true);

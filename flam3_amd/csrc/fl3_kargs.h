@@ -82,6 +82,7 @@ struct IterArgs {
 
 #define FL3_BIN_CHUNK_SAMPLES (1LL << 28)
 #define FL3_CHUNK_BUFS 2            // record buffers in rotation: the walkers run one chunk ahead of the sort
+#define FL3_PACKED_SHIFT 12          // tiles of the packed accumulation: 4096 cells
 #define FL3_BIN_ITEM_RECORDS (1 << 18)
 #define FL3_BIN_MIN_SAMPLES (1LL << 20)
 
@@ -102,6 +103,10 @@ struct BinArgs {
    long long rows;                 // record rows in this chunk
    unsigned *bin_total;            // [tile] record counts (summed by the walkers)
    unsigned *bin_start, *item_start, *item_counter;
+   // packed accumulation: tiles of several work items (their count first), per
+   // tile the place of its first item among the partial sums, and these
+   unsigned *multi, *tile_part;
+   void *partial;
    // two-pass sort: walker order -> super-tiles of FL3_SUPER tiles (sorted)
    // -> tiles (final, the record buffer reused)
    unsigned *soff;                 // [walker workgroup][super-tile] first slot in sorted
@@ -112,6 +117,7 @@ struct BinArgs {
    int nbins;                      // tiles
    int chunk;                      // records per accumulation work item
    int round;                      // 4-byte records: records per LDS round (0: not packed)
+   int alpha;                      // packed accumulation: the alpha of every palette entry, all below 256 (-1: no such)
    int width, height;
    // job records: palette (floor and float) and xform visibility per job
    const uint32_t *dmapu_all;      // [job][1024]

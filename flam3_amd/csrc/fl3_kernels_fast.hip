@@ -65,17 +65,21 @@ extern "C" int fl3k_launch_apply_fp32(const unsigned char *job, int xi, const do
 #endif
 
 // One workgroup: exclusive scans of the tile counts and of the work items
-// (ceil(count / chunk) per tile).  It also leaves the tile counts at zero
-// for their next use and resets the accumulation's item counter.
+// (ceil(count / chunk) per tile), and the list of the tiles of several items
+// with the place of their first in the array of partial sums.  It also leaves
+// the tile counts at zero for their next use and resets the accumulation's
+// item counter.
 __global__ __launch_bounds__(1024) void k_bin_scan(BinArgs a) {
+   // records | (items of tiles of several) << 32, items | (such tiles) << 32
    __shared__ unsigned long long part[1024], ipart[1024];
    const int t = threadIdx.x, per = (a.nbins + 1023) / 1024;
    if (t == 0) *a.item_counter = 0u;
    const int b0 = t * per, b1 = min(a.nbins, b0 + per);
    unsigned long long s = 0, si = 0;
    for (int b = b0; b < b1; b++) {
-      s += a.bin_total[b];
-      si += (a.bin_total[b] + a.chunk - 1) / a.chunk;
+      const unsigned n = a.bin_total[b], ni = (unsigned)(((unsigned long long)n + a.chunk - 1) / a.chunk);
+      s += n + ((unsigned long long)(ni > 1 ? ni : 0u) << 32);
+      si += ni + ((unsigned long long)(ni > 1) << 32);
    }
    part[t] = s;
    ipart[t] = si;
@@ -89,16 +93,20 @@ __global__ __launch_bounds__(1024) void k_bin_scan(BinArgs a) {
    }
    unsigned long long run = t ? part[t - 1] : 0, irun = t ? ipart[t - 1] : 0;
    for (int b = b0; b < b1; b++) {
+      const unsigned n = a.bin_total[b], ni = (unsigned)(((unsigned long long)n + a.chunk - 1) / a.chunk);
       a.bin_start[b] = (unsigned)run;
       a.cursor[b] = (unsigned)run;
       a.item_start[b] = (unsigned)irun;
-      run += a.bin_total[b];
-      irun += (a.bin_total[b] + a.chunk - 1) / a.chunk;
+      a.tile_part[b] = (unsigned)(run >> 32);
+      if (ni > 1) a.multi[1 + (unsigned)(irun >> 32)] = (unsigned)b;
+      run += n + ((unsigned long long)(ni > 1 ? ni : 0u) << 32);
+      irun += ni + ((unsigned long long)(ni > 1) << 32);
       a.bin_total[b] = 0u;
    }
    if (t == 1023) {
       a.bin_start[a.nbins] = (unsigned)part[1023];
       a.item_start[a.nbins] = (unsigned)ipart[1023];
+      a.multi[0] = (unsigned)(ipart[1023] >> 32);
    }
 }
 
@@ -437,159 +445,222 @@ __global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum(BinArgs a) {
 // Accumulation of records of visibility 1 with a stepped palette (a record
 // adds its palette entry and 255 hits): 4-byte records, or job records that
 // carry the entry's bytes (palettes of entries below 256).  The tile's cells
-// live in LDS as two packed 64-bit words, R:24 | G:24 | count:16 and B:32 | A:32, so a record
-// costs two LDS atomics (and, for 4-byte records, one 16-byte read of its
-// palette entry, kept in LDS in that packed form); a round of at most `round` records keeps every
-// field below its width, after which each thread folds the CPT cells it
-// owns into registers and clears them.  The tile is then added to the
-// histogram from the registers (non-atomic saturating add if the tile has
-// one work item).
-template <int CPT, bool JOB>
+// live in LDS as packed sums, and a round of at most `round` records keeps
+// every field below its width, after which each thread folds the CPT cells it
+// owns into registers and clears them.  The sums of a tile of one work item
+// are then added to the histogram; those of the items of a fuller tile go to an
+// array of partial sums, which k_bin_merge adds up.  (Atomic adds from every
+// item's 20 channels a thread ran at 1e11 a second: 0.2 us an item.)
+// Bound by LDS atomics, so a record makes as few as its fields allow.  RGB:
+// every palette entry is below 256 and has alpha a.alpha, so alpha is a
+// multiple of the count and a cell is R:24 | G:24 | count:16 and B:32 (one
+// 64-bit and one 32-bit atomic, after a 4-byte read of the palette entry for
+// 4-byte records); otherwise R:24 | G:24 | count:16 and B:32 | A:32 (two 64-bit
+// atomics after a 16-byte read).  Per 64 records of a tile, that is 22 against
+// 31 clocks of a CU's LDS.  The next records are loaded while the ones before
+// them are added, and the work item after the next is drawn and the next one
+// looked up meanwhile, so that its first records are under way while this
+// one's sums are stored.
+// At 1920x1080 with 2x2 supersampling (2^28 records of 4 bytes a launch) 606 us
+// with 2^18-record items added by atomics, 470 us so with the merge (LDS active
+// half of the time, 4 TB/s); 256x256 (3.6M records) 94 and 17 us, 640x480
+// (15M) 105 and 48 us; 48 previews' 8-byte records 398 and 339 us.
+#define FL3_ACC_AHEAD 8   // records a thread loads ahead
+// 16-byte words of an item's partial sums: per cell R, G, B, count, then the
+// alphas if they are not a multiple of the count
+__host__ __device__ __forceinline__ size_t part_words(unsigned cells, bool rgb) {
+   return rgb ? cells : cells + cells / 4;
+}
+__device__ __forceinline__ uint32_t add_u32_sat(uint32_t x, uint32_t y) {
+   const uint32_t t = x + y;
+   return t < x ? 0xffffffffu : t;
+}
+template <bool JOB, bool RGB>
 __global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum_narrow(BinArgs a) {
    typedef typename std::conditional<JOB, unsigned long long, unsigned>::type RT;
+   typedef typename std::conditional<RGB, unsigned, unsigned long long>::type PT;
    const fl3_job_hdr *h = (const fl3_job_hdr *)a.job;
-   const int tile_cells = CPT * FL3_ACC_THREADS;
+   constexpr int tile_cells = 1 << FL3_PACKED_SHIFT, CPT = tile_cells / FL3_ACC_THREADS, U = FL3_ACC_AHEAD, step = U * FL3_ACC_THREADS;
    unsigned long long *p0 = (unsigned long long *)fl3_lds;   // tile_cells
-   unsigned long long *p1 = p0 + tile_cells;                  // tile_cells
-   ulonglong2 *pal = (ulonglong2 *)(p1 + tile_cells);          // 256
-   __shared__ int item_sh;
+   PT *p1 = (PT *)(p0 + tile_cells);                           // tile_cells
+   ulonglong2 *pal = (ulonglong2 *)(p1 + tile_cells);          // 256 (RGB: bytes R, G, B)
+   unsigned *pal8 = (unsigned *)pal;
+   // work items, alternating: the one drawn after the next, and of the next its
+   // tile, first record, records, and place among the partial sums + 1 (0: the
+   // tile's only item)
+   __shared__ unsigned drawn[2];
+   __shared__ uint4 found[2];
+   const int tid = threadIdx.x;
    const double *pd = (const double *)(a.job + h->off_dmap);
    if (!JOB)
-      for (int e = threadIdx.x; e < 256; e += blockDim.x) {
+      for (int e = tid; e < 256; e += FL3_ACC_THREADS) {
          const uint32_t r = (uint32_t)pd[4 * e], g = (uint32_t)pd[4 * e + 1], bb = (uint32_t)pd[4 * e + 2], al = (uint32_t)pd[4 * e + 3];
-         ulonglong2 w;
-         w.x = (unsigned long long)r | ((unsigned long long)g << 24) | (1ull << 48);
-         w.y = (unsigned long long)bb | ((unsigned long long)al << 32);
-         pal[e] = w;
+         if (RGB)
+            pal8[e] = r | g << 8 | bb << 16;
+         else {
+            ulonglong2 w;
+            w.x = (unsigned long long)r | ((unsigned long long)g << 24) | (1ull << 48);
+            w.y = (unsigned long long)bb | ((unsigned long long)al << 32);
+            pal[e] = w;
+         }
       }
-   for (int e = threadIdx.x; e < tile_cells; e += blockDim.x) {
+   for (int e = tid; e < tile_cells; e += FL3_ACC_THREADS) {
       p0[e] = 0;
       p1[e] = 0;
    }
-   const long long total_items = a.item_start[a.nbins];
-   const RT *sorted = (const RT *)a.final;
-   const long long step = (long long)FL3_ACC_UNROLL * FL3_ACC_THREADS;
-   for (;;) {
-      __syncthreads();
-      if (threadIdx.x == 0) item_sh = (int)atomicAdd(a.item_counter, 1u);
-      __syncthreads();
-      const long long item = item_sh;
-      if (item >= total_items) break;
-      int lo = 0, hi = a.nbins - 1;
-      while (lo < hi) {  // last tile whose first item is <= item
-         const int mid = (lo + hi + 1) >> 1;
-         if ((long long)a.item_start[mid] <= item) lo = mid;
-         else hi = mid - 1;
-      }
-      const int b = lo;
-      const long long k = item - a.item_start[b];
-      const long long r0 = (long long)a.bin_start[b] + k * a.chunk;
-      const long long r1 = min((long long)a.bin_start[b + 1], r0 + a.chunk);
-      const bool single = (a.item_start[b + 1] - a.item_start[b]) == 1;
-      const unsigned cell0 = a.cell_base + ((unsigned)b << a.shift);
-      uint32_t acc[CPT][5];
-      for (int j = 0; j < CPT; j++)
-         for (int c = 0; c < 5; c++) acc[j][c] = 0;
-      for (long long rs = r0; rs < r1; rs += a.round) {
-         const long long re = min(rs + a.round, r1);
-         for (long long rb = rs; rb < re; rb += step) {
-            RT v[FL3_ACC_UNROLL];
-            for (int u = 0; u < FL3_ACC_UNROLL; u++) {
-               const long long r = rb + u * FL3_ACC_THREADS + threadIdx.x;
-               v[u] = r < re ? sorted[r] : (RT)FL3_REC_NONE;
-            }
-            for (int u = 0; u < FL3_ACC_UNROLL; u++) {
-               if ((unsigned)v[u] == FL3_REC_NONE) continue;
-               // 4-byte record: cell | palette index << 24; job record: cell
-               // | the palette entry's bytes R, G, B, A << 32
-               if (JOB) {
-                  const unsigned local = (unsigned)v[u] - cell0;
-                  const unsigned c = (unsigned)(v[u] >> 32);
-                  atomicAdd(&p0[local], (unsigned long long)(c & 0xffu) | ((unsigned long long)((c >> 8) & 0xffu) << 24) |
-                                            (1ull << 48));
-                  atomicAdd(&p1[local], (unsigned long long)((c >> 16) & 0xffu) | ((unsigned long long)(c >> 24) << 32));
-               } else {
-                  const unsigned local = ((unsigned)v[u] & 0xffffffu) - cell0;
-                  const ulonglong2 w = pal[(unsigned)v[u] >> 24];
-                  atomicAdd(&p0[local], w.x);
-                  atomicAdd(&p1[local], w.y);
-               }
-            }
+   const unsigned total_items = a.item_start[a.nbins];
+   const int round_steps = a.round / step;
+   auto look_up = [&](unsigned item, int slot) {
+      for (int b = tid; b < a.nbins; b += FL3_ACC_THREADS) {
+         const unsigned i0 = a.item_start[b], i1 = a.item_start[b + 1], r0 = a.bin_start[b], r1 = a.bin_start[b + 1];
+         const unsigned p = a.tile_part[b];
+         if (i0 <= item && item < i1) {
+            const unsigned k = item - i0, first = r0 + k * (unsigned)a.chunk;
+            found[slot] = make_uint4((unsigned)b, first, min(r1 - first, (unsigned)a.chunk), i1 - i0 == 1 ? 0u : p + k + 1u);
          }
+      }
+   };
+   // (the first two items of a workgroup are its own, the others drawn)
+   unsigned item = blockIdx.x, next = gridDim.x + blockIdx.x;
+   if (item >= total_items) return;
+   look_up(item, 0);
+   __syncthreads();
+   auto in_item = [&](int slot, int c) { return __builtin_amdgcn_readfirstlane(((const unsigned *)&found[slot])[c]); };
+   unsigned b = in_item(0, 0), first = in_item(0, 1), place = in_item(0, 3);
+   int n = (int)in_item(0, 2);
+   auto fetch = [&](RT(&v)[U], int at) {
+      const RT *in = (const RT *)a.final + first;
+      for (int u = 0; u < U; u++) v[u] = in[min(at + u * FL3_ACC_THREADS + tid, n - 1)];
+   };
+   RT v[U], nx[U];
+   fetch(nx, 0);
+   for (int slot = 1;; slot ^= 1) {
+      const unsigned cell0 = a.cell_base + (b << a.shift), place_now = place;
+      unsigned draw = 0;
+      if (tid == 0) draw = 2u * gridDim.x + atomicAdd(a.item_counter, 1u);
+      if (next < total_items) look_up(next, slot);
+      uint32_t acc[CPT][RGB ? 4 : 5];
+      for (int j = 0; j < CPT; j++)
+         for (int c = 0; c < (RGB ? 4 : 5); c++) acc[j][c] = 0;
+      auto add = [&](RT v) {
+         const unsigned local = (unsigned)v & (unsigned)(tile_cells - 1);   // (a tile starts at a multiple of its cells)
+         if (RGB) {
+            const unsigned c = JOB ? (unsigned)((unsigned long long)v >> 32) : pal8[(unsigned)v >> 24];
+            atomicAdd(&p0[local], (unsigned long long)((c & 0xffu) | (c >> 8) << 24) | 1ull << 48);
+            atomicAdd(&p1[local], (PT)((c >> 16) & 0xffu));
+         } else if (JOB) {
+            const unsigned c = (unsigned)((unsigned long long)v >> 32);
+            atomicAdd(&p0[local], (unsigned long long)(c & 0xffu) | ((unsigned long long)((c >> 8) & 0xffu) << 24) | (1ull << 48));
+            atomicAdd(&p1[local], (PT)((unsigned long long)((c >> 16) & 0xffu) | ((unsigned long long)(c >> 24) << 32)));
+         } else {
+            const ulonglong2 w = pal[(unsigned)v >> 24];
+            atomicAdd(&p0[local], w.x);
+            atomicAdd(&p1[local], (PT)w.y);
+         }
+      };
+      for (int at = 0, steps = 0; at < n; at += step) {
+         for (int u = 0; u < U; u++) v[u] = nx[u];
+         if (at + step < n) fetch(nx, at + step);
+         if (at + step <= n)
+            for (int u = 0; u < U; u++) add(v[u]);
+         else
+            for (int u = 0; u < U; u++)
+               if (at + u * FL3_ACC_THREADS + tid < n) add(v[u]);
+         if (++steps < round_steps && at + step < n) continue;
+         steps = 0;
+         if (tid == 0) drawn[slot] = draw;
          __syncthreads();
          for (int j = 0; j < CPT; j++) {
-            const int e = threadIdx.x + j * FL3_ACC_THREADS;
-            const unsigned long long x0 = p0[e], x1 = p1[e];
+            const int e = tid + j * FL3_ACC_THREADS;
+            const unsigned long long x0 = p0[e];
+            const PT x1 = p1[e];
             p0[e] = 0;
             p1[e] = 0;
             acc[j][0] += (uint32_t)(x0 & 0xffffffu);
             acc[j][1] += (uint32_t)((x0 >> 24) & 0xffffffu);
             acc[j][2] += (uint32_t)x1;
-            acc[j][3] += (uint32_t)(x1 >> 32);
-            acc[j][4] += 255u * (uint32_t)(x0 >> 48);
+            acc[j][3] += (uint32_t)(x0 >> 48);
+            if (!RGB) acc[j][RGB ? 0 : 4] += (uint32_t)((unsigned long long)x1 >> 32);
          }
          __syncthreads();
       }
-      uint32_t *bk = (uint32_t *)a.buckets + (size_t)cell0 * 5;
-      const long long ncells = (long long)a.width * a.height;
-      const int nvalid = (int)min((long long)tile_cells, ncells - (long long)cell0);
-      // every load (or atomic add) of the thread's cells is issued before
-      // any result is used, so that their latencies overlap
-      uint32_t old[CPT][5];
-      if (nvalid == tile_cells) {
-         // (a tile inside the histogram: straight-line code over all its
-         // cells, so that no store waits for an earlier one; a tile of one
-         // work item owns its cells, and adding zero leaves a cell as it is)
-         uint32_t *bt = bk + (size_t)threadIdx.x * 5;
-         if (single) {
-            for (int j = 0; j < CPT; j++)
-               for (int c = 0; c < 5; c++) old[j][c] = bt[(size_t)j * FL3_ACC_THREADS * 5 + c];
-            for (int j = 0; j < CPT; j++)
-               for (int c = 0; c < 5; c++) {
-                  const unsigned long long s2 = (unsigned long long)old[j][c] + acc[j][c];
-                  old[j][c] = s2 > 0xffffffffull ? 0xffffffffu : (uint32_t)s2;
-               }
-            for (int j = 0; j < CPT; j++)
-               for (int c = 0; c < 5; c++) bt[(size_t)j * FL3_ACC_THREADS * 5 + c] = old[j][c];
-         } else {
-            for (int j = 0; j < CPT; j++)
-               for (int c = 0; c < 5; c++) old[j][c] = atomicAdd(bt + (size_t)j * FL3_ACC_THREADS * 5 + c, acc[j][c]);
-            for (int j = 0; j < CPT; j++)
-               for (int c = 0; c < 5; c++)
-                  if (old[j][c] > 0xffffffffu - acc[j][c])
-                     atomicExch(bt + (size_t)j * FL3_ACC_THREADS * 5 + c, 0xffffffffu);
+      const bool more = next < total_items;
+      if (more) {
+         b = in_item(slot, 0);
+         first = in_item(slot, 1);
+         n = (int)in_item(slot, 2);
+         place = in_item(slot, 3);
+         fetch(nx, 0);
+      }
+      next = __builtin_amdgcn_readfirstlane(drawn[slot]);
+      if (place_now) {
+         uint4 *out = (uint4 *)a.partial + (size_t)(place_now - 1) * part_words(tile_cells, RGB);
+         for (int j = 0; j < CPT; j++) {
+            const int e = tid + j * FL3_ACC_THREADS;
+            out[e] = make_uint4(acc[j][0], acc[j][1], acc[j][2], acc[j][3]);
+            if (!RGB) ((unsigned *)(out + tile_cells))[e] = acc[j][RGB ? 0 : 4];
          }
-      } else if (single) {
+      } else {
+         uint32_t *bk = (uint32_t *)a.buckets + (size_t)cell0 * 5;
+         const int nvalid = (int)min((long long)tile_cells, (long long)a.width * a.height - (long long)cell0);
+         // every load of the thread's cells is issued before any result is
+         // used, so that their latencies overlap (adding zero leaves a cell as
+         // it is, and the tile is this workgroup's alone)
+         uint32_t sum[CPT][5], old[CPT][5];
+         for (int j = 0; j < CPT; j++) {
+            for (int c = 0; c < 3; c++) sum[j][c] = acc[j][c];
+            sum[j][3] = RGB ? acc[j][3] * (unsigned)a.alpha : acc[j][RGB ? 0 : 4];
+            sum[j][4] = acc[j][3] * 255u;
+         }
          for (int j = 0; j < CPT; j++)
             for (int c = 0; c < 5; c++) {
-               const int e = threadIdx.x + j * FL3_ACC_THREADS;
-               old[j][c] = e < nvalid && acc[j][c] ? bk[(size_t)e * 5 + c] : 0u;
+               const int e = tid + j * FL3_ACC_THREADS;
+               old[j][c] = e < nvalid ? bk[(size_t)e * 5 + c] : 0u;
             }
          // (the sums first, each in a register of its own, so that no store
          // waits for an earlier one to release its data register)
          for (int j = 0; j < CPT; j++)
-            for (int c = 0; c < 5; c++) {
-               const unsigned long long s2 = (unsigned long long)old[j][c] + acc[j][c];
-               old[j][c] = s2 > 0xffffffffull ? 0xffffffffu : (uint32_t)s2;
-            }
+            for (int c = 0; c < 5; c++) old[j][c] = add_u32_sat(old[j][c], sum[j][c]);
          for (int j = 0; j < CPT; j++)
             for (int c = 0; c < 5; c++) {
-               const int e = threadIdx.x + j * FL3_ACC_THREADS;
-               if (e < nvalid && acc[j][c]) bk[(size_t)e * 5 + c] = old[j][c];
+               const int e = tid + j * FL3_ACC_THREADS;
+               if (e < nvalid) bk[(size_t)e * 5 + c] = old[j][c];
             }
-      } else {
-         for (int j = 0; j < CPT; j++)
-            for (int c = 0; c < 5; c++) {
-               const int e = threadIdx.x + j * FL3_ACC_THREADS;
-               old[j][c] = e < nvalid && acc[j][c] ? atomicAdd(bk + (size_t)e * 5 + c, acc[j][c]) : 0u;
-            }
-         // (a saturating add: the sum stops at UINT_MAX, as sat_add)
-         for (int j = 0; j < CPT; j++)
-            for (int c = 0; c < 5; c++) {
-               const int e = threadIdx.x + j * FL3_ACC_THREADS;
-               const uint32_t v = acc[j][c];
-               if (e < nvalid && v && old[j][c] > 0xffffffffu - v) atomicExch(bk + (size_t)e * 5 + c, 0xffffffffu);
-            }
+      }
+      if (!more) break;
+   }
+}
+
+// Adds up the partial sums of the tiles of several work items and adds them
+// to the histogram: a workgroup takes 256 cells of a tile at a time.
+template <bool RGB>
+__global__ __launch_bounds__(256) void k_bin_merge(BinArgs a) {
+   const unsigned cells = 1u << a.shift, parts = cells / 256, units = a.multi[0] * parts;
+   const size_t words = part_words(cells, RGB);
+   for (unsigned u = blockIdx.x; u < units; u += gridDim.x) {
+      const unsigned b = a.multi[1 + u / parts], e = u % parts * 256 + threadIdx.x;
+      const unsigned n = a.item_start[b + 1] - a.item_start[b];
+      const uint4 *in = (const uint4 *)a.partial + (size_t)a.tile_part[b] * words;
+      const size_t cell = (size_t)a.cell_base + ((size_t)b << a.shift) + e;
+      unsigned long long sum[5] = {0, 0, 0, 0, 0};
+#pragma unroll 4
+      for (unsigned i = 0; i < n; i++) {
+         const uint4 v = in[i * words + e];
+         sum[0] += v.x;
+         sum[1] += v.y;
+         sum[2] += v.z;
+         sum[4] += v.w;
+         if (!RGB) sum[3] += ((const unsigned *)(in + i * words + cells))[e];
+      }
+      if (cell >= (size_t)a.width * a.height) continue;
+      if (RGB) sum[3] = sum[4] * (unsigned)a.alpha;
+      sum[4] *= 255u;
+      uint32_t *bk = (uint32_t *)a.buckets + cell * 5;
+      uint32_t old[5];
+      for (int c = 0; c < 5; c++) old[c] = bk[c];
+      for (int c = 0; c < 5; c++) {
+         const unsigned long long t = old[c] + sum[c];
+         bk[c] = t > 0xffffffffull ? 0xffffffffu : (uint32_t)t;
       }
    }
 }
@@ -753,8 +824,23 @@ __global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum_f64(BinArgs a) {
 
 extern "C" size_t fl3k_bin_f64_lds_bytes(int shift) { return (size_t)40 * ((size_t)1 << shift) + 8 * (1024 + 1024 + 256) + 64; }
 
-extern "C" size_t fl3k_bin_narrow_lds_bytes(int shift) { return (size_t)16 * ((size_t)1 << shift) + 4 * 1024 + 64; }
-extern "C" int fl3k_bin_pass_records(void) { return FL3_ACC_UNROLL * FL3_ACC_THREADS; }
+extern "C" int fl3k_bin_pass_records(void) { return FL3_ACC_AHEAD * FL3_ACC_THREADS; }
+template <bool JOB, bool RGB>
+static void launch_narrow(const BinArgs *a, int ncu, hipStream_t s) {
+   const size_t cells = (size_t)1 << FL3_PACKED_SHIFT;
+   const size_t lds = RGB ? 12 * cells + 1024 : 16 * cells + 4096;
+   if (lds > 65536)
+      (void)hipFuncSetAttribute((const void *)k_bin_accum_narrow<JOB, RGB>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+   hipLaunchKernelGGL((k_bin_accum_narrow<JOB, RGB>), dim3(2u * (unsigned)ncu), dim3(FL3_ACC_THREADS), lds, s, *a);
+   hipLaunchKernelGGL((k_bin_merge<RGB>), dim3(8u * (unsigned)ncu), dim3(256), 0, s, *a);
+}
+// Bytes of the packed accumulation's partial sums for `records` in a chunk
+// (a tile of several items has more than an item's records, so at most two
+// items for every item's worth of records).
+extern "C" size_t fl3k_bin_partial_bytes(const BinArgs *a, long long records) {
+   return 16 * part_words(1u << a->shift, a->alpha >= 0) * (size_t)(2 * records / a->chunk + 1);
+}
 
 extern "C" size_t fl3k_bin_lds_bytes(int shift) {
    return (size_t)20 * ((size_t)1 << shift) + 8 * 1024 + 4 * 256 + 64;
@@ -769,7 +855,6 @@ extern "C" int fl3k_launch_bin(const BinArgs *a, int ncu, int format, hipStream_
    const size_t lds = fl3k_bin_lds_bytes(a->shift);
    const unsigned gacc = (unsigned)ncu * (lds > 65536 ? 1 : 3);
    const int big = lds > 65536;
-   const int cpt = (1 << a->shift) / FL3_ACC_THREADS;
    if (format == FL3_BIN_F64_WIDE || format == FL3_BIN_F64_NARROW) {
       // double buckets: 8- or 4-byte records, accumulated in double
       const size_t lf = fl3k_bin_f64_lds_bytes(a->shift);
@@ -794,7 +879,7 @@ extern "C" int fl3k_launch_bin(const BinArgs *a, int ncu, int format, hipStream_
       }
       return hipGetLastError() != hipSuccess;
    }
-   if ((format == 1 || format == 2) && a->round > 0 && (cpt == 2 || cpt == 4)) {
+   if ((format == 1 || format == 2) && a->round > 0 && a->shift == FL3_PACKED_SHIFT) {
       const bool job = format == 2;
       if (job) {
          hipLaunchKernelGGL(k_bin_part1<unsigned long long>, dim3(a->nblk), dim3(256), 0, s, *a);
@@ -806,19 +891,11 @@ extern "C" int fl3k_launch_bin(const BinArgs *a, int ncu, int format, hipStream_
             hipLaunchKernelGGL(k_bin_part1<unsigned>, dim3(a->nblk), dim3(256), 0, s, *a);
          if (g2) hipLaunchKernelGGL(k_bin_part2<unsigned>, dim3(g2), dim3(256), lds2_4, s, *a);
       }
-      const size_t ln = fl3k_bin_narrow_lds_bytes(a->shift);
-      const unsigned gn = (unsigned)ncu * (ln > 65536 ? 2 : 3);
-      const void *kf = job ? (cpt == 4 ? (const void *)k_bin_accum_narrow<4, true> : (const void *)k_bin_accum_narrow<2, true>)
-                           : (cpt == 4 ? (const void *)k_bin_accum_narrow<4, false> : (const void *)k_bin_accum_narrow<2, false>);
-      if (ln > 65536) (void)hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ln);
-      if (job && cpt == 4)
-         hipLaunchKernelGGL((k_bin_accum_narrow<4, true>), dim3(gn), dim3(FL3_ACC_THREADS), ln, s, *a);
-      else if (job)
-         hipLaunchKernelGGL((k_bin_accum_narrow<2, true>), dim3(gn), dim3(FL3_ACC_THREADS), ln, s, *a);
-      else if (cpt == 4)
-         hipLaunchKernelGGL((k_bin_accum_narrow<4, false>), dim3(gn), dim3(FL3_ACC_THREADS), ln, s, *a);
+      const bool rgb = a->alpha >= 0;
+      if (job)
+         rgb ? launch_narrow<true, true>(a, ncu, s) : launch_narrow<true, false>(a, ncu, s);
       else
-         hipLaunchKernelGGL((k_bin_accum_narrow<2, false>), dim3(gn), dim3(FL3_ACC_THREADS), ln, s, *a);
+         rgb ? launch_narrow<false, true>(a, ncu, s) : launch_narrow<false, false>(a, ncu, s);
    } else if (format == 1) {
       if (a->rows >= FL3_PART1_STAGED_ROWS)
          hipLaunchKernelGGL(k_bin_part1_staged<unsigned>, dim3(a->nblk), dim3(256), 0, s, *a);

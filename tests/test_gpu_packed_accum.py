@@ -1,0 +1,59 @@
+"""The packed accumulation of tile-sorted records (partial sums of the work
+items of a full tile, alpha as a multiple of the count where the palettes
+allow it) against per-sample atomics: the same integers, so the same image."""
+import numpy as np
+import pytest
+
+from flam3_amd import genome as G
+
+pytestmark = pytest.mark.gpu
+
+
+class _Shaded(G.Genome):
+    """Palette entries of one alpha below 1, of differing alphas, or of values
+    that bytes don't hold."""
+    shade = "bytes"
+
+    def to_struct(self):
+        gp = super().to_struct()
+        for i in range(256):
+            c = gp.contents.palette[i].color
+            if self.shade == "veiled":
+                c[3] = 0.3
+            elif self.shade == "alpha":
+                c[3] = (i % 7) / 6.0
+            elif self.shade == "bright":
+                for k in range(3):
+                    c[k] *= 3.0
+        return gp
+
+
+def _shaded(g, shade):
+    g.__class__ = _Shaded
+    g.shade = shade
+    g.estimator_radius = 0.0
+    return g
+
+
+@pytest.mark.parametrize("shade", ["bytes", "veiled", "alpha", "bright"])
+@pytest.mark.parametrize("size,quality,walkers,chunk", [
+    ((64, 64), 300, 1024, 1024 * 700),      # one tile, many items
+    ((64, 65), 260, 256, 256 * 64),         # items of exactly a chunk's records and a ragged last tile
+    ((640, 481), 4, 1024, 0),               # sparse tiles of one item
+    ((333, 217), 90, 2048, 2048 * 2000)])   # both, over chunks
+def test_packed_accumulation_equals_atomics(prod, shade, size, quality, walkers, chunk):
+    g = _shaded(G.synthetic_small(seed=40, width=size[0], height=size[1], quality=quality), shade)
+    a, _ = prod.render(g, seed="acc", nwalkers=walkers, deposit=1, nchan=4, transp=1)
+    b, _ = prod.render(g, seed="acc", nwalkers=walkers, deposit=2, chunk_samples=chunk, nchan=4, transp=1)
+    assert np.array_equal(a, b)
+    assert a[..., :3].mean() > 1.0
+
+
+@pytest.mark.parametrize("shades", [("bytes", "bytes", "bytes"), ("bytes", "veiled", "alpha"),
+                                    ("bytes", "bright", "veiled")])
+def test_renders_of_several_palettes_together(prod, shades):
+    items = [{"genomes": _shaded(G.synthetic_preview(60 + k, size=s, quality=60), sh), "seed": "p%d" % k, "nchan": 4,
+              "transp": 1} for k, (s, sh) in enumerate(zip((64, 200, 129), shades))]
+    for it, (img, _) in zip(items, prod.render_many(items)):
+        want, _ = prod.render(it["genomes"], seed=it["seed"], nchan=4, transp=1, deposit=1)
+        assert np.array_equal(img, want), it["seed"]
