@@ -64,6 +64,45 @@ extern "C" const char *fl3h_last_error(void) { return g_err; }
 #define FL3_IMAGE_STRIPS 4
 #define FL3_STRIP_MIN_BYTES (2u << 20)
 
+// Pinned host memory that a call fills and copies to the device without
+// waiting: the copy after it waits, on the host, until the one before has left
+// the memory.  (2 MB of jobs through a new std::vector took 690 us, page faults
+// and the runtime's own staging most of it.)  It grows to the largest set of
+// jobs, as their device buffer does.
+struct PinBuf {
+   unsigned char *p = nullptr;
+   size_t cap = 0;
+   hipEvent_t left = nullptr;
+   bool sent = false;
+   unsigned char *take(size_t bytes) {
+      if (sent && hipEventSynchronize(left) != hipSuccess) return nullptr;
+      sent = false;
+      if (bytes > cap) {
+         if (p) (void)hipHostFree(p);
+         cap = 0;
+         p = nullptr;
+         const size_t want = bytes + bytes / 2;
+         if (hipHostMalloc((void **)&p, want, hipHostMallocDefault) != hipSuccess) {
+            snprintf(g_err, sizeof(g_err), "hipHostMalloc of %zu bytes failed", want);
+            (void)hipGetLastError();
+            p = nullptr;
+            return nullptr;
+         }
+         cap = want;
+      }
+      return p;
+   }
+   int send(void *dev, size_t bytes, hipStream_t s) {
+      if ((!left && hipEventCreateWithFlags(&left, hipEventDisableTiming) != hipSuccess) ||
+          hipMemcpyAsync(dev, p, bytes, hipMemcpyHostToDevice, s) != hipSuccess || hipEventRecord(left, s) != hipSuccess) {
+         snprintf(g_err, sizeof(g_err), "copy of %zu bytes from pinned memory failed", bytes);
+         return 1;
+      }
+      sent = true;
+      return 0;
+   }
+};
+
 struct DevBuf {
    void *p = nullptr;
    size_t cap = 0;
@@ -120,6 +159,7 @@ struct Ctx {
    hipEvent_t ev_band = nullptr;
    hipEvent_t ev_strip[FL3_IMAGE_STRIPS] = {};   // fl3d_images_fetch: strip k of the image is in staging
    unsigned long long *counters = nullptr;   // [0] badvals, [1] saturation flag
+   PinBuf job_pin, tab_pin;                   // jobs, and their tables, on the way to the device
    void *staging = nullptr;                   // pinned host buffer for the image download
    size_t staging_cap = 0;
    void *slot[2] = {nullptr, nullptr};        // pinned buffers of fl3d_images_download
@@ -624,6 +664,14 @@ static bool same_narrow_tables(const fl3_job_hdr *a, const fl3_job_hdr *b) {
    if (!narrow_records_ok(a, 0) || !narrow_records_ok(b, 0)) return false;
    const double *da = (const double *)((const unsigned char *)a + a->off_dmap);
    const double *db = (const double *)((const unsigned char *)b + b->off_dmap);
+   // (without an exit, and in 32-bit integers where they hold the entries, four
+   // entries at a time: 100 jobs took 130 us one by one)
+   int differ = 0, wide = 0;
+   for (int e = 0; e < 1024; e++) {
+      wide |= !(da[e] > -1.0 && da[e] < 2147483648.0) | !(db[e] > -1.0 && db[e] < 2147483648.0);
+      differ |= (int)da[e] ^ (int)db[e];
+   }
+   if (!wide) return differ == 0;
    for (int e = 0; e < 1024; e++)
       if ((uint32_t)da[e] != (uint32_t)db[e]) return false;
    return true;
@@ -640,8 +688,12 @@ extern "C" int fl3d_jobs_share_palette(const void *job0, const void *job) {
 static int upload_job_tables(const fl3_job_hdr *const *h, int n, int nxf_max, BinArgs *b,
                              const uint32_t **pal8 = nullptr) {
    const int vs = nxf_max > 0 ? nxf_max : 1;
-   std::vector<uint32_t> du((size_t)n * 1024), pb((size_t)n * 256);
-   std::vector<float> df((size_t)n * 1024), vis((size_t)n * vs, 1.0f);
+   const size_t nb = (size_t)n * 4096, vb = (size_t)n * vs * 4, pbb = (size_t)n * 1024;
+   if (g_ctx.jobtab.ensure(2 * nb + vb + pbb)) return 1;
+   unsigned char *host = g_ctx.tab_pin.take(2 * nb + vb + pbb);
+   if (!host) return 1;
+   uint32_t *du = (uint32_t *)host, *pb = (uint32_t *)(host + 2 * nb + vb);
+   float *df = (float *)(host + nb), *vis = (float *)(host + 2 * nb);
    bool bytes = true;
    for (int j = 0; j < n; j++) {
       const unsigned char *hb = (const unsigned char *)h[j];
@@ -656,21 +708,15 @@ static int upload_job_tables(const fl3_job_hdr *const *h, int n, int nxf_max, Bi
          const uint32_t *c = &du[(size_t)j * 1024 + 4 * e];
          pb[(size_t)j * 256 + e] = (c[0] & 0xffu) | (c[1] & 0xffu) << 8 | (c[2] & 0xffu) << 16 | (c[3] & 0xffu) << 24;
       }
-      for (int e = 0; e < h[j]->nxf; e++) vis[(size_t)j * vs + e] = (float)px[e].vis;
+      for (int e = 0; e < vs; e++) vis[(size_t)j * vs + e] = e < h[j]->nxf ? (float)px[e].vis : 1.0f;
    }
-   const size_t nb = du.size() * 4, fb = df.size() * 4, vb = vis.size() * 4, pbb = pb.size() * 4;
-   if (g_ctx.jobtab.ensure(nb + fb + vb + pbb)) return 1;
    unsigned char *t = (unsigned char *)g_ctx.jobtab.p;
-   HIPCHK(hipMemcpyAsync(t, du.data(), nb, hipMemcpyHostToDevice, g_ctx.stream));
-   HIPCHK(hipMemcpyAsync(t + nb, df.data(), fb, hipMemcpyHostToDevice, g_ctx.stream));
-   HIPCHK(hipMemcpyAsync(t + nb + fb, vis.data(), vb, hipMemcpyHostToDevice, g_ctx.stream));
-   HIPCHK(hipMemcpyAsync(t + nb + fb + vb, pb.data(), pbb, hipMemcpyHostToDevice, g_ctx.stream));
-   HIPCHK(hipStreamSynchronize(g_ctx.stream));  // the host vectors go out of scope
+   if (g_ctx.tab_pin.send(t, 2 * nb + vb + pbb, g_ctx.stream)) return 1;
    b->dmapu_all = (const uint32_t *)t;
    b->dmapf_all = (const float *)(t + nb);
-   b->vis_all = (const float *)(t + nb + fb);
+   b->vis_all = (const float *)(t + 2 * nb);
    b->vis_stride = vs;
-   if (pal8) *pal8 = bytes ? (const uint32_t *)(t + nb + fb + vb) : nullptr;
+   if (pal8) *pal8 = bytes ? (const uint32_t *)(t + 2 * nb + vb) : nullptr;
    return 0;
 }
 
@@ -851,12 +897,13 @@ static int iterate_binned(IterArgs a, long long W, long long Wj, const JobSet &j
    const int wshift = band ? band - FL3_SUPER_SHIFT : shift;   // the walkers' counting tiles
    const int nbins = (int)((ncells + (1LL << wshift) - 1) >> wshift);
    bool narrow = !band && narrow_records_ok(js.h[0], ncells);
-   for (int j = 1; narrow && j < js.n; j++) narrow = same_narrow_tables(js.h[0], js.h[j]);
+   for (int j = 1; narrow && !js.same_tables && j < js.n; j++) narrow = same_narrow_tables(js.h[0], js.h[j]);
    // double buckets of a banded histogram: the walkers write 8-byte records,
    // the band pass 4-byte ones (cells within a 2^24-cell band) when the
    // tables allow
    bool band_narrow = band == 24 && g_ctx.bits == 64 && narrow_records_ok(js.h[0], -1);
-   for (int j = 1; band_narrow && j < js.n; j++) band_narrow = same_narrow_tables(js.h[0], js.h[j]);
+   for (int j = 1; band_narrow && !js.same_tables && j < js.n; j++)
+      band_narrow = same_narrow_tables(js.h[0], js.h[j]);
    // one palette for all jobs: narrow or wide records; else the job index
    // rides in the record (step palettes only: it takes the fraction's bits);
    // double buckets take narrow or wide records
@@ -914,7 +961,9 @@ static int iterate_binned(IterArgs a, long long W, long long Wj, const JobSet &j
    b.nbins = nbins;
    b.width = g_ctx.width;
    b.height = g_ctx.height;
-   b.chunk = item_records(js.h, js.n, format >= FL3_BIN_F64_WIDE);
+   // (jobs of 4-byte records have the first one's palette integers)
+   const int npal = narrow || band_narrow ? 1 : js.n;
+   b.chunk = item_records(js.h, npal, format >= FL3_BIN_F64_WIDE);
    const uint32_t *pal8 = nullptr;
    if (format == 2 && upload_job_tables(js.h, js.n, js.nxf_max, &b, &pal8)) return 1;
    a.rec_mode = narrow ? 2 : (format == 2 ? 3 : 1);
@@ -929,8 +978,8 @@ static int iterate_binned(IterArgs a, long long W, long long Wj, const JobSet &j
    a.pal_off = (unsigned)((lds_rec + 15) & ~(size_t)15);
    if (colour) lds_rec = a.pal_off + 1024;
    lds_rec = with_shuffle(a, lds_rec, jobs_wave_ok(js.h, js.n));
-   b.round = narrow || colour ? narrow_round(js.h, js.n) : 0;
-   b.alpha = b.round > 0 ? narrow_alpha(js.h, js.n) : -1;
+   b.round = narrow || colour ? narrow_round(js.h, npal) : 0;
+   b.alpha = b.round > 0 ? narrow_alpha(js.h, npal) : -1;
    if (b.round > 0 && packed_items(&b, W * per)) return 1;
    // chunk k: walkers on the render stream, then its sort and accumulation
    // on the bin stream, which chunk k + 2's walkers wait for before they
@@ -1022,10 +1071,11 @@ extern "C" int fl3d_iterate_batch(const void *const *jobs, const size_t *job_byt
       // after the jobs: byte offsets, walker keys and (if given) sample counts
       const size_t tab = sizeof(long long) * njobs + sizeof(uint64_t) * 2 * njobs +
                          (p->job_nsamples ? sizeof(long long) * njobs : 0);
-      std::vector<unsigned char> host(total + tab);
-      for (int j = 0; j < njobs; j++) memcpy(host.data() + off[j], jobs[j], job_bytes[j]);
-      memcpy(host.data() + total, off.data(), sizeof(long long) * njobs);
-      memcpy(host.data() + total + sizeof(long long) * njobs, keys, sizeof(uint64_t) * 2 * njobs);
+      unsigned char *host = g_ctx.job_pin.take(total + tab);
+      if (!host) return 1;
+      for (int j = 0; j < njobs; j++) memcpy(host + off[j], jobs[j], job_bytes[j]);
+      memcpy(host + total, off.data(), sizeof(long long) * njobs);
+      memcpy(host + total + sizeof(long long) * njobs, keys, sizeof(uint64_t) * 2 * njobs);
       if (p->job_nsamples)
          for (int j = 0; j < njobs; j++) {
             if (p->job_nsamples[j] < 0 || p->job_nsamples[j] > p->nsamples) {
@@ -1033,12 +1083,11 @@ extern "C" int fl3d_iterate_batch(const void *const *jobs, const size_t *job_byt
                return 1;
             }
             const long long v = p->job_nsamples[j];
-            memcpy(host.data() + total + (sizeof(long long) + 2 * sizeof(uint64_t)) * njobs + sizeof(long long) * j,
+            memcpy(host + total + (sizeof(long long) + 2 * sizeof(uint64_t)) * njobs + sizeof(long long) * j,
                    &v, sizeof(long long));
          }
       if (g_ctx.job.ensure(total + tab)) return 1;
-      HIPCHK(hipMemcpyAsync(g_ctx.job.p, host.data(), total + tab, hipMemcpyHostToDevice, g_ctx.stream));
-      HIPCHK(hipStreamSynchronize(g_ctx.stream));  // host is a local buffer
+      if (g_ctx.job_pin.send(g_ctx.job.p, total + tab, g_ctx.stream)) return 1;
       js.dev_all = (const unsigned char *)g_ctx.job.p;
       js.dev_off = (const long long *)(js.dev_all + total);
       js.dev_keys = (const unsigned long long *)(js.dev_all + total + sizeof(long long) * njobs);
@@ -1213,12 +1262,13 @@ extern "C" int fl3d_iterate_multi(const fl3d_multi_job *jobs, int njobs, int fus
    for (int j = 0; j < njobs; j++)
       for (int b = 0; b < d[j].nblocks; b++) blk[(size_t)(gstart[grp[j]] + d[j].block0 + b)] = j;
    const size_t dbytes = sizeof(JobDesc) * njobs, bbytes = sizeof(int) * (size_t)blocks;
-   std::vector<unsigned char> host(total + dbytes + bbytes);
-   for (int j = 0; j < njobs; j++) memcpy(host.data() + d[j].off, jobs[j].job, jobs[j].bytes);
-   memcpy(host.data() + total, d.data(), dbytes);
-   memcpy(host.data() + total + dbytes, blk.data(), bbytes);
-   if (g_ctx.job.ensure(host.size())) return 1;
-   HIPCHK(hipMemcpyAsync(g_ctx.job.p, host.data(), host.size(), hipMemcpyHostToDevice, g_ctx.stream));
+   if (g_ctx.job.ensure(total + dbytes + bbytes)) return 1;
+   unsigned char *host = g_ctx.job_pin.take(total + dbytes + bbytes);
+   if (!host) return 1;
+   for (int j = 0; j < njobs; j++) memcpy(host + d[j].off, jobs[j].job, jobs[j].bytes);
+   memcpy(host + total, d.data(), dbytes);
+   memcpy(host + total + dbytes, blk.data(), bbytes);
+   if (g_ctx.job_pin.send(g_ctx.job.p, total + dbytes + bbytes, g_ctx.stream)) return 1;
    HIPCHK(hipMemsetAsync(g_ctx.rcount.p, 0, 16 * (size_t)nrenders, g_ctx.stream));
    IterArgs a;
    memset(&a, 0, sizeof(a));

@@ -7,7 +7,6 @@
  * per-row step breakpoints instead of 32 KB tables.
  */
 #include <math.h>
-#include <pthread.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -395,96 +394,76 @@ unsigned short *fl3_create_xform_distrib(flam3_genome *cp, int *nrows) {
    return t;
 }
 
-/* Breakpoints of the selection rows the walkers use, without the table:
- * each row filled as fl3_create_xform_distrib fills it, into one row buffer,
- * and reduced to its breakpoints.  The last STARTS_CACHE inputs (weights
- * and, with xaos, the xaos rows) and their breakpoints are kept, since the
- * temporal samples of a frame, and the frames of an animation, usually share
- * their weights; the lookup compares the inputs bit for bit. */
-#define STARTS_CACHE 8
-typedef struct {
-   double *key;
-   size_t nkey;
-   int *starts;
-   int nstarts, rows;
-} starts_entry;
-static starts_entry starts_cache[STARTS_CACHE];
-static int starts_next;
-static pthread_mutex_t starts_mu = PTHREAD_MUTEX_INITIALIZER;
+/* Breakpoints of one row as fill_row fills it, without the row: starts[j] is
+ * the first slot i whose sum of i steps, rounded at each, reaches the edge of
+ * xform j.  16384 dependent additions took 20 us a row; while the sum stays in
+ * one binade and a step is not midway between two of its neighbours, each
+ * addition adds the same multiple of the sum's last place, so the slots up to
+ * the next edge or power of two are counted at once. */
+static int row_starts(const flam3_genome *cp, int from, int ns, int *starts) {
+   int i, j = 0;
+   double total = 0.0, step, acc = 0.0, edge;
+   for (i = 0; i < ns; i++) {
+      double d = cp->xform[i].density;
+      if (from >= 0) d *= cp->chaos[from][i];
+      if (d < 0.0) {
+         fprintf(stderr, "xform weight must be non-negative, not %g.\n", d);
+         return 1;
+      }
+      total += d;
+   }
+   if (total == 0.0) {
+      fprintf(stderr, "cannot iterate empty flame.\n");
+      return 1;
+   }
+   step = total / FL3_CHOOSE_GRAIN;
+   edge = cp->xform[0].density * (from >= 0 ? cp->chaos[from][0] : 1.0);
+   starts[0] = 0;
+   for (i = 0; i < FL3_CHOOSE_GRAIN && j < ns - 1; i++) {
+      while (acc >= edge && j < ns - 1) {
+         starts[++j] = i;
+         edge += cp->xform[j].density * (from >= 0 ? cp->chaos[from][j] : 1.0);
+      }
+      if (acc >= 1e-200 && acc < edge && edge < 1e200) {
+         int e;
+         double top, place, d;
+         frexp(acc, &e);
+         top = ldexp(1.0, e);             /* acc in [top / 2, top) */
+         place = ldexp(1.0, e - 53);      /* its last place */
+         d = (acc + step) - acc;
+         if (acc + step < top && fabs(step - d) * 2 < place) {
+            const double lim = edge < top ? edge : top;
+            const long long most = (long long)((lim - acc) / place), by = (long long)(d / place);
+            long long k = (most - 1) / by;   /* the most steps that leave acc below lim */
+            if (k > FL3_CHOOSE_GRAIN - 1 - i) k = FL3_CHOOSE_GRAIN - 1 - i;
+            acc += (double)(k * by) * place;
+            i += (int)k;
+         }
+      }
+      acc += step;
+   }
+   for (j++; j < ns; j++) starts[j] = FL3_CHOOSE_GRAIN;
+   return 0;
+}
 
+/* Breakpoints of the selection rows the walkers use, without the table. */
 int fl3_xform_starts(flam3_genome *cp, int *starts, int *nrows) {
-   int ns = num_std(cp), i, j, r, unity = 1, rows, e;
-   size_t nkey, k = 0;
-   double *key;
-   unsigned short *row;
+   int ns = num_std(cp), i, j, r, unity = 1;
    for (i = 0; i < ns; i++)
       for (j = 0; j < ns; j++)
          if (fabs(cp->chaos[i][j] - 1.0) > FL3_EPS) unity = 0;
    cp->chaos_enable = !unity;
-   rows = unity ? 1 : ns + 1;
-   nkey = 2 + (size_t)ns + (unity ? 0 : (size_t)ns * ns);
-   key = (double *)malloc(sizeof(double) * nkey);
-   if (!key) return 1;
-   key[k++] = ns;
-   key[k++] = cp->final_xform_index;
-   for (i = 0; i < ns; i++) key[k++] = cp->xform[i].density;
-   if (!unity)
-      for (i = 0; i < ns; i++)
-         for (j = 0; j < ns; j++) key[k++] = cp->chaos[i][j];
-   pthread_mutex_lock(&starts_mu);
-   for (e = 0; e < STARTS_CACHE; e++) {
-      const starts_entry *c = &starts_cache[e];
-      if (c->key && c->nkey == nkey && memcmp(c->key, key, sizeof(double) * nkey) == 0) {
-         memcpy(starts, c->starts, sizeof(int) * (size_t)c->nstarts);
-         pthread_mutex_unlock(&starts_mu);
-         free(key);
-         if (nrows) *nrows = rows;
-         return 0;
-      }
-   }
-   pthread_mutex_unlock(&starts_mu);
-   row = (unsigned short *)malloc(sizeof(unsigned short) * FL3_CHOOSE_GRAIN);
-   if (!row) {
-      free(key);
-      return 1;
-   }
-   if (fill_row(cp, -1, row)) goto fail;
-   fl3_distrib_breakpoints(row, 1, ns, starts);
+   if (row_starts(cp, -1, ns, starts)) return 1;
    if (!unity) {
       r = 0;
       for (i = 0; i < cp->num_xforms; i++) {
          if (i == cp->final_xform_index) continue;
          r++;
-         if (fill_row(cp, i, row)) goto fail;
-         fl3_distrib_breakpoints(row, 1, ns, starts + (size_t)r * ns);
+         if (row_starts(cp, i, ns, starts + (size_t)r * ns)) return 1;
       }
    }
-   free(row);
-   {
-      int *copy = (int *)malloc(sizeof(int) * (size_t)rows * ns);
-      if (copy) {
-         memcpy(copy, starts, sizeof(int) * (size_t)rows * ns);
-         pthread_mutex_lock(&starts_mu);
-         starts_entry *c = &starts_cache[starts_next];
-         starts_next = (starts_next + 1) % STARTS_CACHE;
-         free(c->key);
-         free(c->starts);
-         c->key = key;
-         c->nkey = nkey;
-         c->starts = copy;
-         c->nstarts = rows * ns;
-         c->rows = rows;
-         pthread_mutex_unlock(&starts_mu);
-         key = NULL;
-      }
-   }
-   free(key);
-   if (nrows) *nrows = rows;
+   if (nrows) *nrows = unity ? 1 : ns + 1;
    return 0;
-fail:
-   free(row);
-   free(key);
-   return 1;
 }
 
 void fl3_distrib_breakpoints(const unsigned short *distrib, int nrows, int nstd, int *starts) {

@@ -42,6 +42,15 @@ int fl3_genome_add_xforms(flam3_genome *g, int n, int padding, int final_flag);
 /* Genome at time t from a time-sorted list (flam3.c:717-802).  Returns 0 on
  * success.  dst must be zeroed or previously produced by this library. */
 int fl3_interpolate(const flam3_genome *cps, int ncps, double t, double stagger, flam3_genome *dst);
+/* The same with the aligned control points of t's segment shared between calls
+ * (those of s if t lies in its segment, else its own; s may be NULL).  A
+ * segment is only read by these calls, from any thread; its control points are
+ * cps' as they were when it was opened (NULL for one control point). */
+typedef struct fl3_segment fl3_segment;
+fl3_segment *fl3_segment_open(const flam3_genome *cps, int ncps, double t);
+void fl3_segment_close(fl3_segment *s);
+int fl3_interpolate_in(const fl3_segment *s, const flam3_genome *cps, int ncps, double t, double stagger,
+                       flam3_genome *dst);
 
 /* Active-variation lists and precalc flags for every xform (variations.c:2016). */
 int fl3_prepare_precalc_flags(flam3_genome *cp);

@@ -422,7 +422,29 @@ static double stagger_weight(double t, double stagger, int nx, int i) {
 
 /* ---------------------------------------------------------------- blend */
 
-static void blend_palette(flam3_genome *res, const flam3_genome *cpi, int n, const double *c) {
+/* Hue, saturation and value of the control points' palettes, as the blend
+ * takes them. */
+static void palette_hsv(const flam3_genome *cpi, int n, double hsv[][256][3]) {
+   const int mode = cpi[0].palette_interpolation;
+   int i, k;
+   if (mode == flam3_palette_interpolation_sweep) return;
+   for (k = n - 1; k >= 0; k--)
+      for (i = 0; i < 256; i++) {
+         double *h = hsv[k][i];
+         fl3_rgb2hsv(cpi[k].palette[i].color, h);
+         if (n == 2 && k == 0 && mode == flam3_palette_interpolation_hsv_circular) {
+            /* hue of the first point moved so the blend takes the short way round */
+            const double h2 = hsv[1][i][0];
+            if (h2 - h[0] > 3.0)
+               h[0] += 6.0;
+            else if (h2 - h[0] < -3.0)
+               h[0] -= 6.0;
+         }
+      }
+}
+
+static void blend_palette(flam3_genome *res, const flam3_genome *cpi, int n, const double *c,
+                          double palhsv[][256][3]) {
    int i, k, l;
    const int mode = cpi[0].palette_interpolation;
    if (mode == flam3_palette_interpolation_sweep) {
@@ -439,17 +461,7 @@ static void blend_palette(flam3_genome *res, const flam3_genome *cpi, int n, con
       int opaque = 1;
       for (k = 0; k < n; k++) {
          const flam3_palette_entry *e = &cpi[k].palette[i];
-         double h[3];
-         fl3_rgb2hsv(e->color, h);
-         if (n == 2 && k == 0 && mode == flam3_palette_interpolation_hsv_circular) {
-            /* hue of the first point moved so the blend takes the short way round */
-            double h2[3];
-            fl3_rgb2hsv(cpi[1].palette[i].color, h2);
-            if (h2[0] - h[0] > 3.0)
-               h[0] += 6.0;
-            else if (h2[0] - h[0] < -3.0)
-               h[0] -= 6.0;
-         }
+         const double *h = palhsv[k][i];
          for (l = 0; l < 3; l++) {
             rgb[l] += c[k] * e->color[l];
             hsv[l] += c[k] * h[l];
@@ -496,10 +508,11 @@ static double lin(const double *c, int n, const flam3_genome *cpi, size_t off) {
 
 /* res: cleared genome with the aligned xform layout.  c is modified and
  * restored when staggering (interpolation.c:373-708). */
-static void blend(flam3_genome *res, int n, const flam3_genome *cpi, double *c, double stagger) {
+static void blend(flam3_genome *res, int n, const flam3_genome *cpi, double palhsv[][256][3], double *c,
+                  double stagger) {
    int i, j, k, numstd;
    size_t f;
-   blend_palette(res, cpi, n, c);
+   blend_palette(res, cpi, n, c, palhsv);
    res->palette_index = -1;
    res->symmetry = 0;
    res->spatial_filter_select = cpi[0].spatial_filter_select;
@@ -589,11 +602,19 @@ static void free_all(flam3_genome *g, int n) {
    for (i = 0; i < n; i++) fl3_genome_free(&g[i]);
 }
 
-int fl3_interpolate_multi(const flam3_genome *cps, int ncps, double t, double stagger, flam3_genome *dst) {
-   int i1, i2, smooth = 0, nalign, rc = 1;
-   double c[4];
+/* The aligned control points of the segment a time lies in, with their
+ * palettes' HSV: what all temporal samples of a frame in that segment share.
+ * Only read once it is open. */
+struct fl3_segment {
+   int i1, smooth;
    flam3_genome cpi[4];
-   memset(cpi, 0, sizeof(cpi));
+   double palhsv[4][256][3];
+};
+
+/* First control point of t's segment; *smooth: it takes four. */
+static int find_segment(const flam3_genome *cps, int ncps, double t, int *smooth, int report) {
+   int i1, i2;
+   *smooth = 0;
    if (cps[0].time >= t) {
       i1 = 0;
       i2 = 1;
@@ -606,21 +627,65 @@ int fl3_interpolate_multi(const flam3_genome *cps, int ncps, double t, double st
       i1--;
       i2 = i1 + 1;
    }
-   c[0] = (cps[i2].time - t) / (cps[i2].time - cps[i1].time);
-   c[1] = 1.0 - c[0];
-
    if (cps[i1].interpolation != flam3_interpolation_linear) {
       /* Catmull-Rom over four control points needs one on each side; the
        * reference reports the first and last segments and then reads past
        * the array; here they fall back to linear. */
-      if (i1 == 0 || i2 == ncps - 1)
+      if (i1 != 0 && i2 != ncps - 1)
+         *smooth = 1;
+      else if (report)
          fprintf(stderr, "error: cannot use smooth interpolation on %s segment.\nreverting to linear interpolation.\n",
                  i1 == 0 ? "first" : "last");
-      else
-         smooth = 1;
    }
-   nalign = smooth ? 4 : 2;
-   if (align(cpi, smooth ? &cps[i1 - 1] : &cps[i1], nalign)) goto out;
+   return i1;
+}
+
+static int open_segment(fl3_segment *s, const flam3_genome *cps, int i1, int smooth) {
+   const int n = smooth ? 4 : 2;
+   s->i1 = i1;
+   s->smooth = smooth;
+   memset(s->cpi, 0, sizeof(s->cpi));
+   if (align(s->cpi, smooth ? &cps[i1 - 1] : &cps[i1], n)) return 1;
+   palette_hsv(s->cpi, n, s->palhsv);
+   return 0;
+}
+
+void fl3_segment_close(fl3_segment *s) {
+   if (!s) return;
+   free_all(s->cpi, s->smooth ? 4 : 2);
+   free(s);
+}
+
+fl3_segment *fl3_segment_open(const flam3_genome *cps, int ncps, double t) {
+   fl3_segment *s;
+   int i1, smooth;
+   if (ncps < 2) return NULL;
+   s = (fl3_segment *)malloc(sizeof(fl3_segment));
+   if (!s) return NULL;
+   i1 = find_segment(cps, ncps, t, &smooth, 0);
+   if (open_segment(s, cps, i1, smooth)) {
+      fl3_segment_close(s);
+      return NULL;
+   }
+   return s;
+}
+
+int fl3_interpolate_multi(const fl3_segment *shared, const flam3_genome *cps, int ncps, double t, double stagger,
+                          flam3_genome *dst) {
+   fl3_segment *own = NULL;
+   const fl3_segment *s = shared;
+   const flam3_genome *cpi;
+   int smooth, rc = 1;
+   double c[4];
+   const int i1 = find_segment(cps, ncps, t, &smooth, 1);
+   c[0] = (cps[i1 + 1].time - t) / (cps[i1 + 1].time - cps[i1].time);
+   c[1] = 1.0 - c[0];
+   if (!s || s->i1 != i1 || s->smooth != smooth) {
+      s = own = (fl3_segment *)malloc(sizeof(fl3_segment));
+      if (!own) return 1;
+      if (open_segment(own, cps, i1, smooth)) goto out;
+   }
+   cpi = s->cpi;
 
    fl3_genome_free(dst);
    fl3_genome_defaults(dst, 1);
@@ -641,7 +706,7 @@ int fl3_interpolate_multi(const flam3_genome *cps, int ncps, double t, double st
    dst->hsv_rgb_palette_blend = 0.0;
 
    if (!smooth) {
-      blend(dst, 2, cpi, c, stagger);
+      blend(dst, 2, cpi, (double(*)[256][3])s->palhsv, c, stagger);
    } else {
       /* Catmull-Rom weights at u = c[1] (interpolation.c:326-337) */
       const double u = c[1], u2 = u * u, u3 = u2 * u;
@@ -650,10 +715,10 @@ int fl3_interpolate_multi(const flam3_genome *cps, int ncps, double t, double st
       w[1] = (3 * u3 - 5 * u2 + 2) / 2;
       w[2] = (4 * u2 - 3 * u3 + u) / 2;
       w[3] = (u3 - u2) / 2;
-      blend(dst, 4, cpi, w, 0);
+      blend(dst, 4, cpi, (double(*)[256][3])s->palhsv, w, 0);
    }
    rc = 0;
 out:
-   free_all(cpi, nalign);
+   fl3_segment_close(own);
    return rc;
 }

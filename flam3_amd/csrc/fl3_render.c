@@ -198,6 +198,7 @@ typedef struct {
    double vibrancy, gamma, background[3], badvals;
    int vib_gam_n;
    uint64_t *keys;                /* two per temporal sample */
+   fl3_segment *segment;          /* the control points around the frame's time (NULL for a still) */
    uint32_t *walker_states;       /* replay: 36 words per reference thread */
    time_t tstart;
 } render_plan;
@@ -206,6 +207,7 @@ static void plan_close(render_plan *P) {
    free(P->filter);
    free(P->temporal_filter);
    free(P->temporal_deltas);
+   fl3_segment_close(P->segment);
    free(P->cam);
    free(P->walker_states);
    free(P->keys);
@@ -238,7 +240,8 @@ static int plan_open(render_plan *P, flam3_frame *spec, void *out, int field, in
    /* apophysis palettes use 255 entries (rect.c:587) */
    P->cmap_size = 256 - env_int("apo_palette", 0);
 
-   if (fl3_interpolate(spec->genomes, spec->ngenomes, spec->time, 0, &P->cp)) goto fail;
+   if (spec->ngenomes > 1) P->segment = fl3_segment_open(spec->genomes, spec->ngenomes, spec->time);
+   if (fl3_interpolate_in(P->segment, spec->genomes, spec->ngenomes, spec->time, 0, &P->cp)) goto fail;
    P->oversample = P->cp.spatial_oversample;
    P->nbatches = P->cp.nbatches;
    P->nts = P->cp.ntemporal_samples;
@@ -300,7 +303,7 @@ fail:
  * temporal sample (rect.c:726-747). */
 static int plan_batch_de(render_plan *P, int batch_num, fl3_de_filters *de) {
    memset(de, 0, sizeof(*de));
-   if (fl3_interpolate(P->spec->genomes, P->spec->ngenomes,
+   if (fl3_interpolate_in(P->segment, P->spec->genomes, P->spec->ngenomes,
                        P->spec->time + P->temporal_deltas[batch_num * P->nts], 0, &P->cp))
       return 1;
    if (P->cp.estimator < 0.0 || P->cp.estimator_minimum < 0.0) {
@@ -331,7 +334,8 @@ static int plan_ts_job(render_plan *P, int tidx, int first, void **job, size_t *
    int *starts;
    int i, j, nrows, ns;
    *job = NULL;
-   if (fl3_interpolate(P->spec->genomes, P->spec->ngenomes, P->spec->time + P->temporal_deltas[tidx], 0, cp))
+   if (fl3_interpolate_in(P->segment, P->spec->genomes, P->spec->ngenomes,
+                          P->spec->time + P->temporal_deltas[tidx], 0, cp))
       return 1;
    if (fl3_prepare_precalc_flags(cp)) {
       fprintf(stderr, "prepare xform pointers returned error: aborting.\n");

@@ -45,7 +45,7 @@ FL3_HD void fl3_hsv2rgb(const double *hsv, double *rgb) {
    int j;
    while (h >= 6.0) h = h - 6.0;
    while (h < 0.0) h = h + 6.0;
-   j = (int)floor(h);
+   j = (int)h;
    f = h - j;
    p = v * (1 - s);
    q = v * (1 - (s * f));
