@@ -530,9 +530,14 @@ __device__ __forceinline__ void point_color(const GenL<R> &G, R c, int &ci, R &f
 // Deposit one plotted point (rect.c:419-516).  BITS 32/33: uint32 cells of
 // 5 channels with truncated, saturating adds; 64: double cells.  The cell
 // index is computed like the reference (truncation of ws0*x - wb0s0) with
-// contraction off, and cells outside the histogram are dropped.
+// contraction off, and cells outside the histogram are dropped.  bytes: no
+// sum of the histogram can reach 2^32 and every delta is below 256, so nothing
+// is read back and channels that share an aligned 64-bit word are added to it
+// together: few walkers wait for the atomics they read back in every step (one
+// workgroup's 41000 samples of 64x64: 298 us, and 156 us so; 0.96M samples of
+// 400x300 447 and 247 us).
 template <typename R, int BITS, bool EXACT>
-__device__ __forceinline__ void deposit(const GenL<R> &G, const R *q, void *buckets, uint32_t *sat) {
+__device__ __forceinline__ void deposit(const GenL<R> &G, const R *q, void *buckets, uint32_t *sat, bool bytes = false) {
 #pragma clang fp contract(off)
    R x = q[0], y = q[1];
    if (G.rotate) {
@@ -585,6 +590,14 @@ __device__ __forceinline__ void deposit(const GenL<R> &G, const R *q, void *buck
    d[4] = (vis == R(1.0)) ? 255u : (uint32_t)(vis * R(255.0));
    if (EXACT) {
       for (int k = 0; k < 5; k++) sat_add(b + k, d[k]);
+   } else if (bytes) {
+      // (an odd word's cell: its first channel alone, then two pairs)
+      const bool odd = ((uintptr_t)b & 4u) != 0;
+      unsigned long long *w = (unsigned long long *)(b + (odd ? 1 : 0));
+      auto pair = [](uint32_t lo, uint32_t hi) { return (unsigned long long)lo | (unsigned long long)hi << 32; };
+      atomicAdd(w, odd ? pair(d[1], d[2]) : pair(d[0], d[1]));
+      atomicAdd(w + 1, odd ? pair(d[3], d[4]) : pair(d[2], d[3]));
+      atomicAdd(b + (odd ? 0 : 4), odd ? d[0] : d[4]);
    } else {
       // Colour deltas never exceed the count delta (palette <= 1), so only
       // the count channel can reach UINT_MAX first; if it does, the caller

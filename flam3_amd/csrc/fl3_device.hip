@@ -171,6 +171,7 @@ struct Ctx {
    std::vector<long long> rcell0;
    std::vector<int> rwidth, rheight;
    long long cell0 = 0;
+   double deposited = 0.0;   // samples the begun histograms may hold at most
    DevBuf rcount, descs;   // per-render counters, job descriptors + workgroup table
 };
 
@@ -370,6 +371,7 @@ extern "C" int fl3d_begin_many(const int *width, const int *height, int n, int b
    g_ctx.bits = bits;
    HIPCHK(hipMemsetAsync(g_ctx.accum.p, 0, cells * accum_bytes(bits), g_ctx.stream));
    HIPCHK(hipMemsetAsync(g_ctx.buckets.p, 0, cells * bucket_bytes(bits), g_ctx.stream));
+   g_ctx.deposited = 0.0;
    return fl3d_select(0);
 }
 
@@ -410,6 +412,7 @@ extern "C" int fl3d_select(int r) {
 extern "C" int fl3d_clear_buckets(void) {
    size_t n = (size_t)g_ctx.width * g_ctx.height;
    HIPCHK(hipMemsetAsync(cur_buckets(), 0, n * bucket_bytes(g_ctx.bits), g_ctx.stream));
+   if (g_ctx.rcell0.size() == 1) g_ctx.deposited = 0.0;
    return 0;
 }
 
@@ -794,6 +797,23 @@ static int packed_items(BinArgs *b, long long records) {
    return 0;
 }
 
+// Whether `samples` more deposits of these jobs leave every sum of the begun
+// histograms below 2^32, and each adds less than 256 to a channel.
+static bool byte_deposits(const fl3_job_hdr *const *h, int n, double samples) {
+   g_ctx.deposited += samples;
+   if (g_ctx.bits == 64 || g_ctx.deposited * 255.0 > 4294967295.0) return false;
+   for (int j = 0; j < n; j++) {
+      const unsigned char *hb = (const unsigned char *)h[j];
+      const double *dm = (const double *)(hb + h[j]->off_dmap);
+      const fl3_xform_pack *px = (const fl3_xform_pack *)(hb + h[j]->off_xf);
+      bool ok = true;
+      for (int e = 0; e < 1024; e++) ok &= dm[e] >= 0.0 && dm[e] < 256.0;
+      for (int e = 0; e < h[j]->nxf; e++) ok &= px[e].vis >= 0.0 && px[e].vis <= 1.0;
+      if (!ok) return false;
+   }
+   return true;
+}
+
 // Genomes whose walkers draw the xform per wavefront: no xaos, and room in
 // LDS for the exchange buffers beside the largest genome image, tile counts
 // and palette bytes any launch of them can need (so that the choice does
@@ -1128,6 +1148,8 @@ extern "C" int fl3d_iterate_batch(const void *const *jobs, const size_t *job_byt
       }
       const bool binned =
           binnable && (p->deposit == 2 || (p->deposit == 0 && p->nsamples * njobs >= FL3_BIN_MIN_SAMPLES));
+      // (binned deposits too count toward what later direct ones may reach)
+      const bool direct_bytes = byte_deposits(js.h, js.n, (double)p->nsamples * njobs);
       if (p->job_nsamples && njobs > 1)
          for (int j = 0; j < njobs; j++) g_prof.samples += p->job_nsamples[j];
       else
@@ -1137,6 +1159,7 @@ extern "C" int fl3d_iterate_batch(const void *const *jobs, const size_t *job_byt
       } else {
          const int pk = prof_begin(ST_ITER);
          const size_t lw = with_shuffle(a, js.lds, jobs_wave_ok(js.h, js.n));
+         a.bytes = direct_bytes;
          const int lrc =
              fl3k_launch_iter_fast(&a, (unsigned)(W / 256), lw, g_ctx.stream, g_ctx.bits, p->exact, js.tier);
          prof_end(pk);
@@ -1277,6 +1300,7 @@ extern "C" int fl3d_iterate_multi(const fl3d_multi_job *jobs, int njobs, int fus
    a.buckets = g_ctx.buckets.p;
    a.badvals = (unsigned long long *)g_ctx.rcount.p;
    a.fuse = fuse;
+   a.bytes = byte_deposits(hs.data(), njobs, (double)samples);
    const int *blk_dev = (const int *)(a.jobs + total + dbytes);
    g_prof.samples += samples;
    const size_t lds_lane = lds;

@@ -40,6 +40,7 @@ struct IterArgs {
    unsigned long long key0, key1;
    unsigned long long *badvals;
    uint32_t *sat;
+   int bytes;               // direct deposits: no sum reaches 2^32 and no delta 256
    // replay
    uint32_t *isaac;         // 36 words per walker, updated in place
    double batch_size;       // replay: samples per walker (double, rect.c:840)

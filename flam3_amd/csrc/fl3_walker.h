@@ -315,7 +315,7 @@ __global__ __launch_bounds__(256, walker_waves<TIER>()) void k_iter_fast(IterArg
              cell == FL3_REC_NONE ? FL3_REC_NONE : (cell | ((unsigned)(r >> 32) & 0xffu) << 24);
          if (cell != FL3_REC_NONE) atomicAdd(&bh[cell >> a.bin_shift], 1u);
       } else
-         deposit<float, BITS, EXACT>(G, v, buckets, satp);
+         deposit<float, BITS, EXACT>(G, v, buckets, satp, a.bytes != 0);
    };
    if constexpr (WAVE) {
       // One xform per wavefront and step (drawn from a hash of the

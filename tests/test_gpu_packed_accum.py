@@ -57,3 +57,17 @@ def test_renders_of_several_palettes_together(prod, shades):
     for it, (img, _) in zip(items, prod.render_many(items)):
         want, _ = prod.render(it["genomes"], seed=it["seed"], nchan=4, transp=1, deposit=1)
         assert np.array_equal(img, want), it["seed"]
+
+
+@pytest.mark.parametrize("quality", [4112, 4113])
+@pytest.mark.parametrize("opacity", [1.0, 0.5, 1.5])
+def test_direct_deposits_on_both_sides_of_their_bound(prod, quality, opacity):
+    """Channels added in pairs, without reading them back, while 255 times the
+    samples stays below 2^32 and no delta passes 255 (4112 x 64 x 64 samples
+    and visibility 1); one by one beyond."""
+    g = _shaded(G.synthetic_small(seed=41, width=64, height=64, quality=quality), "alpha")
+    g.xforms[1].opacity = opacity
+    a, sa = prod.render(g, seed="pairs", deposit=1, nchan=4, transp=1)
+    b, sb = prod.render(g, seed="pairs", deposit=2, nchan=4, transp=1)
+    assert sa["num_iters"] == sb["num_iters"] == quality * 64 * 64
+    assert np.array_equal(a, b)
