@@ -135,7 +135,7 @@ struct Ctx {
    hipStream_t stream = nullptr;
    // The tile-binned deposit sorts and accumulates chunk k on bin_stream
    // while the walkers produce the next chunks on stream: chunk k's records
-   // and tile counts are set k % FL3_CHUNK_BUFS of crec/cblk/ctot.
+   // and tile counts are set k % FL3_CHUNK_BUFS of crec/ctot.
    hipStream_t bin_stream = nullptr;
    hipEvent_t ev_walk[FL3_CHUNK_BUFS] = {}, ev_bin[FL3_CHUNK_BUFS] = {}, ev_join = nullptr;
    DevBuf buckets, accum, job, table, image, isaac, points, misc, findex;
@@ -148,13 +148,13 @@ struct Ctx {
    int de_up_kind = 0;               // 1 the exact gather's coefficients, 2 / 3 double / float tables
    size_t de_up_tab = 0;             // the tables' bytes, and how many of them LDS takes
    int de_up_lds = 0;
-   DevBuf crec[FL3_CHUNK_BUFS], cblk[FL3_CHUNK_BUFS], ctot[FL3_CHUNK_BUFS];   // tile-binned deposit
-   DevBuf sorted, wstate, bins, jobtab, soff, partial;
+   DevBuf crec[FL3_CHUNK_BUFS], ctot[FL3_CHUNK_BUFS];   // tile-binned deposit
+   DevBuf sorted, wstate, bins, jobtab, partial;
    DevBuf srcv, srcl;                  // density estimation per-source values
    DevBuf detab, deargs;               // batched density estimation: tables, per-render arguments
    DevBuf deblk;                       // DE: widest source kernel per 16x16 block
    DevBuf detaps;                      // DE gather footprint counters (stage profile)
-   DevBuf blk2, soff2, bins2;          // banded histograms: second-level block counts, offsets, counters
+   DevBuf bins2;                       // banded histograms: second-level counters
    unsigned *band_host = nullptr;      // pinned: first-level tile starts of the last chunk
    hipEvent_t ev_band = nullptr;
    hipEvent_t ev_strip[FL3_IMAGE_STRIPS] = {};   // fl3d_images_fetch: strip k of the image is in staging
@@ -212,12 +212,12 @@ extern "C" int fl3d_device_memory(double *avail, double *total) {
    HIPCHK(hipMemGetInfo(&fr, &tot));
    const DevBuf *bufs[] = {&g_ctx.buckets, &g_ctx.accum, &g_ctx.job, &g_ctx.table, &g_ctx.image, &g_ctx.isaac,
                            &g_ctx.points, &g_ctx.misc, &g_ctx.findex, &g_ctx.sorted, &g_ctx.partial, &g_ctx.wstate, &g_ctx.bins,
-                           &g_ctx.jobtab, &g_ctx.soff, &g_ctx.srcv, &g_ctx.srcl, &g_ctx.detab, &g_ctx.deargs,
+                           &g_ctx.jobtab, &g_ctx.srcv, &g_ctx.srcl, &g_ctx.detab, &g_ctx.deargs,
                            &g_ctx.rcount, &g_ctx.descs, &g_ctx.deblk};
    double held = 0.0;
    for (const DevBuf *b : bufs) held += (double)b->cap;
    for (int i = 0; i < FL3_CHUNK_BUFS; i++)
-      held += (double)(g_ctx.crec[i].cap + g_ctx.cblk[i].cap + g_ctx.ctot[i].cap);
+      held += (double)(g_ctx.crec[i].cap + g_ctx.ctot[i].cap);
    if (avail) *avail = (double)fr + held;
    if (total) *total = (double)tot;
    return 0;
@@ -556,13 +556,12 @@ static int pick_tier(const fl3_job_hdr *h) {
    return FL3_TIER_FULL;
 }
 
-// Record, per-workgroup count and tile-total buffers of the chunks of a
+// Record and tile-total buffers of the chunks of a
 // binned deposit (as many sets as chunks, at most FL3_CHUNK_BUFS).
-static int ensure_chunk_bufs(long long nchunks, size_t rec_bytes, size_t blk_bytes, size_t tot_bytes) {
+static int ensure_chunk_bufs(long long nchunks, size_t rec_bytes, size_t tot_bytes) {
    const int nb = nchunks < FL3_CHUNK_BUFS ? (nchunks > 0 ? (int)nchunks : 1) : FL3_CHUNK_BUFS;
    for (int i = 0; i < nb; i++)
-      if (g_ctx.crec[i].ensure(rec_bytes) || g_ctx.cblk[i].ensure(blk_bytes) || g_ctx.ctot[i].ensure(tot_bytes))
-         return 1;
+      if (g_ctx.crec[i].ensure(rec_bytes) || g_ctx.ctot[i].ensure(tot_bytes)) return 1;
    return 0;
 }
 
@@ -847,13 +846,21 @@ static size_t with_shuffle(IterArgs &a, size_t lds, bool want) {
    return lds;
 }
 
+// A chunk's records sorted and added to the histogram on stream bs; the sort
+// is the last to read the walkers' buffers, `free` after it.
+static int sort_and_accumulate(const BinArgs &b, int format, hipEvent_t free, hipStream_t bs) {
+   if (fl3k_launch_bin_sort(&b, format, bs)) return 1;
+   HIPCHK(hipEventRecord(free, bs));
+   return fl3k_launch_bin_accum(&b, g_ctx.ncu, format, bs);
+}
+
 // Binned deposit: the walkers write records in chunks of `per` rows (the
 // walker state carries over between chunks, so the trajectories are those of
 // a single launch); each chunk is tile-sorted and accumulated.
 // One chunk of a banded histogram on stream bs: the first level (scans of
 // the walkers' counts, records grouped by band into b1.sorted), then per
-// band with records: a counting pass, the two sort passes (through the
-// walker buffer) back into the band's range and the accumulation.  The
+// band with records: a counting pass, the sort into the walker buffer and the
+// accumulation.  The
 // host reads the band boundaries, so it waits for this chunk's walkers.
 static int bin_banded(const BinArgs &b1, int format, int band, int shift, hipStream_t bs) {
    // double buckets of 2^24-cell bands, visibility 1, stepped palette: the
@@ -868,7 +875,8 @@ static int bin_banded(const BinArgs &b1, int format, int band, int shift, hipStr
    const int rows2 = 64;   // second-level blocks: 64 x 256 records
    const size_t rsz = narrow ? 4 : 8;
    const unsigned *st = g_ctx.band_host;
-   for (int j = 0; j < b1.nsuper; j++) {
+   const int nbands = (b1.nbins + (1 << FL3_SUPER_SHIFT) - 1) >> FL3_SUPER_SHIFT;
+   for (int j = 0; j < nbands; j++) {
       const int t0 = j << FL3_SUPER_SHIFT, t1 = std::min(b1.nbins, t0 + (1 << FL3_SUPER_SHIFT));
       const long long n = (long long)st[t1] - st[t0];
       if (n <= 0) continue;
@@ -883,12 +891,6 @@ static int bin_banded(const BinArgs &b1, int format, int band, int shift, hipStr
       b.shift = shift;
       const long long cells = std::min(ncells - (long long)b.cell_base, 1LL << band);
       b.nbins = (int)((cells + (1LL << shift) - 1) >> shift);
-      b.nsuper = (b.nbins + (1 << FL3_SUPER_SHIFT) - 1) >> FL3_SUPER_SHIFT;
-      if (g_ctx.blk2.ensure(sizeof(unsigned) * (size_t)b.nblk * b.nsuper) ||
-          g_ctx.soff2.ensure(sizeof(unsigned) * (size_t)b.nblk * b.nsuper))
-         return 1;
-      b.blk_hist = (unsigned *)g_ctx.blk2.p;
-      b.soff = (unsigned *)g_ctx.soff2.p;
       // the bands' counters, at fixed places for any tile count (the tile
       // counts start at zero and each scan leaves them there)
       unsigned *bw = (unsigned *)g_ctx.bins2.p;
@@ -900,8 +902,10 @@ static int bin_banded(const BinArgs &b1, int format, int band, int shift, hipStr
       b.tile_part = bw + 4 * FL3_MAX_BINS + 4;
       b.multi = bw + 5 * FL3_MAX_BINS + 4;
       b.sorted = (void *)b1.rec;                                // the walker buffer, free after the band pass
-      b.final = (unsigned char *)b1.sorted + rsz * st[t0];      // the band's own range
-      if (fl3k_launch_bin_count(&b, narrow, bs) || fl3k_launch_bin(&b, g_ctx.ncu, format, bs)) return 1;
+      b.band_cursor = nullptr;
+      if (fl3k_launch_bin_count(&b, narrow, bs) || fl3k_launch_bin_sort(&b, format, bs) ||
+          fl3k_launch_bin_accum(&b, g_ctx.ncu, format, bs))
+         return 1;
    }
    return 0;
 }
@@ -948,16 +952,12 @@ static int iterate_binned(IterArgs a, long long W, long long Wj, const JobSet &j
    const long long nchunks = (p->nsamples + Wj * per - 1) / (Wj * per);
    if (g_ctx.sorted.ensure(rec_bytes)) return 1;
    if (g_ctx.wstate.ensure(sizeof(uint32_t) * 10 * (size_t)W)) return 1;
-   const size_t nsup = (size_t)((nbins + (1 << FL3_SUPER_SHIFT) - 1) >> FL3_SUPER_SHIFT);
-   if (ensure_chunk_bufs(nchunks, rec_bytes, sizeof(unsigned) * (size_t)nblk * nsup, sizeof(unsigned) * (size_t)nbins))
-      return 1;
-   const int nsuper = (nbins + (1 << FL3_SUPER_SHIFT) - 1) >> FL3_SUPER_SHIFT;
-   if (g_ctx.bins.ensure(sizeof(unsigned) * (6 * (size_t)nbins + 16))) return 1;
+   if (ensure_chunk_bufs(nchunks, rec_bytes, sizeof(unsigned) * (size_t)nbins)) return 1;
+   if (g_ctx.bins.ensure(sizeof(unsigned) * (6 * (size_t)nbins + 16 + 256))) return 1;   // (and 256 bands)
    if (band) {
       if (g_ctx.bins2.ensure(sizeof(unsigned) * (6 * (size_t)FL3_MAX_BINS + 16))) return 1;
       HIPCHK(hipMemsetAsync(g_ctx.bins2.p, 0, sizeof(unsigned) * FL3_MAX_BINS, g_ctx.stream));
    }
-   if (g_ctx.soff.ensure(sizeof(unsigned) * (size_t)nblk * nsuper)) return 1;
    unsigned *bw = (unsigned *)g_ctx.bins.p;
    BinArgs b;
    memset(&b, 0, sizeof(b));
@@ -965,7 +965,6 @@ static int iterate_binned(IterArgs a, long long W, long long Wj, const JobSet &j
    b.buckets = a.buckets;
    b.rec = g_ctx.crec[0].p;
    b.sorted = g_ctx.sorted.p;
-   b.blk_hist = (unsigned *)g_ctx.cblk[0].p;
    b.nblk = (int)nblk;
    b.walkers = W;
    b.bin_total = bw;
@@ -975,8 +974,7 @@ static int iterate_binned(IterArgs a, long long W, long long Wj, const JobSet &j
    b.cursor = bw + 3 * nbins + 4;
    b.tile_part = bw + 4 * nbins + 4;
    b.multi = bw + 5 * nbins + 4;
-   b.soff = (unsigned *)g_ctx.soff.p;
-   b.nsuper = nsuper;
+   b.band_cursor = band ? bw + 6 * nbins + 16 : nullptr;
    b.shift = wshift;
    b.nbins = nbins;
    b.width = g_ctx.width;
@@ -1016,7 +1014,6 @@ static int iterate_binned(IterArgs a, long long W, long long Wj, const JobSet &j
       a.ns_row0 = done / Wj;   // (done: whole rows of every walker)
       a.resume = done > 0;
       a.rec = (unsigned long long *)g_ctx.crec[buf].p;
-      a.blk_hist = (unsigned *)g_ctx.cblk[buf].p;
       a.bin_total = (unsigned *)g_ctx.ctot[buf].p;
       if (k >= FL3_CHUNK_BUFS) HIPCHK(hipStreamWaitEvent(ws, g_ctx.ev_bin[buf], 0));
       HIPCHK(hipMemsetAsync(a.bin_total, 0, sizeof(unsigned) * (size_t)nbins, ws));
@@ -1030,21 +1027,19 @@ static int iterate_binned(IterArgs a, long long W, long long Wj, const JobSet &j
       HIPCHK(hipEventRecord(g_ctx.ev_walk[buf], ws));
       HIPCHK(hipStreamWaitEvent(bs, g_ctx.ev_walk[buf], 0));
       b.rec = a.rec;
-      b.final = a.rec;   // the walker buffer takes the tile-grouped records
-      b.blk_hist = a.blk_hist;
       b.bin_total = a.bin_total;
       b.rows = a.rows_out;
       pk = prof_begin(ST_BIN, bs);
-      if (band)
+      if (band) {
          lrc = bin_banded(b, format, band, shift, bs);
-      else
-         lrc = fl3k_launch_bin(&b, g_ctx.ncu, format, bs);
+         if (!lrc) HIPCHK(hipEventRecord(g_ctx.ev_bin[buf], bs));
+      } else
+         lrc = sort_and_accumulate(b, format, g_ctx.ev_bin[buf], bs);
       prof_end(pk, bs);
       if (lrc) {
          set_err("binned deposit launch failed");
          return 1;
       }
-      HIPCHK(hipEventRecord(g_ctx.ev_bin[buf], bs));
       done += c;
    }
    // the render stream continues once every chunk is accumulated
@@ -1349,14 +1344,9 @@ extern "C" int fl3d_iterate_multi(const fl3d_multi_job *jobs, int njobs, int fus
       const size_t rec_bytes = (narrow ? 4 : 8) * (size_t)Wrec * per;
       if (g_ctx.sorted.ensure(rec_bytes)) return 1;
       if (g_ctx.wstate.ensure(sizeof(uint32_t) * 10 * (size_t)Wrec)) return 1;
-      const size_t nsup = (size_t)((nbins + (1 << FL3_SUPER_SHIFT) - 1) >> FL3_SUPER_SHIFT);
-      if (ensure_chunk_bufs(nchunks, rec_bytes, sizeof(unsigned) * (size_t)nblk * nsup,
-                            sizeof(unsigned) * (size_t)nbins))
-         return 1;
-      const int nsuper = (nbins + (1 << FL3_SUPER_SHIFT) - 1) >> FL3_SUPER_SHIFT;
+      if (ensure_chunk_bufs(nchunks, rec_bytes, sizeof(unsigned) * (size_t)nbins)) return 1;
       if (g_ctx.bins.ensure(sizeof(unsigned) * (6 * (size_t)nbins + 16))) return 1;
-      if (g_ctx.soff.ensure(sizeof(unsigned) * (size_t)nblk * nsuper)) return 1;
-      unsigned *bw = (unsigned *)g_ctx.bins.p;
+         unsigned *bw = (unsigned *)g_ctx.bins.p;
       BinArgs b;
       memset(&b, 0, sizeof(b));
       b.job = a.jobs + d[jrec].off;   // the palette of 4-byte records
@@ -1371,8 +1361,6 @@ extern "C" int fl3d_iterate_multi(const fl3d_multi_job *jobs, int njobs, int fus
       b.cursor = bw + 3 * nbins + 4;
       b.tile_part = bw + 4 * nbins + 4;
       b.multi = bw + 5 * nbins + 4;
-      b.soff = (unsigned *)g_ctx.soff.p;
-      b.nsuper = nsuper;
       b.shift = shift;
       b.nbins = nbins;
       b.width = (int)(tcells < 0x7fffffffLL ? tcells : 0x7fffffffLL);
@@ -1414,7 +1402,6 @@ extern "C" int fl3d_iterate_multi(const fl3d_multi_job *jobs, int njobs, int fus
          ar.rows_out = rows_total - ar.row0 < per ? rows_total - ar.row0 : per;
          ar.resume = k > 0;
          ar.rec = (unsigned long long *)g_ctx.crec[buf].p;
-         ar.blk_hist = (unsigned *)g_ctx.cblk[buf].p;
          ar.bin_total = (unsigned *)g_ctx.ctot[buf].p;
          if (k >= FL3_CHUNK_BUFS) HIPCHK(hipStreamWaitEvent(ws, g_ctx.ev_bin[buf], 0));
          HIPCHK(hipMemsetAsync(ar.bin_total, 0, sizeof(unsigned) * (size_t)nbins, ws));
@@ -1435,18 +1422,15 @@ extern "C" int fl3d_iterate_multi(const fl3d_multi_job *jobs, int njobs, int fus
          HIPCHK(hipEventRecord(g_ctx.ev_walk[buf], ws));
          HIPCHK(hipStreamWaitEvent(bs, g_ctx.ev_walk[buf], 0));
             b.rec = ar.rec;
-         b.final = ar.rec;
-         b.blk_hist = ar.blk_hist;
          b.bin_total = ar.bin_total;
             b.rows = ar.rows_out;
          const int pk = prof_begin(ST_BIN, bs);
-         const int lrc = fl3k_launch_bin(&b, g_ctx.ncu, narrow ? 1 : 2, bs);
+         const int lrc = sort_and_accumulate(b, narrow ? 1 : 2, g_ctx.ev_bin[buf], bs);
          prof_end(pk, bs);
          if (lrc) {
             set_err("binned deposit launch failed");
             return 1;
          }
-         HIPCHK(hipEventRecord(g_ctx.ev_bin[buf], bs));
       }
       HIPCHK(hipEventRecord(g_ctx.ev_join, bs));
       HIPCHK(hipStreamWaitEvent(ws, g_ctx.ev_join, 0));

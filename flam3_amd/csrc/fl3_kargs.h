@@ -52,7 +52,6 @@ struct IterArgs {
                               // 3 8-byte records carrying the job instead of the palette fraction
    unsigned long long *rec;   // 8-byte records, or 4-byte ones in the same buffer
    long long rows_out;
-   unsigned *blk_hist;        // [workgroup][super-tile] record counts
    unsigned *bin_total;       // [tile] record counts over all workgroups (added atomically)
    int bin_shift, nbins;
    unsigned hist_off;         // LDS byte offset of the workgroup's tile counts
@@ -79,7 +78,7 @@ struct IterArgs {
 // tiles of a frame (2.2e6 of a chunk's 2.6e8 records at 1080p, against a mean
 // of 1.3e5) over several workgroups, so that the last items do not trail.
 #define FL3_MAX_BINS 8192
-#define FL3_SUPER_SHIFT 5           // tiles per super-tile = 32
+#define FL3_SUPER_SHIFT 5           // tiles a band is counted in: 32
 
 #define FL3_BIN_CHUNK_SAMPLES (1LL << 28)
 #define FL3_CHUNK_BUFS 2            // record buffers in rotation: the walkers run one chunk ahead of the sort
@@ -98,7 +97,6 @@ struct BinArgs {
    void *buckets;
    const void *rec;                // records in walker order, one block of rows x 256 per workgroup
    void *sorted;                   // records grouped by tile
-   unsigned *blk_hist;             // [walker workgroup][super-tile] counts
    int nblk;                       // walker workgroups (256 walkers each)
    long long walkers;              // row stride of rec
    long long rows;                 // record rows in this chunk
@@ -108,12 +106,8 @@ struct BinArgs {
    // tile the place of its first item among the partial sums, and these
    unsigned *multi, *tile_part;
    void *partial;
-   // two-pass sort: walker order -> super-tiles of FL3_SUPER tiles (sorted)
-   // -> tiles (final, the record buffer reused)
-   unsigned *soff;                 // [walker workgroup][super-tile] first slot in sorted
-   unsigned *cursor;               // [tile] next free slot of the tile in final
-   void *final;
-   int nsuper;
+   unsigned *cursor;               // [tile] next free slot of the tile in sorted
+   unsigned *band_cursor;          // [band] the same for bands of 1 << FL3_SUPER_SHIFT tiles (nullptr: none)
    int shift;                      // cells per tile = 1 << shift
    int nbins;                      // tiles
    int chunk;                      // records per accumulation work item

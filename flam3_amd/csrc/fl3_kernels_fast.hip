@@ -96,6 +96,7 @@ __global__ __launch_bounds__(1024) void k_bin_scan(BinArgs a) {
       const unsigned n = a.bin_total[b], ni = (unsigned)(((unsigned long long)n + a.chunk - 1) / a.chunk);
       a.bin_start[b] = (unsigned)run;
       a.cursor[b] = (unsigned)run;
+      if (a.band_cursor && (b & ((1 << FL3_SUPER_SHIFT) - 1)) == 0) a.band_cursor[b >> FL3_SUPER_SHIFT] = (unsigned)run;
       a.item_start[b] = (unsigned)irun;
       a.tile_part[b] = (unsigned)(run >> 32);
       if (ni > 1) a.multi[1 + (unsigned)(irun >> 32)] = (unsigned)b;
@@ -130,200 +131,103 @@ __device__ __forceinline__ RT rec_at(const BinArgs &a, const RT *rec, long long 
    return a.rec_count == 0 || idx < a.rec_count ? rec[idx] : (RT)FL3_REC_NONE;
 }
 
-// First slot of each walker workgroup's records of each super-tile in the
-// super-tile-grouped array: workgroup s scans super-tile s's counts over the
-// walker workgroups.
-__global__ __launch_bounds__(256) void k_super_off(BinArgs a) {
-   __shared__ unsigned part[256];
-   const int s = blockIdx.x, t = threadIdx.x;
-   const int b0 = s << FL3_SUPER_SHIFT;
-   const int per = (a.nblk + 255) / 256;
-   const int k0 = t * per, k1 = min(a.nblk, k0 + per);
-   unsigned sum = 0;
-   for (int k = k0; k < k1; k++) sum += a.blk_hist[(size_t)k * a.nsuper + s];
-   part[t] = sum;
-   __syncthreads();
-   for (int off = 1; off < 256; off <<= 1) {
-      const unsigned v = t >= off ? part[t - off] : 0;
-      __syncthreads();
-      part[t] += v;
-      __syncthreads();
-   }
-   unsigned run = a.bin_start[b0] + (t ? part[t - 1] : 0);
-   for (int k = k0; k < k1; k++) {
-      a.soff[(size_t)k * a.nsuper + s] = run;
-      run += a.blk_hist[(size_t)k * a.nsuper + s];
-   }
+#define FL3_SCATTER_UNROLL 16
+// The record as the sort writes it: unchanged, or (OT 4 bytes from 8-byte
+// records, the band pass of a histogram of 2^24-cell bands, visibility 1
+// and a stepped palette) its cell within the band of 1 << sh cells | palette
+// index << 24.
+template <typename RT, typename OT>
+__device__ __forceinline__ OT sorted_rec(RT v, int sh) {
+   if (sizeof(OT) == sizeof(RT)) return (OT)v;
+   const unsigned long long x = (unsigned long long)v;
+   return (OT)(((unsigned)x & ((1u << sh) - 1u)) | (((unsigned)(x >> 32) & 0xffu) << 24));
 }
 
-// Exclusive prefix sum over a 256-thread workgroup (v from each thread);
-// *total gets the sum.  wsum: 4 words of LDS.  Ends with a barrier.
-__device__ __forceinline__ unsigned wg_excl_scan256(unsigned v, unsigned *wsum, unsigned *total) {
-   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-   unsigned x = v;
+// The records grouped by tile of 1 << sh cells, for at most MT tiles: a
+// workgroup takes NT x P records in walker order, counts them by tile in LDS,
+// reserves each tile's slots in a.sorted with one global atomic (cursor holds
+// each tile's next one), orders the records by tile in LDS and writes them from
+// there, consecutive lanes to consecutive slots.  The order within a tile is
+// arbitrary: the accumulation adds integers.  Bound by memory latency in those
+// phases, with one workgroup of 16 wavefronts a CU, and by the atomics (512
+// records a tile's reservation at 64 tiles, 16 at 2000); a workgroup takes as
+// many records as LDS holds, so that a tile's run is some cache lines long.  Two
+// passes (to groups of 32 tiles, then to tiles) moved every record twice:
+// 3.6M records to 18 tiles 79 us, 12 so; 15M to 75 tiles 156 and 41 us; 184M to
+// 900 tiles 745 and 437 us; 2^28 to 2060 tiles 910 and 520 us; 126M of 8
+// bytes to 3600 2.8 and 1.5 ms.  (Persistent workgroups that load the next
+// records meanwhile: 439 and 601 us; half the records: 532 and 591 us.)
+template <typename RT, typename OT, int NT, int P, int MT, bool FEW>
+__global__ __launch_bounds__(NT) void k_bin_sort(BinArgs a, int sh, unsigned *cursor) {
+   constexpr int N = NT * P, PER = (MT + NT - 1) / NT;
+   RT *stage = (RT *)fl3_lds;                 // [N]
+   unsigned *gofs = (unsigned *)(stage + N);    // [MT] counts, then the tile's slots less its first place in stage
+   uint16_t *lofs = (uint16_t *)(gofs + MT);   // [MT] that place
+   __shared__ unsigned wsum[NT / 64];
+   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+   const long long slots = a.rec_count ? a.rec_count : a.walkers * a.rows, r0 = (long long)blockIdx.x * N;
+   const RT *in = (const RT *)a.rec + r0;
+   const int n = (int)(slots - r0 < N ? slots - r0 : N);
+   RT v[P];
+   for (int k = 0; k < P; k++) {
+      const int r = k * NT + tid;
+      v[k] = r < n ? in[r] : (RT)FL3_REC_NONE;
+   }
+   for (int t = tid; t < MT; t += NT) gofs[t] = 0;
+   __syncthreads();
+   unsigned rank[P];
+   auto counter = [&](RT x) {
+      const unsigned t = rel_cell(a, x) >> sh;
+      return FEW ? t * 64u + (unsigned)lane : t;
+   };
+   for (int k = 0; k < P; k++)
+      if (!rec_none(v[k])) rank[k] = atomicAdd(&gofs[counter(v[k])], 1u);
+   __syncthreads();
+   // (the slots are on their way while the counts are scanned)
+   unsigned g[PER], c[PER], sum = 0;
+   for (int j = 0; j < PER; j++) {
+      const int t = j * NT + tid;
+      const unsigned ct = t < MT ? gofs[t] : 0u;
+      g[j] = 0;
+      if (!FEW && ct) g[j] = atomicAdd(&cursor[t], ct);
+   }
+   for (int j = 0; j < PER; j++) {
+      c[j] = PER * tid + j < MT ? gofs[PER * tid + j] : 0u;
+      sum += c[j];
+   }
+   unsigned x = sum;
    for (int o = 1; o < 64; o <<= 1) {
       const unsigned y = __shfl_up(x, o, 64);
       if (lane >= o) x += y;
    }
-   if (lane == 63) wsum[w] = x;
+   if (lane == 63) wsum[wave] = x;
    __syncthreads();
-   unsigned pre = 0;
-   for (int k = 0; k < w; k++) pre += wsum[k];
-   *total = wsum[0] + wsum[1] + wsum[2] + wsum[3];
-   __syncthreads();
-   return pre + x - v;
-}
-
-// Pass 1: workgroup k moves the records of walkers [256k, 256k + 256) (one
-// column block of the record matrix) to its range of each super-tile.  With
-// at most 256 super-tiles per workgroup the partly written lines stay in L2
-// until they fill.
-#define FL3_SCATTER_UNROLL 16
-// The record as pass 1 writes it: unchanged, or (OT 4 bytes from 8-byte
-// records, the band pass of a histogram of 2^24-cell bands, visibility 1
-// and a stepped palette) its cell within the super-tile | palette index << 24.
-template <typename RT, typename OT>
-__device__ __forceinline__ OT part1_out(RT v, int ss) {
-   if (sizeof(OT) == sizeof(RT)) return (OT)v;
-   const unsigned long long x = (unsigned long long)v;
-   return (OT)(((unsigned)x & ((1u << ss) - 1u)) | (((unsigned)(x >> 32) & 0xffu) << 24));
-}
-
-template <typename RT, typename OT = RT>
-__global__ __launch_bounds__(256) void k_bin_part1(BinArgs a) {
-   __shared__ unsigned base[256], cnt[256];
-   const int ss = a.shift + FL3_SUPER_SHIFT;
-   for (int s = threadIdx.x; s < a.nsuper; s += blockDim.x) {
-      base[s] = a.soff[(size_t)blockIdx.x * a.nsuper + s];
-      cnt[s] = 0;
+   unsigned pre = x - sum, tot = 0;
+   for (int w = 0; w < NT / 64; w++) {
+      if (w < wave) pre += wsum[w];
+      tot += wsum[w];
    }
+   for (int j = 0; j < PER; j++)
+      if (PER * tid + j < MT) {
+         lofs[PER * tid + j] = (uint16_t)pre;
+         pre += c[j];
+      }
    __syncthreads();
-   const RT *rec = (const RT *)a.rec;
+   if (!FEW) {
+      for (int j = 0; j < PER; j++)
+         if (j * NT + tid < MT) gofs[j * NT + tid] = g[j] - lofs[j * NT + tid];
+   } else if (tid < MT / 64) {
+      const unsigned l0 = lofs[tid * 64], ct = (tid < MT / 64 - 1 ? lofs[tid * 64 + 64] : tot) - l0;
+      gofs[tid] = (ct ? atomicAdd(&cursor[tid], ct) : 0u) - l0;
+   }
+   for (int k = 0; k < P; k++)
+      if (!rec_none(v[k])) stage[lofs[counter(v[k])] + rank[k]] = v[k];
+   __syncthreads();
    OT *out = (OT *)a.sorted;
-   long long i = 0;
-   for (; i + FL3_SCATTER_UNROLL <= a.rows; i += FL3_SCATTER_UNROLL) {
-      RT v[FL3_SCATTER_UNROLL];
-      for (int k = 0; k < FL3_SCATTER_UNROLL; k++) v[k] = rec_at(a, rec, (blockIdx.x * a.rows + i + k) * 256 + threadIdx.x);
-      for (int k = 0; k < FL3_SCATTER_UNROLL; k++) {
-         if (rec_none(v[k])) continue;
-         const unsigned s = rel_cell(a, v[k]) >> ss;
-         out[base[s] + atomicAdd(&cnt[s], 1u)] = part1_out<RT, OT>(v[k], ss);
-      }
+   for (unsigned j = tid; j < tot; j += NT) {
+      const RT w = stage[j];
+      out[gofs[rel_cell(a, w) >> sh] + j] = sorted_rec<RT, OT>(w, sh);
    }
-   for (; i < a.rows; i++) {
-      const RT v = rec_at(a, rec, (blockIdx.x * a.rows + i) * 256 + threadIdx.x);
-      if (rec_none(v)) continue;
-      const unsigned s = rel_cell(a, v) >> ss;
-      out[base[s] + atomicAdd(&cnt[s], 1u)] = part1_out<RT, OT>(v, ss);
-   }
-}
-
-// The same for 4-byte records of tall blocks (many rows per chunk): the
-// block is taken in batches of 16 rows, each batch ordered by super-tile in
-// LDS (counting sort) and written out from there, so consecutive lanes store
-// consecutive slots of one super-tile's range (a few cache lines per store
-// instead of one per lane).  Faster from a few dozen rows on; for short
-// blocks the batches' scans and barriers cost more than they save.
-#define FL3_PART1_STAGED_ROWS 64
-template <typename RT>
-__global__ __launch_bounds__(256) void k_bin_part1_staged(BinArgs a) {
-   constexpr int P = sizeof(RT) == 4 ? 16 : 8;   // rows per batch
-   __shared__ unsigned gnext[256];   // this workgroup's next slot in each super-tile
-   __shared__ unsigned lcnt[256], loff[256], wsum[4];
-   __shared__ RT stage[256 * P];
-   const int ss = a.shift + FL3_SUPER_SHIFT;
-   const int t = threadIdx.x;
-   gnext[t] = t < a.nsuper ? a.soff[(size_t)blockIdx.x * a.nsuper + t] : 0u;
-   const RT *rec = (const RT *)a.rec;
-   RT *out = (RT *)a.sorted;
-   for (long long i0 = 0; i0 < a.rows; i0 += P) {
-      lcnt[t] = 0;
-      __syncthreads();
-      RT v[P];
-      unsigned rk[P];
-      for (int k = 0; k < P; k++) {
-         const long long row = i0 + k;
-         v[k] = row < a.rows ? rec_at(a, rec, (blockIdx.x * a.rows + row) * 256 + t) : (RT)FL3_REC_NONE;
-      }
-      for (int k = 0; k < P; k++)
-         if (!rec_none(v[k])) rk[k] = atomicAdd(&lcnt[rel_cell(a, v[k]) >> ss], 1u);
-      __syncthreads();
-      unsigned tot;
-      loff[t] = wg_excl_scan256(lcnt[t], wsum, &tot);
-      __syncthreads();
-      for (int k = 0; k < P; k++)
-         if (!rec_none(v[k])) stage[loff[rel_cell(a, v[k]) >> ss] + rk[k]] = v[k];
-      __syncthreads();
-      for (unsigned j = t; j < tot; j += 256) {
-         const RT w = stage[j];
-         const unsigned sp = rel_cell(a, w) >> ss;
-         out[gnext[sp] + (j - loff[sp])] = w;
-      }
-      __syncthreads();
-      gnext[t] += lcnt[t];
-   }
-}
-
-// Pass 2: workgroup c moves the super-tile-grouped records
-// [c * FL3_PART2_RECORDS, ...) to their tiles.  The records of a workgroup
-// usually span fewer than 256 tiles (a few super-tiles): ranks within the
-// workgroup from LDS counters of that span, each tile's slots reserved with
-// one global atomic, and 4-byte records ordered by tile in LDS first and
-// written out from there, consecutive lanes to consecutive slots (8-byte
-// records would need twice the LDS and halve the workgroups a CU holds, so
-// they are written from registers).  A wider span (records of many sparse
-// tiles) reserves one slot per record.  The order within a tile is
-// arbitrary: the accumulation adds integers (or doubles, whose sums then
-// differ in rounding only).
-#define FL3_PART2_PER 32
-#define FL3_PART2_RECORDS (256 * FL3_PART2_PER)
-template <typename RT>
-__global__ __launch_bounds__(256) void k_bin_part2(BinArgs a) {
-   RT *stage = (RT *)fl3_lds;   // 4-byte records: [FL3_PART2_RECORDS]
-   __shared__ unsigned lcnt[256], lofs[256], gofs[256], wsum[4];
-   const long long total = a.bin_start[a.nbins];
-   const long long r0 = (long long)blockIdx.x * FL3_PART2_RECORDS;
-   if (r0 >= total) return;
-   const RT *in = (const RT *)a.sorted;
-   RT *out = (RT *)a.final;
-   RT v[FL3_PART2_PER];
-   for (int k = 0; k < FL3_PART2_PER; k++) {
-      const long long r = r0 + k * 256 + threadIdx.x;
-      v[k] = r < total ? in[r] : (RT)FL3_REC_NONE;
-   }
-   const long long rl = (total < r0 + FL3_PART2_RECORDS ? total : r0 + FL3_PART2_RECORDS) - 1;
-   const int t_lo = (int)((rel_cell(a, in[r0]) >> a.shift) & ~((1u << FL3_SUPER_SHIFT) - 1u));
-   const int t_hi = (int)((rel_cell(a, in[rl]) >> a.shift) | ((1u << FL3_SUPER_SHIFT) - 1u));
-   if (t_hi - t_lo >= 256) {
-      for (int k = 0; k < FL3_PART2_PER; k++)
-         if (!rec_none(v[k])) out[atomicAdd(&a.cursor[rel_cell(a, v[k]) >> a.shift], 1u)] = v[k];
-      return;
-   }
-   lcnt[threadIdx.x] = 0;
-   __syncthreads();
-   unsigned rank[FL3_PART2_PER];
-   for (int k = 0; k < FL3_PART2_PER; k++)
-      if (!rec_none(v[k])) rank[k] = atomicAdd(&lcnt[(rel_cell(a, v[k]) >> a.shift) - t_lo], 1u);
-   __syncthreads();
-   const int b = t_lo + (int)threadIdx.x;
-   const unsigned c = lcnt[threadIdx.x];   // (zero past t_hi and the last tile)
-   unsigned tot;
-   const unsigned l = wg_excl_scan256(c, wsum, &tot);
-   lofs[threadIdx.x] = l;
-   gofs[threadIdx.x] = c ? atomicAdd(&a.cursor[b], c) : 0u;
-   __syncthreads();
-   if (sizeof(RT) == 4) {
-      for (int k = 0; k < FL3_PART2_PER; k++)
-         if (!rec_none(v[k])) stage[lofs[(rel_cell(a, v[k]) >> a.shift) - t_lo] + rank[k]] = v[k];
-      __syncthreads();
-      for (unsigned j = threadIdx.x; j < tot; j += 256) {
-         const RT w = stage[j];
-         const unsigned bb = (rel_cell(a, w) >> a.shift) - (unsigned)t_lo;
-         out[gofs[bb] + (j - lofs[bb])] = w;
-      }
-   } else
-      for (int k = 0; k < FL3_PART2_PER; k++)
-         if (!rec_none(v[k])) out[gofs[(rel_cell(a, v[k]) >> a.shift) - t_lo] + rank[k]] = v[k];
 }
 
 // Persistent workgroups take work items (tile, chunk of its records) from a
@@ -351,7 +255,7 @@ __global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum(BinArgs a) {
    for (int e = threadIdx.x; e < h->nxf && e < 256; e += blockDim.x) vis[e] = (float)px[e].vis;
    const int linear = h->palette_mode == 1;
    const long long total_items = a.item_start[a.nbins];
-   const RT *sorted = (const RT *)a.final;
+   const RT *sorted = (const RT *)a.sorted;
    for (;;) {
       __syncthreads();
       if (threadIdx.x == 0) item_sh = (int)atomicAdd(a.item_counter, 1u);
@@ -529,7 +433,7 @@ __global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum_narrow(BinArgs a)
    unsigned b = in_item(0, 0), first = in_item(0, 1), place = in_item(0, 3);
    int n = (int)in_item(0, 2);
    auto fetch = [&](RT(&v)[U], int at) {
-      const RT *in = (const RT *)a.final + first;
+      const RT *in = (const RT *)a.sorted + first;
       for (int u = 0; u < U; u++) v[u] = in[min(at + u * FL3_ACC_THREADS + tid, n - 1)];
    };
    RT v[U], nx[U];
@@ -667,8 +571,7 @@ __global__ __launch_bounds__(256) void k_bin_merge(BinArgs a) {
 
 // Counting pass of a band (the walkers' counting for records sorted by band
 // first): workgroup k counts the records of its block of rows x 256 slots
-// per tile in LDS, adds the counts to bin_total and stores its counts per
-// super-tile at blk_hist[k][super-tile].
+// per tile in LDS and adds the counts to bin_total.
 template <typename RT>
 __global__ __launch_bounds__(256) void k_bin_count(BinArgs a) {
    unsigned *hist = (unsigned *)fl3_lds;   // [nbins]
@@ -691,12 +594,6 @@ __global__ __launch_bounds__(256) void k_bin_count(BinArgs a) {
    __syncthreads();
    for (int b = threadIdx.x; b < a.nbins; b += blockDim.x)
       if (hist[b]) atomicAdd(&a.bin_total[b], hist[b]);
-   for (int sp = threadIdx.x; sp < a.nsuper; sp += blockDim.x) {
-      const int b0 = sp << FL3_SUPER_SHIFT, b1 = min(a.nbins, b0 + (1 << FL3_SUPER_SHIFT));
-      unsigned c = 0;
-      for (int b = b0; b < b1; b++) c += hist[b];
-      a.blk_hist[(size_t)blockIdx.x * a.nsuper + sp] = c;
-   }
 }
 
 // Accumulation into bits-64 (double) buckets.  Each record adds what the
@@ -734,7 +631,7 @@ __global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum_f64(BinArgs a) {
    const int linear = h->palette_mode == 1;
    const unsigned long long hits = (unsigned long long)__double2ll_rn(255.0 * FL3_F64_FIX);
    const long long total_items = a.item_start[a.nbins];
-   const RT *sorted = (const RT *)a.final;
+   const RT *sorted = (const RT *)a.sorted;
    for (;;) {
       __syncthreads();
       if (threadIdx.x == 0) item_sh = (int)atomicAdd(a.item_counter, 1u);
@@ -846,99 +743,104 @@ extern "C" size_t fl3k_bin_lds_bytes(int shift) {
    return (size_t)20 * ((size_t)1 << shift) + 8 * 1024 + 4 * 256 + 64;
 }
 
-extern "C" int fl3k_launch_bin(const BinArgs *a, int ncu, int format, hipStream_t s) {
+template <typename RT, typename OT, int NT, int P, int MT, bool FEW = false>
+static void launch_sort(const BinArgs *a, int sh, unsigned *cursor, hipStream_t s) {
+   const size_t lds = sizeof(RT) * NT * P + 6 * (size_t)MT;
+   if (lds > 65536)
+      (void)hipFuncSetAttribute((const void *)k_bin_sort<RT, OT, NT, P, MT, FEW>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+   const long long slots = a->rec_count ? a->rec_count : a->walkers * a->rows;
+   const unsigned g = (unsigned)((slots + (long long)NT * P - 1) / ((long long)NT * P));
+   if (g) hipLaunchKernelGGL((k_bin_sort<RT, OT, NT, P, MT, FEW>), dim3(g), dim3(NT), lds, s, *a, sh, cursor);
+}
+
+// Scans of the walkers' counts, and the records grouped by tile into a->sorted:
+// with 128 KB of records a workgroup, or half that where two workgroups then
+// fit a CU (15M records to 75 tiles: 41 us, 63 us with half as many wavefronts)
+// and 96 KB where the tiles' counts need the room.
+template <typename RT>
+static void sort_records(const BinArgs *a, hipStream_t s) {
+   constexpr int P = 128 / sizeof(RT);
    hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(1024), 0, s, *a);
-   hipLaunchKernelGGL(k_super_off, dim3(a->nsuper), dim3(256), 0, s, *a);
-   const unsigned g2 = (unsigned)(((long long)a->walkers * a->rows + FL3_PART2_RECORDS - 1) / FL3_PART2_RECORDS);
-   // the staging area of 4-byte records (8-byte records: none)
-   const size_t lds2_4 = 4 * (size_t)FL3_PART2_RECORDS, lds2_8 = 0;
+   if (a->nbins <= 256)
+      launch_sort<RT, RT, 1024, P / 2, 256>(a, a->shift, a->cursor, s);
+   else if (a->nbins <= 1024)
+      launch_sort<RT, RT, 1024, P, 1024>(a, a->shift, a->cursor, s);
+   else if (a->nbins <= 3072)
+      launch_sort<RT, RT, 1024, P, 3072>(a, a->shift, a->cursor, s);
+   else if (a->nbins <= 5120)
+      launch_sort<RT, RT, 1024, P, 5120>(a, a->shift, a->cursor, s);
+   else
+      launch_sort<RT, RT, 1024, P * 3 / 4, FL3_MAX_BINS>(a, a->shift, a->cursor, s);
+}
+
+extern "C" int fl3k_launch_bin_sort(const BinArgs *a, int format, hipStream_t s) {
+   if (format == 1 || format == FL3_BIN_F64_NARROW)
+      sort_records<unsigned>(a, s);
+   else
+      sort_records<unsigned long long>(a, s);
+   return hipGetLastError() != hipSuccess;
+}
+
+template <typename RT>
+static void launch_f64(const BinArgs *a, int ncu, hipStream_t s) {
+   const size_t lf = fl3k_bin_f64_lds_bytes(a->shift);
+   const unsigned gf = (unsigned)ncu * (lf > 81920 ? 1 : (lf > 54000 ? 2 : 3));
+   if (lf > 65536)
+      (void)hipFuncSetAttribute((const void *)k_bin_accum_f64<RT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lf);
+   hipLaunchKernelGGL(k_bin_accum_f64<RT>, dim3(gf), dim3(FL3_ACC_THREADS), lf, s, *a);
+}
+template <typename RT, bool JOBREC>
+static void launch_accum(const BinArgs *a, int ncu, hipStream_t s) {
    const size_t lds = fl3k_bin_lds_bytes(a->shift);
    const unsigned gacc = (unsigned)ncu * (lds > 65536 ? 1 : 3);
-   const int big = lds > 65536;
-   if (format == FL3_BIN_F64_WIDE || format == FL3_BIN_F64_NARROW) {
-      // double buckets: 8- or 4-byte records, accumulated in double
-      const size_t lf = fl3k_bin_f64_lds_bytes(a->shift);
-      const unsigned gf = (unsigned)ncu * (lf > 81920 ? 1 : (lf > 54000 ? 2 : 3));
-      if (format == FL3_BIN_F64_NARROW) {
-         if (a->rows >= FL3_PART1_STAGED_ROWS)
-            hipLaunchKernelGGL(k_bin_part1_staged<unsigned>, dim3(a->nblk), dim3(256), 0, s, *a);
-         else
-            hipLaunchKernelGGL(k_bin_part1<unsigned>, dim3(a->nblk), dim3(256), 0, s, *a);
-         if (g2) hipLaunchKernelGGL(k_bin_part2<unsigned>, dim3(g2), dim3(256), lds2_4, s, *a);
-         if (lf > 65536)
-            (void)hipFuncSetAttribute((const void *)k_bin_accum_f64<unsigned>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lf);
-         hipLaunchKernelGGL(k_bin_accum_f64<unsigned>, dim3(gf), dim3(FL3_ACC_THREADS), lf, s, *a);
-      } else {
-         hipLaunchKernelGGL(k_bin_part1<unsigned long long>, dim3(a->nblk), dim3(256), 0, s, *a);
-         if (g2) hipLaunchKernelGGL(k_bin_part2<unsigned long long>, dim3(g2), dim3(256), lds2_8, s, *a);
-         if (lf > 65536)
-            (void)hipFuncSetAttribute((const void *)k_bin_accum_f64<unsigned long long>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lf);
-         hipLaunchKernelGGL(k_bin_accum_f64<unsigned long long>, dim3(gf), dim3(FL3_ACC_THREADS), lf, s, *a);
-      }
-      return hipGetLastError() != hipSuccess;
-   }
-   if ((format == 1 || format == 2) && a->round > 0 && a->shift == FL3_PACKED_SHIFT) {
-      const bool job = format == 2;
-      if (job) {
-         hipLaunchKernelGGL(k_bin_part1<unsigned long long>, dim3(a->nblk), dim3(256), 0, s, *a);
-         if (g2) hipLaunchKernelGGL(k_bin_part2<unsigned long long>, dim3(g2), dim3(256), lds2_8, s, *a);
-      } else {
-         if (a->rows >= FL3_PART1_STAGED_ROWS)
-            hipLaunchKernelGGL(k_bin_part1_staged<unsigned>, dim3(a->nblk), dim3(256), 0, s, *a);
-         else
-            hipLaunchKernelGGL(k_bin_part1<unsigned>, dim3(a->nblk), dim3(256), 0, s, *a);
-         if (g2) hipLaunchKernelGGL(k_bin_part2<unsigned>, dim3(g2), dim3(256), lds2_4, s, *a);
-      }
+   if (lds > 65536)
+      (void)hipFuncSetAttribute((const void *)k_bin_accum<RT, JOBREC>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+   hipLaunchKernelGGL((k_bin_accum<RT, JOBREC>), dim3(gacc), dim3(FL3_ACC_THREADS), lds, s, *a);
+}
+
+// The sorted records added to the histogram.
+extern "C" int fl3k_launch_bin_accum(const BinArgs *a, int ncu, int format, hipStream_t s) {
+   if (format == FL3_BIN_F64_WIDE)
+      launch_f64<unsigned long long>(a, ncu, s);
+   else if (format == FL3_BIN_F64_NARROW)
+      launch_f64<unsigned>(a, ncu, s);
+   else if ((format == 1 || format == 2) && a->round > 0 && a->shift == FL3_PACKED_SHIFT) {
       const bool rgb = a->alpha >= 0;
-      if (job)
+      if (format == 2)
          rgb ? launch_narrow<true, true>(a, ncu, s) : launch_narrow<true, false>(a, ncu, s);
       else
          rgb ? launch_narrow<false, true>(a, ncu, s) : launch_narrow<false, false>(a, ncu, s);
-   } else if (format == 1) {
-      if (a->rows >= FL3_PART1_STAGED_ROWS)
-         hipLaunchKernelGGL(k_bin_part1_staged<unsigned>, dim3(a->nblk), dim3(256), 0, s, *a);
-      else
-         hipLaunchKernelGGL(k_bin_part1<unsigned>, dim3(a->nblk), dim3(256), 0, s, *a);
-      if (g2) hipLaunchKernelGGL(k_bin_part2<unsigned>, dim3(g2), dim3(256), lds2_4, s, *a);
-      if (big)
-         (void)hipFuncSetAttribute((const void *)k_bin_accum<unsigned, false>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      hipLaunchKernelGGL((k_bin_accum<unsigned, false>), dim3(gacc), dim3(FL3_ACC_THREADS), lds, s, *a);
-   } else {
-      hipLaunchKernelGGL(k_bin_part1<unsigned long long>, dim3(a->nblk), dim3(256), 0, s, *a);
-      if (g2) hipLaunchKernelGGL(k_bin_part2<unsigned long long>, dim3(g2), dim3(256), lds2_8, s, *a);
-      if (format == 2) {
-         if (big)
-            (void)hipFuncSetAttribute((const void *)k_bin_accum<unsigned long long, true>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-         hipLaunchKernelGGL((k_bin_accum<unsigned long long, true>), dim3(gacc), dim3(FL3_ACC_THREADS), lds, s, *a);
-      } else {
-         if (big)
-            (void)hipFuncSetAttribute((const void *)k_bin_accum<unsigned long long, false>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-         hipLaunchKernelGGL((k_bin_accum<unsigned long long, false>), dim3(gacc), dim3(FL3_ACC_THREADS), lds, s, *a);
-      }
-   }
-   return hipGetLastError() != hipSuccess;
-}
-
-// Banded histograms, first level: the walkers' 8-byte records grouped by
-// super-tile (the bands) into a->sorted: scans of the walkers' counts and the
-// first sort pass only.
-extern "C" int fl3k_launch_bin_split(const BinArgs *a, int narrow_out, hipStream_t s) {
-   hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(1024), 0, s, *a);
-   hipLaunchKernelGGL(k_super_off, dim3(a->nsuper), dim3(256), 0, s, *a);
-   if (narrow_out)
-      hipLaunchKernelGGL((k_bin_part1<unsigned long long, unsigned>), dim3(a->nblk), dim3(256), 0, s, *a);
+   } else if (format == 1)
+      launch_accum<unsigned, false>(a, ncu, s);
+   else if (format == 2)
+      launch_accum<unsigned long long, true>(a, ncu, s);
    else
-      hipLaunchKernelGGL(k_bin_part1<unsigned long long>, dim3(a->nblk), dim3(256), 0, s, *a);
+      launch_accum<unsigned long long, false>(a, ncu, s);
    return hipGetLastError() != hipSuccess;
 }
 
-// Banded histograms, second level: per-tile and per-block counts of one
-// band's 8-byte records (a->rec, a->rec_count of them, as a->nblk blocks of
+// Banded histograms, first level: scans of the walkers' counts, and the
+// walkers' 8-byte records grouped by band (1 << FL3_SUPER_SHIFT of the tiles
+// that they counted) into a->sorted.
+extern "C" int fl3k_launch_bin_split(const BinArgs *a, int narrow_out, hipStream_t s) {
+   typedef unsigned long long u64;
+   const int sh = a->shift + FL3_SUPER_SHIFT;
+   hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(1024), 0, s, *a);
+   // with a few bands nearly all of a wavefront's records meet at one counter: 64
+   // counters a band then, one for each lane (4 bands, 2^28 records: 1.1 ms with
+   // one, 0.8 ms so)
+   const bool few = a->nbins <= 16 << FL3_SUPER_SHIFT;
+   if (narrow_out)
+      few ? launch_sort<u64, unsigned, 1024, 16, 1024, true>(a, sh, a->band_cursor, s)
+          : launch_sort<u64, unsigned, 1024, 16, 256>(a, sh, a->band_cursor, s);
+   else
+      few ? launch_sort<u64, u64, 1024, 16, 1024, true>(a, sh, a->band_cursor, s)
+          : launch_sort<u64, u64, 1024, 16, 256>(a, sh, a->band_cursor, s);
+   return hipGetLastError() != hipSuccess;
+}
+
+// Banded histograms, second level: per-tile counts of one band's 8-byte records (a->rec, a->rec_count of them, as a->nblk blocks of
 // a->rows x 256), before fl3k_launch_bin sorts and accumulates them.
 extern "C" int fl3k_launch_bin_count(const BinArgs *a, int narrow, hipStream_t s) {
    const size_t l = sizeof(unsigned) * (size_t)a->nbins;   // at most FL3_MAX_BINS: 32 KiB

@@ -19,7 +19,8 @@ int fl3k_launch_apply_fp32_tier(const unsigned char *job, int xi, const double *
                                 unsigned long long key, size_t lds, hipStream_t s, int tier);
 /* format: 0 8-byte records, 1 4-byte records, 2 8-byte job records;
  * FL3_BIN_F64_WIDE / FL3_BIN_F64_NARROW: 8- / 4-byte records into double buckets */
-int fl3k_launch_bin(const BinArgs *a, int ncu, int format, hipStream_t s);
+int fl3k_launch_bin_sort(const BinArgs *a, int format, hipStream_t s);
+int fl3k_launch_bin_accum(const BinArgs *a, int ncu, int format, hipStream_t s);
 /* banded histograms: the first level (scans and the band pass, writing
  * 4-byte band records when narrow_out), the second level's counting pass */
 int fl3k_launch_bin_split(const BinArgs *a, int narrow_out, hipStream_t s);

@@ -19,8 +19,7 @@
 // start, the per-sub-batch procedure of rect.c:393-400 with one long
 // sub-batch per walker; with WAVE (genomes without xaos) the xform is drawn
 // per wavefront and the workgroup's points change lanes after every step.  In
-// record mode each workgroup also counts its records per tile in LDS and
-// stores them per super-tile at blk_hist[block][super-tile].
+// record mode each workgroup also counts its records per tile in LDS.
 // Waves per SIMD the walker kernel is compiled for: the classic tier (the
 // variations of most genomes) at 8, which holds it to 64 VGPRs (a few
 // spills; 7 waves at its natural 67-78 VGPRs ran 11% slower per launch),
@@ -540,19 +539,11 @@ __global__ __launch_bounds__(256, walker_waves<TIER>()) void k_iter_fast(IterArg
       for (long long i = n; i < a.rows_out; i++)
          ((unsigned *)a.rec)[(blk * a.rows_out + i) * 256 + threadIdx.x] = FL3_REC_NONE;
    if (RECORDS) {
-      // tile counts summed over workgroups, and this workgroup's counts per
-      // super-tile (FL3_SUPER tiles) for the first sort pass
+      // tile counts summed over workgroups
       __syncthreads();
       for (int b = threadIdx.x; b < a.nbins; b += blockDim.x) {
          const unsigned c = bh[b];
          if (c) atomicAdd(&a.bin_total[b], c);
-      }
-      const int nsuper = (a.nbins + (1 << FL3_SUPER_SHIFT) - 1) >> FL3_SUPER_SHIFT;
-      for (int sp = threadIdx.x; sp < nsuper; sp += blockDim.x) {
-         const int b0 = sp << FL3_SUPER_SHIFT, b1 = min(a.nbins, b0 + (1 << FL3_SUPER_SHIFT));
-         unsigned c = 0;
-         for (int b = b0; b < b1; b++) c += bh[b];
-         a.blk_hist[(size_t)blk * nsuper + sp] = c;
       }
    }
    if (ws) {

@@ -71,3 +71,18 @@ def test_direct_deposits_on_both_sides_of_their_bound(prod, quality, opacity):
     b, sb = prod.render(g, seed="pairs", deposit=2, nchan=4, transp=1)
     assert sa["num_iters"] == sb["num_iters"] == quality * 64 * 64
     assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("opacity", [1.0, 0.5])
+@pytest.mark.parametrize("width,height,quality", [
+    (40, 30, 3), (1000, 1024, 3), (1040, 1024, 3), (2040, 2040, 2), (2060, 2060, 2),      # about 256, 1024 tiles
+    (3060, 4070, 1), (3100, 4096, 1), (4560, 4570, 0.5), (4640, 4640, 0.5), (5760, 5760, 0.4)])   # 3072, 5120, 8192
+def test_sort_by_the_number_of_tiles(prod, width, height, quality, opacity):
+    """Records of 4 and (an opacity below 1, or 2^24 cells) 8 bytes, sorted by
+    each form's workgroups, the last of a chunk partly filled."""
+    g = _shaded(G.synthetic_small(seed=43, width=width, height=height, quality=quality), "bytes")
+    g.xforms[1].opacity = opacity
+    a, _ = prod.render(g, seed="sort", deposit=1)
+    b, _ = prod.render(g, seed="sort", deposit=2, chunk_samples=700001)
+    assert np.array_equal(a, b)
+    assert a.any()
