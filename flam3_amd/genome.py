@@ -177,12 +177,15 @@ class Genome:
         g.temporal_filter_width = self.temporal_filter_width
         g.temporal_filter_exp = self.temporal_filter_exp
         pal = self.palette if self.palette is not None else np.full((256, 3), 255.0)
-        for i in range(256):
-            e = g.palette[i]
-            e.color[3] = 255.0 / 255.0
-            for k in range(3):
-                e.color[k] = e.color[3] * float(pal[i][k]) / 255.0
-            e.index = float(i)
+        # (index, colour and alpha of every entry at once: entry by entry took
+        # longer than a small preview's render)
+        pal = np.asarray(pal, dtype=np.float64)
+        if len(pal) < 256:
+            raise IndexError("a palette has 256 entries, not %d" % len(pal))
+        entries = np.ones((256, 5))
+        entries[:, 0] = np.arange(256)
+        entries[:, 1:4] = pal[:256, :3] / 255.0
+        ctypes.memmove(g.palette, entries.ctypes.data, entries.nbytes)
         xf = ctypes.cast(g.xform, abi.XFORM_P)
         nstd = len(self.xforms)
         for i, x in enumerate(self.xforms):
