@@ -567,12 +567,9 @@ static int ensure_chunk_bufs(long long nchunks, size_t rec_bytes, size_t tot_byt
 
 // Tile shift of the binned deposit for the current histogram (cells per
 // tile = 1 << shift), or 0 when the histogram is too large for it.
-static int bin_shift_cells(long long ncells);
 static int bin_shift_cells(long long ncells) {
-   // 4096-cell tiles when LDS allows (fewer, larger scatter runs), else 2048
-   for (int sh = 12; sh >= 11; sh--)
-      if (((ncells + (1LL << sh) - 1) >> sh) <= FL3_MAX_BINS && fl3k_bin_lds_bytes(sh) <= g_ctx.lds_max) return sh;
-   return 0;
+   const int sh = FL3_TILE_SHIFT;
+   return ((ncells + (1LL << sh) - 1) >> sh) <= FL3_MAX_BINS && fl3k_bin_lds_bytes() <= g_ctx.lds_max ? sh : 0;
 }
 
 // Tile shift of the accumulation into double buckets (bits 64: five doubles
@@ -590,9 +587,8 @@ static int acc_tile_shift(long long ncells, int bits, int *band) {
    int sh = 0;
    if (bits == 64)
       sh = f64_tile_shift();
-   else
-      for (int t = 12; t >= 11 && !sh; t--)
-         if (fl3k_bin_lds_bytes(t) <= g_ctx.lds_max) sh = t;
+   else if (fl3k_bin_lds_bytes() <= g_ctx.lds_max)
+      sh = FL3_TILE_SHIFT;
    *band = 0;
    if (!sh) return 0;
    if (((ncells + (1LL << sh) - 1) >> sh) > FL3_MAX_BINS) {
@@ -727,7 +723,7 @@ static int upload_job_tables(const fl3_job_hdr *const *h, int n, int nxf_max, Bi
 // entries below 256, the tiles hold 4096 cells and the walker's LDS
 // has room for the palette after its tile counts.
 static bool colour_records(const fl3_job_hdr *const *h, int n, const uint32_t *pal8, int shift, size_t lds_walker) {
-   return pal8 && shift == FL3_PACKED_SHIFT && job_records_packed(h, n) &&
+   return pal8 && shift == FL3_TILE_SHIFT && job_records_packed(h, n) &&
           ((lds_walker + 15) & ~(size_t)15) + 1024 <= g_ctx.lds_max;
 }
 
@@ -781,16 +777,17 @@ static int item_records(const fl3_job_hdr *const *h, int n, int fixed64 = 0) {
    return c < 1 ? 1 : c;
 }
 
-// Work items of the packed accumulation for chunks of up to `records`, and
+// Work items of the accumulation for chunks of up to `records`, and
 // room for their partial sums: one for each of two workgroups a CU, of at least
 // two of their steps and at most 2^17 records.  (3.6M records on 256 CUs: items
 // of 2^14 take 17 us with the merge, of 2^13 24 us, of 2^18 69 us.  2^28 records:
 // of 2^17 470 us, of 2^16 535 us, as more partial sums are written and read,
 // of 2^18 486 us, as the last ones run alone.)
-static int packed_items(BinArgs *b, long long records) {
+static int accum_items(BinArgs *b, long long records) {
    const int step = fl3k_bin_pass_records();
    const long long c = records / (2 * g_ctx.ncu) / step * step;
-   b->chunk = (int)std::min((long long)b->chunk, std::min(std::max(c, 2LL * step), 1LL << 17));
+   const long long most = records > 1LL << 30 ? 1LL << 18 : 1LL << 17;   // (less room for partial sums)
+   b->chunk = (int)std::min((long long)b->chunk, std::min(std::max(c, 2LL * step), most));
    if (g_ctx.partial.ensure(fl3k_bin_partial_bytes(b, records))) return 1;
    b->partial = g_ctx.partial.p;
    return 0;
@@ -998,7 +995,7 @@ static int iterate_binned(IterArgs a, long long W, long long Wj, const JobSet &j
    lds_rec = with_shuffle(a, lds_rec, jobs_wave_ok(js.h, js.n));
    b.round = narrow || colour ? narrow_round(js.h, npal) : 0;
    b.alpha = b.round > 0 ? narrow_alpha(js.h, npal) : -1;
-   if (b.round > 0 && packed_items(&b, W * per)) return 1;
+   if (g_ctx.bits != 64 && accum_items(&b, W * per)) return 1;
    // chunk k: walkers on the render stream, then its sort and accumulation
    // on the bin stream, which chunk k + 2's walkers wait for before they
    // overwrite the same record buffer
@@ -1388,7 +1385,7 @@ extern "C" int fl3d_iterate_multi(const fl3d_multi_job *jobs, int njobs, int fus
          if (colour) lds_r = ar.pal_off + 1024;
          b.round = narrow || colour ? narrow_round(rh.data(), (int)rh.size()) : 0;
          b.alpha = b.round > 0 ? narrow_alpha(rh.data(), (int)rh.size()) : -1;
-         if (b.round > 0 && packed_items(&b, Wrec * per)) return 1;
+         if (accum_items(&b, Wrec * per)) return 1;
       }
       const size_t lds_r_lane = lds_r;
       lds_r = with_shuffle(ar, lds_r, true);

@@ -82,7 +82,7 @@ struct IterArgs {
 
 #define FL3_BIN_CHUNK_SAMPLES (1LL << 28)
 #define FL3_CHUNK_BUFS 2            // record buffers in rotation: the walkers run one chunk ahead of the sort
-#define FL3_PACKED_SHIFT 12          // tiles of the packed accumulation: 4096 cells
+#define FL3_TILE_SHIFT 12            // tiles of 32-bit histograms: 4096 cells
 #define FL3_BIN_ITEM_RECORDS (1 << 18)
 #define FL3_BIN_MIN_SAMPLES (1LL << 20)
 

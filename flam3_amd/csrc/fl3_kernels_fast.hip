@@ -230,131 +230,21 @@ __global__ __launch_bounds__(NT) void k_bin_sort(BinArgs a, int sh, unsigned *cu
    }
 }
 
-// Persistent workgroups take work items (tile, chunk of its records) from a
-// counter.  The tile's channels live in LDS as two 64-bit pairs (R|G, B|A)
-// and the hit count: a work item adds at most 2^18 deltas of at most 255 to
-// a cell, so no 32-bit half carries into the other.  A tile that has one
-// work item is added to the histogram without atomics.
-template <typename RT, bool JOBREC>
-__global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum(BinArgs a) {
-   const fl3_job_hdr *h = (const fl3_job_hdr *)a.job;
-   const int tile_cells = 1 << a.shift;
-   unsigned long long *rg = (unsigned long long *)fl3_lds;   // tile_cells
-   unsigned long long *ba = rg + tile_cells;                  // tile_cells
-   uint32_t *hits = (uint32_t *)(ba + tile_cells);            // tile_cells
-   uint32_t *dmapu = hits + tile_cells;                       // 1024
-   float *dmapf = (float *)(dmapu + 1024);                    // 1024
-   float *vis = dmapf + 1024;                                 // 256
-   __shared__ int item_sh;
-   const double *pd = (const double *)(a.job + h->off_dmap);
-   const fl3_xform_pack *px = (const fl3_xform_pack *)(a.job + h->off_xf);
-   for (int e = threadIdx.x; e < 1024; e += blockDim.x) {
-      dmapu[e] = (uint32_t)pd[e];
-      dmapf[e] = (float)pd[e];
-   }
-   for (int e = threadIdx.x; e < h->nxf && e < 256; e += blockDim.x) vis[e] = (float)px[e].vis;
-   const int linear = h->palette_mode == 1;
-   const long long total_items = a.item_start[a.nbins];
-   const RT *sorted = (const RT *)a.sorted;
-   for (;;) {
-      __syncthreads();
-      if (threadIdx.x == 0) item_sh = (int)atomicAdd(a.item_counter, 1u);
-      for (int e = threadIdx.x; e < tile_cells; e += blockDim.x) {
-         rg[e] = 0;
-         ba[e] = 0;
-         hits[e] = 0;
-      }
-      __syncthreads();
-      const long long item = item_sh;
-      if (item >= total_items) break;
-      int lo = 0, hi = a.nbins - 1;
-      while (lo < hi) {  // last tile whose first item is <= item
-         const int mid = (lo + hi + 1) >> 1;
-         if ((long long)a.item_start[mid] <= item) lo = mid;
-         else hi = mid - 1;
-      }
-      const int b = lo;
-      const long long k = item - a.item_start[b];
-      const long long r0 = (long long)a.bin_start[b] + k * a.chunk;
-      const long long r1 = min((long long)a.bin_start[b + 1], r0 + a.chunk);
-      const bool single = (a.item_start[b + 1] - a.item_start[b]) == 1;
-      const unsigned cell0 = a.cell_base + ((unsigned)b << a.shift);
-      for (long long rb = r0; rb < r1; rb += FL3_ACC_UNROLL * blockDim.x) {
-         RT v[FL3_ACC_UNROLL];
-         for (int u = 0; u < FL3_ACC_UNROLL; u++) {
-            const long long r = rb + u * blockDim.x + threadIdx.x;
-            v[u] = r < r1 ? sorted[r] : (RT)FL3_REC_NONE;
-         }
-         for (int u = 0; u < FL3_ACC_UNROLL; u++) {
-            if (rec_none(v[u])) continue;
-            const unsigned local = rec_cell(v[u]) - cell0;
-            uint32_t d[5];
-            if (sizeof(RT) == 4) {
-               const int ci = (int)((unsigned)v[u] >> 24);
-               for (int c = 0; c < 4; c++) d[c] = dmapu[ci * 4 + c];
-               d[4] = 255u;
-            } else if (JOBREC) {
-               // the record's job selects palette and visibility (stepped palette)
-               const unsigned long long w = (unsigned long long)v[u];
-               const int ci = (int)((w >> 32) & 0xff), fn = (int)((w >> 40) & 0xff), jb = (int)(w >> 48);
-               const float vv = a.vis_all[jb * a.vis_stride + fn];
-               const uint32_t *du = a.dmapu_all + jb * 1024 + ci * 4;
-               if (vv == 1.0f) {
-                  for (int c = 0; c < 4; c++) d[c] = du[c];
-                  d[4] = 255u;
-               } else {
-                  const float *df = a.dmapf_all + jb * 1024 + ci * 4;
-                  for (int c = 0; c < 4; c++) d[c] = (uint32_t)(vv * df[c]);
-                  d[4] = (uint32_t)(vv * 255.0f);
-               }
-            } else {
-               const unsigned long long w = (unsigned long long)v[u];
-               const int ci = (int)((w >> 32) & 0xff), fn = (int)((w >> 40) & 0xff);
-               const float vv = vis[fn];
-               if (linear) {
-                  const float f = (float)(w >> 48) * (1.0f / 65535.0f);
-                  for (int c = 0; c < 4; c++) {
-                     const float col = dmapf[ci * 4 + c] * (1.0f - f) + dmapf[ci * 4 + 4 + c] * f;
-                     d[c] = (uint32_t)(vv == 1.0f ? col : vv * col);
-                  }
-               } else if (vv == 1.0f) {
-                  for (int c = 0; c < 4; c++) d[c] = dmapu[ci * 4 + c];
-               } else {
-                  for (int c = 0; c < 4; c++) d[c] = (uint32_t)(vv * dmapf[ci * 4 + c]);
-               }
-               d[4] = vv == 1.0f ? 255u : (uint32_t)(vv * 255.0f);
-            }
-            atomicAdd(&rg[local], (unsigned long long)d[0] | ((unsigned long long)d[1] << 32));
-            atomicAdd(&ba[local], (unsigned long long)d[2] | ((unsigned long long)d[3] << 32));
-            atomicAdd(&hits[local], d[4]);
-         }
-      }
-      __syncthreads();
-      uint32_t *bk = (uint32_t *)a.buckets + (size_t)cell0 * 5;
-      const long long ncells = (long long)a.width * a.height;
-      const int nvalid = (int)min((long long)tile_cells, ncells - (long long)cell0);
-      for (int e = threadIdx.x; e < nvalid * 5; e += blockDim.x) {
-         const int cl = e / 5, ch = e % 5;
-         const uint32_t v = ch == 4 ? hits[cl] : (uint32_t)((ch < 2 ? rg[cl] : ba[cl]) >> (32 * (ch & 1)));
-         if (!v) continue;
-         if (single) {
-            const unsigned long long s2 = (unsigned long long)bk[e] + v;
-            bk[e] = s2 > 0xffffffffull ? 0xffffffffu : (uint32_t)s2;
-         } else
-            sat_add(bk + e, v);
-      }
-   }
-}
-
-// Accumulation of records of visibility 1 with a stepped palette (a record
-// adds its palette entry and 255 hits): 4-byte records, or job records that
-// carry the entry's bytes (palettes of entries below 256).  The tile's cells
-// live in LDS as packed sums, and a round of at most `round` records keeps
-// every field below its width, after which each thread folds the CPT cells it
-// owns into registers and clears them.  The sums of a tile of one work item
+// Accumulation of the sorted records: persistent workgroups take work items (a
+// tile's records, or a.chunk of them), sum them in LDS and fold the sums into
+// registers, a thread the CPT cells it owns.  The sums of a tile of one work item
 // are then added to the histogram; those of the items of a fuller tile go to an
 // array of partial sums, which k_bin_merge adds up.  (Atomic adds from every
 // item's 20 channels a thread ran at 1e11 a second: 0.2 us an item.)
+//
+// ACC_NARROW (4-byte records) and ACC_COLOUR (job records that carry the
+// entry's bytes, palettes of entries below 256) are of visibility 1 with a stepped
+// palette: a record adds its palette entry and 255 hits.  The tile's cells are
+// packed sums, and a round of at most `round` records keeps every field below its
+// width.  The others (linear palettes, visibilities below 1, entries too bright for
+// a round) take one round, in two 64-bit pairs (R|G, B|A) and a hit count: an item
+// adds at most 2^18 deltas of at most 255 to a cell, so no 32-bit half carries.
+//
 // Bound by LDS atomics, so a record makes as few as its fields allow.  RGB:
 // every palette entry is below 256 and has alpha a.alpha, so alpha is a
 // multiple of the count and a cell is R:24 | G:24 | count:16 and B:32 (one
@@ -368,7 +258,9 @@ __global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum(BinArgs a) {
 // At 1920x1080 with 2x2 supersampling (2^28 records of 4 bytes a launch) 606 us
 // with 2^18-record items added by atomics, 470 us so with the merge (LDS active
 // half of the time, 4 TB/s); 256x256 (3.6M records) 94 and 17 us, 640x480
-// (15M) 105 and 48 us; 48 previews' 8-byte records 398 and 339 us.
+// (15M) 105 and 48 us; 48 previews' 8-byte records 398 and 339 us; 47M records of
+// a linear palette and visibilities below 1 483 us and 242 us.
+enum { ACC_NARROW, ACC_COLOUR, ACC_PLAIN4, ACC_WIDE, ACC_JOB };
 #define FL3_ACC_AHEAD 8   // records a thread loads ahead
 // 16-byte words of an item's partial sums: per cell R, G, B, count, then the
 // alphas if they are not a multiple of the count
@@ -379,16 +271,22 @@ __device__ __forceinline__ uint32_t add_u32_sat(uint32_t x, uint32_t y) {
    const uint32_t t = x + y;
    return t < x ? 0xffffffffu : t;
 }
-template <bool JOB, bool RGB>
-__global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum_narrow(BinArgs a) {
-   typedef typename std::conditional<JOB, unsigned long long, unsigned>::type RT;
+template <int KIND, bool RGB>
+__global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum(BinArgs a) {
+   constexpr bool PACKED = KIND == ACC_NARROW || KIND == ACC_COLOUR;
+   typedef typename std::conditional<KIND == ACC_NARROW || KIND == ACC_PLAIN4, unsigned, unsigned long long>::type RT;
    typedef typename std::conditional<RGB, unsigned, unsigned long long>::type PT;
    const fl3_job_hdr *h = (const fl3_job_hdr *)a.job;
-   constexpr int tile_cells = 1 << FL3_PACKED_SHIFT, CPT = tile_cells / FL3_ACC_THREADS, U = FL3_ACC_AHEAD, step = U * FL3_ACC_THREADS;
+   constexpr int tile_cells = 1 << FL3_TILE_SHIFT, CPT = tile_cells / FL3_ACC_THREADS, U = FL3_ACC_AHEAD, step = U * FL3_ACC_THREADS;
    unsigned long long *p0 = (unsigned long long *)fl3_lds;   // tile_cells
    PT *p1 = (PT *)(p0 + tile_cells);                           // tile_cells
    ulonglong2 *pal = (ulonglong2 *)(p1 + tile_cells);          // 256 (RGB: bytes R, G, B)
    unsigned *pal8 = (unsigned *)pal;
+   // (not packed:)
+   uint32_t *hits = (uint32_t *)(p1 + tile_cells);             // tile_cells
+   uint32_t *dmapu = hits + tile_cells;                        // 1024
+   float *dmapf = (float *)(dmapu + 1024);                     // 1024
+   float *vis = dmapf + 1024;                                  // 256
    // work items, alternating: the one drawn after the next, and of the next its
    // tile, first record, records, and place among the partial sums + 1 (0: the
    // tile's only item)
@@ -396,7 +294,16 @@ __global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum_narrow(BinArgs a)
    __shared__ uint4 found[2];
    const int tid = threadIdx.x;
    const double *pd = (const double *)(a.job + h->off_dmap);
-   if (!JOB)
+   if (!PACKED) {
+      const fl3_xform_pack *px = (const fl3_xform_pack *)(a.job + h->off_xf);
+      for (int e = tid; e < 1024; e += FL3_ACC_THREADS) {
+         dmapu[e] = (uint32_t)pd[e];
+         dmapf[e] = (float)pd[e];
+      }
+      for (int e = tid; e < h->nxf && e < 256; e += FL3_ACC_THREADS) vis[e] = (float)px[e].vis;
+   }
+   const int linear = h->palette_mode == 1;
+   if (KIND == ACC_NARROW)
       for (int e = tid; e < 256; e += FL3_ACC_THREADS) {
          const uint32_t r = (uint32_t)pd[4 * e], g = (uint32_t)pd[4 * e + 1], bb = (uint32_t)pd[4 * e + 2], al = (uint32_t)pd[4 * e + 3];
          if (RGB)
@@ -411,9 +318,10 @@ __global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum_narrow(BinArgs a)
    for (int e = tid; e < tile_cells; e += FL3_ACC_THREADS) {
       p0[e] = 0;
       p1[e] = 0;
+      if (!PACKED) hits[e] = 0;
    }
    const unsigned total_items = a.item_start[a.nbins];
-   const int round_steps = a.round / step;
+   const int round_steps = PACKED ? a.round / step : INT_MAX;
    auto look_up = [&](unsigned item, int slot) {
       for (int b = tid; b < a.nbins; b += FL3_ACC_THREADS) {
          const unsigned i0 = a.item_start[b], i1 = a.item_start[b + 1], r0 = a.bin_start[b], r1 = a.bin_start[b + 1];
@@ -448,18 +356,52 @@ __global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum_narrow(BinArgs a)
          for (int c = 0; c < (RGB ? 4 : 5); c++) acc[j][c] = 0;
       auto add = [&](RT v) {
          const unsigned local = (unsigned)v & (unsigned)(tile_cells - 1);   // (a tile starts at a multiple of its cells)
-         if (RGB) {
-            const unsigned c = JOB ? (unsigned)((unsigned long long)v >> 32) : pal8[(unsigned)v >> 24];
-            atomicAdd(&p0[local], (unsigned long long)((c & 0xffu) | (c >> 8) << 24) | 1ull << 48);
-            atomicAdd(&p1[local], (PT)((c >> 16) & 0xffu));
-         } else if (JOB) {
-            const unsigned c = (unsigned)((unsigned long long)v >> 32);
-            atomicAdd(&p0[local], (unsigned long long)(c & 0xffu) | ((unsigned long long)((c >> 8) & 0xffu) << 24) | (1ull << 48));
-            atomicAdd(&p1[local], (PT)((unsigned long long)((c >> 16) & 0xffu) | ((unsigned long long)(c >> 24) << 32)));
-         } else {
+         if constexpr (KIND == ACC_COLOUR || (KIND == ACC_NARROW && RGB)) {
+            const unsigned c = KIND == ACC_COLOUR ? (unsigned)((unsigned long long)v >> 32) : pal8[(unsigned)v >> 24];
+            atomicAdd(&p0[local], (unsigned long long)((c & 0xffu) | ((c >> 8) & 0xffu) << 24) | 1ull << 48);
+            atomicAdd(&p1[local], (PT)((c >> 16) & 0xffu) | (RGB ? 0 : (PT)((unsigned long long)(c >> 24) << 32)));
+         } else if constexpr (KIND == ACC_NARROW) {
             const ulonglong2 w = pal[(unsigned)v >> 24];
             atomicAdd(&p0[local], w.x);
             atomicAdd(&p1[local], (PT)w.y);
+         } else {
+            uint32_t d[5];
+            const int ci = (int)(((unsigned long long)v >> (KIND == ACC_PLAIN4 ? 24 : 32)) & 0xff);
+            const int fn = KIND == ACC_PLAIN4 ? 0 : (int)(((unsigned long long)v >> 40) & 0xff);
+            const int top = KIND == ACC_PLAIN4 ? 0 : (int)((unsigned long long)v >> 48);
+            if (KIND == ACC_PLAIN4) {
+               for (int c = 0; c < 4; c++) d[c] = dmapu[ci * 4 + c];
+               d[4] = 255u;
+            } else if (KIND == ACC_JOB) {
+               // the record's job selects palette and visibility (stepped palette)
+               const float vv = a.vis_all[top * a.vis_stride + fn];
+               const uint32_t *du = a.dmapu_all + top * 1024 + ci * 4;
+               if (vv == 1.0f) {
+                  for (int c = 0; c < 4; c++) d[c] = du[c];
+                  d[4] = 255u;
+               } else {
+                  const float *df = a.dmapf_all + top * 1024 + ci * 4;
+                  for (int c = 0; c < 4; c++) d[c] = (uint32_t)(vv * df[c]);
+                  d[4] = (uint32_t)(vv * 255.0f);
+               }
+            } else {
+               const float vv = vis[fn];
+               if (linear) {
+                  const float f = (float)top * (1.0f / 65535.0f);
+                  for (int c = 0; c < 4; c++) {
+                     const float col = dmapf[ci * 4 + c] * (1.0f - f) + dmapf[ci * 4 + 4 + c] * f;
+                     d[c] = (uint32_t)(vv == 1.0f ? col : vv * col);
+                  }
+               } else if (vv == 1.0f) {
+                  for (int c = 0; c < 4; c++) d[c] = dmapu[ci * 4 + c];
+               } else {
+                  for (int c = 0; c < 4; c++) d[c] = (uint32_t)(vv * dmapf[ci * 4 + c]);
+               }
+               d[4] = vv == 1.0f ? 255u : (uint32_t)(vv * 255.0f);
+            }
+            atomicAdd(&p0[local], (unsigned long long)d[0] | ((unsigned long long)d[1] << 32));
+            atomicAdd(&p1[local], (PT)((unsigned long long)d[2] | ((unsigned long long)d[3] << 32)));
+            atomicAdd(&hits[local], d[4]);
          }
       };
       for (int at = 0, steps = 0; at < n; at += step) {
@@ -480,10 +422,11 @@ __global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum_narrow(BinArgs a)
             const PT x1 = p1[e];
             p0[e] = 0;
             p1[e] = 0;
-            acc[j][0] += (uint32_t)(x0 & 0xffffffu);
-            acc[j][1] += (uint32_t)((x0 >> 24) & 0xffffffu);
+            acc[j][0] += PACKED ? (uint32_t)(x0 & 0xffffffu) : (uint32_t)x0;
+            acc[j][1] += PACKED ? (uint32_t)((x0 >> 24) & 0xffffffu) : (uint32_t)(x0 >> 32);
             acc[j][2] += (uint32_t)x1;
-            acc[j][3] += (uint32_t)(x0 >> 48);
+            acc[j][3] += PACKED ? (uint32_t)(x0 >> 48) : hits[e];
+            if (!PACKED) hits[e] = 0;
             if (!RGB) acc[j][RGB ? 0 : 4] += (uint32_t)((unsigned long long)x1 >> 32);
          }
          __syncthreads();
@@ -514,7 +457,7 @@ __global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum_narrow(BinArgs a)
          for (int j = 0; j < CPT; j++) {
             for (int c = 0; c < 3; c++) sum[j][c] = acc[j][c];
             sum[j][3] = RGB ? acc[j][3] * (unsigned)a.alpha : acc[j][RGB ? 0 : 4];
-            sum[j][4] = acc[j][3] * 255u;
+            sum[j][4] = acc[j][3] * (PACKED ? 255u : 1u);
          }
          for (int j = 0; j < CPT; j++)
             for (int c = 0; c < 5; c++) {
@@ -537,7 +480,7 @@ __global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum_narrow(BinArgs a)
 
 // Adds up the partial sums of the tiles of several work items and adds them
 // to the histogram: a workgroup takes 256 cells of a tile at a time.
-template <bool RGB>
+template <bool RGB, unsigned HIT>
 __global__ __launch_bounds__(256) void k_bin_merge(BinArgs a) {
    const unsigned cells = 1u << a.shift, parts = cells / 256, units = a.multi[0] * parts;
    const size_t words = part_words(cells, RGB);
@@ -558,7 +501,7 @@ __global__ __launch_bounds__(256) void k_bin_merge(BinArgs a) {
       }
       if (cell >= (size_t)a.width * a.height) continue;
       if (RGB) sum[3] = sum[4] * (unsigned)a.alpha;
-      sum[4] *= 255u;
+      sum[4] *= HIT;
       uint32_t *bk = (uint32_t *)a.buckets + cell * 5;
       uint32_t old[5];
       for (int c = 0; c < 5; c++) old[c] = bk[c];
@@ -722,26 +665,25 @@ __global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum_f64(BinArgs a) {
 extern "C" size_t fl3k_bin_f64_lds_bytes(int shift) { return (size_t)40 * ((size_t)1 << shift) + 8 * (1024 + 1024 + 256) + 64; }
 
 extern "C" int fl3k_bin_pass_records(void) { return FL3_ACC_AHEAD * FL3_ACC_THREADS; }
-template <bool JOB, bool RGB>
-static void launch_narrow(const BinArgs *a, int ncu, hipStream_t s) {
-   const size_t cells = (size_t)1 << FL3_PACKED_SHIFT;
-   const size_t lds = RGB ? 12 * cells + 1024 : 16 * cells + 4096;
+template <int KIND, bool RGB = false>
+static void launch_accum(const BinArgs *a, int ncu, hipStream_t s) {
+   constexpr bool packed = KIND == ACC_NARROW || KIND == ACC_COLOUR;
+   const size_t cells = (size_t)1 << FL3_TILE_SHIFT;
+   const size_t lds = RGB ? 12 * cells + 1024 : packed ? 16 * cells + 4096 : 20 * cells + 9 * 1024;
    if (lds > 65536)
-      (void)hipFuncSetAttribute((const void *)k_bin_accum_narrow<JOB, RGB>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-   hipLaunchKernelGGL((k_bin_accum_narrow<JOB, RGB>), dim3(2u * (unsigned)ncu), dim3(FL3_ACC_THREADS), lds, s, *a);
-   hipLaunchKernelGGL((k_bin_merge<RGB>), dim3(8u * (unsigned)ncu), dim3(256), 0, s, *a);
+      (void)hipFuncSetAttribute((const void *)k_bin_accum<KIND, RGB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+   hipLaunchKernelGGL((k_bin_accum<KIND, RGB>), dim3((packed ? 2u : 1u) * (unsigned)ncu), dim3(FL3_ACC_THREADS), lds, s, *a);
+   hipLaunchKernelGGL((k_bin_merge<RGB, packed ? 255 : 1>), dim3(8u * (unsigned)ncu), dim3(256), 0, s, *a);
 }
-// Bytes of the packed accumulation's partial sums for `records` in a chunk
+// Bytes of the accumulation's partial sums for `records` in a chunk
 // (a tile of several items has more than an item's records, so at most two
 // items for every item's worth of records).
 extern "C" size_t fl3k_bin_partial_bytes(const BinArgs *a, long long records) {
    return 16 * part_words(1u << a->shift, a->alpha >= 0) * (size_t)(2 * records / a->chunk + 1);
 }
 
-extern "C" size_t fl3k_bin_lds_bytes(int shift) {
-   return (size_t)20 * ((size_t)1 << shift) + 8 * 1024 + 4 * 256 + 64;
-}
+// LDS of the accumulation into 32-bit histograms, at most.
+extern "C" size_t fl3k_bin_lds_bytes(void) { return (size_t)20 * ((size_t)1 << FL3_TILE_SHIFT) + 9 * 1024 + 256; }
 
 template <typename RT, typename OT, int NT, int P, int MT, bool FEW = false>
 static void launch_sort(const BinArgs *a, int sh, unsigned *cursor, hipStream_t s) {
@@ -790,33 +732,22 @@ static void launch_f64(const BinArgs *a, int ncu, hipStream_t s) {
       (void)hipFuncSetAttribute((const void *)k_bin_accum_f64<RT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lf);
    hipLaunchKernelGGL(k_bin_accum_f64<RT>, dim3(gf), dim3(FL3_ACC_THREADS), lf, s, *a);
 }
-template <typename RT, bool JOBREC>
-static void launch_accum(const BinArgs *a, int ncu, hipStream_t s) {
-   const size_t lds = fl3k_bin_lds_bytes(a->shift);
-   const unsigned gacc = (unsigned)ncu * (lds > 65536 ? 1 : 3);
-   if (lds > 65536)
-      (void)hipFuncSetAttribute((const void *)k_bin_accum<RT, JOBREC>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-   hipLaunchKernelGGL((k_bin_accum<RT, JOBREC>), dim3(gacc), dim3(FL3_ACC_THREADS), lds, s, *a);
-}
-
 // The sorted records added to the histogram.
 extern "C" int fl3k_launch_bin_accum(const BinArgs *a, int ncu, int format, hipStream_t s) {
    if (format == FL3_BIN_F64_WIDE)
       launch_f64<unsigned long long>(a, ncu, s);
    else if (format == FL3_BIN_F64_NARROW)
       launch_f64<unsigned>(a, ncu, s);
-   else if ((format == 1 || format == 2) && a->round > 0 && a->shift == FL3_PACKED_SHIFT) {
-      const bool rgb = a->alpha >= 0;
-      if (format == 2)
-         rgb ? launch_narrow<true, true>(a, ncu, s) : launch_narrow<true, false>(a, ncu, s);
-      else
-         rgb ? launch_narrow<false, true>(a, ncu, s) : launch_narrow<false, false>(a, ncu, s);
-   } else if (format == 1)
-      launch_accum<unsigned, false>(a, ncu, s);
+   else if (format == 1 && a->round > 0)
+      a->alpha >= 0 ? launch_accum<ACC_NARROW, true>(a, ncu, s) : launch_accum<ACC_NARROW>(a, ncu, s);
+   else if (format == 2 && a->round > 0)
+      a->alpha >= 0 ? launch_accum<ACC_COLOUR, true>(a, ncu, s) : launch_accum<ACC_COLOUR>(a, ncu, s);
+   else if (format == 1)
+      launch_accum<ACC_PLAIN4>(a, ncu, s);
    else if (format == 2)
-      launch_accum<unsigned long long, true>(a, ncu, s);
+      launch_accum<ACC_JOB>(a, ncu, s);
    else
-      launch_accum<unsigned long long, false>(a, ncu, s);
+      launch_accum<ACC_WIDE>(a, ncu, s);
    return hipGetLastError() != hipSuccess;
 }
 
