@@ -513,7 +513,7 @@ __device__ __forceinline__ unsigned de_prep_cell(const DEArgs &a, int i, int j, 
          for (int ii = -ss; ii <= ss; ii++)
             for (int jj = -ss; jj <= ss; jj++) {
                const int y = j + jj;
-               if (y < H) fsel += (double)b[((i + ii) + (long)y * W) * 5 + 4] / 255.0;
+               if (y < H) fsel += fl3_div255((double)b[((i + ii) + (long)y * W) * 5 + 4]);
             }
          if (scf) fsel *= scfact;
          int fi;
@@ -1005,7 +1005,7 @@ __global__ __launch_bounds__(256) void k_logscale(const BT *b, AT *acc, long nce
 
 __device__ __forceinline__ void tone_pixel(const double *t, double *out_rgb, double &alpha, const TMArgs &a) {
    double ls, newrgb[3];
-   const double tmp = t[3] / FL3_PREFILTER_WHITE;
+   const double tmp = fl3_div255(t[3]);
    if (t[3] <= 0) {
       alpha = 0.0;
       ls = 0.0;
@@ -1016,9 +1016,12 @@ __device__ __forceinline__ void tone_pixel(const double *t, double *out_rgb, dou
       if (alpha > 1.0) alpha = 1.0;
    }
    fl3_calc_newrgb(t, ls, a.highpow, newrgb);
+   // (of vibrancy 1 the term is zero times a power that is finite)
+   const bool whole = a.vibrancy == 1.0 && a.g >= 0.0 && a.g <= 1.0;
    for (int k = 0; k < 3; k++) {
       double v = newrgb[k];
-      v += (1.0 - a.vibrancy) * 256.0 * pow(t[k] / FL3_PREFILTER_WHITE, a.g);
+      if (!(whole && t[k] >= 0.0 && t[k] <= 1e300))
+         v += (1.0 - a.vibrancy) * 256.0 * pow(fl3_div255(t[k]), a.g);
       if (a.nchan <= 3 || a.transp == 0)
          v += ((1.0 - alpha) * a.bg[k]);
       else

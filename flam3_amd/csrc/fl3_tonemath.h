@@ -18,6 +18,20 @@
 
 #define FL3_PREFILTER_WHITE 255.0
 
+/* x / 255, correctly rounded like the division: on the GPU by Markstein's
+ * correction of a product with the reciprocal (three instructions instead of
+ * eleven), exact where nothing underflows or overflows. */
+FL3_HD double fl3_div255(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+   const double m = fabs(x);
+   if (m <= 1e300 && (m >= 1e-280 || m == 0.0)) {
+      const double q = x * (1.0 / 255.0);
+      return __builtin_fma(__builtin_fma(-255.0, q, x), 1.0 / 255.0, q);
+   }
+#endif
+   return x / 255.0;
+}
+
 FL3_HD void fl3_rgb2hsv(const double *rgb, double *hsv) {
    double rd = rgb[0], gd = rgb[1], bd = rgb[2], h, s, v, mx, mn, del;
    if (rd >= gd) mx = (rd >= bd) ? rd : bd;
@@ -65,9 +79,9 @@ FL3_HD void fl3_hsv2rgb(const double *hsv, double *rgb) {
 
 /* Alpha from normalised density, with a linear ramp below linrange. */
 FL3_HD double fl3_calc_alpha(double dnorm, double gamma, double linrange) {
-   double funcval = pow(linrange, gamma);
    if (dnorm > 0) {
       if (dnorm < linrange) {
+         double funcval = pow(linrange, gamma);
          double frac = dnorm / linrange;
          return (1.0 - frac) * dnorm * (funcval / linrange) + frac * pow(dnorm, gamma);
       }
@@ -86,17 +100,17 @@ FL3_HD void fl3_calc_newrgb(const double *cbuf, double ls, double highpow, doubl
       return;
    }
    for (k = 0; k < 3; k++) {
-      a = ls * (cbuf[k] / FL3_PREFILTER_WHITE);
+      a = ls * (fl3_div255(cbuf[k]));
       if (a > maxa) {
          maxa = a;
-         maxc = cbuf[k] / FL3_PREFILTER_WHITE;
+         maxc = fl3_div255(cbuf[k]);
       }
    }
    if (maxa > 255 && highpow >= 0.0) {
       double hsv[3], lsratio;
       newls = 255.0 / maxc;
       lsratio = pow(newls / ls, highpow);
-      for (k = 0; k < 3; k++) newrgb[k] = newls * (cbuf[k] / FL3_PREFILTER_WHITE) / 255.0;
+      for (k = 0; k < 3; k++) newrgb[k] = newls * (fl3_div255(cbuf[k])) / 255.0;
       fl3_rgb2hsv(newrgb, hsv);
       hsv[1] *= lsratio;
       fl3_hsv2rgb(hsv, newrgb);
@@ -107,7 +121,7 @@ FL3_HD void fl3_calc_newrgb(const double *cbuf, double ls, double highpow, doubl
       if (adjhlp > 1) adjhlp = 1;
       if (maxa <= 255) adjhlp = 1.0;
       for (k = 0; k < 3; k++)
-         newrgb[k] = ((1.0 - adjhlp) * newls + adjhlp * ls) * (cbuf[k] / FL3_PREFILTER_WHITE);
+         newrgb[k] = ((1.0 - adjhlp) * newls + adjhlp * ls) * (fl3_div255(cbuf[k]));
    }
 }
 
