@@ -41,6 +41,8 @@ typedef struct {
    int64_t chunk;       /* binned: samples per chunk, 0 = library choice */
    const int64_t *job_nsamples;   /* fl3d_iterate_batch: job j plots job_nsamples[j] (at most
                                      nsamples); NULL: nsamples each */
+   int defer;           /* fl3d_iterate_batch may return before the device is done, with *badvals 0: the
+                           count is then in fl3d_deferred_badvals' */
 } fl3d_iter_params;
 
 /* Iterate one job (one genome at one temporal sample) and deposit into the
@@ -75,6 +77,12 @@ int fl3d_iterate_multi(const fl3d_multi_job *jobs, int njobs, int fuse, int exac
  * keys[2j], keys[2j+1]. */
 int fl3d_iterate_batch(const void *const *jobs, const size_t *job_bytes, int njobs, const fl3d_iter_params *p,
                        const uint64_t *keys, double *badvals, int *saturated);
+/* Bad values of the deferred launches since fl3d_begin.  Waits for the device,
+ * unless fl3d_tonemap has since. */
+double fl3d_deferred_badvals(void);
+/* Bad values of render r of a fl3d_iterate_multi without badvals and saturated,
+ * once the device's work up to it is known to be done (an image is here). */
+double fl3d_multi_badvals(int r);
 
 typedef struct {
    int oversample;

@@ -158,7 +158,12 @@ struct Ctx {
    unsigned *band_host = nullptr;      // pinned: first-level tile starts of the last chunk
    hipEvent_t ev_band = nullptr;
    hipEvent_t ev_strip[FL3_IMAGE_STRIPS] = {};   // fl3d_images_fetch: strip k of the image is in staging
-   unsigned long long *counters = nullptr;   // [0] badvals, [1] saturation flag
+   // [0] badvals, [1] saturation flag; [2] badvals of deferred launches, whether
+   // there are any, and whether their copy in counts is on its way; counts:
+   // pinned, that or fl3d_iterate_multi's counters
+   unsigned long long *counters = nullptr, *counts = nullptr;
+   size_t counts_cap = 0;
+   bool deferred = false, deferred_copied = false;
    PinBuf job_pin, tab_pin;                   // jobs, and their tables, on the way to the device
    void *staging = nullptr;                   // pinned host buffer for the image download
    size_t staging_cap = 0;
@@ -372,6 +377,7 @@ extern "C" int fl3d_begin_many(const int *width, const int *height, int n, int b
    HIPCHK(hipMemsetAsync(g_ctx.accum.p, 0, cells * accum_bytes(bits), g_ctx.stream));
    HIPCHK(hipMemsetAsync(g_ctx.buckets.p, 0, cells * bucket_bytes(bits), g_ctx.stream));
    g_ctx.deposited = 0.0;
+   g_ctx.deferred = g_ctx.deferred_copied = false;
    return fl3d_select(0);
 }
 
@@ -420,6 +426,39 @@ static int upload_job(const void *job, size_t bytes) {
    if (g_ctx.job.ensure(bytes)) return 1;
    HIPCHK(hipMemcpyAsync(g_ctx.job.p, job, bytes, hipMemcpyHostToDevice, g_ctx.stream));
    return 0;
+}
+
+static int ensure_counts(size_t n) {
+   if (2 * n <= g_ctx.counts_cap) return 0;
+   HIPCHK(hipStreamSynchronize(g_ctx.stream));   // (a copy into it may be under way)
+   if (g_ctx.counts) (void)hipHostFree(g_ctx.counts);
+   g_ctx.counts = nullptr;
+   g_ctx.counts_cap = 0;
+   HIPCHK(hipHostMalloc((void **)&g_ctx.counts, sizeof(unsigned long long) * 2 * n, hipHostMallocDefault));
+   g_ctx.counts_cap = 2 * n;
+   return 0;
+}
+
+static int copy_deferred() {
+   if (!g_ctx.deferred || g_ctx.deferred_copied) return 0;
+   if (ensure_counts(1)) return 1;
+   HIPCHK(hipMemcpyAsync(g_ctx.counts, g_ctx.counters + 2, sizeof(unsigned long long), hipMemcpyDeviceToHost, g_ctx.stream));
+   g_ctx.deferred_copied = true;
+   return 0;
+}
+
+extern "C" double fl3d_deferred_badvals(void) {
+   std::lock_guard<std::recursive_mutex> lk(g_mu);
+   if (!g_ctx.deferred) return 0.0;
+   const bool here = g_ctx.deferred_copied;
+   if (copy_deferred() || (!here && hipStreamSynchronize(g_ctx.stream) != hipSuccess)) return 0.0;
+   g_ctx.deferred = g_ctx.deferred_copied = false;
+   return (double)g_ctx.counts[0];
+}
+
+extern "C" double fl3d_multi_badvals(int r) {
+   std::lock_guard<std::recursive_mutex> lk(g_mu);
+   return (double)g_ctx.counts[2 * r];
 }
 
 static int read_counters(double *badvals, int *saturated) {
@@ -1072,7 +1111,11 @@ extern "C" int fl3d_iterate_batch(const void *const *jobs, const size_t *job_byt
    js.h = hs.data();
    std::vector<long long> off((size_t)njobs);
    if (njobs == 1) {
-      if (upload_job(jobs[0], job_bytes[0])) return 1;
+      if (g_ctx.job.ensure(job_bytes[0])) return 1;
+      unsigned char *host = g_ctx.job_pin.take(job_bytes[0]);
+      if (!host) return 1;
+      memcpy(host, jobs[0], job_bytes[0]);
+      if (g_ctx.job_pin.send(g_ctx.job.p, job_bytes[0], g_ctx.stream)) return 1;
       js.dev_one = (const unsigned char *)g_ctx.job.p;
    } else {
       size_t total = 0;
@@ -1106,7 +1149,8 @@ extern "C" int fl3d_iterate_batch(const void *const *jobs, const size_t *job_byt
       if (p->job_nsamples)
          js.dev_ns = (const long long *)(js.dev_all + total + (sizeof(long long) + 2 * sizeof(uint64_t)) * njobs);
    }
-   HIPCHK(hipMemsetAsync(g_ctx.counters, 0, 16, g_ctx.stream));
+   // a launch that cannot saturate leaves nothing to wait for
+   bool defer = false;
    if (p->nsamples > 0) {
       IterArgs a;
       memset(&a, 0, sizeof(a));
@@ -1121,8 +1165,6 @@ extern "C" int fl3d_iterate_batch(const void *const *jobs, const size_t *job_byt
       a.fuse = p->fuse;
       a.key0 = keys[0];
       a.key1 = keys[1];
-      a.badvals = g_ctx.counters;
-      a.sat = (uint32_t *)(g_ctx.counters + 1);
       // walkers: a multiple of 256 per job
       const long long Wj = job_walkers(p->nsamples, njobs, p->nwalkers);
       const long long W = Wj * njobs;
@@ -1142,6 +1184,11 @@ extern "C" int fl3d_iterate_batch(const void *const *jobs, const size_t *job_byt
           binnable && (p->deposit == 2 || (p->deposit == 0 && p->nsamples * njobs >= FL3_BIN_MIN_SAMPLES));
       // (binned deposits too count toward what later direct ones may reach)
       const bool direct_bytes = byte_deposits(js.h, js.n, (double)p->nsamples * njobs);
+      defer = p->defer && (binned || direct_bytes || g_ctx.bits == 64);
+      a.badvals = g_ctx.counters + (defer ? 2 : 0);
+      a.sat = (uint32_t *)(g_ctx.counters + 1);
+      if (!defer || !g_ctx.deferred) HIPCHK(hipMemsetAsync(a.badvals, 0, 16, g_ctx.stream));
+      g_ctx.deferred = g_ctx.deferred || defer;
       if (p->job_nsamples && njobs > 1)
          for (int j = 0; j < njobs; j++) g_prof.samples += p->job_nsamples[j];
       else
@@ -1160,6 +1207,11 @@ extern "C" int fl3d_iterate_batch(const void *const *jobs, const size_t *job_byt
             return 1;
          }
       }
+   }
+   if (defer || p->nsamples <= 0) {
+      if (badvals) *badvals = 0.0;
+      if (saturated) *saturated = 0;
+      return 0;
    }
    return read_counters(badvals, saturated);
 }
@@ -1432,9 +1484,11 @@ extern "C" int fl3d_iterate_multi(const fl3d_multi_job *jobs, int njobs, int fus
       HIPCHK(hipEventRecord(g_ctx.ev_join, bs));
       HIPCHK(hipStreamWaitEvent(ws, g_ctx.ev_join, 0));
    }
-   std::vector<unsigned long long> c(2 * (size_t)nrenders);
-   HIPCHK(hipMemcpyAsync(c.data(), g_ctx.rcount.p, 16 * (size_t)nrenders, hipMemcpyDeviceToHost, g_ctx.stream));
-   HIPCHK(hipStreamSynchronize(g_ctx.stream));   // also keeps host alive for the upload
+   if (ensure_counts((size_t)nrenders)) return 1;
+   const unsigned long long *c = g_ctx.counts;
+   HIPCHK(hipMemcpyAsync(g_ctx.counts, g_ctx.rcount.p, 16 * (size_t)nrenders, hipMemcpyDeviceToHost, g_ctx.stream));
+   if (!badvals && !saturated) return 0;   // (fl3d_multi_badvals, later)
+   HIPCHK(hipStreamSynchronize(g_ctx.stream));
    for (int r = 0; r < nrenders; r++) {
       if (badvals) badvals[r] = (double)c[2 * r];
       if (saturated) saturated[r] = (c[2 * r + 1] & 0xffffffffull) != 0;
@@ -2073,7 +2127,7 @@ extern "C" int fl3d_tonemap(const fl3d_tm_params *p, const double *filter, void 
    if (fl3d_images_begin(d.row_bytes * (size_t)p->image_height,
                          sizeof(double) * p->filter_width * p->filter_width))
       return 1;
-   if (fl3d_tonemap_async(p, filter, 0, 0)) return 1;
+   if (fl3d_tonemap_async(p, filter, 0, 0) || copy_deferred()) return 1;
    return fl3d_images_fetch(&d, 1);
 }
 

@@ -70,6 +70,7 @@ static int flush_batch(void **jobs, size_t *bytes, int *n, const int64_t *nsampl
    ip.nwalkers = opts ? opts->nwalkers : 0;
    ip.deposit = opts ? opts->deposit : 0;
    ip.chunk = opts ? opts->chunk_samples : 0;
+   ip.defer = 1;
    rc = fl3d_iterate_batch((const void *const *)jobs, bytes, *n, &ip, keys, bad, sat);
    for (t = 0; t < *n; t++) {
       free(jobs[t]);
@@ -700,8 +701,10 @@ int fl3h_render(flam3_frame *spec, void *out, int field, int nchan, int transp, 
       fl3d_tm_params tp;
       plan_tm(&P, &tp);
       if (fl3d_tonemap(&tp, P.filter, P.out, plan_out_stride(&P))) goto devfail;
+      P.badvals += fl3d_deferred_badvals();
       plan_finish(&P);
    } else {
+      P.badvals += fl3d_deferred_badvals();
       stats->badvals = P.badvals;
       stats->render_seconds = (int)(time(NULL) - P.tstart);
    }
@@ -1049,8 +1052,7 @@ static int many_density(render_plan *Q, fl3_de_filters *de) {
  * (per kernel tier), their density estimation and tone maps, one image
  * download. */
 static int many_group(fl3_many *B, int i0, int i1) {
-   int *widths, *heights, *sat, i, ok = 0;
-   double *bad;
+   int *widths, *heights, i, ok = 0;
    fl3d_multi_job *mj;
    fl3d_image_dst *dst;
    size_t img_total = 0, filt_total = 0;
@@ -1059,11 +1061,9 @@ static int many_group(fl3_many *B, int i0, int i1) {
    if (nl <= 0) return 0;
    widths = (int *)malloc(sizeof(int) * (size_t)nl);
    heights = (int *)malloc(sizeof(int) * (size_t)nl);
-   bad = (double *)calloc((size_t)nl, sizeof(double));
-   sat = (int *)calloc((size_t)nl, sizeof(int));
    dst = (fl3d_image_dst *)calloc((size_t)nl, sizeof(fl3d_image_dst));
    mj = (fl3d_multi_job *)malloc(sizeof(fl3d_multi_job) * (size_t)(B->nmj > 0 ? B->nmj : 1));
-   if (widths && heights && bad && sat && dst && mj) {
+   if (widths && heights && dst && mj) {
       for (i = 0; i < nl; i++) {
          const int r = B->live[i0 + i];
          const render_plan *Q = &B->P[r];
@@ -1082,7 +1082,7 @@ static int many_group(fl3_many *B, int i0, int i1) {
          nm += B->njob[r];
       }
       ok = fl3d_begin_many(widths, heights, nl, B->bits) == 0 &&
-           fl3d_iterate_multi(mj, nm, FUSE_WALKER, 0, nl, bad, sat) == 0;
+           fl3d_iterate_multi(mj, nm, FUSE_WALKER, 0, nl, NULL, NULL) == 0;
       if (ok) {
          /* density estimation (or log scaling) of the group in one launch pair */
          fl3d_de_params *dps = (fl3d_de_params *)calloc((size_t)nl, sizeof(fl3d_de_params));
@@ -1091,7 +1091,6 @@ static int many_group(fl3_many *B, int i0, int i1) {
          for (i = 0; ok && i < nl; i++) {
             render_plan *Q = &B->P[B->live[i0 + i]];
             const fl3_de_filters *d = &B->de[B->live[i0 + i]];
-            Q->badvals = bad[i];
             plan_de_params(Q, &dps[i]);
             des[i] = d->max_filter_index > 0 ? d : NULL;
          }
@@ -1136,6 +1135,7 @@ static int many_group(fl3_many *B, int i0, int i1) {
                ok = 0;
                im->host = NULL;
             }
+            for (i = 0; ok && i < nl; i++) B->P[B->live[i0 + i]].badvals = fl3d_multi_badvals(i);
             B->dv.hand_over(B->dv.ctx, im);   /* also a failed one: it frees the slot */
             im = NULL;
          }
@@ -1146,6 +1146,7 @@ static int many_group(fl3_many *B, int i0, int i1) {
          if (ok) ok = fl3d_images_fetch(dst, nl) == 0;
          if (!ok) fprintf(stderr, "flam3_amd: device error: %s\n", fl3d_error());
          for (i = 0; ok && i < nl; i++) {
+            B->P[B->live[i0 + i]].badvals = fl3d_multi_badvals(i);
             plan_finish(&B->P[B->live[i0 + i]]);
             B->reqs[B->live[i0 + i]].rc = 0;
          }
@@ -1153,8 +1154,6 @@ static int many_group(fl3_many *B, int i0, int i1) {
    }
    free(mj);
    free(dst);
-   free(sat);
-   free(bad);
    free(heights);
    free(widths);
    return ok ? 0 : 1;
