@@ -1180,8 +1180,8 @@ extern "C" int fl3d_iterate_batch(const void *const *jobs, const size_t *job_byt
                  "", (long)FL3_MAX_BINS);
          return 1;
       }
-      const bool binned =
-          binnable && (p->deposit == 2 || (p->deposit == 0 && p->nsamples * njobs >= FL3_BIN_MIN_SAMPLES));
+      const long long min_binned = js.linear || g_ctx.bits == 64 ? FL3_BIN_MIN_SAMPLES : FL3_BIN_MIN_STEPPED;
+      const bool binned = binnable && (p->deposit == 2 || (p->deposit == 0 && p->nsamples * njobs >= min_binned));
       // (binned deposits too count toward what later direct ones may reach)
       const bool direct_bytes = byte_deposits(js.h, js.n, (double)p->nsamples * njobs);
       defer = p->defer && (binned || direct_bytes || g_ctx.bits == 64);

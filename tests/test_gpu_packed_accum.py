@@ -86,3 +86,15 @@ def test_sort_by_the_number_of_tiles(prod, width, height, quality, opacity):
     b, _ = prod.render(g, seed="sort", deposit=2, chunk_samples=700001)
     assert np.array_equal(a, b)
     assert a.any()
+
+
+@pytest.mark.parametrize("quality", [15.99, 16])
+@pytest.mark.parametrize("opacity", [1.0, 0.5])
+def test_small_renders_on_both_sides_of_the_sorted_deposit(prod, quality, opacity):
+    """The library's own choice of deposit around 65536 samples."""
+    g = _shaded(G.synthetic_small(seed=44, width=64, height=64, quality=quality), "alpha")
+    g.xforms[1].opacity = opacity
+    a, sa = prod.render(g, seed="line", nchan=4, transp=1)
+    b, sb = prod.render(g, seed="line", deposit=1, nchan=4, transp=1)
+    assert (sa["badvals"], sa["num_iters"]) == (sb["badvals"], sb["num_iters"])
+    assert np.array_equal(a, b)
