@@ -735,13 +735,18 @@ __device__ __forceinline__ void de_gather_body(const DEArgs &a, int bx, int by) 
 // At 1920x1080 with 2x2 supersampling (8.4M cells, radius 9): 876 us with a
 // workgroup's shared lists and tests per tap, 671 us so (2.75e8 vector
 // instructions instead of 5.7e8; LDS is active for 60% of the time); 3840x2160
-// with 3x3 in FP64 44.0 ms (each term formed per tap) against 21.2 ms.
+// with 3x3 in FP64 44.0 ms (each term formed per tap) against 19.5 ms (the vector
+// caches' 64 addresses a tap).
 // Wavefronts of a workgroup: they share the tables, NW / 2 blocks across and two
 // down.
 constexpr int de_waves(int cells) { return cells == 2 ? 8 : 4; }
 template <typename AT, int CELLS>
 __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
-   constexpr int SH = sizeof(AT) == 4 ? 2 : 3, BH = 8 * CELLS, NW = de_waves(CELLS), TURN = 32, CAP = TURN + 64;
+   constexpr int SH = sizeof(AT) == 4 ? 2 : 3, NW = de_waves(CELLS), TURN = 32, CAP = TURN + 64;
+   // a wavefront's block: BW cells across, CELLS times RW down (FP64 tables are
+   // read from the vector caches: 21.4 ms with 8 across, 19.5 with 16, 22.4 with 32
+   // in the 3840x2160 case above; FP32 ones from LDS: no difference)
+   constexpr int BW = sizeof(AT) == 4 ? 8 : 16, RW = 64 / BW, BH = RW * CELLS, ACROSS = 4 * NW / BW;
    typedef typename std::conditional<sizeof(AT) == 4, float4, double4>::type V4;
    __shared__ int4 s_src[NW][CAP];   // per wavefront: x, y, its table's place, radius + 1
    __shared__ unsigned s_stride[NW][CAP];   // bytes of a row of its square
@@ -756,25 +761,25 @@ __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
    const int W = a.width, H = a.height;
    const int tid = threadIdx.x, lane = tid & 63;
    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // (so that what depends on it is scalar)
-   const int mx0 = (bx * (NW / 2) + wave % (NW / 2)) * 8, my0 = (by * 2 + wave / (NW / 2)) * BH;
-   const int mx1 = min(mx0 + 8, W) - 1, my1 = min(my0 + BH, H) - 1;
-   const int x = mx0 + (lane & 7), y = my0 + (lane >> 3);
+   const int mx0 = (bx * ACROSS + wave % ACROSS) * BW, my0 = (by * (NW / ACROSS) + wave / ACROSS) * BH;
+   const int mx1 = min(mx0 + BW, W) - 1, my1 = min(my0 + BH, H) - 1;
+   const int x = mx0 + lane % BW, y = my0 + lane / BW;
 #pragma unroll 4
    for (int e = tid; e < a.tab_bytes / 16; e += 64 * NW) ((uint4 *)fl3_lds)[e] = ((const uint4 *)a.tab)[e];
    for (int e = tid; e <= nf; e += 64 * NW)
       s_info[e] = e < nf ? make_int2((a.info[2 * e] << SH) + lds0, a.info[2 * e + 1]) : make_int2(lds0, -(1 << 20));
-   // acc[j][i]: FP32, channel lane & 3 of cell (px + i, y + 8 j) of this lane's
-   // four, as the matrix instruction leaves them; FP64, channel i of (x, y + 8 j)
+   // acc[j][i]: FP32, channel lane & 3 of cell (px + i, y + RW j) of this lane's
+   // four, as the matrix instruction leaves them; FP64, channel i of (x, y + RW j)
    constexpr bool MAT = sizeof(AT) == 4;
-   const int px = MAT ? mx0 + (lane & 4) : x;
+   const int px = MAT ? mx0 + (lane & (BW - 4)) : x;
    typedef AT AV __attribute__((ext_vector_type(4)));
    AV acc[CELLS];
    auto at_acc = [&](int j, int i) {
-      return (AT *)a.accum + ((px + (MAT ? i : 0)) + (long)(y + 8 * j) * W) * 4 + (MAT ? lane & 3 : i);
+      return (AT *)a.accum + ((px + (MAT ? i : 0)) + (long)(y + RW * j) * W) * 4 + (MAT ? lane & 3 : i);
    };
    for (int j = 0; j < CELLS; j++)
       for (int i = 0; i < 4; i++)
-         acc[j][i] = px + (MAT ? i : 0) < W && y + 8 * j < H ? *at_acc(j, i) : (AT)0;
+         acc[j][i] = px + (MAT ? i : 0) < W && y + RW * j < H ? *at_acc(j, i) : (AT)0;
    // this block's halo, as de_halo finds a region's
    int E = a.half;
    if (a.blkmax) {
@@ -807,7 +812,7 @@ __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
          const unsigned ax = min(__builtin_amdgcn_sad_u16((unsigned)x, (unsigned)src.x, 0u), w);
          const unsigned row = (ax << SH) + (unsigned)src.z, stride = s_stride[wave][i];
          for (int j = 0; j < CELLS; j++) {
-            const unsigned ay = min(__builtin_amdgcn_sad_u16((unsigned)(y + 8 * j), (unsigned)src.y, 0u), w);
+            const unsigned ay = min(__builtin_amdgcn_sad_u16((unsigned)(y + RW * j), (unsigned)src.y, 0u), w);
             const AT coef = coef_at(__umul24(ay, stride) + row);
             if constexpr (MAT)
                acc[j] = __builtin_amdgcn_mfma_f32_4x4x1f32(coef, ((const float *)&s_val[wave][i])[lane & 3], acc[j], 0, 0, 0);
@@ -842,7 +847,7 @@ __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
       int4 src = make_int4(0, 0, 0, 0);
       V4 val = {(AT)0, (AT)0, (AT)0, (AT)0};
       // (a block reaches as far as its distances from twice its middle)
-      const unsigned mid2x = (unsigned)(2 * mx0 + 7), mid2y = (unsigned)(2 * my0 + BH - 1);
+      const unsigned mid2x = (unsigned)(2 * mx0 + BW - 1), mid2y = (unsigned)(2 * my0 + BH - 1);
       for (int base = 0; base < nh + 64; base += 64) {   // (one turn more for the last 64's)
          const int f = fnext, cx = sx, cy = sy;
          const unsigned cc = cell;
@@ -864,7 +869,7 @@ __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
          listed = found;
          at = -1;
          const int dx2 = abs(2 * cx - (int)mid2x), dy2 = abs(2 * cy - (int)mid2y);
-         const bool reach = dx2 <= 2 * in.y + 7 && dy2 <= 2 * in.y + BH - 1;
+         const bool reach = dx2 <= 2 * in.y + BW - 1 && dy2 <= 2 * in.y + BH - 1;
          const unsigned long long m = __builtin_amdgcn_ballot_w64(reach);
          if (listed >= TURN) {
             __builtin_amdgcn_wave_barrier();
@@ -894,7 +899,7 @@ __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
       scan([&](unsigned o) { return *(const AT *)((const unsigned char *)a.tab + o); });
    for (int j = 0; j < CELLS; j++)
       for (int i = 0; i < 4; i++)
-         if (px + (MAT ? i : 0) < W && y + 8 * j < H) *at_acc(j, i) = acc[j][i];
+         if (px + (MAT ? i : 0) < W && y + RW * j < H) *at_acc(j, i) = acc[j][i];
 }
 
 __global__ __launch_bounds__(256) void k_fill_i32(int *p, long n, int v) {
