@@ -733,7 +733,7 @@ __device__ __forceinline__ void de_gather_body(const DEArgs &a, int bx, int by) 
 // wavefront scans its own block's halo and lists its sources in LDS of its
 // own: no barriers, and a tighter halo than a workgroup's.
 // At 1920x1080 with 2x2 supersampling (8.4M cells, radius 9): 876 us with a
-// workgroup's shared lists and tests per tap, 671 us so (2.75e8 vector
+// workgroup's shared lists and tests per tap, 635 us so (2.75e8 vector
 // instructions instead of 5.7e8; LDS is active for 60% of the time); 3840x2160
 // with 3x3 in FP64 44.0 ms (each term formed per tap) against 19.5 ms (the vector
 // caches' 64 addresses a tap).
@@ -803,28 +803,45 @@ __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
    const int hy0 = max(0, my0 - E), hy1 = min(H, my1 + 1 + E);
    const int hw = hx1 - hx0, nh = E < 0 || mx0 >= W || my0 >= H ? 0 : hw * (hy1 - hy0);
    const V4 *srcv = (const V4 *)a.srcv;
-   auto taps = [&](int n, auto coef_at) {
-#pragma unroll 4
-      for (int i = 0; i < n; i++) {
-         const int4 src = s_src[wave][i];
+   // U sources from the i-th on: all their reads before the first sum (the matrix
+   // instruction keeps the compiler from unrolling a loop of single ones)
+   auto taps_of = [&](int i, auto count, auto coef_at) {
+      constexpr int U = decltype(count)::value;
+      AT coef[U][CELLS];
+      V4 val[U];
+      float chan[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+         const int4 src = s_src[wave][i + u];
          const unsigned w = (unsigned)src.w;
          // (|x - y| of coordinates below 65536, whose high halves are zero)
          const unsigned ax = min(__builtin_amdgcn_sad_u16((unsigned)x, (unsigned)src.x, 0u), w);
-         const unsigned row = (ax << SH) + (unsigned)src.z, stride = s_stride[wave][i];
+         const unsigned row = (ax << SH) + (unsigned)src.z, stride = s_stride[wave][i + u];
          for (int j = 0; j < CELLS; j++) {
             const unsigned ay = min(__builtin_amdgcn_sad_u16((unsigned)(y + RW * j), (unsigned)src.y, 0u), w);
-            const AT coef = coef_at(__umul24(ay, stride) + row);
-            if constexpr (MAT)
-               acc[j] = __builtin_amdgcn_mfma_f32_4x4x1f32(coef, ((const float *)&s_val[wave][i])[lane & 3], acc[j], 0, 0, 0);
-            else {
-               const V4 v = s_val[wave][i];
-               acc[j][0] = fma(coef, v.x, acc[j][0]);
-               acc[j][1] = fma(coef, v.y, acc[j][1]);
-               acc[j][2] = fma(coef, v.z, acc[j][2]);
-               acc[j][3] = fma(coef, v.w, acc[j][3]);
-            }
+            coef[u][j] = coef_at(__umul24(ay, stride) + row);
          }
+         if constexpr (MAT)
+            chan[u] = ((const float *)&s_val[wave][i + u])[lane & 3];
+         else
+            val[u] = s_val[wave][i + u];
       }
+#pragma unroll
+      for (int u = 0; u < U; u++)
+         for (int j = 0; j < CELLS; j++)
+            if constexpr (MAT)
+               acc[j] = __builtin_amdgcn_mfma_f32_4x4x1f32(coef[u][j], chan[u], acc[j], 0, 0, 0);
+            else {
+               acc[j][0] = fma(coef[u][j], val[u].x, acc[j][0]);
+               acc[j][1] = fma(coef[u][j], val[u].y, acc[j][1]);
+               acc[j][2] = fma(coef[u][j], val[u].z, acc[j][2]);
+               acc[j][3] = fma(coef[u][j], val[u].w, acc[j][3]);
+            }
+   };
+   auto taps = [&](int n, auto coef_at) {
+      int i = 0;
+      for (; i + 4 <= n; i += 4) taps_of(i, std::integral_constant<int, 4>(), coef_at);
+      for (; i < n; i++) taps_of(i, std::integral_constant<int, 1>(), coef_at);
    };
    auto scan = [&](auto coef_at) {
       // the lane's cell of the next 64 halo cells (its place, its index), and
@@ -956,7 +973,7 @@ __global__ __launch_bounds__(64 * de_waves(CELLS)) void k_de_taps_many(const DEA
 // Cells a lane of the production gather holds, for regions of `blocks` 16x16
 // blocks of cells in all: two where that leaves every CU several workgroups,
 // one otherwise, where the gather is bound by how long a workgroup takes.
-// Kernel time with one and two: 640x480 (1271 blocks) 40 and 59 us; 7.7k blocks
+// Kernel time with one and two: 640x480 (1271 blocks) 40 and 59 us, 7.7k blocks
 // 263 and 235 us, 32k blocks 838 and 672 us.
 extern "C" int fl3k_de_cells(long long blocks) { return blocks >= 4096 ? 2 : 1; }
 // Cells across and down of a workgroup's region.
