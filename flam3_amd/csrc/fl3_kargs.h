@@ -86,11 +86,11 @@ struct IterArgs {
 #define FL3_BIN_ITEM_RECORDS (1 << 18)
 // Samples from which a render's deposits are sorted by tile.  Stepped palettes in
 // 32-bit histograms (the same integers either way): direct deposits of 41000
-// samples take 264-367 us a render over eight genomes, sorted ones 293-305;
-// of 164000 319-504 and 337-347; of 960000 349-908 and 316-326 (more than
-// 5 ms where most samples meet in a cell).  Linear palettes and double
-// histograms round otherwise in records and keep to the older line.
-#define FL3_BIN_MIN_STEPPED (1LL << 16)
+// samples take 264-367 us a render over eight genomes (585 over others), sorted
+// ones 293-305; of 164000 319-504 and 337-347; of 960000 349-908 (8 ms where most
+// samples meet in a cell) and 316-326.  Linear palettes and double histograms
+// round otherwise in records and keep to the older line.
+#define FL3_BIN_MIN_STEPPED (1LL << 15)
 #define FL3_BIN_MIN_SAMPLES (1LL << 20)
 
 // Record formats of fl3k_launch_bin beyond 0 (8-byte records), 1 (4-byte

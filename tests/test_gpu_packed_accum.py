@@ -88,10 +88,10 @@ def test_sort_by_the_number_of_tiles(prod, width, height, quality, opacity):
     assert a.any()
 
 
-@pytest.mark.parametrize("quality", [15.99, 16])
+@pytest.mark.parametrize("quality", [7.99, 8])
 @pytest.mark.parametrize("opacity", [1.0, 0.5])
 def test_small_renders_on_both_sides_of_the_sorted_deposit(prod, quality, opacity):
-    """The library's own choice of deposit around 65536 samples."""
+    """The library's own choice of deposit around 32768 samples."""
     g = _shaded(G.synthetic_small(seed=44, width=64, height=64, quality=quality), "alpha")
     g.xforms[1].opacity = opacity
     a, sa = prod.render(g, seed="line", nchan=4, transp=1)
