@@ -632,7 +632,7 @@ static int acc_tile_shift(long long ncells, int bits, int *band) {
    if (!sh) return 0;
    if (((ncells + (1LL << sh) - 1) >> sh) > FL3_MAX_BINS) {
       const int bs = sh + 13;   // FL3_MAX_BINS = 2^13 tiles per band
-      // bands are the first level's super-tiles: at most 256 of them, and
+      // bands: at most 256 of them (the band sort's counters), and
       // 32-bit record cells
       if (((ncells + (1LL << bs) - 1) >> bs) > 256 || ncells >= (1LL << 31)) return 0;
       *band = bs;
@@ -949,7 +949,7 @@ static int bin_banded(const BinArgs &b1, int format, int band, int shift, hipStr
 // shift: the accumulation tiles' (cells per tile = 1 << shift); band: 0, or
 // the band shift of a histogram of more than FL3_MAX_BINS tiles: the
 // walkers then count their records per 2^(band - FL3_SUPER_SHIFT)-cell tile,
-// the first sort pass groups them by band, and each band is counted, sorted
+// a first sort groups them by band, and each band is counted, sorted by tile
 // and accumulated on its own (iterate_banded_chunk).
 static int iterate_binned(IterArgs a, long long W, long long Wj, const JobSet &js, const fl3d_iter_params *p,
                           int shift, int band) {

@@ -127,7 +127,7 @@ struct BinArgs {
    const float *vis_all;           // [job][vis_stride]
    int vis_stride;
    // banded histograms: the records' cells are relative to cell_base; the
-   // input of the first sort pass (or count pass) holds rec_count records
+   // input of the sort (or count pass) holds rec_count records
    // (0: every slot of the blocks is a record or FL3_REC_NONE)
    unsigned cell_base;
    long long rec_count;

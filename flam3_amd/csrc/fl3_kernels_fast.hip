@@ -1,5 +1,5 @@
-// fl3_kernels_fast.hip - FP32 production walkers (compiled with FP
-// contraction on).
+// fl3_kernels_fast.hip - launches of the FP32 production walkers, and the
+// binned deposit's kernels (compiled with FP contraction on).
 #include "fl3_walker.h"
 #include "fl3_launch.h"
 
@@ -551,8 +551,9 @@ __global__ __launch_bounds__(256) void k_bin_count(BinArgs a) {
 // additions.
 // 4-byte records (stepped palette, visibility 1; each adds exactly 255 to
 // the count, which is then a 32-bit record count scaled at the flush) or
-// 8-byte records (make_record).  Persistent workgroups take work items as
-// in k_bin_accum; a tile with one item is added without atomics.
+// 8-byte records (make_record).  Persistent workgroups take work items
+// (up to a.chunk records of one tile) from a counter; a tile with one item is
+// added without atomics.
 #define FL3_F64_FIX 4294967296.0    // 2^32: the fixed-point scale of the LDS sums
 template <typename RT>
 __global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum_f64(BinArgs a) {
