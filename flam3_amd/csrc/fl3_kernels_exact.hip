@@ -737,8 +737,7 @@ __device__ __forceinline__ void de_gather_body(const DEArgs &a, int bx, int by) 
 // instructions instead of 5.7e8; LDS is active for 60% of the time); 3840x2160
 // with 3x3 in FP64 44.0 ms (each term formed per tap) against 19.5 ms (the vector
 // caches' 64 addresses a tap).
-// Wavefronts of a workgroup: they share the tables, NW / 2 blocks across and two
-// down.
+// Wavefronts of a workgroup (they share the tables).
 constexpr int de_waves(int cells) { return cells == 2 ? 8 : 4; }
 template <typename AT, int CELLS>
 __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
@@ -1067,23 +1066,23 @@ __global__ __launch_bounds__(256) void k_earlyclip(AT *acc, long ncells, TMArgs 
    ac[3] = (AT)alpha;
 }
 
+// The filtered sum of a pixel from the cells at acc (rows `stride` cells apart).
 template <typename AT>
-__device__ __forceinline__ void tonemap_body(const TMArgs &a, int bx, int by) {
-   const int i = bx * blockDim.x + threadIdx.x;
-   const int j = by;
-   if (i >= a.iw || j >= a.ih) return;
-   const AT *acc = (const AT *)a.accum;
-   const int x = a.de_offset + i * a.os, y = a.de_offset + j * a.os;
-   double t[4] = {0.0, 0.0, 0.0, 0.0};
+__device__ __forceinline__ void filter_pixel(const TMArgs &a, const AT *acc, long stride, double *t) {
+   for (int k = 0; k < 4; k++) t[k] = 0.0;
    for (int ii = 0; ii < a.fw; ii++)
       for (int jj = 0; jj < a.fw; jj++) {
          const double k = a.filter[ii + jj * a.fw];
-         const AT *ac = acc + ((x + ii) + (long)(y + jj) * a.W) * 4;
+         const AT *ac = acc + (ii + jj * stride) * 4;
          t[0] += k * (double)ac[0];
          t[1] += k * (double)ac[1];
          t[2] += k * (double)ac[2];
          t[3] += k * (double)ac[3];
       }
+}
+
+// Tone maps, clips and writes pixel (i, j) with the filtered sum t.
+__device__ __forceinline__ void write_pixel(const TMArgs &a, int i, int j, double *t) {
    if (!a.earlyclip) {
       double rgb[3], alpha;
       tone_pixel(t, rgb, alpha, a);
@@ -1111,6 +1110,17 @@ __device__ __forceinline__ void tonemap_body(const TMArgs &a, int bx, int by) {
          else p[3] = 255;
       }
    }
+}
+
+template <typename AT>
+__device__ __forceinline__ void tonemap_body(const TMArgs &a, int bx, int by) {
+   const int i = bx * blockDim.x + threadIdx.x;
+   const int j = by;
+   if (i >= a.iw || j >= a.ih) return;
+   const int x = a.de_offset + i * a.os, y = a.de_offset + j * a.os;
+   double t[4];
+   filter_pixel<AT>(a, (const AT *)a.accum + (x + (long)y * a.W) * 4, a.W, t);
+   write_pixel(a, i, j, t);
 }
 
 // ------------------------------------------------------------------ launchers
@@ -1208,6 +1218,48 @@ __global__ __launch_bounds__(256) void k_tonemap(TMArgs a) {
    tonemap_body<AT>(a, blockIdx.x, blockIdx.y);
 }
 
+// The same by tiles of 32 x 4 pixels whose cells are read once, into LDS.  A
+// wavefront of 64 pixels of k_tonemap walks fw rows of 64 os cells for each of
+// its fw columns, more than a CU's vector cache holds for all of its wavefronts
+// when cells are doubles, so every tap goes out to the L2 (3840x2160,
+// supersample 3, 5 x 5 taps: 2.75 ms, 0.67 ms from LDS).
+#define TM_TX 32
+#define TM_TY 4
+template <typename AT>
+__global__ __launch_bounds__(TM_TX * TM_TY) void k_tonemap_lds(TMArgs a) {
+   typedef AT v16 __attribute__((ext_vector_type(16 / sizeof(AT))));
+   constexpr int PARTS = 4 * sizeof(AT) / 16;   // 16-byte loads per cell
+   v16 *tile = (v16 *)fl3_lds;
+   const int i0 = blockIdx.x * TM_TX, j0 = blockIdx.y * TM_TY;
+   // the cells of the tile's pixels inside the image
+   const int cols = (min(TM_TX, a.iw - i0) - 1) * a.os + a.fw, rows = (min(TM_TY, a.ih - j0) - 1) * a.os + a.fw;
+   const v16 *acc = (const v16 *)a.accum + ((a.de_offset + i0 * a.os) + (long)(a.de_offset + j0 * a.os) * a.W) * PARTS;
+   const int rowp = cols * PARTS, n = rows * rowp, step = TM_TX * TM_TY, stepr = step / rowp, stepc = step % rowp;
+   int r = (int)threadIdx.x / rowp, c = (int)threadIdx.x % rowp;
+   for (int e = threadIdx.x; e < n; e += 8 * step) {
+      v16 v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+         if (e + u * step < n) v[u] = acc[(long)r * a.W * PARTS + c];
+         r += stepr;
+         c += stepc;
+         if (c >= rowp) {
+            c -= rowp;
+            r++;
+         }
+      }
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+         if (e + u * step < n) tile[e + u * step] = v[u];
+   }
+   __syncthreads();
+   const int lx = threadIdx.x % TM_TX, ly = threadIdx.x / TM_TX;
+   if (i0 + lx >= a.iw || j0 + ly >= a.ih) return;
+   double t[4];
+   filter_pixel<AT>(a, (const AT *)fl3_lds + (lx + ly * cols) * a.os * 4, cols, t);
+   write_pixel(a, i0 + lx, j0 + ly, t);
+}
+
 // Tone maps of several renders in one launch (workgroup prefixes as for
 // k_de_gather_many; rows of 256 pixels).
 template <typename AT>
@@ -1241,9 +1293,21 @@ extern "C" int fl3k_launch_earlyclip(void *acc, long n, const TMArgs *a, hipStre
    return hipGetLastError() != hipSuccess;
 }
 
+// Tiles of up to this many bytes, so that three workgroups share a CU; 1920x1080,
+// direct and from LDS, us: supersample 1 with 3 x 3 taps 43 and 45 (floats), 49
+// and 45 (doubles), 2 with 4 x 4 71 and 52, 147 and 81, 3 with 5 x 5 239 and 89,
+// 581 and 186, 1 with 20 x 20 565 and 432, 969 and 518.
+#define TM_LDS (52 << 10)
 extern "C" int fl3k_launch_tonemap(const TMArgs *a, hipStream_t s, int bits) {
    const dim3 grid((a->iw + 255) / 256, a->ih), block(256);
-   if (bits == 64)
+   const long lds = (((long)TM_TX - 1) * a->os + a->fw) * (((long)TM_TY - 1) * a->os + a->fw) * 4 *
+                    (bits == 64 ? sizeof(double) : sizeof(float));
+   const dim3 gt((a->iw + TM_TX - 1) / TM_TX, (a->ih + TM_TY - 1) / TM_TY), bt(TM_TX * TM_TY);
+   if (bits == 64 && lds <= TM_LDS)
+      hipLaunchKernelGGL((k_tonemap_lds<double>), gt, bt, (size_t)lds, s, *a);
+   else if (bits == 33 && lds <= TM_LDS)
+      hipLaunchKernelGGL((k_tonemap_lds<float>), gt, bt, (size_t)lds, s, *a);
+   else if (bits == 64)
       hipLaunchKernelGGL((k_tonemap<double>), grid, block, 0, s, *a);
    else if (bits == 33)
       hipLaunchKernelGGL((k_tonemap<float>), grid, block, 0, s, *a);
