@@ -1538,21 +1538,21 @@ static size_t align16(size_t n) { return (n + 15) & ~(size_t)15; }
 
 // Entries of a bank's tables (DeTables), and whether the production gather's
 // 32-bit byte offsets reach them all; a larger bank takes the exact gather.
-static double de_table_entries(const fl3_de_filters *de) {
+static double de_table_entries(const fl3_de_filters *de, size_t entry) {
    double n = 0;
    for (int i = 0; i <= de->max_filter_index; i++) {
       const double side = ceil(de->filter_widths[i]) + 1;
-      if (side > 0) n += side * side;
+      if (side > 0) n += side * (side + fl3k_de_cols(entry) - 2);
    }
    return n;
 }
 static bool de_tables_ok(const fl3_de_filters *de, size_t entry) {
-   return de_table_entries(de) * (double)entry < 0x7fff0000;
+   return de_table_entries(de, entry) * (double)entry < 0x7fff0000;
 }
 
 // A filter bank as the production gather reads it (DEArgs::tab, info): of
 // kernel i, radius r = ceil(width) - 1, a square of the coefficients by |dy|,
-// |dx| with a row and a column of zeros beyond the radius.  (A bank whose rows
+// |dx| with a row and a column (doubles: two) of zeros beyond the radius.  (A bank whose rows
 // are shorter than their radius asks for goes on in the next row, as the
 // reference's index does; past its end there are zeros.)
 template <typename T>
@@ -1570,12 +1570,12 @@ struct DeTables {
          if (r < -1) r = -1;   // (reaches nothing, whatever its width below zero)
          info[2 * i] = (int)n;
          info[2 * i + 1] = r;
-         n += (size_t)(r + 2) * (r + 2);
+         n += (size_t)(r + 2) * (r + fl3k_de_cols(sizeof(T)));
       }
       if (n * sizeof(T) + 8 * (size_t)(nf + 1) <= FL3_DE_LDS_BYTES) lds_bytes = (int)align16(n * sizeof(T));
       tab.assign(n, (T)0);
       for (int i = 0; i < nf; i++) {
-         const int r = info[2 * i + 1], side = r + 2;
+         const int r = info[2 * i + 1], side = r + fl3k_de_cols(sizeof(T));
          T *t = tab.data() + info[2 * i];
          for (int y = 0; y <= r; y++)
             for (int x = 0; x <= r; x++) {

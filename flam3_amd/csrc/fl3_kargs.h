@@ -176,6 +176,10 @@ struct DEArgs {
 };
 #define FL3_DE_LDS_BYTES 49152   // most LDS bytes of tables and info a gather workgroup takes
 
+// Columns of a production gather's table (entries of this size) beyond the
+// radius: its own zero column, and one more where two entries are read at once.
+static inline __host__ __device__ constexpr int fl3k_de_cols(size_t entry) { return entry == 8 ? 3 : 2; }
+
 struct TMArgs {
    const void *accum;
    const double *filter;

@@ -736,8 +736,9 @@ __device__ __forceinline__ void de_gather_body(const DEArgs &a, int bx, int by) 
 // coefficients lie in a square table with a zero row and column at its edge,
 // and the distances are clamped to that edge, so a tap costs three
 // instructions for its address, without tests (a missed tap adds zero); the tables are in LDS where they fit (a wavefront
-// reads 64 scattered coefficients per source).  A lane holds CELLS cells, 8
-// rows apart, which share the source's read and the x distance.  In FP32 the
+// reads 64 scattered coefficients per source).  A lane holds CELLS cells, some
+// rows apart, which share the source's read and the x distance (FP64: side by
+// side).  In FP32 the
 // four channels are one matrix instruction, an outer product of four cells'
 // coefficients and four channels whose every sum is one fused multiply-add
 // with the bits of fmaf.  Each
@@ -746,8 +747,8 @@ __device__ __forceinline__ void de_gather_body(const DEArgs &a, int bx, int by) 
 // At 1920x1080 with 2x2 supersampling (8.4M cells, radius 9): 876 us with a
 // workgroup's shared lists and tests per tap, 635 us so (2.75e8 vector
 // instructions instead of 5.7e8; LDS is active for 60% of the time); 3840x2160
-// with 3x3 in FP64 44.0 ms (each term formed per tap) against 19.5 ms (the vector
-// caches' 64 addresses a tap).
+// with 3x3 in FP64 44.0 ms (each term formed per tap) against 17.2 ms (vector
+// instructions and the vector caches' 64 addresses a load).
 // Wavefronts of a workgroup (they share the tables).
 constexpr int de_waves(int cells) { return cells == 2 ? 8 : 4; }
 template <typename AT, int CELLS>
@@ -756,7 +757,11 @@ __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
    // a wavefront's block: BW cells across, CELLS times RW down (FP64 tables are
    // read from the vector caches: 21.4 ms with 8 across, 19.5 with 16, 22.4 with 32
    // in the 3840x2160 case above; FP32 ones from LDS: no difference)
-   constexpr int BW = sizeof(AT) == 4 ? 8 : 16, RW = 64 / BW, BH = RW * CELLS, ACROSS = 4 * NW / BW;
+   constexpr int BW = sizeof(AT) == 4 ? 8 : 16, ACROSS = 4 * NW / BW;
+   // FP64, two cells: side by side, so that one load of 16 bytes has both
+   // coefficients (rows apart, a load each: 19.6 ms in that case, 17.2 so)
+   constexpr bool PAIR = sizeof(AT) == 8 && CELLS == 2;
+   constexpr int LW = PAIR ? BW / 2 : BW, RW = 64 / LW, BH = PAIR ? RW : RW * CELLS;
    typedef typename std::conditional<sizeof(AT) == 4, float4, double4>::type V4;
    __shared__ int4 s_src[NW][CAP];   // per wavefront: x, y, its table's place, radius + 1
    __shared__ unsigned s_stride[NW][CAP];   // bytes of a row of its square
@@ -765,7 +770,9 @@ __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
    // the tables (tab_bytes), then per kernel its table's place (LDS address, or
    // byte offset in tab) and radius, and one that reaches nothing
    int2 *s_info = (int2 *)(fl3_lds + a.tab_bytes);
-   typedef const __attribute__((address_space(3))) AT lds_at;
+   typedef double two __attribute__((ext_vector_type(2), aligned(8)));
+   typedef typename std::conditional<PAIR, two, AT>::type C;
+   typedef const __attribute__((address_space(3))) C lds_at;
    const int nf = a.max_filter_index + 1;
    const int lds0 = a.tab_bytes ? (int)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)fl3_lds : 0;
    const int W = a.width, H = a.height;
@@ -773,23 +780,25 @@ __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // (so that what depends on it is scalar)
    const int mx0 = (bx * ACROSS + wave % ACROSS) * BW, my0 = (by * (NW / ACROSS) + wave / ACROSS) * BH;
    const int mx1 = min(mx0 + BW, W) - 1, my1 = min(my0 + BH, H) - 1;
-   const int x = mx0 + lane % BW, y = my0 + lane / BW;
+   const int x = mx0 + lane % LW * (BW / LW), y = my0 + lane / LW;
 #pragma unroll 4
    for (int e = tid; e < a.tab_bytes / 16; e += 64 * NW) ((uint4 *)fl3_lds)[e] = ((const uint4 *)a.tab)[e];
    for (int e = tid; e <= nf; e += 64 * NW)
       s_info[e] = e < nf ? make_int2((a.info[2 * e] << SH) + lds0, a.info[2 * e + 1]) : make_int2(lds0, -(1 << 20));
    // acc[j][i]: FP32, channel lane & 3 of cell (px + i, y + RW j) of this lane's
    // four, as the matrix instruction leaves them; FP64, channel i of (x, y + RW j)
+   // or (x + j, y)
    constexpr bool MAT = sizeof(AT) == 4;
    const int px = MAT ? mx0 + (lane & (BW - 4)) : x;
+   constexpr int DX = PAIR ? 1 : 0, DY = PAIR ? 0 : RW;   // from a lane's cell to its next
    typedef AT AV __attribute__((ext_vector_type(4)));
    AV acc[CELLS];
    auto at_acc = [&](int j, int i) {
-      return (AT *)a.accum + ((px + (MAT ? i : 0)) + (long)(y + RW * j) * W) * 4 + (MAT ? lane & 3 : i);
+      return (AT *)a.accum + ((px + DX * j + (MAT ? i : 0)) + (long)(y + DY * j) * W) * 4 + (MAT ? lane & 3 : i);
    };
    for (int j = 0; j < CELLS; j++)
       for (int i = 0; i < 4; i++)
-         acc[j][i] = px + (MAT ? i : 0) < W && y + RW * j < H ? *at_acc(j, i) : (AT)0;
+         acc[j][i] = px + DX * j + (MAT ? i : 0) < W && y + DY * j < H ? *at_acc(j, i) : (AT)0;
    // this block's halo, as de_halo finds a region's
    int E = a.half;
    if (a.blkmax) {
@@ -825,12 +834,21 @@ __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
          const int4 src = s_src[wave][i + u];
          const unsigned w = (unsigned)src.w;
          // (|x - y| of coordinates below 65536, whose high halves are zero)
-         const unsigned ax = min(__builtin_amdgcn_sad_u16((unsigned)x, (unsigned)src.x, 0u), w);
+         unsigned ax = min(__builtin_amdgcn_sad_u16((unsigned)x, (unsigned)src.x, 0u), w);
+         if constexpr (PAIR) ax = min(ax, __builtin_amdgcn_sad_u16((unsigned)x + 1u, (unsigned)src.x, 0u));
          const unsigned row = (ax << SH) + (unsigned)src.z, stride = s_stride[wave][i + u];
-         for (int j = 0; j < CELLS; j++) {
-            const unsigned ay = min(__builtin_amdgcn_sad_u16((unsigned)(y + RW * j), (unsigned)src.y, 0u), w);
-            coef[u][j] = coef_at(__umul24(ay, stride) + row);
-         }
+         if constexpr (PAIR) {
+            // the nearer cell's coefficient and the next one: the right cell is
+            // the nearer to a source at its right
+            const unsigned ay = min(__builtin_amdgcn_sad_u16((unsigned)y, (unsigned)src.y, 0u), w);
+            const auto c = coef_at(__umul24(ay, stride) + row);
+            coef[u][0] = src.x > x ? c.y : c.x;
+            coef[u][CELLS - 1] = src.x > x ? c.x : c.y;
+         } else
+            for (int j = 0; j < CELLS; j++) {
+               const unsigned ay = min(__builtin_amdgcn_sad_u16((unsigned)(y + RW * j), (unsigned)src.y, 0u), w);
+               coef[u][j] = coef_at(__umul24(ay, stride) + row);
+            }
          if constexpr (MAT)
             chan[u] = ((const float *)&s_val[wave][i + u])[lane & 3];
          else
@@ -890,7 +908,7 @@ __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
          const int2 in = s_info[min(f, nf)];
          if (at >= 0) {
             s_src[wave][at] = src;
-            s_stride[wave][at] = ((unsigned)src.w << SH) + (1u << SH);
+            s_stride[wave][at] = (unsigned)(src.w + fl3k_de_cols(sizeof(AT)) - 1) << SH;
             s_val[wave][at] = val;
          }
          listed = found;
@@ -923,10 +941,10 @@ __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
    if (a.tab_bytes)
       scan([&](unsigned o) { return *(lds_at *)(uintptr_t)o; });
    else
-      scan([&](unsigned o) { return *(const AT *)((const unsigned char *)a.tab + o); });
+      scan([&](unsigned o) { return *(const C *)((const unsigned char *)a.tab + o); });
    for (int j = 0; j < CELLS; j++)
       for (int i = 0; i < 4; i++)
-         if (px + (MAT ? i : 0) < W && y + RW * j < H) *at_acc(j, i) = acc[j][i];
+         if (px + DX * j + (MAT ? i : 0) < W && y + DY * j < H) *at_acc(j, i) = acc[j][i];
 }
 
 __global__ __launch_bounds__(256) void k_fill_i32(int *p, long n, int v) {
