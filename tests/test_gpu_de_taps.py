@@ -106,3 +106,34 @@ def _compare(prod, bits, W, H, bank, fill, mfi=None):
     np.testing.assert_allclose(got, exact, rtol=tol, atol=0)
     if fill == 1.0:
         assert (got > start).any()
+
+
+@pytest.mark.parametrize("curve", [0.25, 0.4, 0.5, 0.9, 1.0, 3.0, 5.5])
+def test_kernel_index_beyond_100_hits(prod, curve):
+    """Kernel 100 + floor((hits - 100)^curve): every kernel reaches its own cell
+    alone, with a coefficient that tells its index.  Counts at and beside the
+    powers' integers and anywhere between.  (At an integer itself either side of
+    it is right: the power there is a matter of its last bit.)"""
+    nf = 1000
+    widths, coefs = np.full(nf, 0.9), np.arange(1.0, nf + 1)[:, None].copy()
+    rng = np.random.default_rng(7)
+    x = np.arange(1, 920) ** (1 / curve)
+    x = np.concatenate([x, x * (1 + 1e-7), x * (1 - 1e-7), x * (1 + 3e-6), x * (1 - 3e-6), np.round(x),
+                        np.exp(rng.uniform(-3, np.log(1000.0) / curve, 20000))])
+    W = 128
+    x = np.resize(x, (len(x) // W, W))
+    b = np.zeros(x.shape + (5,))
+    b[..., 3] = 255.0
+    b[..., 4] = 255.0 * (x + 100)
+    fsel = b[..., 4] / 255.0
+    acc = np.zeros(x.shape + (4,))
+    assert prod.lib().fl3h_density_estimate(
+        b.ctypes.data_as(ctypes.c_void_p), W, x.shape[0], 64, 1, 1068.0, 1.0 / 2000.0, curve, 2**31 - 1, nf - 1, 1, nf,
+        widths.ctypes.data_as(ctypes.c_void_p), coefs.ctypes.data_as(ctypes.c_void_p),
+        acc.ctypes.data_as(ctypes.c_void_p)) == 0, prod.last_error()
+    got = np.rint(acc[..., 3] / (1068.0 * np.log(1.0 + 255.0 / 2000.0))).astype(int) - 1
+    p = (fsel - 100) ** curve
+    ok = (fsel > 100) & (fsel < 2**31 - 1)
+    lo, hi = (np.minimum(100 + np.floor(p * f), nf - 1) for f in (1 - 1e-12, 1 + 1e-12))
+    assert ok.sum() > 10000
+    assert ((got >= lo) & (got <= hi))[ok].all()
