@@ -1804,7 +1804,7 @@ static int de_many_batch(const fl3d_de_params *p, const fl3_de_filters *const *d
    for (int k = 0; k < nd; k++)
       blocks += (long long)((g_ctx.rwidth[dej[k]] + DG_REGION_HOST - 1) / DG_REGION_HOST) *
                 ((g_ctx.rheight[dej[k]] + DG_REGION_HOST - 1) / DG_REGION_HOST);
-   const int cells = fl3k_de_cells(blocks);
+   const int cells = fl3k_de_cells(blocks, 33);
    int rw, rh;   // a gather workgroup's region
    fl3k_de_region(cells, &rw, &rh);
    size_t lds = 0;

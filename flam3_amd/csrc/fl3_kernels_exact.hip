@@ -747,7 +747,7 @@ __device__ __forceinline__ void de_gather_body(const DEArgs &a, int bx, int by) 
 // At 1920x1080 with 2x2 supersampling (8.4M cells, radius 9): 876 us with a
 // workgroup's shared lists and tests per tap, 635 us so (2.75e8 vector
 // instructions instead of 5.7e8; LDS is active for 60% of the time); 3840x2160
-// with 3x3 in FP64 44.0 ms (each term formed per tap) against 17.2 ms (vector
+// with 3x3 in FP64 44.0 ms (each term formed per tap) against 15.3 ms (vector
 // instructions and the vector caches' 64 addresses a load).
 // Wavefronts of a workgroup (they share the tables).
 constexpr int de_waves(int cells) { return cells == 2 ? 8 : 4; }
@@ -758,10 +758,11 @@ __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
    // read from the vector caches: 21.4 ms with 8 across, 19.5 with 16, 22.4 with 32
    // in the 3840x2160 case above; FP32 ones from LDS: no difference)
    constexpr int BW = sizeof(AT) == 4 ? 8 : 16, ACROSS = 4 * NW / BW;
-   // FP64, two cells: side by side, so that one load of 16 bytes has both
-   // coefficients (rows apart, a load each: 19.6 ms in that case, 17.2 so)
-   constexpr bool PAIR = sizeof(AT) == 8 && CELLS == 2;
-   constexpr int LW = PAIR ? BW / 2 : BW, RW = 64 / LW, BH = PAIR ? RW : RW * CELLS;
+   // FP64: two cells side by side, so that one load of 16 bytes has both
+   // coefficients (in that case two cells rows apart took 19.6 ms, side by side
+   // 17.2, two and two 15.3)
+   constexpr bool PAIR = sizeof(AT) == 8 && CELLS >= 2;
+   constexpr int LW = PAIR ? BW / 2 : BW, RW = 64 / LW, BH = PAIR ? RW * CELLS / 2 : RW * CELLS;
    typedef typename std::conditional<sizeof(AT) == 4, float4, double4>::type V4;
    __shared__ int4 s_src[NW][CAP];   // per wavefront: x, y, its table's place, radius + 1
    __shared__ unsigned s_stride[NW][CAP];   // bytes of a row of its square
@@ -786,19 +787,20 @@ __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
    for (int e = tid; e <= nf; e += 64 * NW)
       s_info[e] = e < nf ? make_int2((a.info[2 * e] << SH) + lds0, a.info[2 * e + 1]) : make_int2(lds0, -(1 << 20));
    // acc[j][i]: FP32, channel lane & 3 of cell (px + i, y + RW j) of this lane's
-   // four, as the matrix instruction leaves them; FP64, channel i of (x, y + RW j)
-   // or (x + j, y)
+   // four, as the matrix instruction leaves them; FP64, channel i of the lane's j-th
    constexpr bool MAT = sizeof(AT) == 4;
    const int px = MAT ? mx0 + (lane & (BW - 4)) : x;
-   constexpr int DX = PAIR ? 1 : 0, DY = PAIR ? 0 : RW;   // from a lane's cell to its next
+   // from a lane's first cell to its j-th
+   auto dxj = [](int j) { return PAIR ? j & 1 : 0; };
+   auto dyj = [](int j) { return PAIR ? RW * (j >> 1) : RW * j; };
    typedef AT AV __attribute__((ext_vector_type(4)));
    AV acc[CELLS];
    auto at_acc = [&](int j, int i) {
-      return (AT *)a.accum + ((px + DX * j + (MAT ? i : 0)) + (long)(y + DY * j) * W) * 4 + (MAT ? lane & 3 : i);
+      return (AT *)a.accum + ((px + dxj(j) + (MAT ? i : 0)) + (long)(y + dyj(j)) * W) * 4 + (MAT ? lane & 3 : i);
    };
    for (int j = 0; j < CELLS; j++)
       for (int i = 0; i < 4; i++)
-         acc[j][i] = px + DX * j + (MAT ? i : 0) < W && y + DY * j < H ? *at_acc(j, i) : (AT)0;
+         acc[j][i] = px + dxj(j) + (MAT ? i : 0) < W && y + dyj(j) < H ? *at_acc(j, i) : (AT)0;
    // this block's halo, as de_halo finds a region's
    int E = a.half;
    if (a.blkmax) {
@@ -840,10 +842,12 @@ __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
          if constexpr (PAIR) {
             // the nearer cell's coefficient and the next one: the right cell is
             // the nearer to a source at its right
-            const unsigned ay = min(__builtin_amdgcn_sad_u16((unsigned)y, (unsigned)src.y, 0u), w);
-            const auto c = coef_at(__umul24(ay, stride) + row);
-            coef[u][0] = src.x > x ? c.y : c.x;
-            coef[u][CELLS - 1] = src.x > x ? c.x : c.y;
+            for (int j = 0; j < CELLS; j += 2) {
+               const unsigned ay = min(__builtin_amdgcn_sad_u16((unsigned)(y + dyj(j)), (unsigned)src.y, 0u), w);
+               const auto c = coef_at(__umul24(ay, stride) + row);
+               coef[u][j] = src.x > x ? c.y : c.x;
+               coef[u][j + 1] = src.x > x ? c.x : c.y;
+            }
          } else
             for (int j = 0; j < CELLS; j++) {
                const unsigned ay = min(__builtin_amdgcn_sad_u16((unsigned)(y + RW * j), (unsigned)src.y, 0u), w);
@@ -944,7 +948,7 @@ __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
       scan([&](unsigned o) { return *(const C *)((const unsigned char *)a.tab + o); });
    for (int j = 0; j < CELLS; j++)
       for (int i = 0; i < 4; i++)
-         if (px + DX * j + (MAT ? i : 0) < W && y + DY * j < H) *at_acc(j, i) = acc[j][i];
+         if (px + dxj(j) + (MAT ? i : 0) < W && y + dyj(j) < H) *at_acc(j, i) = acc[j][i];
 }
 
 __global__ __launch_bounds__(256) void k_fill_i32(int *p, long n, int v) {
@@ -1002,8 +1006,10 @@ __global__ __launch_bounds__(64 * de_waves(CELLS)) void k_de_taps_many(const DEA
 // blocks of cells in all: two where that leaves every CU several workgroups,
 // one otherwise, where the gather is bound by how long a workgroup takes.
 // Kernel time with one and two: 640x480 (1271 blocks) 40 and 59 us, 7.7k blocks
-// 263 and 235 us, 32k blocks 838 and 672 us.
-extern "C" int fl3k_de_cells(long long blocks) { return blocks >= 4096 ? 2 : 1; }
+// 263 and 235 us, 32k blocks 838 and 672 us.  In FP64 four on large ones; one,
+// two and four: 4.1k blocks 837, 660 and 684 us, 8.1k 1614, 1292 and 1356, 10.8k
+// 2134, 1743 and 1729, the 3840x2160 case (147k) 17.2 ms with two, 15.3 with four.
+extern "C" int fl3k_de_cells(long long blocks, int bits) { return blocks < 4096 ? 1 : bits != 64 || blocks < 16384 ? 2 : 4; }
 // Cells across and down of a workgroup's region.
 extern "C" void fl3k_de_region(int cells, int *w, int *h) {
    *w = 4 * de_waves(cells);
@@ -1199,7 +1205,7 @@ extern "C" int fl3k_launch_deposit(const unsigned char *job, const double *pts, 
 extern "C" int fl3k_launch_de_tiled(const DEArgs *a, hipStream_t s, int bits, int exact) {
    const dim3 g1((a->width + 255) / 256, a->height), b1(256), b3(DG_CHUNK);
    const dim3 g3((a->width + DG_REGION - 1) / DG_REGION, (a->height + DG_REGION - 1) / DG_REGION);
-   const int cells = fl3k_de_cells((long long)g3.x * g3.y);
+   const int cells = fl3k_de_cells((long long)g3.x * g3.y, bits);
    int tw, th;
    fl3k_de_region(cells, &tw, &th);
    const dim3 gt((a->width + tw - 1) / tw, (a->height + th - 1) / th), bt(64 * de_waves(cells));
@@ -1211,7 +1217,9 @@ extern "C" int fl3k_launch_de_tiled(const DEArgs *a, hipStream_t s, int bits, in
    if (nblk) hipLaunchKernelGGL(k_fill_i32, dim3((unsigned)((nblk + 255) / 256)), dim3(256), 0, s, clear, nblk, 0);
    if (bits == 64) {
       hipLaunchKernelGGL((k_de_prep<double, double>), g1, b1, 0, s, *a);
-      if (!exact && cells == 2)
+      if (!exact && cells == 4)
+         hipLaunchKernelGGL((k_de_taps<double, 4>), gt, bt, lds, s, *a);
+      else if (!exact && cells == 2)
          hipLaunchKernelGGL((k_de_taps<double, 2>), gt, bt, lds, s, *a);
       else if (!exact)
          hipLaunchKernelGGL((k_de_taps<double, 1>), gt, bt, lds, s, *a);

@@ -37,7 +37,7 @@ int fl3k_launch_preview(const unsigned char *job, int xi, double range, int numv
 int fl3k_launch_deposit(const unsigned char *job, const double *pts, long long n, void *buckets, uint32_t *sat,
                         unsigned grid, size_t lds, hipStream_t s, int bits);
 int fl3k_launch_de_tiled(const DEArgs *a, hipStream_t s, int bits, int exact);
-int fl3k_de_cells(long long blocks);
+int fl3k_de_cells(long long blocks, int bits);
 void fl3k_de_region(int cells, int *w, int *h);
 int fl3k_launch_de_many(const DEArgs *as, const unsigned *prep_first, unsigned prep_blocks,
                         const unsigned *gather_first, unsigned gather_blocks, int n, hipStream_t s,

@@ -38,7 +38,8 @@ BANKS = {
 @pytest.mark.parametrize("W,H,bank,fill", [
     (1, 1, "flame", 1.0), (7, 5, "flame", 1.0), (8, 16, "one", 0.5), (9, 17, "flame", 0.3),
     (16, 16, "points", 0.7), (33, 31, "wide", 1.0), (65, 130, "flame", 0.02), (257, 64, "flame", 1.0),
-    (97, 40, "wide", 0.2), (1039, 1025, "flame", 0.1), (1025, 1039, "points", 0.5), (2049, 513, "wide", 0.01)])
+    (97, 40, "wide", 0.2), (1039, 1025, "flame", 0.1), (1025, 1039, "points", 0.5), (2049, 513, "wide", 0.01),
+    (2049, 2033, "flame", 0.05)])
 def test_taps_against_the_bank(prod, bits, W, H, bank, fill):
     """Both sum the same non-negative terms in the same order, so they differ
     by at most the roundings of each sum, one or three per term, and of the
