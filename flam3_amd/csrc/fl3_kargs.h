@@ -176,6 +176,14 @@ struct DEArgs {
 };
 #define FL3_DE_LDS_BYTES 49152   // most LDS bytes of tables and info a gather workgroup takes
 
+// A cell's index and the byte offset of its kernel index: sides are below
+// 65536, so an index fits 32 bits unsigned (46400 x 46400 cells are past 2^31)
+// and the offset does not.
+static inline __host__ __device__ unsigned fl3k_de_cell(int x, int y, int w) {
+   return (unsigned)x + (unsigned)y * (unsigned)w;
+}
+static inline __host__ __device__ size_t fl3k_de_findex_at(unsigned cell) { return (size_t)cell * sizeof(uint16_t); }
+
 // Columns of a production gather's table (entries of this size) beyond the
 // radius: its own zero column, and one more where two entries are read at once.
 static inline __host__ __device__ constexpr int fl3k_de_cols(size_t entry) { return entry == 8 ? 3 : 2; }

@@ -886,10 +886,10 @@ __device__ __forceinline__ void de_taps_body(const DEArgs &a, int bx, int by) {
          stepx = 64 % hw;
          stepy = 64 / hw;
       }
-      unsigned cell = (unsigned)(sx + sy * W);   // (histograms stay below 2^31 cells)
+      unsigned cell = fl3k_de_cell(sx, sy, W);
       const unsigned step = (unsigned)(stepx + stepy * W), wrap = (unsigned)(W - hw);
       auto kernel_at = [&](int k, unsigned c) {
-         return k < nh ? (int)*(const uint16_t *)((const unsigned char *)a.findex + (size_t)(c * 2u)) : (int)DE_SKIP;
+         return k < nh ? (int)*(const uint16_t *)((const unsigned char *)a.findex + fl3k_de_findex_at(c)) : (int)DE_SKIP;
       };
       int fnext = kernel_at(lane, cell);
       int listed = 0, found = 0, at = -1;   // sources in the list, and with the last 64's
@@ -1001,6 +1001,10 @@ __global__ __launch_bounds__(64 * de_waves(CELLS)) void k_de_taps_many(const DEA
    const unsigned local = blockIdx.x - first[j], cols = (unsigned)(a.width + 4 * de_waves(CELLS) - 1) / (4 * de_waves(CELLS));
    de_taps_body<float, CELLS>(a, (int)(local % cols), (int)(local / cols));
 }
+
+// Byte offset of the kernel index of cell (x, y), as the gather forms it (for
+// tests).
+extern "C" unsigned long long fl3k_de_findex_offset(int x, int y, int w) { return fl3k_de_findex_at(fl3k_de_cell(x, y, w)); }
 
 // Cells a lane of the production gather holds, for regions of `blocks` 16x16
 // blocks of cells in all: two where that leaves every CU several workgroups,

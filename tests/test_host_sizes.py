@@ -1,0 +1,17 @@
+"""Sizes, offsets and rules that the host works out for the kernels, at the
+ends of their ranges.  All CPU; no GPU calls."""
+import ctypes
+
+import pytest
+
+
+@pytest.mark.parametrize("x,y,w", [
+    (0, 0, 1), (46339, 46340, 46341), (46399, 46399, 46400), (65534, 32767, 65535), (0, 65534, 65535),
+    (65534, 65534, 65535)])
+def test_de_kernel_index_offset_past_2_31_cells(prod_lib, x, y, w):
+    """Byte offset of a cell's kernel index in the density estimation's gather:
+    two bytes a cell, beyond 32 bits from 2^31 cells on."""
+    f = prod_lib.fl3k_de_findex_offset
+    f.argtypes = [ctypes.c_int] * 3
+    f.restype = ctypes.c_ulonglong
+    assert f(x, y, w) == 2 * (x + y * w)
