@@ -551,7 +551,11 @@ int fl3h_render(flam3_frame *spec, void *out, int field, int nchan, int transp, 
       if (plan_batch_de(&P, batch_num, &de)) goto fail;
       /* every batch starts from empty buckets; its density estimate adds to
        * the accumulator (rect.c:709-721) */
-      if (batch_num > 0 && fl3d_clear_buckets()) goto devfail_de;
+      if (batch_num > 0) {
+         /* (the launches counted below on the device are this batch's) */
+         P.badvals += fl3d_deferred_badvals();
+         if (fl3d_clear_buckets()) goto devfail_de;
+      }
 
       /* Pass 0 uses fast deposits; if a hit counter saturated, pass 1
        * repeats the batch with saturating adds on every channel, reusing
@@ -561,6 +565,7 @@ int fl3h_render(flam3_frame *spec, void *out, int field, int nchan, int transp, 
             if (!saturated || P.replay) break;
             exact = 1;
             P.badvals -= batch_bad;
+            (void)fl3d_deferred_badvals();   /* those of pass 0 */
             batch_bad = 0.0;
             if (fl3d_clear_buckets()) goto devfail_de;
          }
