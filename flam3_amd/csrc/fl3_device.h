@@ -77,9 +77,10 @@ int fl3d_iterate_multi(const fl3d_multi_job *jobs, int njobs, int fuse, int exac
  * keys[2j], keys[2j+1]. */
 int fl3d_iterate_batch(const void *const *jobs, const size_t *job_bytes, int njobs, const fl3d_iter_params *p,
                        const uint64_t *keys, double *badvals, int *saturated);
-/* Bad values of the deferred launches since fl3d_begin.  Waits for the device,
- * unless fl3d_tonemap has since. */
-double fl3d_deferred_badvals(void);
+/* Bad values of the deferred launches since fl3d_begin or the last such call.
+ * Waits for the device, unless fl3d_tonemap has since; returns non-zero if the
+ * launches or the wait failed. */
+int fl3d_deferred_badvals(double *badvals);
 /* Bad values of render r of a fl3d_iterate_multi without badvals and saturated,
  * once the device's work up to it is known to be done (an image is here). */
 double fl3d_multi_badvals(int r);

@@ -447,13 +447,16 @@ static int copy_deferred() {
    return 0;
 }
 
-extern "C" double fl3d_deferred_badvals(void) {
+extern "C" int fl3d_deferred_badvals(double *badvals) {
    std::lock_guard<std::recursive_mutex> lk(g_mu);
-   if (!g_ctx.deferred) return 0.0;
+   *badvals = 0.0;
+   if (!g_ctx.deferred) return 0;
    const bool here = g_ctx.deferred_copied;
-   if (copy_deferred() || (!here && hipStreamSynchronize(g_ctx.stream) != hipSuccess)) return 0.0;
+   if (copy_deferred()) return 1;
+   if (!here) HIPCHK(hipStreamSynchronize(g_ctx.stream));
    g_ctx.deferred = g_ctx.deferred_copied = false;
-   return (double)g_ctx.counts[0];
+   *badvals = (double)g_ctx.counts[0];
+   return 0;
 }
 
 extern "C" double fl3d_multi_badvals(int r) {

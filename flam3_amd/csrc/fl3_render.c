@@ -552,9 +552,10 @@ int fl3h_render(flam3_frame *spec, void *out, int field, int nchan, int transp, 
       /* every batch starts from empty buckets; its density estimate adds to
        * the accumulator (rect.c:709-721) */
       if (batch_num > 0) {
-         /* (the launches counted below on the device are this batch's) */
-         P.badvals += fl3d_deferred_badvals();
-         if (fl3d_clear_buckets()) goto devfail_de;
+         /* (what the device counts from here on is this batch's) */
+         double before = 0.0;
+         if (fl3d_deferred_badvals(&before) || fl3d_clear_buckets()) goto devfail_de;
+         P.badvals += before;
       }
 
       /* Pass 0 uses fast deposits; if a hit counter saturated, pass 1
@@ -565,7 +566,8 @@ int fl3h_render(flam3_frame *spec, void *out, int field, int nchan, int transp, 
             if (!saturated || P.replay) break;
             exact = 1;
             P.badvals -= batch_bad;
-            (void)fl3d_deferred_badvals();   /* those of pass 0 */
+            /* (and the deferred ones of pass 0, dropped) */
+            if (fl3d_deferred_badvals(&batch_bad)) goto devfail_de;
             batch_bad = 0.0;
             if (fl3d_clear_buckets()) goto devfail_de;
          }
@@ -704,12 +706,15 @@ int fl3h_render(flam3_frame *spec, void *out, int field, int nchan, int transp, 
 
    if (!aborted) {
       fl3d_tm_params tp;
+      double bad = 0.0;
       plan_tm(&P, &tp);
-      if (fl3d_tonemap(&tp, P.filter, P.out, plan_out_stride(&P))) goto devfail;
-      P.badvals += fl3d_deferred_badvals();
+      if (fl3d_tonemap(&tp, P.filter, P.out, plan_out_stride(&P)) || fl3d_deferred_badvals(&bad)) goto devfail;
+      P.badvals += bad;
       plan_finish(&P);
    } else {
-      P.badvals += fl3d_deferred_badvals();
+      double bad = 0.0;
+      if (fl3d_deferred_badvals(&bad)) goto devfail;
+      P.badvals += bad;
       stats->badvals = P.badvals;
       stats->render_seconds = (int)(time(NULL) - P.tstart);
    }

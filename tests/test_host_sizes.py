@@ -15,3 +15,13 @@ def test_de_kernel_index_offset_past_2_31_cells(prod_lib, x, y, w):
     f.argtypes = [ctypes.c_int] * 3
     f.restype = ctypes.c_ulonglong
     assert f(x, y, w) == 2 * (x + y * w)
+
+
+def test_deferred_counts_say_whether_they_failed(prod_lib):
+    """fl3d_deferred_badvals returns its status beside the count, so that a
+    failed wait is not a count of zero; nothing deferred is neither."""
+    f = prod_lib.fl3d_deferred_badvals
+    f.argtypes = [ctypes.POINTER(ctypes.c_double)]
+    f.restype = ctypes.c_int
+    n = ctypes.c_double(-1.0)
+    assert f(ctypes.byref(n)) == 0 and n.value == 0.0
