@@ -676,11 +676,13 @@ static void launch_accum(const BinArgs *a, int ncu, hipStream_t s) {
    hipLaunchKernelGGL((k_bin_accum<KIND, RGB>), dim3((packed ? 2u : 1u) * (unsigned)ncu), dim3(FL3_ACC_THREADS), lds, s, *a);
    hipLaunchKernelGGL((k_bin_merge<RGB, packed ? 255 : 1>), dim3(8u * (unsigned)ncu), dim3(256), 0, s, *a);
 }
-// Bytes of the accumulation's partial sums for `records` in a chunk
-// (a tile of several items has more than an item's records, so at most two
-// items for every item's worth of records).
-extern "C" size_t fl3k_bin_partial_bytes(const BinArgs *a, long long records) {
-   return 16 * part_words(1u << a->shift, a->alpha >= 0) * (size_t)(2 * records / a->chunk + 1);
+// Bytes of the accumulation's partial sums for `records` in a chunk (a tile of
+// several items has more than an item's records, so at most two items for every
+// item's worth of records); rgb: the alphas are multiples of the counts.  Tiles
+// are those of the accumulation, also where the walkers count larger ones
+// (banded histograms).
+extern "C" size_t fl3k_bin_partial_bytes(int rgb, long long chunk, long long records) {
+   return 16 * part_words(1u << FL3_TILE_SHIFT, rgb != 0) * (size_t)(2 * records / chunk + 1);
 }
 
 // LDS of the accumulation into 32-bit histograms, at most.

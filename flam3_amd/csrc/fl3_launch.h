@@ -26,7 +26,7 @@ int fl3k_launch_bin_accum(const BinArgs *a, int ncu, int format, hipStream_t s);
 int fl3k_launch_bin_split(const BinArgs *a, int narrow_out, hipStream_t s);
 int fl3k_launch_bin_count(const BinArgs *a, int narrow, hipStream_t s);
 size_t fl3k_bin_f64_lds_bytes(int shift);
-size_t fl3k_bin_partial_bytes(const BinArgs *a, long long records);
+size_t fl3k_bin_partial_bytes(int rgb, long long chunk, long long records);
 int fl3k_bin_pass_records(void);   // records one accumulation workgroup loads per pass
 int fl3k_launch_copy_probe(const void *src, void *dst, long long n16, hipStream_t s);
 size_t fl3k_bin_lds_bytes(void);

@@ -25,3 +25,15 @@ def test_deferred_counts_say_whether_they_failed(prod_lib):
     f.restype = ctypes.c_int
     n = ctypes.c_double(-1.0)
     assert f(ctypes.byref(n)) == 0 and n.value == 0.0
+
+
+@pytest.mark.parametrize("rgb,per_item", [(1, 65536), (0, 81920)])
+@pytest.mark.parametrize("records,chunk", [(1 << 28, 1 << 17), (1 << 31, 1 << 18), (32768, 16384)])
+def test_partial_sums_are_those_of_the_accumulation_tiles(prod_lib, rgb, per_item, records, chunk):
+    """Partial sums hold 4096 cells an item (16 bytes a cell, 20 with alphas),
+    whatever tiles the walkers count: a 7716x4356 still of 2^28 records takes
+    0.3 GB."""
+    f = prod_lib.fl3k_bin_partial_bytes
+    f.argtypes = [ctypes.c_int, ctypes.c_longlong, ctypes.c_longlong]
+    f.restype = ctypes.c_size_t
+    assert f(rgb, chunk, records) == per_item * (2 * records // chunk + 1)
