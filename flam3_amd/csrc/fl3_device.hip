@@ -830,7 +830,14 @@ static int accum_items(BinArgs *b, long long records) {
    const long long c = records / (2 * g_ctx.ncu) / step * step;
    const long long most = records > 1LL << 30 ? 1LL << 18 : 1LL << 17;   // (less room for partial sums)
    b->chunk = (int)std::min((long long)b->chunk, std::min(std::max(c, 2LL * step), most));
-   if (g_ctx.partial.ensure(fl3k_bin_partial_bytes(b->alpha >= 0, b->chunk, records))) return 1;
+   const size_t bytes = fl3k_bin_partial_bytes(b->alpha >= 0, b->chunk, records);
+   b->partial = nullptr;
+   if (!bytes) {
+      if (b->round <= 0) return 0;
+      set_err("binned deposit: no room for partial sums");   // (its items are never that small)
+      return 1;
+   }
+   if (g_ctx.partial.ensure(bytes)) return 1;
    b->partial = g_ctx.partial.p;
    return 0;
 }

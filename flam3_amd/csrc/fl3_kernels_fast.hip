@@ -234,7 +234,8 @@ __global__ __launch_bounds__(NT) void k_bin_sort(BinArgs a, int sh, unsigned *cu
 // tile's records, or a.chunk of them), sum them in LDS and fold the sums into
 // registers, a thread the CPT cells it owns.  The sums of a tile of one work item
 // are then added to the histogram; those of the items of a fuller tile go to an
-// array of partial sums, which k_bin_merge adds up.  (Atomic adds from every
+// array of partial sums, which k_bin_merge adds up (or, where there is no room
+// for one, to the histogram with atomics).  (Atomic adds from every
 // item's 20 channels a thread ran at 1e11 a second: 0.2 us an item.)
 //
 // ACC_NARROW (4-byte records) and ACC_COLOUR (job records that carry the
@@ -440,7 +441,7 @@ __global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum(BinArgs a) {
          fetch(nx, 0);
       }
       next = __builtin_amdgcn_readfirstlane(drawn[slot]);
-      if (place_now) {
+      if (place_now && (PACKED || a.partial)) {
          uint4 *out = (uint4 *)a.partial + (size_t)(place_now - 1) * part_words(tile_cells, RGB);
          for (int j = 0; j < CPT; j++) {
             const int e = tid + j * FL3_ACC_THREADS;
@@ -450,29 +451,37 @@ __global__ __launch_bounds__(FL3_ACC_THREADS) void k_bin_accum(BinArgs a) {
       } else {
          uint32_t *bk = (uint32_t *)a.buckets + (size_t)cell0 * 5;
          const int nvalid = (int)min((long long)tile_cells, (long long)a.width * a.height - (long long)cell0);
-         // every load of the thread's cells is issued before any result is
-         // used, so that their latencies overlap (adding zero leaves a cell as
-         // it is, and the tile is this workgroup's alone)
          uint32_t sum[CPT][5], old[CPT][5];
          for (int j = 0; j < CPT; j++) {
             for (int c = 0; c < 3; c++) sum[j][c] = acc[j][c];
             sum[j][3] = RGB ? acc[j][3] * (unsigned)a.alpha : acc[j][RGB ? 0 : 4];
             sum[j][4] = acc[j][3] * (PACKED ? 255u : 1u);
          }
-         for (int j = 0; j < CPT; j++)
-            for (int c = 0; c < 5; c++) {
-               const int e = tid + j * FL3_ACC_THREADS;
-               old[j][c] = e < nvalid ? bk[(size_t)e * 5 + c] : 0u;
-            }
-         // (the sums first, each in a register of its own, so that no store
-         // waits for an earlier one to release its data register)
-         for (int j = 0; j < CPT; j++)
-            for (int c = 0; c < 5; c++) old[j][c] = add_u32_sat(old[j][c], sum[j][c]);
-         for (int j = 0; j < CPT; j++)
-            for (int c = 0; c < 5; c++) {
-               const int e = tid + j * FL3_ACC_THREADS;
-               if (e < nvalid) bk[(size_t)e * 5 + c] = old[j][c];
-            }
+         if (!PACKED && place_now) {   // (no room for partial sums: others add to the tile too)
+            for (int j = 0; j < CPT; j++)
+               for (int c = 0; c < 5; c++) {
+                  const int e = tid + j * FL3_ACC_THREADS;
+                  if (e < nvalid && sum[j][c]) sat_add(bk + (size_t)e * 5 + c, sum[j][c]);
+               }
+         } else {
+            // every load of the thread's cells is issued before any result is
+            // used, so that their latencies overlap (adding zero leaves a cell as
+            // it is, and the tile is this workgroup's alone)
+            for (int j = 0; j < CPT; j++)
+               for (int c = 0; c < 5; c++) {
+                  const int e = tid + j * FL3_ACC_THREADS;
+                  old[j][c] = e < nvalid ? bk[(size_t)e * 5 + c] : 0u;
+               }
+            // (the sums first, each in a register of its own, so that no store
+            // waits for an earlier one to release its data register)
+            for (int j = 0; j < CPT; j++)
+               for (int c = 0; c < 5; c++) old[j][c] = add_u32_sat(old[j][c], sum[j][c]);
+            for (int j = 0; j < CPT; j++)
+               for (int c = 0; c < 5; c++) {
+                  const int e = tid + j * FL3_ACC_THREADS;
+                  if (e < nvalid) bk[(size_t)e * 5 + c] = old[j][c];
+               }
+         }
       }
       if (!more) break;
    }
@@ -674,14 +683,21 @@ static void launch_accum(const BinArgs *a, int ncu, hipStream_t s) {
    if (lds > 65536)
       (void)hipFuncSetAttribute((const void *)k_bin_accum<KIND, RGB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
    hipLaunchKernelGGL((k_bin_accum<KIND, RGB>), dim3((packed ? 2u : 1u) * (unsigned)ncu), dim3(FL3_ACC_THREADS), lds, s, *a);
-   hipLaunchKernelGGL((k_bin_merge<RGB, packed ? 255 : 1>), dim3(8u * (unsigned)ncu), dim3(256), 0, s, *a);
+   if (a->partial) hipLaunchKernelGGL((k_bin_merge<RGB, packed ? 255 : 1>), dim3(8u * (unsigned)ncu), dim3(256), 0, s, *a);
 }
 // Bytes of the accumulation's partial sums for `records` in a chunk (a tile of
 // several items has more than an item's records, so at most two items for every
 // item's worth of records); rgb: the alphas are multiples of the counts.  Tiles
 // are those of the accumulation, also where the walkers count larger ones
-// (banded histograms).
+// (banded histograms).  0 where they would take more than 256 MiB and the
+// records' 8 bytes each: items of so few records are those of palette entries too
+// bright for more (171 records at 2.5e7, whose sums would take 250 GB for a
+// chunk of 2^28), and their sums go to the histogram with atomics.  Items of
+// 2^14 to 2^18 records, as the launch's size sets them, take at most 130 MB, or
+// 1.3 bytes a record.
 extern "C" size_t fl3k_bin_partial_bytes(int rgb, long long chunk, long long records) {
+   const double n = 16.0 * (double)part_words(1u << FL3_TILE_SHIFT, rgb != 0) * (2.0 * (double)records / (double)chunk + 1.0);
+   if (n > 268435456.0 + 8.0 * (double)records) return 0;
    return 16 * part_words(1u << FL3_TILE_SHIFT, rgb != 0) * (size_t)(2 * records / chunk + 1);
 }
 

@@ -37,3 +37,20 @@ def test_partial_sums_are_those_of_the_accumulation_tiles(prod_lib, rgb, per_ite
     f.argtypes = [ctypes.c_int, ctypes.c_longlong, ctypes.c_longlong]
     f.restype = ctypes.c_size_t
     assert f(rgb, chunk, records) == per_item * (2 * records // chunk + 1)
+
+
+@pytest.mark.parametrize("records", [32768, 1 << 22, 8 << 20, 1 << 26, 1 << 28, 1 << 31])
+@pytest.mark.parametrize("rgb", [0, 1])
+def test_partial_sums_of_ordinary_items_have_room(prod_lib, rgb, records):
+    """Items of 2^14 to 2^18 records as the launch's size sets them on 256 CUs;
+    shorter ones (entries too bright for more) only while their sums take no more
+    than 256 MiB and 8 bytes a record."""
+    f = prod_lib.fl3k_bin_partial_bytes
+    f.argtypes = [ctypes.c_int, ctypes.c_longlong, ctypes.c_longlong]
+    f.restype = ctypes.c_size_t
+    chunk = min(max(records // 512 // 8192 * 8192, 16384), 1 << 18 if records > 1 << 30 else 1 << 17)
+    room = (256 << 20) + 8 * records
+    assert 0 < f(rgb, chunk, records) <= room
+    for few in (1, 171, 5000):
+        want = (81920, 65536)[rgb] * (2 * records // few + 1)
+        assert f(rgb, few, records) in ((0, want) if abs(want / room - 1) < 0.01 else (want if want < room else 0,))
