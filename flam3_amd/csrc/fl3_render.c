@@ -46,9 +46,10 @@
  * and empties the set.  Interpolated sample densities differ in their last
  * bits between temporal samples (rect.c:797, 830-833), so the counts may
  * differ by a few samples: one launch takes them all, its walkers sized by
- * the largest. */
+ * the largest.  wait: return once the launch is done (a progress callback
+ * follows the device, and its abort leaves no launch under way). */
 static int flush_batch(void **jobs, size_t *bytes, int *n, const int64_t *nsamples, const uint64_t *keys, int exact,
-                       const fl3h_render_opts *opts, double *bad, int *sat) {
+                       int wait, const fl3h_render_opts *opts, double *bad, int *sat) {
    fl3d_iter_params ip;
    int rc, t, same = 1;
    int64_t nmax = nsamples[0];
@@ -70,7 +71,7 @@ static int flush_batch(void **jobs, size_t *bytes, int *n, const int64_t *nsampl
    ip.nwalkers = opts ? opts->nwalkers : 0;
    ip.deposit = opts ? opts->deposit : 0;
    ip.chunk = opts ? opts->chunk_samples : 0;
-   ip.defer = 1;
+   ip.defer = !wait;
    rc = fl3d_iterate_batch((const void *const *)jobs, bytes, *n, &ip, keys, bad, sat);
    for (t = 0; t < *n; t++) {
       free(jobs[t]);
@@ -531,6 +532,7 @@ int fl3h_render(flam3_frame *spec, void *out, int field, int nchan, int transp, 
    size_t *bbytes = NULL;
    int64_t *bns = NULL;   /* and their sample counts */
    int bn = 0, bts0 = 0;
+   const int wait = spec->progress != NULL;
 
    if (plan_open(&P, spec, out, field, nchan, transp, stats, opts)) return 1;
    nts = P.nts;
@@ -603,7 +605,7 @@ int fl3h_render(flam3_frame *spec, void *out, int field, int nchan, int transp, 
                plan_keys(&P, ts, batch_num * nts + ts);
                nsamp = plan_nsamples(&P, r->batch_size);
                if (bn == max_batch_jobs(opts)) {
-                  if (flush_batch(bjobs, bbytes, &bn, bns, P.keys + 2 * bts0, exact, opts, &bad, &sat)) {
+                  if (flush_batch(bjobs, bbytes, &bn, bns, P.keys + 2 * bts0, exact, wait, opts, &bad, &sat)) {
                      failed = 2;
                      break;
                   }
@@ -660,7 +662,7 @@ int fl3h_render(flam3_frame *spec, void *out, int field, int nchan, int transp, 
                 * to max_batch_jobs of them. */
                nsamp = plan_nsamples(&P, batch_size);
                if (bn == max_batch_jobs(opts)) {
-                  if (flush_batch(bjobs, bbytes, &bn, bns, P.keys + 2 * bts0, exact, opts, &bad, &sat))
+                  if (flush_batch(bjobs, bbytes, &bn, bns, P.keys + 2 * bts0, exact, wait, opts, &bad, &sat))
                      goto devfail_de;
                   if (sat) saturated = 1;
                }
@@ -678,7 +680,7 @@ int fl3h_render(flam3_frame *spec, void *out, int field, int nchan, int transp, 
          if (!aborted && bn > 0) {
             double bad = 0.0;
             int sat = 0;
-            if (flush_batch(bjobs, bbytes, &bn, bns, P.keys + 2 * bts0, exact, opts, &bad, &sat)) goto devfail_de;
+            if (flush_batch(bjobs, bbytes, &bn, bns, P.keys + 2 * bts0, exact, wait, opts, &bad, &sat)) goto devfail_de;
             P.badvals += bad;
             batch_bad += bad;
             if (sat) saturated = 1;
