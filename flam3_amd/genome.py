@@ -178,13 +178,14 @@ class Genome:
         g.temporal_filter_exp = self.temporal_filter_exp
         pal = self.palette if self.palette is not None else np.full((256, 3), 255.0)
         # (index, colour and alpha of every entry at once: entry by entry took
-        # longer than a small preview's render)
-        pal = np.asarray(pal, dtype=np.float64)
-        if len(pal) < 256:
-            raise IndexError("a palette has 256 entries, not %d" % len(pal))
+        # longer than a small preview's render; what is no array of rows of
+        # numbers is read entry by entry)
+        if not (type(pal) is np.ndarray and pal.ndim == 2 and pal.shape[0] >= 256 and pal.shape[1] >= 3
+                and pal.dtype.kind in "fiu"):
+            pal = np.array([[float(pal[i][k]) for k in range(3)] for i in range(256)])
         entries = np.ones((256, 5))
         entries[:, 0] = np.arange(256)
-        entries[:, 1:4] = pal[:256, :3] / 255.0
+        entries[:, 1:4] = pal[:256, :3].astype(np.float64) / 255.0
         ctypes.memmove(g.palette, entries.ctypes.data, entries.nbytes)
         xf = ctypes.cast(g.xform, abi.XFORM_P)
         nstd = len(self.xforms)
