@@ -2223,7 +2223,8 @@ extern "C" int fl3h_iterate(flam3_genome *cp, int n, int fuse, double *samples,
       a.n = n;
       a.fuse = fuse;
       a.nwalkers = nwalkers;
-      if (fl3k_launch_points(&a, lds_bytes_for<double>(h), lds_bytes_for<double>(h, false), g_ctx.stream, pick_tier(h))) {
+      if (fl3k_launch_points(&a, lds_bytes_for<double>(h), lds_bytes_for<double>(h, false), g_ctx.lds_max, g_ctx.ncu,
+                             g_ctx.stream, pick_tier(h))) {
          set_err("k_iterate_points launch failed");
          free(starts);
          break;

@@ -31,7 +31,7 @@ int fl3k_bin_pass_records(void);   // records one accumulation workgroup loads p
 int fl3k_launch_copy_probe(const void *src, void *dst, long long n16, hipStream_t s);
 size_t fl3k_bin_lds_bytes(void);
 int fl3k_launch_replay(const IterArgs *a, unsigned grid, size_t lds, hipStream_t s, int bits);
-int fl3k_launch_points(const PointsArgs *a, size_t lds, size_t lds_lone, hipStream_t s, int tier);
+int fl3k_launch_points(const PointsArgs *a, size_t lds, size_t lds_lone, size_t lds_max, int ncu, hipStream_t s, int tier);
 int fl3k_launch_preview(const unsigned char *job, int xi, double range, int numvals, int depth, double *result,
                         uint32_t *isaac, size_t lds, hipStream_t s);
 int fl3k_launch_deposit(const unsigned char *job, const double *pts, long long n, void *buckets, uint32_t *sat,

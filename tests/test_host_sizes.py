@@ -54,3 +54,16 @@ def test_partial_sums_of_ordinary_items_have_room(prod_lib, rgb, records):
     for few in (1, 171, 5000):
         want = (81920, 65536)[rgb] * (2 * records // few + 1)
         assert f(rgb, few, records) in ((0, want) if abs(want / room - 1) < 0.01 else (want if want < room else 0,))
+
+
+@pytest.mark.parametrize("lds,walkers", [
+    (1000, 4096), (32767, 4096), (32769, 3072), (50000, 2048), (73728, 2048), (73729, 1024), (100000, 1024),
+    (160000, 1024)])
+def test_walkers_that_run_one_per_wavefront(prod_lib, lds, walkers):
+    """fl3h_iterate takes a wavefront per walker up to four rounds of those that
+    a 256-CU chip of 160 KB LDS holds, at most four a CU (8 KB of LDS each beside
+    the genome's)."""
+    f = prod_lib.fl3k_lone_walkers
+    f.argtypes = [ctypes.c_size_t, ctypes.c_size_t, ctypes.c_int]
+    f.restype = ctypes.c_int
+    assert f(lds, 160 << 10, 256) == walkers
