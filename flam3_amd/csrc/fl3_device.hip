@@ -1560,6 +1560,15 @@ static bool de_tables_ok(const fl3_de_filters *de, size_t entry) {
    return de_table_entries(de, entry) * (double)entry < 0x7fff0000;
 }
 
+// Whether the values that a 32-bit cell adds, at most 2^32 times
+// k1 log(1 + 2^32 k2), are finite as floats.  The production gather multiplies them
+// by zero beyond their kernel, so where they may not be (a negative contrast
+// takes the logarithm of negative numbers) the exact gather sums them.
+extern "C" int fl3k_de_values_finite(double k1, double k2) {
+   const double most = 4294967296.0;
+   return k2 >= 0.0 && fabs(k1) * log(1.0 + most * k2) * most <= 1e38;
+}
+
 // A filter bank as the production gather reads it (DEArgs::tab, info): of
 // kernel i, radius r = ceil(width) - 1, a square of the coefficients by |dy|,
 // |dx| with a row and a column (doubles: two) of zeros beyond the radius.  (A bank whose rows
@@ -1659,7 +1668,8 @@ extern "C" int fl3d_density(const fl3d_de_params *p, const fl3_de_filters *de) {
    std::lock_guard<std::recursive_mutex> lk(g_mu);
    DEArgs a;
    memset(&a, 0, sizeof(a));
-   const int exact = p->exact || !de_tables_ok(de, g_ctx.bits == 64 ? 8 : 4);
+   const int exact = p->exact || !de_tables_ok(de, g_ctx.bits == 64 ? 8 : 4) ||
+                     (g_ctx.bits != 64 && !fl3k_de_values_finite(p->k1, p->k2));
    if (de->max_filter_index >= 1024) {
       set_err("density estimation: more than 1024 kernels");
       return 1;
@@ -1729,7 +1739,7 @@ extern "C" int fl3d_density_many(const fl3d_de_params *p, const fl3_de_filters *
       tcells += (long long)g_ctx.rwidth[i] * g_ctx.rheight[i];
       const bool has = de[i] && de[i]->max_filter_index > 0;
       if (has && batched && !p[i].exact && de[i]->max_filter_index < 1024 && g_ctx.rwidth[i] < 65536 &&
-          g_ctx.rheight[i] < 65536 && de_tables_ok(de[i], sizeof(float))) {
+          g_ctx.rheight[i] < 65536 && de_tables_ok(de[i], sizeof(float)) && fl3k_de_values_finite(p[i].k1, p[i].k2)) {
          dej.push_back(i);
       }
    }

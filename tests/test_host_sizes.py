@@ -67,3 +67,17 @@ def test_walkers_that_run_one_per_wavefront(prod_lib, lds, walkers):
     f.argtypes = [ctypes.c_size_t, ctypes.c_size_t, ctypes.c_int]
     f.restype = ctypes.c_int
     assert f(lds, 160 << 10, 256) == walkers
+
+
+@pytest.mark.parametrize("k1,k2,finite", [
+    (1068.0, 1 / 2000.0, 1), (-1068.0, 1 / 2000.0, 1), (0.0, 0.0, 1), (1e25, 1e10, 1), (1e27, 1e10, 0),
+    (1068.0, -1 / 2000.0, 0), (1068.0, float("inf"), 0), (0.0, float("inf"), 0), (float("nan"), 1.0, 0),
+    (1.0, float("nan"), 0), (float("inf"), 1.0, 0)])
+def test_values_that_the_float_gather_may_multiply_by_zero(prod_lib, k1, k2, finite):
+    """A 32-bit cell adds at most 2^32 k1 log(1 + 2^32 k2) to a channel: the
+    production gather takes those below 1e38 only (1e25 and 1e10 give 1.9e36,
+    100 times that is too much)."""
+    f = prod_lib.fl3k_de_values_finite
+    f.argtypes = [ctypes.c_double] * 2
+    f.restype = ctypes.c_int
+    assert f(k1, k2) == finite
