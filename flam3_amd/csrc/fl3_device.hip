@@ -614,6 +614,10 @@ static int bin_shift_cells(long long ncells) {
    return ((ncells + (1LL << sh) - 1) >> sh) <= FL3_MAX_BINS && fl3k_bin_lds_bytes() <= g_ctx.lds_max ? sh : 0;
 }
 
+// Records form a point's cell with a 24-bit product of the width and the row:
+// histograms with a longer side take direct deposits.
+extern "C" int fl3k_record_sides(int width, int height) { return width < 1 << 24 && height < 1 << 24; }
+
 // Tile shift of the accumulation into double buckets (bits 64: five doubles
 // per cell in LDS), 0 if LDS is too small.
 static int f64_tile_shift() {
@@ -1191,7 +1195,8 @@ extern "C" int fl3d_iterate_batch(const void *const *jobs, const size_t *job_byt
          return 1;
       }
       const long long min_binned = js.linear || g_ctx.bits == 64 ? FL3_BIN_MIN_SAMPLES : FL3_BIN_MIN_STEPPED;
-      const bool binned = binnable && (p->deposit == 2 || (p->deposit == 0 && p->nsamples * njobs >= min_binned));
+      const bool binned = binnable && fl3k_record_sides(g_ctx.width, g_ctx.height) &&
+                          (p->deposit == 2 || (p->deposit == 0 && p->nsamples * njobs >= min_binned));
       // (binned deposits too count toward what later direct ones may reach)
       const bool direct_bytes = byte_deposits(js.h, js.n, (double)p->nsamples * njobs);
       defer = p->defer && (binned || direct_bytes || g_ctx.bits == 64);
@@ -1287,6 +1292,7 @@ extern "C" int fl3d_iterate_multi(const fl3d_multi_job *jobs, int njobs, int fus
    const int shift = g_ctx.bits != 64 && njobs < 65536 && nxf_max <= 256 ? bin_shift_cells(tcells) : 0;
    const int nbins = shift > 0 ? (int)((tcells + (1LL << shift) - 1) >> shift) : 0;
    bool use_rec = shift > 0 && tcells < 0xffffffffLL;
+   for (size_t r = 0; r < g_ctx.rcell0.size(); r++) use_rec = use_rec && fl3k_record_sides(g_ctx.rwidth[r], g_ctx.rheight[r]);
    std::vector<JobDesc> d((size_t)njobs);
    long long gblocks[MG_N] = {0};
    for (int j = 0; j < njobs; j++) {

@@ -81,3 +81,13 @@ def test_values_that_the_float_gather_may_multiply_by_zero(prod_lib, k1, k2, fin
     f.argtypes = [ctypes.c_double] * 2
     f.restype = ctypes.c_int
     assert f(k1, k2) == finite
+
+
+@pytest.mark.parametrize("width,height,ok", [
+    ((1 << 24) - 1, 2, 1), (1 << 24, 2, 0), (2, (1 << 24) - 1, 1), (1, 1 << 24, 0), (65535, 65535, 1), (1, 1, 1)])
+def test_sides_that_records_can_hold(prod_lib, width, height, ok):
+    """A record's cell is a 24-bit product of the width and the row: longer sides
+    take direct deposits."""
+    assert prod_lib.fl3k_record_sides(width, height) == ok
+    low = (1 << 24) - 1
+    assert ok == ((width & low) * (height & low) == width * height)
