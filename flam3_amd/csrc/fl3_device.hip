@@ -685,6 +685,7 @@ struct JobSet {
    size_t lds_rec = 0;                     // the same without the palette (record modes)
    int tier = 0, nxf_max = 0;
    bool same_tables = true;                // one palette and visibility set for all jobs
+   int narrow = -1;                        // jobs_narrow's answer, if it was asked
    bool linear = false;
 };
 
@@ -960,18 +961,34 @@ static int bin_banded(const BinArgs &b1, int format, int band, int shift, hipStr
    return 0;
 }
 
+// Whether 4-byte records hold the jobs' samples in a histogram of ncells cells.
+static bool jobs_narrow(JobSet &js, long long ncells) {
+   if (js.narrow < 0) {
+      bool narrow = narrow_records_ok(js.h[0], ncells);
+      for (int j = 1; narrow && !js.same_tables && j < js.n; j++) narrow = same_narrow_tables(js.h[0], js.h[j]);
+      js.narrow = narrow;
+   }
+   return js.narrow != 0;
+}
+
+// Samples from which a launch's deposits are sorted by tile (FL3_BIN_MIN_*);
+// rounds: records round otherwise than direct deposits; tables: each job brings
+// a palette of its own.
+extern "C" long long fl3k_bin_min_samples(int rounds, int njobs, int tables) {
+   return rounds || (tables && njobs > FL3_BIN_FEW_TABLES) ? FL3_BIN_MIN_SAMPLES : FL3_BIN_MIN_STEPPED;
+}
+
 // shift: the accumulation tiles' (cells per tile = 1 << shift); band: 0, or
 // the band shift of a histogram of more than FL3_MAX_BINS tiles: the
 // walkers then count their records per 2^(band - FL3_SUPER_SHIFT)-cell tile,
 // a first sort groups them by band, and each band is counted, sorted by tile
 // and accumulated on its own (iterate_banded_chunk).
-static int iterate_binned(IterArgs a, long long W, long long Wj, const JobSet &js, const fl3d_iter_params *p,
+static int iterate_binned(IterArgs a, long long W, long long Wj, JobSet &js, const fl3d_iter_params *p,
                           int shift, int band) {
    const long long ncells = (long long)g_ctx.width * g_ctx.height;
    const int wshift = band ? band - FL3_SUPER_SHIFT : shift;   // the walkers' counting tiles
    const int nbins = (int)((ncells + (1LL << wshift) - 1) >> wshift);
-   bool narrow = !band && narrow_records_ok(js.h[0], ncells);
-   for (int j = 1; narrow && !js.same_tables && j < js.n; j++) narrow = same_narrow_tables(js.h[0], js.h[j]);
+   const bool narrow = !band && jobs_narrow(js, ncells);
    // double buckets of a banded histogram: the walkers write 8-byte records,
    // the band pass 4-byte ones (cells within a 2^24-cell band) when the
    // tables allow
@@ -1194,7 +1211,10 @@ extern "C" int fl3d_iterate_batch(const void *const *jobs, const size_t *job_byt
                  "", (long)FL3_MAX_BINS);
          return 1;
       }
-      const long long min_binned = js.linear || g_ctx.bits == 64 ? FL3_BIN_MIN_SAMPLES : FL3_BIN_MIN_STEPPED;
+      const bool rounds = js.linear || g_ctx.bits == 64;
+      const bool tables = !rounds && binnable && !js.same_tables && njobs > FL3_BIN_FEW_TABLES &&
+                          !jobs_narrow(js, (long long)g_ctx.width * g_ctx.height);
+      const long long min_binned = fl3k_bin_min_samples(rounds, njobs, tables);
       const bool binned = binnable && fl3k_record_sides(g_ctx.width, g_ctx.height) &&
                           (p->deposit == 2 || (p->deposit == 0 && p->nsamples * njobs >= min_binned));
       // (binned deposits too count toward what later direct ones may reach)

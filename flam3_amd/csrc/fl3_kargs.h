@@ -89,9 +89,13 @@ struct IterArgs {
 // samples take 264-367 us a render over eight genomes (585 over others), sorted
 // ones 293-305; of 164000 319-504 and 337-347; of 960000 349-908 (8 ms where most
 // samples meet in a cell) and 316-326.  Linear palettes and double histograms
-// round otherwise in records and keep to the older line.
+// round otherwise in records and keep to the older line, as do launches of more
+// than a few jobs with a palette each, which the host lays out for job records at 2
+// us a job: 1000 jobs of 41000 to 960000 samples in all 2.3 ms with direct
+// deposits, 4.5 ms sorted; 100 jobs 0.50-0.80 and 0.73 ms.
 #define FL3_BIN_MIN_STEPPED (1LL << 15)
 #define FL3_BIN_MIN_SAMPLES (1LL << 20)
+#define FL3_BIN_FEW_TABLES 32
 
 // Record formats of fl3k_launch_bin beyond 0 (8-byte records), 1 (4-byte
 // records) and 2 (job records): the same records into double buckets.
