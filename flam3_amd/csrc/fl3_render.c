@@ -201,6 +201,8 @@ typedef struct {
    int vib_gam_n;
    uint64_t *keys;                /* two per temporal sample */
    fl3_segment *segment;          /* the control points around the frame's time (NULL for a still) */
+   int *starts, starts_chaos;     /* a still's selection breakpoints, which its temporal samples share, and whether
+                                     they are those of xaos rows (NULL: each sample has its own) */
    uint32_t *walker_states;       /* replay: 36 words per reference thread */
    time_t tstart;
 } render_plan;
@@ -210,6 +212,7 @@ static void plan_close(render_plan *P) {
    free(P->temporal_filter);
    free(P->temporal_deltas);
    fl3_segment_close(P->segment);
+   free(P->starts);
    free(P->cam);
    free(P->walker_states);
    free(P->keys);
@@ -301,6 +304,19 @@ fail:
    return 1;
 }
 
+/* The selection table's breakpoints (what a job holds) of cp; NULL after a
+ * message if it has none. */
+static int *selection_starts(flam3_genome *cp) {
+   const int ns = cp->num_xforms - (cp->final_xform_index >= 0);
+   int nrows, *starts = (int *)malloc(sizeof(int) * (size_t)(ns + 1) * (size_t)(ns > 0 ? ns : 1));
+   if (!starts || fl3_xform_starts(cp, starts, &nrows)) {
+      free(starts);
+      fprintf(stderr, "create xform distrib returned error: aborting.\n");
+      return NULL;
+   }
+   return starts;
+}
+
 /* The batch's density-estimation filters, from the genome at its first
  * temporal sample (rect.c:726-747). */
 static int plan_batch_de(render_plan *P, int batch_num, fl3_de_filters *de) {
@@ -324,6 +340,16 @@ static int plan_batch_de(render_plan *P, int batch_num, fl3_de_filters *de) {
       }
    } else
       de->max_filter_index = 0;
+   /* (one control point: the same weights at every time.  63 xforms with xaos
+    * take 6 us a sample.) */
+   if (P->spec->ngenomes == 1 && P->nts > 1 && !P->starts) {
+      P->starts = selection_starts(&P->cp);
+      P->starts_chaos = P->cp.chaos_enable;
+      if (!P->starts) {
+         fl3_free_de_filters(de);
+         return 1;
+      }
+   }
    return 0;
 }
 
@@ -333,8 +359,8 @@ static int plan_batch_de(render_plan *P, int batch_num, fl3_de_filters *de) {
 static int plan_ts_job(render_plan *P, int tidx, int first, void **job, size_t *job_bytes, double *batch_size) {
    flam3_genome *cp = &P->cp;
    const double color_scalar = P->temporal_filter[tidx];
-   int *starts;
-   int i, j, nrows, ns;
+   int *own = NULL;
+   int i, j;
    *job = NULL;
    if (fl3_interpolate_in(P->segment, P->spec->genomes, P->spec->ngenomes,
                           P->spec->time + P->temporal_deltas[tidx], 0, cp))
@@ -344,21 +370,17 @@ static int plan_ts_job(render_plan *P, int tidx, int first, void **job, size_t *
       return 1;
    }
    for (i = 0; i < cp->num_xforms; i++) fl3_xform_precalc(&cp->xform[i]);
-   /* the selection table's breakpoints (what the job holds) */
-   ns = cp->num_xforms - (cp->final_xform_index >= 0);
-   starts = (int *)malloc(sizeof(int) * (size_t)(ns + 1) * (size_t)(ns > 0 ? ns : 1));
-   if (!starts || fl3_xform_starts(cp, starts, &nrows)) {
-      free(starts);
-      fprintf(stderr, "create xform distrib returned error: aborting.\n");
+   if (P->starts)
+      cp->chaos_enable = P->starts_chaos;
+   else if (!(own = selection_starts(cp)))
       return 1;
-   }
    /* palette scaled to the white level and the temporal weight (rect.c:778-782) */
    for (j = 0; j < 256; j++)
       for (i = 0; i < 4; i++) P->cam->dmap[j][i] = cp->palette[j].color[i] * WHITE_LEVEL * color_scalar;
    P->cam->cmap_size = P->cmap_size;
    P->cam->palette_mode = cp->palette_mode;
    if (setup_camera(P->spec, cp, P->field, P->oversample, &P->geo, P->cam)) {
-      free(starts);
+      free(own);
       return 1;
    }
    *batch_size = P->geo.sample_density * P->geo.image_width * P->geo.image_height / (P->nbatches * P->nts);
@@ -371,8 +393,8 @@ static int plan_ts_job(render_plan *P, int tidx, int first, void **job, size_t *
       P->background[2] += cp->background[2];
       P->vib_gam_n++;
    }
-   *job = fl3_pack_job_starts(cp, starts, P->cam, job_bytes);
-   free(starts);
+   *job = fl3_pack_job_starts(cp, P->starts ? P->starts : own, P->cam, job_bytes);
+   free(own);
    return *job ? 0 : 1;
 }
 
