@@ -201,8 +201,8 @@ typedef struct {
    int vib_gam_n;
    uint64_t *keys;                /* two per temporal sample */
    fl3_segment *segment;          /* the control points around the frame's time (NULL for a still) */
-   int *starts, starts_chaos;     /* a still's selection breakpoints, which its temporal samples share, and whether
-                                     they are those of xaos rows (NULL: each sample has its own) */
+   int *starts, starts_chaos;     /* a still's selection breakpoints, which its temporal samples and batches share,
+                                     and whether they are those of xaos rows (NULL: each has its own) */
    uint32_t *walker_states;       /* replay: 36 words per reference thread */
    time_t tstart;
 } render_plan;
@@ -341,8 +341,8 @@ static int plan_batch_de(render_plan *P, int batch_num, fl3_de_filters *de) {
    } else
       de->max_filter_index = 0;
    /* (one control point: the same weights at every time.  63 xforms with xaos
-    * take 6 us a sample.) */
-   if (P->spec->ngenomes == 1 && P->nts > 1 && !P->starts) {
+    * take 6 us a sample or batch.) */
+   if (P->spec->ngenomes == 1 && P->nts * P->nbatches > 1 && !P->starts) {
       P->starts = selection_starts(&P->cp);
       P->starts_chaos = P->cp.chaos_enable;
       if (!P->starts) {
