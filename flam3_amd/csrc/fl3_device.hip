@@ -973,9 +973,10 @@ static bool jobs_narrow(JobSet &js, long long ncells) {
 
 // Samples from which a launch's deposits are sorted by tile (FL3_BIN_MIN_*);
 // rounds: records round otherwise than direct deposits; tables: each job brings
-// a palette of its own.
-extern "C" long long fl3k_bin_min_samples(int rounds, int njobs, int tables) {
-   return rounds || (tables && njobs > FL3_BIN_FEW_TABLES) ? FL3_BIN_MIN_SAMPLES : FL3_BIN_MIN_STEPPED;
+// a palette of its own; wave: the walkers draw the xform per wavefront.
+extern "C" long long fl3k_bin_min_samples(int rounds, int njobs, int tables, int wave) {
+   if (rounds || (tables && (njobs > FL3_BIN_FEW_TABLES || !wave))) return FL3_BIN_MIN_SAMPLES;
+   return wave ? FL3_BIN_MIN_STEPPED : FL3_BIN_MIN_XAOS;
 }
 
 // shift: the accumulation tiles' (cells per tile = 1 << shift); band: 0, or
@@ -1212,9 +1213,10 @@ extern "C" int fl3d_iterate_batch(const void *const *jobs, const size_t *job_byt
          return 1;
       }
       const bool rounds = js.linear || g_ctx.bits == 64;
-      const bool tables = !rounds && binnable && !js.same_tables && njobs > FL3_BIN_FEW_TABLES &&
+      const bool wave = jobs_wave_ok(js.h, js.n);
+      const bool tables = !rounds && binnable && !js.same_tables && (njobs > FL3_BIN_FEW_TABLES || !wave) &&
                           !jobs_narrow(js, (long long)g_ctx.width * g_ctx.height);
-      const long long min_binned = fl3k_bin_min_samples(rounds, njobs, tables);
+      const long long min_binned = fl3k_bin_min_samples(rounds, njobs, tables, wave);
       const bool binned = binnable && fl3k_record_sides(g_ctx.width, g_ctx.height) &&
                           (p->deposit == 2 || (p->deposit == 0 && p->nsamples * njobs >= min_binned));
       // (binned deposits too count toward what later direct ones may reach)
@@ -1232,7 +1234,7 @@ extern "C" int fl3d_iterate_batch(const void *const *jobs, const size_t *job_byt
          if (iterate_binned(a, W, Wj, js, p, shift, band)) return 1;
       } else {
          const int pk = prof_begin(ST_ITER);
-         const size_t lw = with_shuffle(a, js.lds, jobs_wave_ok(js.h, js.n));
+         const size_t lw = with_shuffle(a, js.lds, wave);
          a.bytes = direct_bytes;
          const int lrc =
              fl3k_launch_iter_fast(&a, (unsigned)(W / 256), lw, g_ctx.stream, g_ctx.bits, p->exact, js.tier);

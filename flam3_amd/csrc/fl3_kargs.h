@@ -92,9 +92,14 @@ struct IterArgs {
 // round otherwise in records and keep to the older line, as do launches of more
 // than a few jobs with a palette each, which the host lays out for job records at 2
 // us a job: 1000 jobs of 41000 to 960000 samples in all 2.3 ms with direct
-// deposits, 4.5 ms sorted; 100 jobs 0.50-0.80 and 0.73 ms.
+// deposits, 4.5 ms sorted; 100 jobs 0.50-0.80 and 0.73 ms.  Walkers with xaos,
+// which take longer over records, in between: direct and sorted 41000 samples of 30
+// xforms 775 and 847 us, 120000 933 and 983, 262000 972 and 1023; of 3 xforms 374-432
+// and 437-483, 496-617 and 485-551, 550-886 and 508-569; with a palette a job
+// 458 and 533 us a launch.
 #define FL3_BIN_MIN_STEPPED (1LL << 15)
 #define FL3_BIN_MIN_SAMPLES (1LL << 20)
+#define FL3_BIN_MIN_XAOS (1LL << 17)
 #define FL3_BIN_FEW_TABLES 32
 
 // Record formats of fl3k_launch_bin beyond 0 (8-byte records), 1 (4-byte

@@ -93,12 +93,14 @@ def test_sides_that_records_can_hold(prod_lib, width, height, ok):
     assert ok == ((width & low) * (height & low) == width * height)
 
 
-@pytest.mark.parametrize("rounds,njobs,tables,samples", [
-    (0, 1, 0, 1 << 15), (0, 1000, 0, 1 << 15), (0, 32, 1, 1 << 15), (0, 33, 1, 1 << 20), (0, 1000, 1, 1 << 20),
-    (1, 1, 0, 1 << 20), (1, 1000, 1, 1 << 20)])
-def test_samples_from_which_deposits_are_sorted(prod_lib, rounds, njobs, tables, samples):
-    """Launches of many jobs with a palette each keep to the line of 2^20 samples."""
+@pytest.mark.parametrize("rounds,njobs,tables,wave,samples", [
+    (0, 1, 0, 1, 1 << 15), (0, 1000, 0, 1, 1 << 15), (0, 32, 1, 1, 1 << 15), (0, 33, 1, 1, 1 << 20),
+    (0, 1000, 1, 1, 1 << 20), (1, 1, 0, 1, 1 << 20), (1, 1000, 1, 0, 1 << 20), (0, 1, 0, 0, 1 << 17),
+    (0, 1000, 0, 0, 1 << 17), (0, 2, 1, 0, 1 << 20), (0, 33, 1, 0, 1 << 20)])
+def test_samples_from_which_deposits_are_sorted(prod_lib, rounds, njobs, tables, wave, samples):
+    """Launches of many jobs with a palette each, or of any with xaos, keep to the
+    line of 2^20 samples; xaos and one palette to 2^17."""
     f = prod_lib.fl3k_bin_min_samples
-    f.argtypes = [ctypes.c_int] * 3
+    f.argtypes = [ctypes.c_int] * 4
     f.restype = ctypes.c_longlong
-    assert f(rounds, njobs, tables) == samples
+    assert f(rounds, njobs, tables, wave) == samples
