@@ -1174,22 +1174,23 @@ extern "C" int fl3k_launch_replay(const IterArgs *a, unsigned grid, size_t lds, 
 
 // Up to this many walkers of a genome whose LDS image without the palette is
 // lds_lone bytes one per wavefront (k_iterate_lone), more of them one per lane
-// (k_iterate_points): four rounds of what the chip holds at once, a wavefront a
-// SIMD or fewer where the workgroups' LDS leaves no room for four a CU.  220 steps of 1
-// / 1024 / 4096 walkers of a genome of six xforms and a final one: 0.74 / 1.6 / 5.3
-// ms per wavefront, 9.1 / 9.8 / 10.7 ms per lane; six xforms of 12 variations
-// of the whole library, 1024 / 4096 walkers: 5.5 / 21.4 and 27.4 / 28.6 ms; 40 such
-// xforms (100 KB, one workgroup a CU), 256 / 1024 / 2048 / 4096 walkers: 7.9 / 30 /
-// 60 / 120 and 50 / 52 / 53 / 52 ms.
-extern "C" int fl3k_lone_walkers(size_t lds_lone, size_t lds_max, int ncu) {
+// (k_iterate_points), whose time does not depend on their number: some rounds of
+// what the chip holds at once, a wavefront a SIMD or fewer where the workgroups'
+// LDS leaves no room for four a CU; four rounds for the classic variations, two for
+// others, whose wavefronts are slower.  120 steps, ms, per wavefront and per lane:
+// six xforms and a final one 1024 walkers 0.40 and 3.8, 4096 1.15 and 3.9; 63 xforms
+// (one workgroup a CU) 1024 1.1 and 2.8, 3072 3.2 and 2.8; three xforms of the whole
+// library 2048 4.3 and 5.6, 3072 6.4 and 5.6; 40 of 12 variations (one a CU) 512 8.0
+// and 25.9, 2048 30.8 and 26.6.
+extern "C" int fl3k_lone_walkers(size_t lds_lone, size_t lds_max, int ncu, int tier) {
    const size_t lds = lds_lone + sizeof(double) * 16 * FL3_MAX_XFORMS, at_once = lds < lds_max ? lds_max / lds : 1;
-   return 4 * ncu * (int)(at_once < 4 ? at_once : 4);
+   return (tier == 0 ? 4 : 2) * ncu * (int)(at_once < 4 ? at_once : 4);
 }
 
 // lds, lds_lone: the genome's LDS image with and without the palette; lds_max: a CU's
 extern "C" int fl3k_launch_points(const PointsArgs *a, size_t lds, size_t lds_lone, size_t lds_max, int ncu,
                                   hipStream_t s, int tier) {
-   if (a->nwalkers > fl3k_lone_walkers(lds_lone, lds_max, ncu))
+   if (a->nwalkers > fl3k_lone_walkers(lds_lone, lds_max, ncu, tier))
       hipLaunchKernelGGL(k_iterate_points, dim3((a->nwalkers + 63) / 64), dim3(64), lds, s, *a);
    else if (tier == 0)
       hipLaunchKernelGGL(k_iterate_lone<0>, dim3(a->nwalkers), dim3(64), lds_lone, s, *a);

@@ -60,13 +60,15 @@ def test_partial_sums_of_ordinary_items_have_room(prod_lib, rgb, records):
     (1000, 4096), (32767, 4096), (32769, 3072), (50000, 2048), (73728, 2048), (73729, 1024), (100000, 1024),
     (160000, 1024)])
 def test_walkers_that_run_one_per_wavefront(prod_lib, lds, walkers):
-    """fl3h_iterate takes a wavefront per walker up to four rounds of those that
-    a 256-CU chip of 160 KB LDS holds, at most four a CU (8 KB of LDS each beside
-    the genome's)."""
+    """fl3h_iterate takes a wavefront per walker up to four rounds (two beyond the
+    classic variations) of those that a 256-CU chip of 160 KB LDS holds, at most four
+    a CU (8 KB of LDS each beside the genome's)."""
     f = prod_lib.fl3k_lone_walkers
-    f.argtypes = [ctypes.c_size_t, ctypes.c_size_t, ctypes.c_int]
+    f.argtypes = [ctypes.c_size_t, ctypes.c_size_t, ctypes.c_int, ctypes.c_int]
     f.restype = ctypes.c_int
-    assert f(lds, 160 << 10, 256) == walkers
+    assert f(lds, 160 << 10, 256, 0) == walkers
+    for tier in (1, 6):
+        assert f(lds, 160 << 10, 256, tier) == walkers // 2
 
 
 @pytest.mark.parametrize("k1,k2,finite", [
