@@ -67,8 +67,12 @@ extern "C" const char *fl3h_last_error(void) { return g_err; }
 // Pinned host memory that a call fills and copies to the device without
 // waiting: the copy after it waits, on the host, until the one before has left
 // the memory.  (2 MB of jobs through a new std::vector took 690 us, page faults
-// and the runtime's own staging most of it.)  It grows to the largest set of
-// jobs, as their device buffer does.
+// and the runtime's own staging most of it.)  It grows with the sets of jobs; a
+// large one is given back by the next call that needs a small one.
+#define FL3_PIN_KEEP ((size_t)128 << 20)   // (a launch of 4096 jobs of 12 KB takes 80 MB)
+extern "C" int fl3k_pin_fits(size_t cap, size_t bytes) {
+   return bytes <= cap && (cap <= FL3_PIN_KEEP || bytes > FL3_PIN_KEEP / 2);
+}
 struct PinBuf {
    unsigned char *p = nullptr;
    size_t cap = 0;
@@ -77,7 +81,7 @@ struct PinBuf {
    unsigned char *take(size_t bytes) {
       if (sent && hipEventSynchronize(left) != hipSuccess) return nullptr;
       sent = false;
-      if (bytes > cap) {
+      if (!fl3k_pin_fits(cap, bytes)) {
          if (p) (void)hipHostFree(p);
          cap = 0;
          p = nullptr;

@@ -106,3 +106,14 @@ def test_samples_from_which_deposits_are_sorted(prod_lib, rounds, njobs, tables,
     f.argtypes = [ctypes.c_int] * 4
     f.restype = ctypes.c_longlong
     assert f(rounds, njobs, tables, wave) == samples
+
+
+@pytest.mark.parametrize("cap,need,fits", [
+    (0, 1, 0), (4096, 4096, 1), (4096, 4097, 0), (128 << 20, 1, 1), ((128 << 20) + 1, 1, 0),
+    (900 << 20, 64 << 20, 0), (900 << 20, (64 << 20) + 1, 1), (900 << 20, 900 << 20, 1), (900 << 20, 901 << 20, 0)])
+def test_pinned_memory_is_given_back(prod_lib, cap, need, fits):
+    """Pinned memory beyond 128 MiB lives until a call needs no more than half of that."""
+    f = prod_lib.fl3k_pin_fits
+    f.argtypes = [ctypes.c_size_t] * 2
+    f.restype = ctypes.c_int
+    assert f(cap, need) == fits
