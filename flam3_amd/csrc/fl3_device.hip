@@ -10,11 +10,12 @@
 //        the frame's ISAAC stream), for production renders;
 //      - k_iter_replay: FP64 walkers that each run exactly one reference
 //        thread's ISAAC stream and sub-batch loop (replay / verification);
-//      - k_iterate_points: FP64 batched flam3_iterate.
+//      - k_iterate_points, k_iterate_lone: FP64 batched flam3_iterate.
+//  * k_bin_*: walkers' records sorted by tile and added to the histogram.
 //  * k_deposit_points: deposit a given point stream (stage test).
-//  * k_de / k_logscale: density estimation or plain log scaling into the
+//  * k_de_* / k_logscale: density estimation or plain log scaling into the
 //    accumulator (rect.c:57-251, 947-974).
-//  * k_earlyclip + k_tonemap: spatial filter, log/gamma/vibrancy/highlight
+//  * k_earlyclip + k_tonemap*: spatial filter, log/gamma/vibrancy/highlight
 //    tone map and quantisation fused into one pass (rect.c:1067-1247).
 #include <hip/hip_runtime.h>
 #include <dlfcn.h>
@@ -987,7 +988,7 @@ extern "C" long long fl3k_bin_min_samples(int rounds, int njobs, int tables, int
 // the band shift of a histogram of more than FL3_MAX_BINS tiles: the
 // walkers then count their records per 2^(band - FL3_SUPER_SHIFT)-cell tile,
 // a first sort groups them by band, and each band is counted, sorted by tile
-// and accumulated on its own (iterate_banded_chunk).
+// and accumulated on its own (bin_banded).
 static int iterate_binned(IterArgs a, long long W, long long Wj, JobSet &js, const fl3d_iter_params *p,
                           int shift, int band) {
    const long long ncells = (long long)g_ctx.width * g_ctx.height;

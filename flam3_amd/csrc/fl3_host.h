@@ -72,8 +72,8 @@ void fl3_distrib_breakpoints(const unsigned short *distrib, int nrows, int nstd,
  * 0..n_std with it; *nrows receives the count) without building the table:
  * what fl3_distrib_breakpoints gives for fl3_create_xform_distrib's table.
  * starts holds (n_std + 1) * n_std ints.  Sets cp->chaos_enable.  Returns 0,
- * or 1 on negative or all-zero weights.  Thread-safe (a small cache of
- * recent inputs and results). */
+ * or 1 on negative or all-zero weights.  Thread-safe (keeps
+ * nothing). */
 int fl3_xform_starts(flam3_genome *cp, int *starts, int *nrows);
 
 /* ---------------- filters (filters.c) ---------------- */

@@ -72,11 +72,10 @@ struct IterArgs {
 
 // Binned deposit limits: tiles per histogram (the sort keeps a counter per
 // tile in LDS), samples per chunk of records, records per accumulation work
-// item and the batch size from which the library prefers binning to atomics.
-// A work item is what one workgroup accumulates alone: 2^18 records keeps a
-// tile cell's partial sum below 2^18 * 255 < 2^32 and splits the densest
-// tiles of a frame (2.2e6 of a chunk's 2.6e8 records at 1080p, against a mean
-// of 1.3e5) over several workgroups, so that the last items do not trail.
+// item at most and the batch sizes from which the library prefers binning to
+// atomics.  A work item is what one workgroup accumulates alone: 2^18 records keep
+// a tile cell's partial sum below 2^18 * 255 < 2^32; 32-bit histograms take fewer by
+// the launch's records (accum_items).
 #define FL3_MAX_BINS 8192
 #define FL3_SUPER_SHIFT 5           // tiles a band is counted in: 32
 
@@ -102,7 +101,7 @@ struct IterArgs {
 #define FL3_BIN_MIN_XAOS (1LL << 17)
 #define FL3_BIN_FEW_TABLES 32
 
-// Record formats of fl3k_launch_bin beyond 0 (8-byte records), 1 (4-byte
+// Record formats of fl3k_launch_bin_sort and fl3k_launch_bin_accum beyond 0 (8-byte records), 1 (4-byte
 // records) and 2 (job records): the same records into double buckets.
 #define FL3_BIN_F64_WIDE 3
 #define FL3_BIN_F64_NARROW 4

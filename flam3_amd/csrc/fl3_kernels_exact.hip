@@ -1022,7 +1022,7 @@ extern "C" void fl3k_de_region(int cells, int *w, int *h) {
 
 // Density estimation of n renders: per-render arguments in device memory,
 // workgroup prefixes prep_first[n + 1] (rows of 256 cells) and
-// gather_first[n + 1] (regions of 16 x 16 cells, 16 x 32 for cells 2).  bits
+// gather_first[n + 1] (regions of fl3k_de_region(cells) cells).  bits
 // 32/33 with the FP32 accumulator (production arithmetic) only.
 // blkmax: a device array of nblk ints the renders' blkmax pointers point
 // into (cleared here), or nullptr.
@@ -1312,7 +1312,7 @@ __global__ __launch_bounds__(TM_TX * TM_TY) void k_tonemap_lds(TMArgs a) {
 }
 
 // Tone maps of several renders in one launch (workgroup prefixes as for
-// k_de_gather_many; rows of 256 pixels).
+// k_de_taps_many; rows of 256 pixels).
 template <typename AT>
 __global__ __launch_bounds__(256) void k_tonemap_many(const TMArgs *as, const unsigned *first, int n) {
    const int j = de_job(first, n, blockIdx.x);

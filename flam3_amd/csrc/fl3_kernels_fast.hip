@@ -49,14 +49,14 @@ extern "C" int fl3k_launch_apply_fp32(const unsigned char *job, int xi, const do
 //
 // The walker kernel writes one record per plotted sample instead of five
 // global atomics, and counts its workgroup's records per tile of 1 << shift
-// cells.  The records are then grouped by tile (a counting sort: per-tile
-// sums and per-workgroup offsets, tile offsets, scatter), and each tile's
+// cells.  The records are then grouped by tile (tile offsets from
+// those counts, then one pass over the records), and each tile's
 // records are accumulated in LDS and added to the histogram once.  Integer
 // sums commute, so the histogram is the one the atomic deposit produces; the
 // tile flush applies the reference's saturation exactly.
 
-// Launch shape of the tile pipeline: threads per accumulation workgroup and
-// records each thread loads before working on them (accumulation, scatter).
+// Threads per accumulation workgroup, and records each thread of the one into
+// double buckets loads before working on them.
 #ifndef FL3_ACC_THREADS
 #define FL3_ACC_THREADS 1024
 #endif
@@ -790,8 +790,9 @@ extern "C" int fl3k_launch_bin_split(const BinArgs *a, int narrow_out, hipStream
    return hipGetLastError() != hipSuccess;
 }
 
-// Banded histograms, second level: per-tile counts of one band's 8-byte records (a->rec, a->rec_count of them, as a->nblk blocks of
-// a->rows x 256), before fl3k_launch_bin sorts and accumulates them.
+// Banded histograms, second level: per-tile counts of one band's records (a->rec,
+// a->rec_count of them, as a->nblk blocks of a->rows x 256; 4 bytes each if
+// narrow), before fl3k_launch_bin_sort and fl3k_launch_bin_accum take them.
 extern "C" int fl3k_launch_bin_count(const BinArgs *a, int narrow, hipStream_t s) {
    const size_t l = sizeof(unsigned) * (size_t)a->nbins;   // at most FL3_MAX_BINS: 32 KiB
    if (narrow)

@@ -41,7 +41,7 @@ constexpr int walker_waves() { return TIER == 0 ? 8 : 1; }
 // thirteen scalar branches per variation, most of a lone wavefront's step.
 // The hashes of 64 steps' draws are computed at once, a step per lane.
 // Measured (kernel trace): a 2.59e8-sample launch of the 1080p still 2.23 ->
-// 1.47 ms, 249 -> about 150 VALU and 203 -> about 90 SALU instructions per
+// 1.47 ms, 249 -> 184 VALU and 203 -> 103 SALU instructions per
 // sample; the 228 steps of a 256 x 256 preview of 28160 walkers, 283 -> 171 us.
 typedef uint32_t fl3_u32x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t fl3_u32x4 __attribute__((ext_vector_type(4)));
