@@ -22,6 +22,11 @@ int fl3d_begin(int width, int height, int bits);
 /* Device bytes a render may use (the device's free memory plus what the
  * library's buffers already hold) and the device's total memory. */
 int fl3d_device_memory(double *avail, double *total);
+/* The device context holds one render's state from fl3d_begin or fl3d_begin_many
+ * until its image is fetched: between these two no other thread's calls come in
+ * (each call alone takes the same lock, which a thread may take again). */
+void fl3d_hold(void);
+void fl3d_release(void);
 /* Zero the histogram (start of each batch, rect.c:721). */
 int fl3d_clear_buckets(void);
 /* Histograms of n renders in one allocation (cleared); fl3d_select(r) makes

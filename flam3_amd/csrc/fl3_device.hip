@@ -188,6 +188,8 @@ struct Ctx {
 static Ctx g_ctx;
 static std::recursive_mutex g_mu;
 static std::atomic<int> g_ready{0};   // g_ctx.ready, for readers without g_mu
+extern "C" void fl3d_hold(void) { g_mu.lock(); }
+extern "C" void fl3d_release(void) { g_mu.unlock(); }
 
 static int ctx_init() {
    if (g_ctx.ready) return 0;

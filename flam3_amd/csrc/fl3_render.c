@@ -558,6 +558,7 @@ int fl3h_render(flam3_frame *spec, void *out, int field, int nchan, int transp, 
 
    if (plan_open(&P, spec, out, field, nchan, transp, stats, opts)) return 1;
    nts = P.nts;
+   fl3d_hold();   /* (until the image is here) */
    if (fl3d_begin(P.geo.width, P.geo.height, spec->bits)) {
       fprintf(stderr, "flam3_amd: %s\n", fl3d_error());
       goto fail;
@@ -750,6 +751,7 @@ devfail:
 fail:
    rv = 1;
 cleanup:
+   fl3d_release();
    for (i = 0; i < bn; i++) free(bjobs[i]);
    free(bjobs);
    free(bbytes);
@@ -1115,6 +1117,7 @@ static int many_group(fl3_many *B, int i0, int i1) {
          for (k = 0; k < B->njob[r]; k++) mj[nm + k].render = i;
          nm += B->njob[r];
       }
+      fl3d_hold();   /* (until the images and counts are here) */
       ok = fl3d_begin_many(widths, heights, nl, B->bits) == 0 &&
            fl3d_iterate_multi(mj, nm, FUSE_WALKER, 0, nl, NULL, NULL) == 0;
       if (ok) {
@@ -1185,6 +1188,7 @@ static int many_group(fl3_many *B, int i0, int i1) {
             B->reqs[B->live[i0 + i]].rc = 0;
          }
       }
+      fl3d_release();
    }
    free(mj);
    free(dst);
@@ -1231,6 +1235,7 @@ static int many_large(fl3_many *B, int r) {
    fl3d_multi_job *m = B->mj + B->job0[r];
    int exact, ts, e, i, saturated = 0;
    fl3d_tm_params tp;
+   fl3d_hold();   /* (until the image is here) */
    if (fl3d_begin(Q->geo.width, Q->geo.height, Q->spec->bits)) goto devfail;
    for (exact = 0; exact < 2; exact++) {
       if (exact) {
@@ -1274,12 +1279,14 @@ static int many_large(fl3_many *B, int r) {
    if (many_density(Q, &B->de[r])) goto devfail;
    plan_tm(Q, &tp);
    if (fl3d_tonemap(&tp, Q->filter, Q->out, plan_out_stride(Q))) goto devfail;
+   fl3d_release();
    plan_finish(Q);
    B->reqs[r].rc = 0;
    (void)i;
    return 0;
 devfail:
    fprintf(stderr, "flam3_amd: device error: %s\n", fl3d_error());
+   fl3d_release();
    return 1;
 }
 
