@@ -45,7 +45,7 @@ typedef struct fin_item {
 
 struct fl3h_server {
    pthread_mutex_t mu;
-   pthread_cond_t cv_work, cv_ready, cv_done, cv_fin, cv_slot;
+   pthread_cond_t cv_work, cv_ready, cv_done, cv_fin;
    pthread_t planner, runner, finisher;
    int threads;
    srv_rec **recs;        /* by ticket */
@@ -61,10 +61,9 @@ struct fl3h_server {
    int ready_n;
    long long batches, renders;
    double prep_s, exec_s;   /* planner and runner busy time */
-   /* finisher queue and the two download slots */
+   /* finisher queue */
    fin_item *fin_head, *fin_tail;
    int runner_done;
-   int slot_busy[2], next_slot;
    double dev_avail;      /* device bytes renders may use (0: unknown) */
 };
 
@@ -179,28 +178,36 @@ static void fin_push(fl3h_server *s, fin_item *it) {
    pthread_mutex_unlock(&s->mu);
 }
 
+/* The two download slots are the device context's, so every server's: an image
+ * in one stays there until its server's finisher has copied it out. */
+static pthread_mutex_t slot_mu = PTHREAD_MUTEX_INITIALIZER;
+static pthread_cond_t cv_slot = PTHREAD_COND_INITIALIZER;
+static int slot_busy[2], next_slot;
+
+static void slot_free(int k) {
+   pthread_mutex_lock(&slot_mu);
+   if (k >= 0) slot_busy[k] = 0;
+   pthread_cond_broadcast(&cv_slot);
+   pthread_mutex_unlock(&slot_mu);
+}
+
 /* fl3_delivery hooks (runner thread) */
 static int slot_acquire(void *ctx) {
-   fl3h_server *s = (fl3h_server *)ctx;
    int k;
-   pthread_mutex_lock(&s->mu);
-   while (s->slot_busy[s->next_slot]) pthread_cond_wait(&s->cv_slot, &s->mu);
-   k = s->next_slot;
-   s->slot_busy[k] = 1;
-   s->next_slot ^= 1;
-   pthread_mutex_unlock(&s->mu);
+   (void)ctx;
+   pthread_mutex_lock(&slot_mu);
+   while (slot_busy[next_slot]) pthread_cond_wait(&cv_slot, &slot_mu);
+   k = next_slot;
+   slot_busy[k] = 1;
+   next_slot ^= 1;
+   pthread_mutex_unlock(&slot_mu);
    return k;
 }
 
 static void images_hand_over(void *ctx, fl3_images *im) {
    fin_item *it = (fin_item *)calloc(1, sizeof(fin_item));
    if (!it) {   /* deliver here rather than lose the group */
-      fl3h_server *s = (fl3h_server *)ctx;
-      const int k = fl3_images_deliver(im);
-      pthread_mutex_lock(&s->mu);
-      if (k >= 0) s->slot_busy[k] = 0;
-      pthread_cond_broadcast(&s->cv_slot);
-      pthread_mutex_unlock(&s->mu);
+      slot_free(fl3_images_deliver(im));
       return;
    }
    it->im = im;
@@ -220,10 +227,8 @@ static void *finisher_main(void *arg) {
       if (!s->fin_head) s->fin_tail = NULL;
       pthread_mutex_unlock(&s->mu);
       if (it->im) {
-         const int k = fl3_images_deliver(it->im);
+         slot_free(fl3_images_deliver(it->im));
          pthread_mutex_lock(&s->mu);
-         if (k >= 0) s->slot_busy[k] = 0;
-         pthread_cond_broadcast(&s->cv_slot);
       } else {
          fl3_many_free(it->B);
          pthread_mutex_lock(&s->mu);
@@ -344,7 +349,6 @@ fl3h_server *fl3h_server_create(const fl3h_server_opts *o) {
    pthread_cond_init(&s->cv_ready, NULL);
    pthread_cond_init(&s->cv_done, NULL);
    pthread_cond_init(&s->cv_fin, NULL);
-   pthread_cond_init(&s->cv_slot, NULL);
    if (fl3d_device_memory(&s->dev_avail, NULL)) s->dev_avail = 0.0;
    {
       /* the device buffers of a full batch, allocated now: growing them
@@ -369,7 +373,6 @@ fl3h_server *fl3h_server_create(const fl3h_server_opts *o) {
    s->threads = 3;
    return s;
 bad:
-   pthread_cond_destroy(&s->cv_slot);
    pthread_cond_destroy(&s->cv_fin);
    pthread_cond_destroy(&s->cv_done);
    pthread_cond_destroy(&s->cv_ready);
@@ -460,7 +463,6 @@ void fl3h_server_destroy(fl3h_server *s) {
    stop_threads(s);
    for (i = 0; i < s->nrecs; i++) free(s->recs[i]);
    free(s->recs);
-   pthread_cond_destroy(&s->cv_slot);
    pthread_cond_destroy(&s->cv_fin);
    pthread_cond_destroy(&s->cv_done);
    pthread_cond_destroy(&s->cv_ready);

@@ -79,3 +79,30 @@ def test_renders_of_several_threads(prod):
     for t in threads:
         t.join()
     assert not bad
+
+
+def test_servers_beside_each_other(prod):
+    """Three servers at once, whose groups pass through the same download slots."""
+    items = [{"genomes": G.synthetic_preview(s, size=64 + 32 * (s % 5), quality=10.0), "seed": str(s)} for s in range(30)]
+    want = [prod.render(it["genomes"], seed=it["seed"])[0] for it in items]
+    bad = []
+
+    def served(order):
+        try:
+            s = Server(max_batch=3)
+            for _ in range(3):
+                ts = [(i, s.submit(**items[i])) for i in order]
+                for i, t in ts:
+                    if not np.array_equal(s.wait(t)[0], want[i]):
+                        bad.append(i)
+            s.close()
+        except Exception as e:
+            bad.append(e)
+
+    n = range(len(items))
+    threads = [threading.Thread(target=served, args=(o,)) for o in (list(n), list(n)[::-1], list(n)[15:] + list(n)[:15])]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
